@@ -103,6 +103,8 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     // planes wider than its LDS) goes on like the 16-bit types and the other kernel sizes.
     int status = conv2d_f32(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
+    status = conv2d_few(p, x->dtype, x->address, w->address, pb, y->address, s);
+    if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     if (pointwise) status = conv2d_k1(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (pointwise && status == TANNIC_UNSUPPORTED_DTYPE) status = conv2d_pointwise(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;

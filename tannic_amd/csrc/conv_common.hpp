@@ -19,6 +19,8 @@ struct ConvProblem {
 
 // Each returns TANNIC_UNSUPPORTED_DTYPE when the problem does not meet its
 // conditions, so that the caller can try the next, more general kernel.
+// 16-bit 1x1 and 3x3 over few output pixels
+int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_k1(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_stem(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
