@@ -492,6 +492,11 @@ int gemm_entry(const tannic_tensor_t* a, const tannic_tensor_t* b, tannic_tensor
                         if (status != TANNIC_UNSUPPORTED_DTYPE) return;   // (refused after all: on with the product as it is)
                     }
                 }
+                if constexpr (std::is_same_v<A, B> && is_16bit<A>::value) {
+                    // at most four rows times narrow matrices that lie row by row: every matrix is read once, along its rows
+                    status = gemm_rows_batch(p, a->dtype, first, second, dst->address, s);
+                    if (status != TANNIC_UNSUPPORTED_DTYPE) return;
+                }
                 constexpr bool shares_k = std::is_same_v<A, B> && (is_16bit<A>::value || std::is_same_v<A, float> || std::is_same_v<A, int8_t>);
                 if (few_results_under_a_long_k(p, shares_k ? 8192 : 32768)) {
                     // (not where the tiles share K or W is streamed: aligned K-contiguous operands of the 16-bit types and

@@ -1,0 +1,140 @@
+// At most four rows times narrow matrices that lie row by row, 16-bit, one product per batch index:
+// y[b][m][n] = sum over k of x[b][m][k] * W[b][k][n], N a multiple of 8 up to 256, K of a thousand or more.  (Attention's probabilities times the
+// cached values for one new token: a group's query heads are the rows, K is the length of the context, whatever it is.)
+//
+// The work is reading W once.  A lane owns eight consecutive columns (one 16-byte load per row of W), LN lanes lie side by side
+// along the columns and 64 / LN rows of W are one load instruction; a block's wavefronts take turns along K, UNROLL rows per
+// lane in flight.  x comes value by value beside it (64 / LN consecutive k per instruction, from the cache), so its row pitch
+// and K may be odd, and nothing here needs alignment.  A lane's sums meet the other rows' by halves (a reduce-scatter: 30 exchanges
+// for 32 sums over 16 lanes where a butterfly takes 128), then the wavefronts' in LDS, in a fixed order; no scratch, one kernel.
+// (src/cpu/matmul.cpp:60-124; fp32 sums, rounded once.)
+#include "gemm_common.hpp"
+
+namespace th {
+
+typedef unsigned int uint4r __attribute__((ext_vector_type(4), aligned(2)));
+
+constexpr int kRowsBatchWaves = 16;
+
+// rows of W a lane has in flight: with few blocks a context of a few thousand is one pass
+constexpr int rows_batch_unroll(int lanes) { return lanes == 2 ? 8 : 4; }
+
+// the sums of the lanes that differ in bits STEP ... 32 of the lane number: N values per lane become N * STEP / 32 / 2 finished ones
+template <int N, int STEP, int LAST>
+__device__ __forceinline__ void scatter_sums(float* v, uint32_t lane, uint32_t& first) {
+    if constexpr (STEP >= LAST) {
+        const bool upper = (lane & STEP) != 0;
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i) {
+            const float keep = upper ? v[i + N / 2] : v[i], send = upper ? v[i] : v[i + N / 2];
+            v[i] = keep + __shfl_xor(send, STEP, 64);
+        }
+        first += upper ? N / 2 : 0;
+        scatter_sums<N / 2, STEP / 2, LAST>(v, lane, first);
+    }
+}
+
+template <class T, int LN>
+__global__ __launch_bounds__(64 * kRowsBatchWaves) void gemm_rows_batch_kernel(const T* x, const T* w, T* y, GemmProblem p) {
+    constexpr int MR = 4;   // rows a lane accumulates, at least M
+    constexpr int ROWS = 64 / LN, UNROLL = rows_batch_unroll(LN);
+    constexpr int LEFT = MR * 8 / ROWS;   // finished sums per lane
+    static_assert(LEFT >= 1, "every lane ends with a sum");
+    __shared__ float part[kRowsBatchWaves][64 * LEFT];
+    const uint32_t lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), waves = blockDim.x / 64;
+    // (workgroups go round the eight dies in turn: with whole eights of products, those that share a product's rows share a die)
+    const uint32_t batch = blockIdx.x % p.batches, group = blockIdx.x / p.batches;
+    int64_t oa, ob, oc;
+    batch_offsets(p, batch, oa, ob, oc);
+    const uint32_t col = (group * LN + lane % LN) * 8, row = lane / LN;
+    const bool active = col < p.N;   // (N is a multiple of 8)
+    const T* wp = w + ob + (active ? col : 0);
+    const T* xp[MR];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) xp[m] = x + oa + static_cast<int64_t>(static_cast<uint32_t>(m) < p.M ? m : 0) * p.a_rs;   // (rows past M are never stored)
+
+    float acc[MR * 8];
+#pragma unroll
+    for (int i = 0; i < MR * 8; ++i) acc[i] = 0.0f;
+    for (uint32_t k0 = wave * ROWS * UNROLL; k0 < p.K; k0 += waves * ROWS * UNROLL) {
+        uint4r bits[UNROLL];
+        T xv[UNROLL][MR];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            const uint32_t k = k0 + u * ROWS + row;
+            const bool live = k < p.K;
+            bits[u] = uint4r{0, 0, 0, 0};
+            if (live) bits[u] = *reinterpret_cast<const uint4r*>(wp + static_cast<int64_t>(k) * p.b_rs);
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                xv[u][m] = T{};
+                if (live) xv[u][m] = xp[m][static_cast<int64_t>(k) * p.a_cs];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            T e[8];
+            __builtin_memcpy(e, &bits[u], 16);
+            float wide[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) wide[i] = static_cast<float>(widen(e[i]));
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                const float f = static_cast<float>(widen(xv[u][m]));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc[m * 8 + i] += f * wide[i];
+            }
+        }
+    }
+    uint32_t first = 0;
+    scatter_sums<MR * 8, 32, LN>(acc, lane, first);
+#pragma unroll
+    for (int i = 0; i < LEFT; ++i) part[wave][i * 64 + lane] = acc[i];
+    __syncthreads();
+    for (uint32_t at = threadIdx.x; at < 64 * LEFT; at += blockDim.x) {
+        // sum `at` is value first + at / 64 of lane at % 64: row value / 8, column value % 8 of that lane's eight
+        float sum = 0.0f;
+        for (uint32_t v = 0; v < waves; ++v) sum += part[v][at];
+        const uint32_t from = at % 64;
+        uint32_t value = at / 64;
+#pragma unroll
+        for (int step = 32, half = MR * 4; step >= LN; step /= 2, half /= 2) value += from & step ? half : 0;
+        const uint32_t m = value / 8, n = (group * LN + from % LN) * 8 + value % 8;
+        if (m < p.M && n < p.N) y[oc + static_cast<int64_t>(m) * p.c_rs + n] = narrow_result<T>(sum);
+    }
+}
+
+template <class T, int LN>
+static int launch_rows_batch(const GemmProblem& p, const void* x, const void* w, void* y, hipStream_t stream) {
+    constexpr uint32_t per_wave = 64 / LN * rows_batch_unroll(LN);   // rows of W a wavefront has in flight
+    const uint32_t groups = (p.N + 8 * LN - 1) / (8 * LN);
+    uint32_t waves = (p.K + per_wave - 1) / per_wave;
+    if (waves > kRowsBatchWaves) waves = kRowsBatchWaves;
+    hipLaunchKernelGGL((gemm_rows_batch_kernel<T, LN>), dim3(groups * p.batches), dim3(64 * waves), 0, stream, static_cast<const T*>(x), static_cast<const T*>(w),
+                       static_cast<T*>(y), p);
+    return launch_status("gemm_rows_batch_kernel");
+}
+
+// Where rows of x that no 16 bytes divide leave the tiles their loaders for any alignment, and there are more results than the
+// kernel for few results takes, up to 8192 columns in all products (bf16, four rows, replayed calls, us here / before:
+// 32 products of 1001 x 128 7.8 / 15.4, 64 of 2049 x 128 11.8 / 32.6, 128 of 4001 x 64 22.2 / 58.2).  With K a multiple of 8 the tiles
+// are as good (64 of 2048 x 128 12.1 / 11.1), and so they are with more products (256 of 4001 x 128 97 / 78: a value of x per
+// row and lane is four loads beside the one of W).
+template <class T>
+static int run_rows_batch(const GemmProblem& p, const void* x, const void* w, void* y, hipStream_t stream) {
+    if (p.M == 0 || p.M > 4 || p.N == 0 || p.N > 256 || p.N % 8 != 0 || p.K < 1000 || p.K >= (1u << 31) || p.K % 8 == 0) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.a_cs != 1 || p.b_cs != 1 || p.b_rs == 1 || p.row_bias || p.c_group || p.b_group_stride) return TANNIC_UNSUPPORTED_DTYPE;
+    const uint64_t columns = static_cast<uint64_t>(p.N) * p.batches;
+    if (columns > 8192 || columns * p.M <= 8192) return TANNIC_UNSUPPORTED_DTYPE;
+    // 64-byte runs of a row where that gives every compute unit a block, else 32
+    if (columns == 8192) return launch_rows_batch<T, 4>(p, x, w, y, stream);
+    return launch_rows_batch<T, 2>(p, x, w, y, stream);
+}
+
+int gemm_rows_batch(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream) {
+    if (dtype == TANNIC_FLOAT16) return run_rows_batch<f16>(p, a, b, c, stream);
+    if (dtype == TANNIC_BFLOAT16) return run_rows_batch<bf16>(p, a, b, c, stream);
+    return TANNIC_UNSUPPORTED_DTYPE;
+}
+
+}  // namespace th
