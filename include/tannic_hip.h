@@ -210,6 +210,14 @@ void tannic_hip_graph_destroy(void* recording);
  * acquisitions, out[1] tensor allocations and releases through tannic_hip_allocate / tannic_hip_deallocate, out[2] the
  * number of workgroups that shared K in the last matrix product that shared it. */
 void tannic_hip_counters(uint64_t out[3]);
+/* Which kernel a convolution of these operands would run, without running it or reading what their addresses point at (for
+ * tests, no reference twin).  out[0] is 1 for the fp32 kernel over the flattened batch, 2 for the 16-bit kernel over few
+ * output pixels, 0 for any other.  After 1: the kernel's side, its template parameters U, PT, NL, RESIDENT, WO and WIDE, then
+ * pixels per tile, tiles of channels, blocks sharing the channels, groups of kernel rows, groups per block, floats from plane to
+ * plane, floats of a plane, rows per image and columns per row with the shared padding.  After 2: the kernel's side, tiles of
+ * 16 channels and of 16 pixels per block, wavefronts, blocks.  The status is the convolution's. */
+int tannic_hip_conv2d_plan(const tannic_tensor_t* x, const tannic_tensor_t* w, const tannic_tensor_t* y, const size_t pad[2],
+                           const size_t stride[2], uint32_t out[20]);
 /* The stream a recording captures: a caller that keeps a device's stream to itself checks that it is this one. */
 tannic_stream_t tannic_hip_graph_stream(void* recording);
 

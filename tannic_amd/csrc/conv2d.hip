@@ -52,7 +52,7 @@ int run_direct(const ConvProblem& p, const void* x, const void* w, const void* b
 }
 
 static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, const tannic_tensor_t* bias, tannic_tensor_t* y,
-                        tannic_stream_t stream, const size_t pad[2], const size_t stride[2]) {
+                        tannic_stream_t stream, const size_t pad[2], const size_t stride[2], uint32_t* plan = nullptr) {
     if (!x || !w || !y || !pad || !stride) return TANNIC_ERROR;
     if (!have_storage(x, w, bias, y)) return TANNIC_ERROR;
     // dispatch on (signal, kernel) dtype first: unsupported pairs report
@@ -94,6 +94,11 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     p.has_bias = bias != nullptr;
     // the bias is read through its stride (a column of a matrix is a valid bias; the CPU path reads b[co], src/cpu/conv2d.cpp:86)
     p.bs = bias ? bias->strides.sizes[0] : 0;
+    if (plan) {
+        for (int i = 0; i < kConvPlanValues; ++i) plan[i] = 0;
+        if (!conv2d_f32_plan(p, x->dtype, x->address, w->address, plan)) conv2d_few_plan(p, x->dtype, plan);
+        return TANNIC_SUCCESS;
+    }
     const void* pb = bias ? bias->address : nullptr;
     hipStream_t s = as_stream(stream);
     // Kernels in order of preference.  A 1x1 kernel has no tap to amortise a staged patch over: its weights stay in
@@ -188,5 +193,11 @@ int tannic_hip_conv2d_biased(const tannic_tensor_t* x, const tannic_tensor_t* w,
                              tannic_stream_t stream, const size_t pad[2], const size_t stride[2]) {
     if (!bias) return TANNIC_ERROR;
     return th::conv2d_entry(x, w, bias, y, stream, pad, stride);
+}
+int tannic_hip_conv2d_plan(const tannic_tensor_t* x, const tannic_tensor_t* w, const tannic_tensor_t* y, const size_t pad[2], const size_t stride[2],
+                           uint32_t out[20]) {
+    if (!y || !out) return TANNIC_ERROR;
+    tannic_tensor_t result = *y;
+    return th::conv2d_entry(x, w, nullptr, &result, tannic_stream_t{}, pad, stride, out);
 }
 }

@@ -509,8 +509,14 @@ static void consider_f32(const ConvProblem& p, bool wide, F32Plan& best, double&
     q.pixels = p.N * p.HO * p.WO;
     q.ptile = 16 * PT * (4 / wo);
     q.co_tiles = (p.O + 32 * wo - 1) / (32 * wo);
-    q.hp = p.H + p.pad_h;
-    q.wp = p.W + p.pad_w;
+    // (padding beyond the kernel's height: the images move apart until no image's first window begins above the last of the one
+    // before, as a tile's windows are counted from its first row on)
+    uint64_t hp = static_cast<uint64_t>(p.H) + p.pad_h;
+    if (static_cast<uint64_t>(p.HO - 1) * p.stride_h > hp) hp = static_cast<uint64_t>(p.HO - 1) * p.stride_h;
+    const uint64_t wp = static_cast<uint64_t>(p.W) + p.pad_w;
+    if (hp >= (1ull << 31) || wp >= (1ull << 31)) return;
+    q.hp = static_cast<uint32_t>(hp);
+    q.wp = static_cast<uint32_t>(wp);
     // the plane of a tile: its sampled pixels, or the rows its windows touch
     uint64_t plane, images;
     if (KS == 1) {
@@ -600,26 +606,25 @@ static int finish_f32(const ConvProblem& p, F32Plan& q, float* y, hipStream_t st
 #define TH_F32_LAUNCH(KS, U, PT, NL, RES, WO, WIDE) \
     if (index == counter++) return launch_f32<KS, U, PT, NL, RES, WO, WIDE>(p, q, x, w, bias, y, partials, stream);
 
-int conv2d_f32(const ConvProblem& p, int dtype, const void* x_, const void* w_, const void* bias_, void* y_, hipStream_t stream) {
-    if (dtype != TANNIC_FLOAT32 || p.KH != p.KW) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0) return TANNIC_SUCCESS;
-    if (p.C == 0) return TANNIC_UNSUPPORTED_DTYPE;
+#define TH_F32_DESCRIBE(KS, U, PT, NL, RES, WO, WIDE) \
+    if (index == counter++) {                         \
+        const uint32_t of[7] = {KS, U, PT, NL, RES, WO, WIDE}; \
+        for (int i = 0; i < 7; ++i) out[1 + i] = of[i];        \
+    }
+
+// The index of the kernel that takes the problem, with its plan; -1 if none does
+static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* w, F32Plan& q) {
+    if (dtype != TANNIC_FLOAT32 || p.KH != p.KW || p.C == 0) return -1;
     const uint64_t K = static_cast<uint64_t>(p.C) * p.KH * p.KW, pixels = static_cast<uint64_t>(p.N) * p.HO * p.WO;
     // contiguous OIHW weights (K runs through memory in order), rows of single floats, results contiguous within an image
-    if (p.ws[3] != 1 || p.ws[2] != p.KW || p.ws[1] != static_cast<int64_t>(p.KH) * p.KW || p.ws[0] != static_cast<int64_t>(K) || reinterpret_cast<uintptr_t>(w_) % 4 != 0)
-        return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.xs[3] != 1 || p.xs[0] < 0 || p.xs[1] < 0 || p.xs[2] < 0 || p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO)) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.KH == 1 && (p.pad_h || p.pad_w)) return TANNIC_UNSUPPORTED_DTYPE;
-    if (K * p.O * 4 >= (1ull << 31) || pixels >= (1ull << 28) || pixels * p.O >= (1ull << 31)) return TANNIC_UNSUPPORTED_DTYPE;
-    const float* x = static_cast<const float*>(x_);
-    const float* w = static_cast<const float*>(w_);
-    const float* bias = static_cast<const float*>(bias_);
-    float* y = static_cast<float*>(y_);
+    if (p.ws[3] != 1 || p.ws[2] != p.KW || p.ws[1] != static_cast<int64_t>(p.KH) * p.KW || p.ws[0] != static_cast<int64_t>(K) || reinterpret_cast<uintptr_t>(w) % 4 != 0) return -1;
+    if (p.xs[3] != 1 || p.xs[0] < 0 || p.xs[1] < 0 || p.xs[2] < 0 || p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO)) return -1;
+    if (p.KH == 1 && (p.pad_h || p.pad_w)) return -1;
+    if (K * p.O * 4 >= (1ull << 31) || pixels >= (1ull << 28) || pixels * p.O >= (1ull << 31)) return -1;
     // 16-byte pieces of the weights (7x7 takes single floats), and of a 1x1 kernel's signal where an image is whole pieces
-    if (p.KH != 7 && (K % 4 != 0 || reinterpret_cast<uintptr_t>(w_) % 16 != 0)) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.KH != 7 && (K % 4 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0)) return -1;
     const bool wide = p.stride_h == 1 && p.stride_w == 1 && p.xs[2] == static_cast<int64_t>(p.W) && (static_cast<uint64_t>(p.H) * p.W) % 4 == 0 && p.xs[0] % 4 == 0 && p.xs[1] % 4 == 0 &&
-                      reinterpret_cast<uintptr_t>(x_) % 16 == 0;
-    F32Plan q{};
+                      reinterpret_cast<uintptr_t>(x) % 16 == 0;
     double time = 1e30;
     int index = -1, counter = 0;
     if (p.KH == 1) {
@@ -629,9 +634,40 @@ int conv2d_f32(const ConvProblem& p, int dtype, const void* x_, const void* w_, 
     } else if (p.KH == 7) {
         TH_F32_K7(TH_F32_CONSIDER)
     }
+    return index;
+}
+
+bool conv2d_f32_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]) {
+    if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0) return false;
+    F32Plan q{};
+    const int index = plan_f32(p, dtype, x, w, q);
+    if (index < 0) return false;
+    int counter = 0;
+    if (p.KH == 1) {
+        TH_F32_K1(TH_F32_DESCRIBE)
+    } else if (p.KH == 3) {
+        TH_F32_K3(TH_F32_DESCRIBE)
+    } else {
+        TH_F32_K7(TH_F32_DESCRIBE)
+    }
+    out[0] = 1;
+    const uint32_t plan[9] = {q.ptile, q.co_tiles, q.splits, q.chunks, q.chunks_per_split, q.pitch, q.plane, q.hp, q.wp};
+    for (int i = 0; i < 9; ++i) out[8 + i] = plan[i];
+    return true;
+}
+
+int conv2d_f32(const ConvProblem& p, int dtype, const void* x_, const void* w_, const void* bias_, void* y_, hipStream_t stream) {
+    if (dtype != TANNIC_FLOAT32 || p.KH != p.KW) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0) return TANNIC_SUCCESS;
+    F32Plan q{};
+    const int index = plan_f32(p, dtype, x_, w_, q);
     if (index < 0) return TANNIC_UNSUPPORTED_DTYPE;
+    const float* x = static_cast<const float*>(x_);
+    const float* w = static_cast<const float*>(w_);
+    const float* bias = static_cast<const float*>(bias_);
+    float* y = static_cast<float*>(y_);
     return finish_f32(p, q, y, stream, [&](float* partials) -> int {
-        counter = 0;
+        int counter = 0;
         if (p.KH == 1) {
             TH_F32_K1(TH_F32_LAUNCH)
         } else if (p.KH == 3) {

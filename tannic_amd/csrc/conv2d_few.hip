@@ -152,11 +152,16 @@ __global__ __launch_bounds__(64 * WAVES) void conv2d_few_kernel(const T* x, cons
 }
 
 template <class T, int KS, int MO, int NP, int WAVES>
-static int launch_few(const ConvProblem& p, FewPlan q, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
+static int launch_few(const ConvProblem& p, FewPlan q, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan) {
     q.pixel_tiles = (q.pixels + 16 * NP - 1) / (16 * NP);
     q.div_tiles = FastDiv(q.pixel_tiles);
     const uint64_t blocks = static_cast<uint64_t>((p.O + 16 * MO - 1) / (16 * MO)) * q.pixel_tiles;
     if (blocks >= (1ull << 31)) return TANNIC_UNSUPPORTED_DTYPE;
+    if (plan) {      // (only asked for)
+        const uint32_t values[6] = {2, KS, MO, NP, WAVES, static_cast<uint32_t>(blocks)};
+        for (int i = 0; i < 6; ++i) plan[i] = values[i];
+        return TANNIC_SUCCESS;
+    }
     hipLaunchKernelGGL((conv2d_few_kernel<T, KS, MO, NP, WAVES>), dim3(static_cast<uint32_t>(blocks)), dim3(64 * WAVES), 0, stream, static_cast<const T*>(x),
                        static_cast<const T*>(w), static_cast<const T*>(bias), static_cast<T*>(y), p, q);
     return launch_status("conv2d_few_kernel");
@@ -185,20 +190,20 @@ static uint64_t most_few_work(const ConvProblem& p) {
 // accumulated tiles fit the static LDS up to eight wavefronts (us with 1, 2 channels, 4 tiles: 3x3 256 @14 batch 1 8.2, 10.1, 13.7, batch 2
 // 13.3, 10.4, 13.8, batch 4 23.4, 17.9, 14.4; 1x1 1024->512 @14 with 1 and 2 pixels 5.8, 5.2, batch 4 14.3, 11.1).
 template <class T, int KS, int WAVES>
-static int few_shape(const ConvProblem& p, const FewPlan& q, uint64_t tiles, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
+static int few_shape(const ConvProblem& p, const FewPlan& q, uint64_t tiles, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan) {
     const bool strided = p.stride_h > 1 || p.stride_w > 1;
-    if (tiles < 300) return launch_few<T, KS, 1, 1, WAVES>(p, q, x, w, bias, y, stream);
+    if (tiles < 300) return launch_few<T, KS, 1, 1, WAVES>(p, q, x, w, bias, y, stream, plan);
     if constexpr (WAVES <= 8) {
-        if (tiles >= 700 && (KS == 3 || strided || WAVES == 8)) return launch_few<T, KS, 2, 2, WAVES>(p, q, x, w, bias, y, stream);
+        if (tiles >= 700 && (KS == 3 || strided || WAVES == 8)) return launch_few<T, KS, 2, 2, WAVES>(p, q, x, w, bias, y, stream, plan);
     }
     if constexpr (KS == 1) {
-        if (!strided) return launch_few<T, KS, 1, 2, WAVES>(p, q, x, w, bias, y, stream);
+        if (!strided) return launch_few<T, KS, 1, 2, WAVES>(p, q, x, w, bias, y, stream, plan);
     }
-    return launch_few<T, KS, 2, 1, WAVES>(p, q, x, w, bias, y, stream);
+    return launch_few<T, KS, 2, 1, WAVES>(p, q, x, w, bias, y, stream, plan);
 }
 
 template <class T, int KS>
-static int run_few(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
+static int run_few(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan) {
     constexpr int64_t TAPS = KS * KS;
     const uint64_t pixels = static_cast<uint64_t>(p.N) * p.HO * p.WO;
     if (pixels == 0 || p.O == 0 || p.C == 0 || p.C % 32 != 0) return TANNIC_UNSUPPORTED_DTYPE;
@@ -223,19 +228,27 @@ static int run_few(const ConvProblem& p, const void* x, const void* w, const voi
     q.div_hw = FastDiv(p.HO * p.WO);
     q.div_wo = FastDiv(p.WO);
     const uint64_t tiles = static_cast<uint64_t>((p.O + 15) / 16) * ((pixels + 15) / 16);
-    if (q.units >= 16) return few_shape<T, KS, 16>(p, q, tiles, x, w, bias, y, stream);
-    if (q.units >= 8) return few_shape<T, KS, 8>(p, q, tiles, x, w, bias, y, stream);
-    if (q.units >= 4) return few_shape<T, KS, 4>(p, q, tiles, x, w, bias, y, stream);
-    return few_shape<T, KS, 2>(p, q, tiles, x, w, bias, y, stream);
+    if (q.units >= 16) return few_shape<T, KS, 16>(p, q, tiles, x, w, bias, y, stream, plan);
+    if (q.units >= 8) return few_shape<T, KS, 8>(p, q, tiles, x, w, bias, y, stream, plan);
+    if (q.units >= 4) return few_shape<T, KS, 4>(p, q, tiles, x, w, bias, y, stream, plan);
+    return few_shape<T, KS, 2>(p, q, tiles, x, w, bias, y, stream, plan);
+}
+
+static int choose_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan) {
+    if (p.KH != p.KW) return TANNIC_UNSUPPORTED_DTYPE;
+    if (dtype == TANNIC_FLOAT16 && p.KH == 1) return run_few<f16, 1>(p, x, w, bias, y, stream, plan);
+    if (dtype == TANNIC_FLOAT16 && p.KH == 3) return run_few<f16, 3>(p, x, w, bias, y, stream, plan);
+    if (dtype == TANNIC_BFLOAT16 && p.KH == 1) return run_few<bf16, 1>(p, x, w, bias, y, stream, plan);
+    if (dtype == TANNIC_BFLOAT16 && p.KH == 3) return run_few<bf16, 3>(p, x, w, bias, y, stream, plan);
+    return TANNIC_UNSUPPORTED_DTYPE;
 }
 
 int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
-    if (p.KH != p.KW) return TANNIC_UNSUPPORTED_DTYPE;
-    if (dtype == TANNIC_FLOAT16 && p.KH == 1) return run_few<f16, 1>(p, x, w, bias, y, stream);
-    if (dtype == TANNIC_FLOAT16 && p.KH == 3) return run_few<f16, 3>(p, x, w, bias, y, stream);
-    if (dtype == TANNIC_BFLOAT16 && p.KH == 1) return run_few<bf16, 1>(p, x, w, bias, y, stream);
-    if (dtype == TANNIC_BFLOAT16 && p.KH == 3) return run_few<bf16, 3>(p, x, w, bias, y, stream);
-    return TANNIC_UNSUPPORTED_DTYPE;
+    return choose_few(p, dtype, x, w, bias, y, stream, nullptr);
+}
+
+bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValues]) {
+    return choose_few(p, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, out) == TANNIC_SUCCESS;
 }
 
 }  // namespace th

@@ -17,6 +17,13 @@ struct ConvProblem {
     bool has_bias;
 };
 
+// The plan of the kernel that would take a problem, for tannic_hip_conv2d_plan: which of the kernels below, then its parameters and
+// the parts of its plan that say where a tile's windows lie (named in include/tannic_hip.h).
+constexpr int kConvPlanValues = 20;
+// true where the kernel takes the problem (conv2d_f32 and conv2d_few launch what these report)
+bool conv2d_f32_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
+bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValues]);
+
 // Each returns TANNIC_UNSUPPORTED_DTYPE when the problem does not meet its
 // conditions, so that the caller can try the next, more general kernel.
 // 16-bit 1x1 and 3x3 over few output pixels

@@ -30,6 +30,9 @@ CASES = {
     "k3_stride_2_odd": ((2, 12, 15, 29), (34, 12, 3, 3), (2, 2), (1, 1)),
     "k3_no_padding": ((2, 8, 12, 10), (16, 8, 3, 3), (1, 1), (0, 0)),
     "k3_wide_padding": ((2, 8, 6, 5), (16, 8, 3, 3), (1, 1), (2, 3)),
+    "k3_padding_of_four": ((8, 16, 14, 14), (64, 16, 3, 3), (1, 1), (4, 4)),
+    "k3_padding_of_five": ((16, 16, 7, 7), (32, 16, 3, 3), (1, 1), (5, 1)),
+    "k3_padding_of_nine": ((3, 8, 5, 9), (33, 8, 3, 3), (1, 1), (9, 9)),
     "k3_rect_stride": ((2, 8, 13, 17), (16, 8, 3, 3), (2, 1), (1, 0)),
     "k3_stride_3": ((2, 8, 20, 20), (16, 8, 3, 3), (3, 3), (1, 1)),
     "k3_small_maps_many_images": ((40, 8, 3, 4), (16, 8, 3, 3), (1, 1), (1, 1)),
@@ -38,6 +41,8 @@ CASES = {
     "k3_many_tiles": ((4, 16, 56, 56), (64, 16, 3, 3), (1, 1), (1, 1)),
     "k7_stem": ((2, 3, 40, 40), (64, 3, 7, 7), (2, 2), (3, 3)),
     "k7_odd_rows": ((3, 3, 23, 29), (70, 3, 7, 7), (2, 2), (3, 3)),
+    "k7_padding_of_eight": ((8, 3, 9, 9), (16, 3, 7, 7), (1, 1), (8, 8)),
+    "k7_padding_of_nine": ((5, 2, 12, 10), (20, 2, 7, 7), (1, 1), (9, 9)),
     "k7_two_channels_stride_1": ((2, 2, 17, 19), (20, 2, 7, 7), (1, 1), (3, 3)),
     "k7_one_channel_no_padding": ((2, 1, 16, 40), (8, 1, 7, 7), (1, 1), (0, 0)),
 }
