@@ -16,7 +16,7 @@
 //  * K = (ci, kh, kw) is walked as the weights lie in memory.  A group of 4 U kernel rows (ci, kh) is U rows for each quarter
 //    of a wavefront; the block's rows of weights for a group are 16-byte pieces of OIHW, loaded to LDS beside the planes.
 //    Three stages of {planes, weights}: one multiplied, one complete by the middle of the group, one on its way.
-//  * Nothing but MFMAs and LDS reads in the loop (see there).
+//  * Nothing but MFMAs and LDS reads in the loop (see there), and the sums of 36 or 64 products that the smaller tiles add up.
 // Pixels are the MFMA's first operand: an accumulator holds four consecutive pixels of the lane's channel, stored as 16 bytes.
 // With few tiles the channels are shared between `splits` blocks per tile: partial sums in fp32, added in split order
 // by a second kernel.  Accumulation starts from the bias (src/cpu/conv2d.cpp:90).
@@ -27,6 +27,7 @@
 // What is left: the last round of tiles, start-up (some 4 us) and the write-out of a round, which a compute unit with one block
 // does not overlap with anything.
 #include "conv_common.hpp"
+#include "gemm_common.hpp"
 
 namespace th {
 
@@ -57,6 +58,15 @@ __device__ __forceinline__ void f32_static_for(F&& f) {
         f32_static_for<N, F, I + 1>(static_cast<F&&>(f));
     }
 }
+
+// After how many groups the sums of a kernel start from zero again, their values added to a second set of accumulators (0: never).
+// An fp32 sum is off by some 1.8e-8 of the result's norm times the root of the additions that are chained, and the products that
+// small problems ran on before share K between four wavefronts or sixteen blocks.  Chains of 36 and 64 products stay below
+// theirs (512 -> 512 3x3 over 7 x 7, nine images: 4.1e-7 there, 5.7e-7 as one chain a block, 1.5e-7 here) and cost 2 - 4 % (31.6
+// -> 32.7 us; 42.7 there).
+// The widest tiles are chosen for problems that are one chain on every path (and have no registers for a second set); a 7x7
+// kernel's K is short.
+constexpr uint32_t chained_groups(int side, int u, int pt) { return pt >= 10 || side == 7 ? 0 : side == 3 ? 1 : 64 / (4 * u); }
 
 // COUNT consecutive floats at a byte offset (all of it in the offset that the buffer's range check sees)
 template <int COUNT>
@@ -430,12 +440,42 @@ __global__ __launch_bounds__(kF32Threads, PT >= 10 ? 1 : 2) void conv2d_f32_kern
         };
         using Yes = std::true_type;
         using No = std::false_type;
-        for (; chunk + 2 < chunk1; ++chunk) run(Yes{}, Yes{});
+        constexpr uint32_t GROUPS = chained_groups(KS, U, PT);
+        float4c total[2][GROUPS ? PT : 1];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < (GROUPS ? PT : 1); ++j) total[i][j] = float4c{0.0f, 0.0f, 0.0f, 0.0f};
+        uint32_t left = GROUPS;
+        auto settle = [&] {
+            if constexpr (GROUPS != 0) {
+                if (--left != 0) return;
+                left = GROUPS;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < PT; ++j) {
+                        total[i][j] += acc[i][j];
+                        acc[i][j] = float4c{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+            }
+        };
+        for (; chunk + 2 < chunk1; ++chunk) {
+            run(Yes{}, Yes{});
+            settle();
+        }
         if (chunk + 1 < chunk1) {
             run(Yes{}, No{});
+            settle();
             ++chunk;
         }
         run(No{}, No{});
+        if constexpr (GROUPS != 0) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < PT; ++j) acc[i][j] = total[i][j] + acc[i][j];
+        }
     }
 
     // ---- results: four consecutive pixels of a channel per lane, as 16 bytes wherever they lie in one image ------------
@@ -551,6 +591,7 @@ static void consider_f32(const ConvProblem& p, bool wide, F32Plan& best, double&
     for (uint32_t splits = 1; splits <= (RESIDENT ? 1 : q.chunks) && splits <= 32; ++splits) {
         const uint32_t per_split = (q.chunks + splits - 1) / splits;
         if (splits > 1 && (per_split * (splits - 1) >= q.chunks || tiles * (splits - 1) >= 2 * COMPUTE_UNITS)) continue;
+        if (splits > 1 && chained_groups(KS, U, PT) == 0) continue;      // (where blocks share the channels, the sums are short chains)
         const uint64_t blocks = tiles * splits;
         if (blocks >= (1ull << 24)) continue;
         // microseconds: a chunk is U * KS steps of 2 PT MFMAs of 32 clocks; start and write-out of a round; the pass over partial sums
@@ -621,10 +662,20 @@ static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* 
     if (p.xs[3] != 1 || p.xs[0] < 0 || p.xs[1] < 0 || p.xs[2] < 0 || p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO)) return -1;
     if (p.KH == 1 && (p.pad_h || p.pad_w)) return -1;
     if (K * p.O * 4 >= (1ull << 31) || pixels >= (1ull << 28) || pixels * p.O >= (1ull << 31)) return -1;
+    const bool dense = p.stride_h == 1 && p.stride_w == 1;
     // 16-byte pieces of the weights (7x7 takes single floats), and of a 1x1 kernel's signal where an image is whole pieces
     if (p.KH != 7 && (K % 4 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0)) return -1;
-    const bool wide = p.stride_h == 1 && p.stride_w == 1 && p.xs[2] == static_cast<int64_t>(p.W) && (static_cast<uint64_t>(p.H) * p.W) % 4 == 0 && p.xs[0] % 4 == 0 && p.xs[1] % 4 == 0 &&
+    const bool wide = dense && p.xs[2] == static_cast<int64_t>(p.W) && (static_cast<uint64_t>(p.H) * p.W) % 4 == 0 && p.xs[0] % 4 == 0 && p.xs[1] % 4 == 0 &&
                       reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    // Few results go to the products that share K more finely than the groups here do, and so round less: 1x1 kernels to the product of
+    // small matrices, which is faster too (512 -> 256 over 20 x 20, two images: 8.6 us and 2.1e-7 there, 12.9 and 4.1e-7 as one chain
+    // here), with a stride, whose samples that product needs copied, under fewer than 256 channels (128 -> 64 over 56 x 56, two images:
+    // 7.2 us and 1.1e-7 there, 8.1 here; under 512 the groups round less, 1.6e-7 against 2.1e-7); 3x3 kernels with at most 8192 results to
+    // the product with a workgroup per 4 x 4 results, unfolded (304 -> 3 over 35 x 37, two images: 1.0e-7 there, 2.9e-7 as chains shared
+    // by eleven blocks here, although in 13 us instead of 49).
+    const uint64_t image = static_cast<uint64_t>(p.HO) * p.WO;
+    if (p.KH == 1 && image % 4 == 0 && (dense ? p.xs[2] == static_cast<int64_t>(p.W) : p.WO % 4 == 0 && p.C < 256) && gemm_small_f32_takes(p.O, image, p.C, p.N)) return -1;
+    if (p.KH == 3 && K >= 320 && (image + 3) / 4 * 4 * p.N * p.O <= 8192) return -1;
     double time = 1e30;
     int index = -1, counter = 0;
     if (p.KH == 1) {

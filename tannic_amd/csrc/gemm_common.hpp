@@ -99,6 +99,11 @@ int gemm_repack(const GemmProblem& p, size_t esize, const void* a, const void* b
                 void* held[2]);
 // fp32 products of a few hundred rows and columns (32 x 32 tiles whose wavefronts split K; gemm_small.hip)
 int gemm_small_f32(const GemmProblem& p, const float* a, const float* b, float* c, hipStream_t stream);
+// its extents: not when the tiles of the large kernels fill the chip, when K is too short to be worth splitting, or when it is long
+inline bool gemm_small_f32_takes(uint64_t M, uint64_t N, uint64_t K, uint64_t batches) {
+    const uint64_t tiles = (M + 31) / 32 * ((N + 31) / 32) * batches;
+    return batches <= 65535 && tiles <= 512 && K >= 64 && K <= 1024 && tiles * K <= 512 * 512;
+}
 // bm x bn tiles (256 x 256, 256 x 128, 128 x 128) filled by direct global -> LDS loads (gemm_dtl.hip); T is f16 or bf16
 template <class T> int gemm16_dtl(const GemmProblem& p, int bm, int bn, const void* a, const void* b, void* c, hipStream_t stream);
 // the 128 x 128 (bm = 128) or 64 x 128 (bm = 64) tiles with K shared between `splits` workgroups per tile (k_chunk elements each, a multiple of 64): fp32

@@ -75,13 +75,13 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_f32_kernel(const 
 }
 
 int gemm_small_f32(const GemmProblem& p, const float* a, const float* b, float* c, hipStream_t stream) {
-    if (p.M == 0 || p.N == 0 || p.K == 0 || p.batches == 0 || p.batches > 65535 || p.c_group) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.M == 0 || p.N == 0 || p.K == 0 || p.batches == 0 || p.c_group) return TANNIC_UNSUPPORTED_DTYPE;
     // Not when the tiles of the large kernels fill the chip, when K is too short to be worth splitting four ways, or when it
     // is long: a wavefront's share of K is one MFMA after the other, 64 clocks for two k, and the large kernels' blocks that
     // share K pass it (NT, us, this kernel against those: 512 x 512 x 512 8.1 / 14.5, 256^3 6.1 / 10.1, 1024 x 512 x 512
     // 11.9 / 16.2, 512 x 1024 x 1024 21.7 / 21.4, 512 x 512 x 2048 23.1 / 22.2, 384 x 384 x 4096 41 / 28).
-    const uint64_t tiles_m = (p.M + 31) / 32, tiles_n = (p.N + 31) / 32, tiles = tiles_m * tiles_n * p.batches;
-    if (tiles > 512 || p.K < 64 || p.K > 1024 || tiles * p.K > 512 * 512) return TANNIC_UNSUPPORTED_DTYPE;
+    if (!gemm_small_f32_takes(p.M, p.N, p.K, p.batches)) return TANNIC_UNSUPPORTED_DTYPE;
+    const uint64_t tiles_m = (p.M + 31) / 32, tiles_n = (p.N + 31) / 32;
     const uint32_t groups = (p.K + 7) / 8, k_per_wave = (groups + kSmallWaves - 1) / kSmallWaves * 8;
     const dim3 grid(static_cast<uint32_t>(tiles_m * tiles_n), p.batches), block(64 * kSmallWaves);
     const bool ak = p.a_cs == 1, bk = p.b_rs == 1;

@@ -10,6 +10,7 @@ import pytest
 import support
 import tannic_amd as ta
 from tannic_amd import ops
+from test_conv_plan import conv_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +73,48 @@ def test_values_beside_the_image_do_not_leak(device):
     want = ops.convolve2d(hx[1:2, :, 2:8, 3:10], hw, None, 1, 1).numpy()
     got = ops.convolve2d(dx[1:2, :, 2:8, 3:10], dw, None, 1, 1).numpy()
     support.assert_close(got, want, 1e-5, 72 * np.finfo(np.float32).eps, "view")
+
+
+# Problems that products with a finely shared K ran before this kernel took them, and some that those keep.  x shape, w shape, stride.
+SUMS = {
+    "k3_seven_wide": ((9, 512, 7, 7), (512, 512, 3, 3), 1),
+    "k3_shared_by_many_blocks": ((3, 512, 7, 7), (512, 512, 3, 3), 1),
+    "k3_one_block_each": ((4, 128, 37, 37), (128, 128, 3, 3), 1),
+    "k3_stride": ((17, 256, 20, 20), (256, 256, 3, 3), 2),
+    "k3_short": ((2, 64, 59, 59), (64, 64, 3, 3), 1),
+    "k3_wide_tile_of_few_channels": ((17, 972, 34, 34), (36, 972, 3, 3), 1),
+    "k3_few_results": ((2, 304, 35, 37), (3, 304, 3, 3), 1),
+    "k1_odd_image": ((3, 512, 37, 37), (128, 512, 1, 1), 1),
+    "k1_long": ((21, 1024, 8, 8), (512, 1024, 1, 1), 1),
+    "k1_seven_wide": ((17, 512, 6, 6), (2048, 512, 1, 1), 1),
+    "k1_stride": ((18, 512, 10, 10), (1024, 512, 1, 1), 2),
+    "k1_stride_short": ((2, 128, 56, 56), (64, 128, 1, 1), 2),
+    "k1_small_product": ((2, 512, 20, 20), (256, 512, 1, 1), 1),
+}
+
+
+@pytest.mark.parametrize("name", list(SUMS))
+def test_sums_are_short_chains(name, device):
+    """The error against 64 bits is what chains of 36 or 64 products, and the sums over groups and blocks, give: n additions of values
+    that grow with their root, each off by an error uniform within half a unit of the last place, 2^-24 / sqrt(3) of the partial sum
+    at most: 2^-24 / sqrt(6) * sqrt(n) of the result's norm."""
+    xs, ws, stride = SUMS[name]
+    pad, side = ws[2] // 2, ws[2]
+    rng = np.random.default_rng(11)
+    x, w = rng.standard_normal(xs, dtype=np.float32), rng.standard_normal(ws, dtype=np.float32)
+    got = ops.convolve2d(ta.tensor(x, ta.float32, device), ta.tensor(w, ta.float32, device), None, stride, pad).numpy()
+    kernel, plan = conv_plan("float32", xs, ws, (stride, stride), (pad, pad))
+    k = ws[1] * side * side
+    if kernel == "f32":
+        additions = (36 if side == 3 else 64) + plan["chunks_per_split"] + plan["splits"]
+    else:       # a wavefront's quarter of K, or a thread's 256th
+        additions = k // 256 + 16 if side == 3 else k // 4 + 4
+    padded = np.pad(x, ((0, 0), (0, 0), (pad, pad), (pad, pad))).astype(np.float64)
+    ho, wo = got.shape[2:]
+    want = np.zeros(got.shape)
+    for i in range(side):
+        for j in range(side):
+            part = padded[:, :, i:i + (ho - 1) * stride + 1:stride, j:j + (wo - 1) * stride + 1:stride]
+            want += np.tensordot(w[:, :, i, j].astype(np.float64), part, (1, 1)).transpose(1, 0, 2, 3)
+    error = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert error <= 2.0 ** -24 / 6 ** 0.5 * additions ** 0.5, (error, additions, kernel, plan)
