@@ -546,6 +546,10 @@ static void consider_f32(const ConvProblem& p, bool wide, F32Plan& best, double&
     if (wo > 1 && p.O <= 16 * wo) return;     // half of the wavefronts would have no channel
     F32Plan q{};
     q.K = p.C * KS * KS;
+    // The widest tiles are one block on a compute unit, and nothing runs beside its write-out: not under a short K (K = 60, 187 channels,
+    // 4 images of 123 x 124: 31 us with them, 26 before this kernel, 21 with the next narrower; K below 32 in more than three rounds, mean of
+    // nine: 1.12 times the time before with them, 0.87 without; K of 64 to 128 in one round or less, mean of thirteen: 0.87 and 0.79).
+    if (KS == 1 && PT >= 10 && q.K < 128) return;
     q.pixels = p.N * p.HO * p.WO;
     q.ptile = 16 * PT * (4 / wo);
     q.co_tiles = (p.O + 32 * wo - 1) / (32 * wo);
@@ -587,6 +591,10 @@ static void consider_f32(const ConvProblem& p, bool wide, F32Plan& best, double&
     const uint64_t span = (images * p.xs[0] + static_cast<uint64_t>(p.C) * p.xs[1] + static_cast<uint64_t>(p.H) * p.xs[2] + p.W) * 4;
     if (span >= (1ull << 31)) return;
     const uint64_t tiles = (q.pixels + q.ptile - 1) / q.ptile * q.co_tiles;
+    // Tiles of 32 pixels under 128 channels (planes so wide that no other tile fits) read the signal often: not beyond half a round of
+    // them under a short K or with channels to spare (time against the kernels before: K = 72, 14 rounds 1.53, K = 144, 4 rounds 1.31, K =
+    // 2916 with 192 channels in two tiles 1.28; K = 1152 with whole tiles 0.77 - 0.93, below half a round 0.54 - 0.76).
+    if (KS == 3 && PT * (4 / WO) == 2 && 2 * tiles > COMPUTE_UNITS && (q.K < 512 || 8 * p.O < 7 * q.co_tiles * 32 * wo)) return;
     const uint32_t resident = PT >= 10 || q.buffer * 4 > 80 * 1024 ? 1 : 2;        // blocks on a compute unit at a time
     for (uint32_t splits = 1; splits <= (RESIDENT ? 1 : q.chunks) && splits <= 32; ++splits) {
         const uint32_t per_split = (q.chunks + splits - 1) / splits;
@@ -676,6 +684,10 @@ static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* 
     const uint64_t image = static_cast<uint64_t>(p.HO) * p.WO;
     if (p.KH == 1 && image % 4 == 0 && (dense ? p.xs[2] == static_cast<int64_t>(p.W) : p.WO % 4 == 0 && p.C < 256) && gemm_small_f32_takes(p.O, image, p.C, p.N)) return -1;
     if (p.KH == 3 && K >= 320 && (image + 3) / 4 * 4 * p.N * p.O <= 8192) return -1;
+    // Very many results under a short K are bound by writing them, behind the sums of a block here and beside those of others in the products
+    // over images (29 images of 122 x 122, 20 -> 991: 544 us there, 717 here; 24 of 84 x 84, 32 -> 437 with a stride: 111 / 149; but 4 -> 739
+    // 640 / 543 and 16 -> 286 307 / 279).
+    if (p.KH == 1 && image % 4 == 0 && K >= 8 && K < 64 && p.O >= 400 && pixels * p.O >= (1ull << 26)) return -1;
     double time = 1e30;
     int index = -1, counter = 0;
     if (p.KH == 1) {
@@ -684,6 +696,9 @@ static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* 
         TH_F32_K3(TH_F32_CONSIDER)
     } else if (p.KH == 7) {
         TH_F32_K7(TH_F32_CONSIDER)
+        // Wide rows: what a tile loads grows beyond what it multiplies (three channels, stride 2, 64 channels, mean of the time against the
+        // gathering tiles by the LDS of a block: up to 32 KB 0.81, to 40 KB 0.88, to 44 KB 0.95, to 50 KB 1.01, to 60 KB 1.2).
+        if (q.buffer * 4 > 40 * 1024) return -1;
     }
     return index;
 }

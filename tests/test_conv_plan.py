@@ -92,3 +92,28 @@ def test_windows_lie_in_their_planes(side, problems):
         stride = (rng.randrange(1, 5), rng.randrange(1, 5)) if rng.random() < 0.5 else (1, 1)
         taken += check_windows((images, channels, height, width), (rng.randrange(1, 200), channels, side, side), stride, padding)
     assert taken >= problems // 4, taken
+
+
+# fp32 problems that the kernels before do in less time: x, w, stride, padding
+FASTER_ELSEWHERE = {
+    "wide_rows_under_a_stem": ((8, 3, 294, 294), (64, 3, 7, 7), 2, 3),
+    "few_channels_wide_rows": ((9, 2, 348, 347), (2, 2, 7, 7), 2, 0),
+    "writing_bound": ((29, 20, 122, 122), (991, 20, 1, 1), 1, 0),
+    "small_tiles_short_k": ((22, 8, 72, 72), (442, 8, 3, 3), 2, 1),
+    "small_tiles_spare_channels": ((6, 324, 74, 76), (192, 324, 3, 3), 2, 1),
+    "small_product": ((2, 512, 20, 20), (256, 512, 1, 1), 1, 0),
+    "small_product_of_samples": ((2, 128, 56, 56), (64, 128, 1, 1), 2, 0),
+}
+
+
+@pytest.mark.parametrize("name", list(FASTER_ELSEWHERE))
+def test_fp32_problems_left_to_other_kernels(name):
+    x, w, stride, padding = FASTER_ELSEWHERE[name]
+    kernel, plan = conv_plan("float32", x, w, (stride, stride), (padding, padding))
+    assert kernel != "f32", plan
+
+
+@pytest.mark.parametrize("x,w", [((4, 60, 123, 124), (187, 60, 1, 1)), ((18, 64, 64, 64), (256, 64, 1, 1))], ids=str)
+def test_short_k_takes_no_tile_that_fills_a_compute_unit(x, w):
+    kernel, plan = conv_plan("float32", x, w, (1, 1), (0, 0))
+    assert kernel == "f32" and plan["pt"] < 10, plan
