@@ -167,34 +167,47 @@ static int launch_few(const ConvProblem& p, FewPlan q, const void* x, const void
     return launch_status("conv2d_few_kernel");
 }
 
-// Multiply-adds up to which this kernel is taken: its loads grow with the work from the first pixel on, the other kernels' time
-// hardly does while their blocks are few.  Where the lines lie (fp16, replayed calls on one box, us, this kernel / the others):
+// Multiply-adds up to which this kernel is taken, its output channels counted in whole tiles of 16 (a tile costs its loads whatever it
+// holds): its loads grow with the work from the first pixel on, the other kernels' time hardly does while their blocks are few.
+// Where the lines lie (fp16, replayed calls on one box, us, this kernel / the others):
 //   3x3, C = 64 or 128 with a stride   240 M   64 @56: batch 1 6.5 / 10.0, 2 8.7 / 10.1, 4 12.3 / 10.3; 128 @56 s2: 8.7 / 13.2, 11.3 / 16.6, 19.4 / 16.8
 //   other 3x3                          470 M   128 @28: batch 1 6.7 / 13.2, 4 12.7 / 19.3, 8 21.4 / 18.8; 256 @14: 8.2 / 26.7, 14.4 / 17.5, 26.8 / 24.8;
 //                                              512 @7: 13.0 / 58.9, 22.5 / 60.6, 37.5 / 20.0
+//   ... C > 512 (a wavefront's second turn), s2 150 M   1248->39 @11x12, batch 9, 175 M: 32.8 / 22.3; 1024->100 @5x7, batch 27, 334 M: 39.3 / 22.6
 //   1x1, images of whole 16 bytes, C < 128      20 M   64->64 @56: batch 1 3.6 / 4.4, 2 4.0 / 3.9, 4 4.5 / 4.0
-//   ... C = 128                                 60 M   128->512 @28: batch 1 4.2 / 4.5, 2 5.1 / 4.6
+//   ... C < 256                                 80 M   128->512 @28: batch 1 4.2 / 4.5, 2 5.1 / 4.6
 //   ... more channels                          110 M   512->128 @28: batch 1 4.2 / 6.7, 2 5.0 / 6.8; 256->128 @56: 4.8 / 5.3, 6.1 / 5.4; 512->256 @28: 5.1 / 6.8, 7.4 / 6.9
 //   1x1, other images, with a stride           210 M   512->1024 @28 s2: batch 1 6.7 / 10.5, 2 10.6 / 10.9, 4 17.5 / 11.4
 //   ... without one                            300 M   256->1024 @14: batch 1 4.1 / 10.7, 4 6.6 / 10.5, 8 9.5 / 10.6; 1024->512 @14: 5.2 / 11.7, 11.1 / 15.1,
 //                                                      20.2 / 16.5; 2048->512 @7: 7.9 / 11.7, 9.3 / 13.6, 15.8 / 16.1
-static uint64_t most_few_work(const ConvProblem& p) {
-    const bool strided = p.stride_h > 1 || p.stride_w > 1;
-    if (p.KH == 3) return p.C < 128 || (strided && p.C < 256) ? 240000000u : 470000000u;
-    if (static_cast<uint64_t>(p.HO) * p.WO % 8 == 0) return p.C < 128 ? 20000000u : p.C == 128 ? 60000000u : 110000000u;
-    return strided ? 210000000u : 300000000u;
+//   ... without one, C < 256                   140 M   192->51 @140x29, batch 5, 250 M: 13.8 / 10.3; 128->54 @79, batch 3, 153 M: 8.4 / 7.2
+//   ... without one, C < 128                   100 M   64->64 @37, batch 32, 179 M: 11.5 / 6.5; 64->109 @83x84, batch 3, 150 M: 8.6 / 6.6
+// Up to 16 output channels under 256 or more channels are worth half a tile (the others' tiles are as empty, and their blocks fewer: 3x3 over
+// 1, 1.4, 2 and 3 times the line, median of the time here over the time there 0.64, 0.60, 0.77 and 1.1; 1x1 over ragged images 0.74, 0.76, 0.80), but not
+// in a 1x1 kernel over whole images (0.77, 1.41 and 1.51).
+// (Before output channels counted in tiles, an output head of one channel came here with sixteen times the loads: 512->1 3x3 @65x112,
+// batch 12, 202 us here, 64 there.)
+static bool few_work(const ConvProblem& p, uint64_t pixels) {
+    const bool strided = p.stride_h > 1 || p.stride_w > 1, whole = static_cast<uint64_t>(p.HO) * p.WO % 8 == 0;
+    double most = strided ? 210e6 : p.C < 128 ? 100e6 : p.C < 256 ? 140e6 : 300e6;
+    if (p.KH == 3) most = p.C < 128 || (strided && p.C < 256) ? 240e6 : strided && p.C > 512 && p.O > 16 ? 150e6 : 470e6;
+    else if (whole) most = p.C < 128 ? 20e6 : p.C < 256 ? 80e6 : 110e6;
+    double channels = (static_cast<uint64_t>(p.O) + 15) / 16 * 16;
+    if (p.O <= 16 && p.C >= 256 && (p.KH == 3 || strided || !whole)) channels = 8;
+    return static_cast<double>(pixels) * channels * p.C * (p.KH * p.KW) <= most;
 }
 
 // Tiles per block: one while there are fewer than some 300, so that every compute unit has a block; then two (output channels where
 // the signal is expensive - nine taps, or every other pixel of a row - and pixels where the weights are), then four, whose
 // accumulated tiles fit the static LDS up to eight wavefronts (us with 1, 2 channels, 4 tiles: 3x3 256 @14 batch 1 8.2, 10.1, 13.7, batch 2
-// 13.3, 10.4, 13.8, batch 4 23.4, 17.9, 14.4; 1x1 1024->512 @14 with 1 and 2 pixels 5.8, 5.2, batch 4 14.3, 11.1).
+// 13.3, 10.4, 13.8, batch 4 23.4, 17.9, 14.4; 1x1 1024->512 @14 with 1 and 2 pixels 5.8, 5.2, batch 4 14.3, 11.1).  Up to 16 output
+// channels are never two tiles of them.
 template <class T, int KS, int WAVES>
 static int few_shape(const ConvProblem& p, const FewPlan& q, uint64_t tiles, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan) {
     const bool strided = p.stride_h > 1 || p.stride_w > 1;
-    if (tiles < 300) return launch_few<T, KS, 1, 1, WAVES>(p, q, x, w, bias, y, stream, plan);
+    if (tiles < 300 || (p.O <= 16 && (KS == 3 || strided))) return launch_few<T, KS, 1, 1, WAVES>(p, q, x, w, bias, y, stream, plan);
     if constexpr (WAVES <= 8) {
-        if (tiles >= 700 && (KS == 3 || strided || WAVES == 8)) return launch_few<T, KS, 2, 2, WAVES>(p, q, x, w, bias, y, stream, plan);
+        if (tiles >= 700 && p.O > 16 && (KS == 3 || strided || WAVES == 8)) return launch_few<T, KS, 2, 2, WAVES>(p, q, x, w, bias, y, stream, plan);
     }
     if constexpr (KS == 1) {
         if (!strided) return launch_few<T, KS, 1, 2, WAVES>(p, q, x, w, bias, y, stream, plan);
@@ -220,7 +233,7 @@ static int run_few(const ConvProblem& p, const void* x, const void* w, const voi
         if (extent[d] > 1) last += (extent[d] - 1) * static_cast<uint64_t>(p.xs[d]);
         if (last >= (1ull << 30)) return TANNIC_UNSUPPORTED_DTYPE;
     }
-    if (pixels >= (1ull << 24) || static_cast<double>(pixels) * p.O * p.C * TAPS > static_cast<double>(most_few_work(p))) return TANNIC_UNSUPPORTED_DTYPE;
+    if (pixels >= (1ull << 24) || !few_work(p, pixels)) return TANNIC_UNSUPPORTED_DTYPE;
     FewPlan q{};
     q.pixels = static_cast<uint32_t>(pixels);
     q.units = p.C / 32;

@@ -117,3 +117,32 @@ def test_fp32_problems_left_to_other_kernels(name):
 def test_short_k_takes_no_tile_that_fills_a_compute_unit(x, w):
     kernel, plan = conv_plan("float32", x, w, (1, 1), (0, 0))
     assert kernel == "f32" and plan["pt"] < 10, plan
+
+
+# 16-bit problems around the lines up to which the kernel over few output pixels is taken: x, w, stride, padding, taken
+FEW_PIXELS = {
+    "one_output_channel_large_maps": ((12, 512, 65, 112), (1, 512, 3, 3), 1, 1, False),
+    "one_output_channel_large_image": ((1, 32, 912, 912), (1, 32, 3, 3), 1, 1, False),
+    "one_output_channel_few_pixels": ((1, 512, 14, 14), (1, 512, 3, 3), 1, 1, True),
+    "ragged_1x1_of_few_channels": ((32, 64, 37, 37), (64, 64, 1, 1), 1, 0, False),
+    "ragged_1x1_below_the_line": ((16, 64, 37, 37), (64, 64, 1, 1), 1, 0, True),
+    "ragged_1x1_of_many_channels": ((7, 1024, 14, 14), (256, 1024, 1, 1), 1, 0, False),
+    "ragged_1x1_of_many_channels_below": ((4, 1024, 14, 10), (512, 1024, 1, 1), 1, 0, True),
+    "stride_of_many_channels": ((27, 1024, 5, 7), (100, 1024, 3, 3), 2, 1, False),
+}
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("name", list(FEW_PIXELS))
+def test_few_pixels(name, dtype):
+    x, w, stride, padding, taken = FEW_PIXELS[name]
+    kernel, plan = conv_plan(dtype, x, w, (stride, stride), (padding, padding))
+    assert (kernel == "few") == taken, plan
+
+
+@pytest.mark.parametrize("outputs", [1, 15, 16])
+@pytest.mark.parametrize("stride", [1, 2])
+def test_sixteen_output_channels_are_one_tile(outputs, stride):
+    for side in (1, 3):
+        kernel, plan = conv_plan("float16", (1, 64, 90 * stride, 91 * stride), (outputs, 64, side, side), (stride, stride), (side // 2, side // 2))
+        assert kernel == "few" and plan["mo"] == 1, plan
