@@ -218,6 +218,9 @@ void tannic_hip_counters(uint64_t out[3]);
  * 16 channels and of 16 pixels per block, wavefronts, blocks.  The status is the convolution's. */
 int tannic_hip_conv2d_plan(const tannic_tensor_t* x, const tannic_tensor_t* w, const tannic_tensor_t* y, const size_t pad[2],
                            const size_t stride[2], uint32_t out[20]);
+/* Whether the product of a few rows with narrow row-major matrices (16-bit, misaligned) takes these operands, asked the same way:
+ * the lanes side by side along its columns, 0 if it does not. */
+int tannic_hip_gemm_rows_batch_lanes(const tannic_tensor_t* a, const tannic_tensor_t* b, const tannic_tensor_t* dst);
 /* The stream a recording captures: a caller that keeps a device's stream to itself checks that it is this one. */
 tannic_stream_t tannic_hip_graph_stream(void* recording);
 

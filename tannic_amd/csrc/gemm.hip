@@ -493,7 +493,7 @@ int gemm_entry(const tannic_tensor_t* a, const tannic_tensor_t* b, tannic_tensor
                     }
                 }
                 if constexpr (std::is_same_v<A, B> && is_16bit<A>::value) {
-                    // at most four rows times narrow matrices that lie row by row: every matrix is read once, along its rows
+                    // two to four rows times narrow matrices that lie row by row, misaligned: every matrix is read once, along its rows
                     status = gemm_rows_batch(p, a->dtype, first, second, dst->address, s);
                     if (status != TANNIC_UNSUPPORTED_DTYPE) return;
                 }
@@ -589,4 +589,12 @@ extern "C" int tannic_hip_gemm_noalloc(const tannic_tensor_t* a, const tannic_te
     if (int rc = scratch_address(&base)) return rc;
     const GemmWorkspace workspace{base, kNoAllocScratchBytes};
     return gemm_entry(a, b, dst, stream, &workspace);
+}
+
+extern "C" int tannic_hip_gemm_rows_batch_lanes(const tannic_tensor_t* a, const tannic_tensor_t* b, const tannic_tensor_t* dst) {
+    if (!a || !b || !dst || a->dtype != b->dtype || !have_storage(a, b, dst)) return 0;
+    GemmProblem p;
+    tannic_tensor_t result = *dst;
+    if (describe_gemm(a, b, &result, p) != TANNIC_SUCCESS) return 0;
+    return static_cast<int>(gemm_rows_batch_lanes(p, a->dtype, a->address, b->address));
 }

@@ -87,7 +87,8 @@ int gemm_skinny_16bit(const GemmProblem& p, int dtype, const void* a, const void
 int gemm_skinny_f32(const GemmProblem& p, const float* a, const float* b, float* c, hipStream_t stream);
 int gemm_skinny_int8(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream);
 int gemm_rows_nn(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
-// 16-bit, at most four rows times narrow row-major matrices under a long, odd K (gemm_rows_batch.hip)
+// 16-bit, two to four rows times narrow row-major matrices under a long K, misaligned (gemm_rows_batch.hip); the lanes it would take, 0 for none
+uint32_t gemm_rows_batch_lanes(const GemmProblem& p, int dtype, const void* a, const void* b);
 int gemm_rows_batch(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 int gemm_few_results(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 int gemm_mfma_f64(const GemmProblem& p, const double* a, const double* b, double* c, hipStream_t stream);

@@ -1,4 +1,4 @@
-// At most four rows times narrow matrices that lie row by row, 16-bit, one product per batch index:
+// Two to four rows times narrow matrices that lie row by row, 16-bit, one product per batch index:
 // y[b][m][n] = sum over k of x[b][m][k] * W[b][k][n], N a multiple of 8 up to 256, K of a thousand or more.  (Attention's probabilities times the
 // cached values for one new token: a group's query heads are the rows, K is the length of the context, whatever it is.)
 //
@@ -19,9 +19,10 @@ constexpr int kRowsBatchWaves = 16;
 // rows of W a lane has in flight: with few blocks a context of a few thousand is one pass
 constexpr int rows_batch_unroll(int lanes) { return lanes == 2 ? 8 : 4; }
 
-// the sums of the lanes that differ in bits STEP ... 32 of the lane number: N values per lane become N * STEP / 32 / 2 finished ones
+// The sums over the lanes that differ in bits LAST ... 32 of the lane number (first call: STEP = 32): N values per lane become N * LAST / 64
+// finished ones, those whose number has the bits of the lane's (the upper half where the lane has bit STEP, and so on).
 template <int N, int STEP, int LAST>
-__device__ __forceinline__ void scatter_sums(float* v, uint32_t lane, uint32_t& first) {
+__device__ __forceinline__ void scatter_sums(float* v, uint32_t lane) {
     if constexpr (STEP >= LAST) {
         const bool upper = (lane & STEP) != 0;
 #pragma unroll
@@ -29,8 +30,7 @@ __device__ __forceinline__ void scatter_sums(float* v, uint32_t lane, uint32_t& 
             const float keep = upper ? v[i + N / 2] : v[i], send = upper ? v[i] : v[i + N / 2];
             v[i] = keep + __shfl_xor(send, STEP, 64);
         }
-        first += upper ? N / 2 : 0;
-        scatter_sums<N / 2, STEP / 2, LAST>(v, lane, first);
+        scatter_sums<N / 2, STEP / 2, LAST>(v, lane);
     }
 }
 
@@ -86,13 +86,12 @@ __global__ __launch_bounds__(64 * kRowsBatchWaves) void gemm_rows_batch_kernel(c
             }
         }
     }
-    uint32_t first = 0;
-    scatter_sums<MR * 8, 32, LN>(acc, lane, first);
+    scatter_sums<MR * 8, 32, LN>(acc, lane);
 #pragma unroll
     for (int i = 0; i < LEFT; ++i) part[wave][i * 64 + lane] = acc[i];
     __syncthreads();
     for (uint32_t at = threadIdx.x; at < 64 * LEFT; at += blockDim.x) {
-        // sum `at` is value first + at / 64 of lane at % 64: row value / 8, column value % 8 of that lane's eight
+        // sum `at` is the (at / 64)th that lane at % 64 finished: row value / 8, column value % 8 of that lane's eight
         float sum = 0.0f;
         for (uint32_t v = 0; v < waves; ++v) sum += part[v][at];
         const uint32_t from = at % 64;
@@ -115,20 +114,46 @@ static int launch_rows_batch(const GemmProblem& p, const void* x, const void* w,
     return launch_status("gemm_rows_batch_kernel");
 }
 
-// Where rows of x that no 16 bytes divide leave the tiles their loaders for any alignment, and there are more results than the
-// kernel for few results takes, up to 8192 columns in all products (bf16, four rows, replayed calls, us here / before:
-// 32 products of 1001 x 128 7.8 / 15.4, 64 of 2049 x 128 11.8 / 32.6, 128 of 4001 x 64 22.2 / 58.2).  With K a multiple of 8 the tiles
-// are as good (64 of 2048 x 128 12.1 / 11.1), and so they are with more products (256 of 4001 x 128 97 / 78: a value of x per
-// row and lane is four loads beside the one of W).
+// Which of the kernels takes a product: its lanes side by side along the columns, or 0 where none does.
+//
+// They are taken where the tiles would read an operand at any alignment (K, or a pitch or an address of x or W, that no 16 bytes divide)
+// and there are more results than the kernel for few results takes, up to one block of 32 columns per compute unit - two where the
+// columns are whole blocks of aligned rows.  bf16, four rows, replayed calls, us here / before:
+//   one block a unit   32 products of 1001 x 128 7.0 / 15.9, 64 of 2049 x 128 12.6 / 33.2, 128 of 4001 x 64 23.2 / 58.4, 85 of 1001 x 72 10.9 / 16.1,
+//                      64 of 1024 x 128 with an odd pitch of x 7.2 / 15.1, of W 7.7 / 15.0
+//   ragged, more       113 of 1001 x 72 18.1 / 16.2, 78 of 1001 x 104 18.8 / 16.0
+//   two a unit         72 of 2049 x 128 18.5 / 33.4, 96 of it 23.1 / 33.7, 128 of it 23.7 / 34.0, of 1001 x 128 14.4 / 19.0
+//   three a unit       192 of 1001 x 128 21.6 / 20.0, of 2049 x 128 38.8 / 34.7
+//   aligned, on tiles  64 of 2048 x 128 12.2 / 11.6, of 4000 x 128 21.5 / 16.8
+// (Up to 64 columns a tile of the product is half empty, and up to 8192 columns in all are taken: 204 of 1001 x 40 13.4 / 17.3.  A K
+// below 1000 is not taken, although 64 of 513 x 128 ran in 6.0 against 11.1.)
+// Lanes: four, 64-byte runs of a row (64 of 2049 x 128 12.6, with two 19.2; 85 of 1001 x 72 10.9, 16.6), but two where the columns are no more than two lanes', or three times two lanes' in more than a round (131 of 2007 x 48 19.4 against 25.5), or a long K is shared
+// by too few blocks (32 of 4001 x 128 14.4 against 19.2, of 2049 x 128 9.2 against 9.4).
+static uint32_t rows_batch_lanes(const GemmProblem& p, const void* x, const void* w) {
+    if (p.M < 2 || p.M > 4 || p.N == 0 || p.N > 256 || p.N % 8 != 0 || p.K < 1000 || p.K >= (1u << 31)) return 0;
+    if (p.a_cs != 1 || p.b_cs != 1 || p.b_rs == 1 || p.row_bias || p.c_group || p.b_group_stride) return 0;
+    bool x_aligned = p.a_rs % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, w_aligned = p.b_rs % 8 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+    for (int d = 0; d < p.batch_rank; ++d) {
+        x_aligned = x_aligned && p.a_bs[d] % 8 == 0;
+        w_aligned = w_aligned && p.b_bs[d] % 8 == 0;
+    }
+    if (p.K % 8 == 0 && x_aligned && w_aligned) return 0;
+    const uint64_t columns = static_cast<uint64_t>(p.N) * p.batches, blocks = static_cast<uint64_t>((p.N + 31) / 32) * p.batches;
+    if (columns * p.M <= 8192) return 0;
+    if (blocks > (p.N % 32 == 0 && w_aligned ? 512 : 256) && !(p.N <= 64 && columns <= 8192)) return 0;
+    if (p.N > 32 && p.N <= 48 && blocks > 256) return 2;
+    return p.N <= 16 || (p.K > 3000 && (p.N + 15) / 16 * static_cast<uint64_t>(p.batches) <= 256) ? 2 : 4;
+}
+
+uint32_t gemm_rows_batch_lanes(const GemmProblem& p, int dtype, const void* a, const void* b) {
+    return dtype == TANNIC_FLOAT16 || dtype == TANNIC_BFLOAT16 ? rows_batch_lanes(p, a, b) : 0;
+}
+
 template <class T>
 static int run_rows_batch(const GemmProblem& p, const void* x, const void* w, void* y, hipStream_t stream) {
-    if (p.M == 0 || p.M > 4 || p.N == 0 || p.N > 256 || p.N % 8 != 0 || p.K < 1000 || p.K >= (1u << 31) || p.K % 8 == 0) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.a_cs != 1 || p.b_cs != 1 || p.b_rs == 1 || p.row_bias || p.c_group || p.b_group_stride) return TANNIC_UNSUPPORTED_DTYPE;
-    const uint64_t columns = static_cast<uint64_t>(p.N) * p.batches;
-    if (columns > 8192 || columns * p.M <= 8192) return TANNIC_UNSUPPORTED_DTYPE;
-    // 64-byte runs of a row where that gives every compute unit a block, else 32
-    if (columns == 8192) return launch_rows_batch<T, 4>(p, x, w, y, stream);
-    return launch_rows_batch<T, 2>(p, x, w, y, stream);
+    const uint32_t lanes = rows_batch_lanes(p, x, w);
+    if (lanes == 0) return TANNIC_UNSUPPORTED_DTYPE;
+    return lanes == 4 ? launch_rows_batch<T, 4>(p, x, w, y, stream) : launch_rows_batch<T, 2>(p, x, w, y, stream);
 }
 
 int gemm_rows_batch(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream) {

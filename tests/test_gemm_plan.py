@@ -1,0 +1,50 @@
+"""Which 16-bit products of a few rows with narrow row-major matrices run on the kernel for them, asked of the library without a GPU
+(``tannic_hip_gemm_rows_batch_lanes``)."""
+import pytest
+
+import tannic_amd as ta
+from test_conv_plan import descriptor
+
+
+def lanes(batches, m, n, k, x_pitch=None, w_pitch=None, x_start=0):
+    x, w, y = (descriptor("bfloat16", s) for s in ((batches, m, k), (batches, k, n), (batches, m, n)))
+    for t, rows, pitch in ((x, m, x_pitch), (w, k, w_pitch)):
+        if pitch:
+            t.strides.sizes[0], t.strides.sizes[1] = rows * pitch, pitch
+    x.address += 2 * x_start
+    return ta.library().gemm_rows_batch_lanes(x, w, y)
+
+
+# batches, M, N, K -> lanes
+PRODUCTS = {
+    "one_block_a_unit": ((64, 4, 128, 2049), 4),
+    "a_product_less": ((63, 4, 128, 2049), 4),
+    "two_blocks_a_unit": ((128, 4, 128, 2049), 4),
+    "more_than_two": ((129, 4, 128, 2049), 0),
+    "ragged_columns_one_block": ((85, 4, 72, 1001), 4),
+    "ragged_columns_more": ((113, 4, 72, 1001), 0),
+    "ragged_columns_of_104": ((78, 4, 104, 2049), 0),
+    "half_a_tile": ((204, 4, 40, 1001), 2),
+    "half_a_tile_one_block": ((128, 4, 40, 1001), 4),
+    "eight_columns": ((1024, 4, 8, 1001), 2),
+    "long_k_few_blocks": ((32, 4, 128, 4001), 2),
+    "long_k_more_blocks": ((33, 4, 128, 4001), 4),
+    "few_results": ((16, 4, 128, 2049), 0),
+    "one_row": ((80, 1, 128, 2049), 0),
+    "aligned": ((64, 4, 128, 2048), 0),
+}
+
+
+@pytest.mark.parametrize("name", list(PRODUCTS))
+def test_products(name):
+    problem, want = PRODUCTS[name]
+    assert lanes(*problem) == want
+
+
+def test_alignment_is_of_rows_and_addresses():
+    """K a multiple of eight is no alignment: a pitch or a start that no 16 bytes divide sends the tiles to their slower loaders."""
+    assert lanes(64, 4, 128, 2048, x_pitch=2056) == 0
+    assert lanes(64, 4, 128, 2048, x_pitch=2049) == 4
+    assert lanes(64, 4, 128, 2048, x_start=1) == 4
+    assert lanes(64, 4, 128, 2048, w_pitch=129) == 4
+    assert lanes(128, 4, 128, 2048, w_pitch=129) == 0
