@@ -641,15 +641,15 @@ static int finish_f32(const ConvProblem& p, F32Plan& q, float* y, hipStream_t st
     return status;
 }
 
-// The kernels compiled: F(KS, U, PT, NL, RESIDENT, WO)
-#define TH_F32_K1W(F, WIDE) F(1, 4, 2, 8, false, 1, WIDE) F(1, 4, 2, 4, false, 2, WIDE) F(1, 8, 2, 4, false, 4, WIDE) F(1, 4, 4, 8, false, 2, WIDE) F(1, 4, 4, 4, false, 4, WIDE) \
+// The kernels compiled: F(KS, U, PT, NL, RESIDENT, WO, WIDE).  (Three more shapes were the plan of 110 of 295 000 random problems.)
+#define TH_F32_K1W(F, WIDE) F(1, 4, 2, 8, false, 1, WIDE) F(1, 4, 2, 4, false, 2, WIDE) F(1, 8, 2, 4, false, 4, WIDE) F(1, 4, 4, 8, false, 2, WIDE) \
     F(1, 8, 4, 8, false, 4, WIDE) F(1, 4, 6, 12, false, 2, WIDE) F(1, 8, 6, 12, false, 4, WIDE) F(1, 8, 8, 16, false, 4, WIDE) F(1, 4, 7, 8, false, 4, WIDE) F(1, 4, 7, 16, false, 2, WIDE) \
     F(1, 4, 13, 16, false, 4, WIDE) F(1, 4, 13, 28, false, 2, WIDE)
 #define TH_F32_K1(F) TH_F32_K1W(F, true) TH_F32_K1W(F, false)
 #define TH_F32_K3(F) F(3, 3, 2, 8, false, 1, false) F(3, 3, 2, 8, false, 2, false) F(3, 3, 2, 8, false, 4, false) F(3, 3, 4, 8, false, 2, false) F(3, 3, 4, 8, false, 4, false) F(3, 3, 5, 8, false, 2, false) \
     F(3, 3, 5, 8, false, 4, false) F(3, 3, 7, 8, false, 2, false) F(3, 3, 7, 6, false, 4, false) F(3, 3, 7, 12, false, 4, false) F(3, 3, 7, 16, false, 2, false) F(3, 3, 10, 10, false, 2, false) F(3, 3, 10, 12, false, 4, false) F(3, 3, 4, 12, false, 2, false) \
     F(3, 3, 13, 12, false, 2, false) F(3, 3, 13, 10, false, 4, false)
-#define TH_F32_K7(F) F(7, 1, 2, 1, true, 1, false) F(7, 1, 2, 1, true, 2, false) F(7, 1, 4, 1, true, 2, false) F(7, 1, 4, 1, true, 4, false) F(7, 1, 7, 1, true, 2, false) F(7, 1, 7, 1, true, 4, false)
+#define TH_F32_K7(F) F(7, 1, 2, 1, true, 1, false) F(7, 1, 2, 1, true, 2, false) F(7, 1, 4, 1, true, 2, false) F(7, 1, 7, 1, true, 2, false)
 
 #define TH_F32_CONSIDER(KS, U, PT, NL, RES, WO, WIDE) consider_f32<KS, U, PT, NL, RES, WO, WIDE>(p, wide, q, time, index, counter++);
 #define TH_F32_LAUNCH(KS, U, PT, NL, RES, WO, WIDE) \
