@@ -367,7 +367,8 @@ __global__ __launch_bounds__(kF32Threads, PT >= 10 ? 1 : 2) void conv2d_f32_kern
                 if constexpr (RUN % 4 == 0) {
                     if (k % 4 == 0) {
                         const float4c v = *reinterpret_cast<lds_float4>(w_at + (i * 16 * (4 * RUN) + k) * 4);
-                        __builtin_memcpy(&wv[i][k], &v, 16);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) wv[i][k + e] = v[e];
                     }
                 } else {
                     wv[i][k] = *reinterpret_cast<lds_float>(w_at + (i * 16 * (4 * RUN) + k) * 4);
