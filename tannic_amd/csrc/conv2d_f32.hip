@@ -1,4 +1,4 @@
-// conv2d in fp32 on v_mfma_f32_16x16x4f32: 1x1, 3x3 and 7x7 kernels, any width, alignment, stride and padding.
+// conv2d in fp32 on v_mfma_f32_16x16x4f32: 1x1, 3x3 and 7x7 kernels, any width, alignment, stride and (3x3, 7x7) padding.
 //
 // The fp32 matrix pipe is sixteen times slower than the 16-bit one (2048 flops in 32 clocks), so a layer is bound by it and by
 // nothing else as long as every SIMD has as much of the work as every other, and nothing makes the pipe wait.  A block of
@@ -21,9 +21,10 @@
 // With few tiles the channels are shared between `splits` blocks per tile: partial sums in fp32, added in split order
 // by a second kernel.  Accumulation starts from the bias (src/cpu/conv2d.cpp:90).
 // Measured, batch 32, us before (gathering tiles; products over images, unfolded or re-pitched) / here, TFLOP/s of 157 here:
-//   64 -> 64 3x3 over 56 x 56 110 / 68, 109; 128 -> 128 over 28 x 28 104 / 70, 106; 256 -> 256 over 14 x 14 116 / 76, 98;
-//   512 -> 512 over 7 x 7 111 / 74, 100; 64 -> 256 1x1 over 56 x 56 55 / 43, 76; 512 -> 256 over 28 x 28 75 / 60, 110;
-//   256 -> 1024 over 14 x 14 44 / 35, 93; 3 -> 64 7x7 s2 over 224 x 224 126 / 117, 65.  One image, 3x3: 22 / 11 ... 26 / 18.
+//   64 -> 64 3x3 over 56 x 56 104 / 67, 111; 128 -> 128 over 28 x 28 104 / 73, 101; 256 -> 256 over 14 x 14 117 / 87, 85;
+//   512 -> 512 over 7 x 7 111 / 77, 96; 64 -> 256 1x1 over 56 x 56 55 / 44, 74; 512 -> 256 over 28 x 28 76 / 61, 108;
+//   256 -> 1024 over 14 x 14 44 / 36, 92; 3 -> 261 7x7 s2 over 40 x 42, batch 27, 36 / 19.  One image, 3x3: 21 / 11 ... 26 / 18.
+// plan_f32 says which problems are left to the kernels before, with both sides.
 // What is left: the last round of tiles, start-up (some 4 us) and the write-out of a round, which a compute unit with one block
 // does not overlap with anything.
 #include "conv_common.hpp"
@@ -302,9 +303,9 @@ __global__ __launch_bounds__(kF32Threads, PT >= 10 ? 1 : 2) void conv2d_f32_kern
         asm volatile("" ::: "memory");
     }
 
-    // The loop.  A vector instruction between two fp32 MFMAs of a wavefront holds the matrix pipe up (some 17 clocks for the
-    // first one, 4 for each that follows; measured with a loop of pairs of MFMAs: 67 clocks a pair, 84 with one addition, 67 with
-    // reads of LDS), so the loop has next to none: addresses are registers plus an immediate, moved on to the next stage once a
+    // The loop.  A vector instruction between two fp32 MFMAs of a wavefront holds the matrix pipe up (14 clocks for the
+    // first one, 4 for each that follows; measured with a loop of pairs of MFMAs: 66.5 clocks a pair, 80.5 with one addition, 67 with
+    // a read of LDS), so the loop has next to none: addresses are registers plus an immediate, moved on to the next stage once a
     // group, all in one place, and operands are replaced in their registers as soon as their last MFMA has been issued: a
     // pixel's value behind that MFMA, a kernel row's (two rows of a 1x1 kernel's) MFMAs before it is needed, the weights at the
     // group's end.

@@ -48,7 +48,7 @@ struct FewPlan {
 };
 
 constexpr uint32_t kFewPitch = 20;              // floats per row of a partial 16 x 16 tile: the four row groups of a write fall on different banks
-constexpr uint32_t kFewOutside = 0x80000000u;   // beyond every signal this kernel takes (records < 2^31): the load gives zero
+constexpr uint32_t kFewOutside = 0x80000000u;   // not below any signal's bytes that this kernel takes (records <= 2^31): the load gives zero
 
 template <class T, int KS, int MO, int NP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void conv2d_few_kernel(const T* x, const T* w, const T* bias, T* y, ConvProblem p, FewPlan q) {

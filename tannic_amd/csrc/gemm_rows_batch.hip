@@ -127,8 +127,9 @@ static int launch_rows_batch(const GemmProblem& p, const void* x, const void* w,
 //   aligned, on tiles  64 of 2048 x 128 12.2 / 11.6, of 4000 x 128 21.5 / 16.8
 // (Up to 64 columns a tile of the product is half empty, and up to 8192 columns in all are taken: 204 of 1001 x 40 13.4 / 17.3.  A K
 // below 1000 is not taken, although 64 of 513 x 128 ran in 6.0 against 11.1.)
-// Lanes: four, 64-byte runs of a row (64 of 2049 x 128 12.6, with two 19.2; 85 of 1001 x 72 10.9, 16.6), but two where the columns are no more than two lanes', or three times two lanes' in more than a round (131 of 2007 x 48 19.4 against 25.5), or a long K is shared
-// by too few blocks (32 of 4001 x 128 14.4 against 19.2, of 2049 x 128 9.2 against 9.4).
+// Lanes: four, 64-byte runs of a row (64 of 2049 x 128 12.6, with two 19.2; 85 of 1001 x 72 10.9, 16.6), but two where the columns are no
+// more than two lanes', or three times two lanes' in more than a round (131 of 2007 x 48 19.4 against 25.5), or a long K is shared by too
+// few blocks (32 of 4001 x 128 14.4 against 19.2, of 2049 x 128 9.2 against 9.4).
 static uint32_t rows_batch_lanes(const GemmProblem& p, const void* x, const void* w) {
     if (p.M < 2 || p.M > 4 || p.N == 0 || p.N > 256 || p.N % 8 != 0 || p.K < 1000 || p.K >= (1u << 31)) return 0;
     if (p.a_cs != 1 || p.b_cs != 1 || p.b_rs == 1 || p.row_bias || p.c_group || p.b_group_stride) return 0;
