@@ -105,7 +105,7 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     // registers when they fit (conv2d_k1.hip), otherwise it is a matrix product per image (conv2d_pointwise.hip).
     const bool pointwise = p.KH == 1 && p.KW == 1;
     // fp32 1x1, 3x3 and 7x7 (few channels) have a kernel of their own; what it refuses (weights that are not whole 16-byte pieces,
-    // planes wider than its LDS) goes on like the 16-bit types and the other kernel sizes.
+    // planes wider than its LDS, few results, what others do in less time: plan_f32) goes on like the 16-bit types and the other kernel sizes.
     int status = conv2d_f32(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     status = conv2d_few(p, x->dtype, x->address, w->address, pb, y->address, s);
