@@ -96,7 +96,7 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     p.bs = bias ? bias->strides.sizes[0] : 0;
     if (plan) {
         for (int i = 0; i < kConvPlanValues; ++i) plan[i] = 0;
-        if (!conv2d_f32_plan(p, x->dtype, x->address, w->address, plan)) conv2d_few_plan(p, x->dtype, plan);
+        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan)) conv2d_few_plan(p, x->dtype, plan);
         return TANNIC_SUCCESS;
     }
     const void* pb = bias ? bias->address : nullptr;
@@ -106,7 +106,9 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     const bool pointwise = p.KH == 1 && p.KW == 1;
     // fp32 1x1, 3x3 and 7x7 (few channels) have a kernel of their own; what it refuses (weights that are not whole 16-byte pieces,
     // planes wider than its LDS, few results, what others do in less time: plan_f32) goes on like the 16-bit types and the other kernel sizes.
-    int status = conv2d_f32(p, x->dtype, x->address, w->address, pb, y->address, s);
+    int status = conv2d_split(p, x->dtype, x->address, w->address, pb, y->address, s);
+    if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
+    status = conv2d_f32(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     status = conv2d_few(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;

@@ -663,8 +663,8 @@ static int finish_f32(const ConvProblem& p, F32Plan& q, float* y, hipStream_t st
         for (int i = 0; i < 7; ++i) out[1 + i] = of[i];        \
     }
 
-// The index of the kernel that takes the problem, with its plan; -1 if none does
-static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* w, F32Plan& q) {
+// The index of the kernel that takes the problem, with its plan and the time (us) it is expected to take; -1 if none does
+static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* w, F32Plan& q, double& time) {
     if (dtype != TANNIC_FLOAT32 || p.KH != p.KW || p.C == 0) return -1;
     const uint64_t K = static_cast<uint64_t>(p.C) * p.KH * p.KW, pixels = static_cast<uint64_t>(p.N) * p.HO * p.WO;
     // contiguous OIHW weights (K runs through memory in order), rows of single floats, results contiguous within an image
@@ -690,7 +690,7 @@ static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* 
     // over images (29 images of 122 x 122, 20 -> 991: 544 us there, 717 here; 24 of 84 x 84, 32 -> 437 with a stride: 111 / 149; but 4 -> 739
     // 640 / 543 and 16 -> 286 307 / 279).
     if (p.KH == 1 && image % 4 == 0 && K >= 8 && K < 64 && p.O >= 400 && pixels * p.O >= (1ull << 26)) return -1;
-    double time = 1e30;
+    time = 1e30;
     int index = -1, counter = 0;
     if (p.KH == 1) {
         TH_F32_K1(TH_F32_CONSIDER)
@@ -705,10 +705,17 @@ static int plan_f32(const ConvProblem& p, int dtype, const void* x, const void* 
     return index;
 }
 
+double conv2d_f32_expected(const ConvProblem& p, int dtype, const void* x, const void* w) {
+    F32Plan q{};
+    double time;
+    return plan_f32(p, dtype, x, w, q, time) < 0 ? -1.0 : time;
+}
+
 bool conv2d_f32_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]) {
     if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0) return false;
     F32Plan q{};
-    const int index = plan_f32(p, dtype, x, w, q);
+    double time;
+    const int index = plan_f32(p, dtype, x, w, q, time);
     if (index < 0) return false;
     int counter = 0;
     if (p.KH == 1) {
@@ -728,7 +735,8 @@ int conv2d_f32(const ConvProblem& p, int dtype, const void* x_, const void* w_, 
     if (dtype != TANNIC_FLOAT32 || p.KH != p.KW) return TANNIC_UNSUPPORTED_DTYPE;
     if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0) return TANNIC_SUCCESS;
     F32Plan q{};
-    const int index = plan_f32(p, dtype, x_, w_, q);
+    double time;
+    const int index = plan_f32(p, dtype, x_, w_, q, time);
     if (index < 0) return TANNIC_UNSUPPORTED_DTYPE;
     const float* x = static_cast<const float*>(x_);
     const float* w = static_cast<const float*>(w_);
