@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void conv_subsample4_kernel(const T* x, T* out
 // Pixel counts that are not a multiple of 16 bytes (14 x 14, 7 x 7 ...): ONE product O x C . C x (N * pitch), pitch the
 // count rounded up to 16 bytes, does the whole batch on whole tiles (a product per image would have 200 or 56 columns) and
 // stores its columns image by image (GemmProblem::c_group), straight into y.  Without a stride it also reads the images
-// where they lie (GemmProblem::b_group_stride).  With one, or when a channel's pixels are not one run of memory, the
+// where they lie (GemmProblem::b_group_stride), an even number of pixels under any number of channels.  With a stride, or when a channel's pixels are not one run of memory, the
 // sampled pixels of every (image, channel) first go to rows of `pitch` elements (the rest zeros), channel by channel with
 // the images side by side:
 // out[(c * N + n) * pitch + pix] = x[n][c][oh * stride_h][ow * stride_w], pix = oh * WO + ow; 16 bytes per thread.
@@ -134,12 +134,12 @@ int run_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w,
         g.c_group_live = static_cast<uint32_t>(pixels);
         g.c_group_stride = p.ys[0];
         g.c_group_div = FastDiv(pitch);
-        if (plane && p.C <= 256) {
-            // The pixels of a channel are one run of memory and there are few channels: the product reads the images where
-            // they lie, its loaders taking 16-byte pieces at whatever address they start.  (Those loads are slower than
-            // aligned ones and the kernel that knows them walks all of K in one block; batch 32, fp16: 256 -> 1024 over
-            // 14 x 14 16.6 against 18.4 us through re-pitched rows, but 1024 -> 256 28 against 22 us, 2048 -> 512 over
-            // 7 x 7 53 against 26 us.)
+        if (plane) {
+            // The pixels of a channel are one run of memory: the product reads the images where they lie, through the
+            // direct-to-LDS tiles for columns in groups (whole steps of channels, an even number of pixels), or, with up to 256 channels,
+            // its loaders take 16-byte pieces at whatever address they start.  (Those loads are slower than aligned ones and
+            // the kernel that knows them walks all of K in one block; batch 32, fp16: 2048 -> 512 over 7 x 7 53 against 26 us through
+            // re-pitched rows.)
             g.b_rs = p.xs[1];
             g.b_group_stride = p.xs[0];
             const int direct = product<T>(g, dtype, w, x, y, stream);
@@ -170,6 +170,22 @@ int run_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w,
     if (dense) {
         if (p.xs[3] != 1 || p.xs[2] != static_cast<int64_t>(p.W)) return TANNIC_UNSUPPORTED_DTYPE;
         g.b_rs = p.xs[1];
+        if (sizeof(T) == 2 && static_cast<uint64_t>(p.N) * pixels < (1ull << 31)) {
+            // the whole batch as one product, tiles running over images (gemm16_dtl_grouped)
+            GemmProblem whole = g;
+            whole.N = static_cast<uint32_t>(p.N * pixels);
+            whole.batch_rank = 0;
+            whole.batches = 1;
+            whole.batch_extent[0] = 1;
+            whole.c_bs[0] = 0;
+            whole.c_group = whole.c_group_live = static_cast<uint32_t>(pixels);
+            whole.c_group_stride = p.ys[0];
+            whole.c_group_div = FastDiv(whole.c_group);
+            whole.b_group_stride = p.xs[0];
+            int status = TANNIC_UNSUPPORTED_DTYPE;
+            if constexpr (sizeof(T) == 2) status = gemm16_dtl_grouped<T>(whole, w, x, y, stream);
+            if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
+        }
         g.b_bs[0] = p.xs[0];
         return product<T>(g, dtype, w, x, y, stream);
     }

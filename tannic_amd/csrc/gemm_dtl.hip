@@ -70,7 +70,8 @@ template <class T> __device__ inline void mfma16x16_in_place(typename DtlTypes<T
 // large tiles to fill the chip; two workgroups of the smallest share a compute unit.
 // SPLIT: `sk.splits` workgroups share a tile, each taking sk.k_chunk of K and storing its fp32 accumulators.
 // A_T, B_T: the operand is contiguous along M (N) and its tile is kept as k-rows.
-template <class T, int BM, int BN, int STAGES, int BLOCKS_PER_CU, bool SPLIT = false, bool A_T = false, bool B_T = false>
+// GROUPED (with B_T): B's columns lie in groups (GemmProblem::b_group_stride), its rows at any multiple of four bytes.
+template <class T, int BM, int BN, int STAGES, int BLOCKS_PER_CU, bool SPLIT = false, bool A_T = false, bool B_T = false, bool GROUPED = false>
 __global__ __launch_bounds__(256, BLOCKS_PER_CU) void gemm16_dtl_kernel(const T* A, const T* B, typename DtlTypes<T>::Out* C, GemmProblem p, uint32_t tiles_m, uint32_t tiles_n, SplitK sk) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass needs the launch stub only (and loses it over the body's device-only builtins)
     constexpr int ES = sizeof(T), BK = 128 / ES, WAVES_N = 2;   // a tile row is 128 bytes: 64 elements of 16 bits, 128 of 8
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void gemm16_dtl_kernel(const T*
     // lanes then read the head of the next k-row, rows or columns of the product that are never stored, and past the
     // last k-row the range check returns zeros.)
     const T* a_base = A + oa + static_cast<int64_t>(m0) * p.a_rs;
-    const T* b_base = B + ob + static_cast<int64_t>(n0) * p.b_cs;
+    const T* b_base = GROUPED ? B : B + ob + static_cast<int64_t>(n0) * p.b_cs;
     auto records = [](uint64_t rows_left, int64_t stride, uint32_t K) -> uint32_t {
         const uint64_t bytes = ((rows_left - 1) * static_cast<uint64_t>(stride) + K) * ES;
         return bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(bytes);
@@ -107,7 +108,11 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void gemm16_dtl_kernel(const T*
     const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<T*>(a_base), 0, A_T ? records(p.K, p.a_cs, p.M - m0 < BM ? p.M - m0 : BM) : records(p.M - m0, p.a_rs, p.K), 0x00020000);
     const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(b_base), 0, B_T ? records(p.K, p.b_rs, p.N - n0 < BN ? p.N - n0 : BN) : records(p.N - n0, p.b_cs, p.K), 0x00020000);
+        const_cast<T*>(b_base), 0,
+        GROUPED ? static_cast<uint32_t>(((p.N / p.c_group - 1) * p.b_group_stride + (p.K - 1) * p.b_rs + p.c_group_live) * ES)
+        : B_T   ? records(p.K, p.b_rs, p.N - n0 < BN ? p.N - n0 : BN)
+                : records(p.N - n0, p.b_cs, p.K),
+        0x00020000);
     // Load j of a wavefront fills 1 KB of a tile (j < LOADS_A: bytes 1024 * (LOADS_A * wave + j) .. of A's, then B's
     // likewise): eight rows of 128 bytes, or 1024 / (2 BM) k-rows; the lane's byte offset from the tile's first element:
     uint32_t voff[LOADS];
@@ -118,6 +123,16 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void gemm16_dtl_kernel(const T*
         if ((of_a && A_T) || (!of_a && B_T)) {
             const uint32_t per_row = (of_a ? BM : BN) / 8, k = slot / per_row, in_row = slot % per_row;
             const uint32_t unit = (in_row / 2) ^ ((k % 4) + 4 * ((k / 8) % 2));
+            if constexpr (GROUPED) {
+                // A piece of eight columns belongs to one group; the last piece of a group that is not whole pieces is moved back, so
+                // that it ends with the group (its first columns are the piece before's last, computed twice, to the same bits).
+                const uint32_t col = n0 + (unit * 2 + in_row % 2) * 8;
+                uint32_t g, in;
+                p.c_group_div.divmod(col, g, in);
+                in = in < p.c_group_live - 8 ? in : p.c_group_live - 8;
+                voff[j] = col < p.N ? (g * static_cast<uint32_t>(p.b_group_stride) + in + k * static_cast<uint32_t>(p.b_rs)) * ES : 0x80000000u;
+                continue;
+            }
             voff[j] = k * static_cast<uint32_t>(of_a ? p.a_cs : p.b_rs) * ES + (unit * 2 + in_row % 2) * 16;
         } else {
             const uint32_t row = slot / 8;
@@ -332,7 +347,13 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void gemm16_dtl_kernel(const T*
         uint32_t live = 0;
         T* first = c;
         if (piece < PIECES && col < p.N) {
-            if (p.c_group) {
+            if constexpr (GROUPED) {
+                uint32_t g, in;
+                p.c_group_div.divmod(col, g, in);
+                in = in < p.c_group_live - 8 ? in : p.c_group_live - 8;
+                first = c + static_cast<int64_t>(g) * p.c_group_stride + in;
+                live = 8;
+            } else if (p.c_group) {
                 first = grouped_piece(c, p, 0, col, 8, live);
             } else {
                 first = c + col;
@@ -359,12 +380,12 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void gemm16_dtl_kernel(const T*
 #endif
 }
 
-template <class T, int BM, int BN, int STAGES, bool SPLIT = false, bool A_T = false, bool B_T = false>
+template <class T, int BM, int BN, int STAGES, bool SPLIT = false, bool A_T = false, bool B_T = false, bool GROUPED = false>
 static int launch_dtl(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream, SplitK sk = SplitK{1, 0, nullptr}) {
     const uint32_t tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
     constexpr size_t tile_bytes = STAGES * (BM + BN) * 128, stage_bytes = sizeof(T) == 2 ? 2 * 4 * (BM / 2) * (BN / 2 + 8) : 0;   // the operand stages; the output staging (16-bit results)
     constexpr size_t lds_bytes = tile_bytes > stage_bytes ? tile_bytes : stage_bytes;
-    auto kernel = gemm16_dtl_kernel<T, BM, BN, STAGES, (lds_bytes <= 80 * 1024 ? 2 : 1), SPLIT, A_T, B_T>;
+    auto kernel = gemm16_dtl_kernel<T, BM, BN, STAGES, (lds_bytes <= 80 * 1024 ? 2 : 1), SPLIT, A_T, B_T, GROUPED>;
     static std::atomic<uint64_t> configured{0};
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_bytes, configured)) return rc;
     hipLaunchKernelGGL(kernel, dim3(tiles_m * tiles_n * sk.splits, p.batches), dim3(256), lds_bytes, stream, static_cast<const T*>(a), static_cast<const T*>(b),
@@ -399,9 +420,36 @@ int gemm16_dtl_krows(const GemmProblem& p, int bm, int bn, bool a_t, bool b_t, S
     if (bm == 128 && bn == 128) return launch_dtl_krows<T, 128, 128, 4, false>(p, a_t, b_t, sk, a, b, c, stream);
     return TANNIC_UNSUPPORTED_DTYPE;
 }
+// B's columns in groups, at any multiple of four bytes (a buffer load of 16 bytes wants its address to be a multiple of four): a 1x1
+// convolution over a whole batch that reads the images where they lie.  Before, images of 14 x 14 were copied into aligned rows first or read
+// by the register-staged tiles for any alignment, and images of 28 x 28 were a product each, with a ragged last tile (fp16, batch 32, us before /
+// here: 1024 -> 256 over 14 x 14 28.2 / 13.8, 256 -> 1024 22.5 / 14.3, 1024 -> 512 29.2 / 17.5, 512 -> 256 over 28 x 28 22.4 / 17.2,
+// 128 -> 512 23.8 / 17.2).  Bound by a tile's start and end: K is 2 to 16 steps.
+template <class T>
+int gemm16_dtl_grouped(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream) {
+    if (p.K == 0 || p.K % 64 != 0 || p.batches != 1 || !p.c_group || p.c_group % 8 != 0 || p.c_group_live < 8 || p.N % p.c_group != 0) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.a_cs != 1 || p.a_rs < static_cast<int64_t>(p.K) || p.a_rs >= (1 << 22) || p.a_rs % 8 != 0 || reinterpret_cast<uintptr_t>(a) % 16 != 0) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.b_cs != 1 || p.b_rs % 2 != 0 || p.b_group_stride % 2 != 0 || p.c_group_live % 2 != 0 || p.b_rs <= 0 || p.b_group_stride <= 0 || reinterpret_cast<uintptr_t>(b) % 4 != 0)
+        return TANNIC_UNSUPPORTED_DTYPE;
+    // byte offsets stay below 2^31, so that a column past the last group is out of range
+    if ((static_cast<uint64_t>(p.N / p.c_group) * p.b_group_stride + static_cast<uint64_t>(p.K) * p.b_rs) * 2 >= (1ull << 31)) return TANNIC_UNSUPPORTED_DTYPE;
+    if (reinterpret_cast<uintptr_t>(c) % 2 != 0) return TANNIC_UNSUPPORTED_DTYPE;
+    // Tiles: 128 x 128 with two stages, two blocks on a compute unit, where there is more than one for each; else blocks enough come first,
+    // 64 x 128 unless the tiles of 128 rows are nearly enough and K is long (fp16, batch 32, us with 128 rows and two stages / 128 and
+    // four / 64 and three: 256 -> 1024 over 14 x 14 (400 tiles of 128 rows) 14.3 / 17.3 / 17.5, 512 -> 256 over 28 x 28 (392)
+    // 17.2 / 20.4 / 20.9, 1024 -> 512 over 14 x 14 (200) 18.2 / 17.5 / 20.8, 512 -> 128 over 28 x 28 (196) 16.9 / 14.8 / 14.2,
+    // 1024 -> 256 over 14 x 14 (100) 22.8 / 17.8 / 13.8; eight images of 256 -> 1024 10.3 / 10.6 / 9.7).
+    const uint64_t tiles = static_cast<uint64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
+    if (p.M > 64 && tiles > 256) return launch_dtl<T, 128, 128, 2, false, false, true, true>(p, a, b, c, stream);
+    if (p.M > 64 && tiles > 160 && p.K >= 768) return launch_dtl<T, 128, 128, 4, false, false, true, true>(p, a, b, c, stream);
+    return launch_dtl<T, 64, 128, 3, false, false, true, true>(p, a, b, c, stream);
+}
+
 #if TH_DTL_PART == 1
+template int gemm16_dtl_grouped<f16>(const GemmProblem&, const void*, const void*, void*, hipStream_t);
 template int gemm16_dtl_krows<f16>(const GemmProblem&, int, int, bool, bool, SplitK, const void*, const void*, void*, hipStream_t);
 #else
+template int gemm16_dtl_grouped<bf16>(const GemmProblem&, const void*, const void*, void*, hipStream_t);
 template int gemm16_dtl_krows<bf16>(const GemmProblem&, int, int, bool, bool, SplitK, const void*, const void*, void*, hipStream_t);
 #endif
 

@@ -655,6 +655,11 @@ int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream
     if (p.b_group_stride) {
         // B's columns in groups: the loaders for any alignment know about them; A is a parameter matrix, K-contiguous
         if (!p.c_group || bk || !ak || p.batches != 1) return TANNIC_UNSUPPORTED_DTYPE;
+        if constexpr (sizeof(T) == 2) {
+            const int rc = gemm16_dtl_grouped<T>(p, a, b, c, stream);
+            if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
+        }
+        if (p.K > 256) return TANNIC_UNSUPPORTED_DTYPE;     // (conv2d_pointwise: faster through aligned rows)
         const uint64_t tiles128 = static_cast<uint64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
         if (p.M > 64 && tiles128 >= 200) return launch16<T, 128, 128, 2, true, false, false, false>(p, a, b, c, stream);
         return launch16<T, 64, 128, 2, true, false, false, false>(p, a, b, c, stream);
