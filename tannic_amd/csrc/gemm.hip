@@ -511,6 +511,10 @@ int gemm_entry(const tannic_tensor_t* a, const tannic_tensor_t* b, tannic_tensor
                         if (!std::is_same_v<A, int8_t> && p.M <= 8 && p.b_cs == 1 && p.b_rs != 1 && p.N >= 256 && p.N % 4 == 0) elsewhere = true;   // gemm_rows_nn
                     }
                     if (!elsewhere) {
+                        if constexpr (std::is_same_v<A, B> && is_16bit<A>::value) {
+                            status = gemm_rows_few(p, a->dtype, first, second, dst->address, s);
+                            if (status != TANNIC_UNSUPPORTED_DTYPE) return;
+                        }
                         status = run_few_results<A, B, D>(p, first, second, dst->address, s);
                         return;
                     }

@@ -114,6 +114,104 @@ static int launch_rows_batch(const GemmProblem& p, const void* x, const void* w,
     return launch_status("gemm_rows_batch_kernel");
 }
 
+// The same for a handful of products (few results: at most 8192), where the latency of one pass over K is the time.  Two lanes side by
+// side, so that there are blocks enough; a block's sixteen wavefronts have all of a pass, 4096 rows of W, on their way at once, and x goes
+// through LDS meanwhile as [k][row] in fp32: one read per k for the four rows (value by value from the cache, four loads of two bytes
+// beside every 16-byte load of W, the path to the cache was as long as the latency).  Eight products of 4 x 128 under 2049: 14.1 us on
+// the kernel for few results before (a workgroup per 4 x 4 results, W's lines 32 times), 8.9 here (one lane, twice the blocks: 9.4);
+// 4 x 128 under 4001 19.5 / 10.8, sixteen of 4 x 128 under 1025 13.5 / 7.8, one row of 64 columns under 3000 13.6 / 9.1.
+constexpr int kRowsFewUnroll = 8;
+constexpr uint32_t kRowsFewPass = 32 * kRowsFewUnroll * kRowsBatchWaves;    // rows of W a block has in flight
+template <class T>
+__global__ __launch_bounds__(64 * kRowsBatchWaves) void gemm_rows_few_kernel(const T* x, const T* w, T* y, GemmProblem p) {
+    constexpr int MR = 4, LN = 2, ROWS = 64 / LN, UNROLL = kRowsFewUnroll;
+    __shared__ float part[kRowsBatchWaves][64];
+    extern __shared__ __align__(16) unsigned char rows_few_lds[];
+    float4* values = reinterpret_cast<float4*>(rows_few_lds);
+    const uint32_t lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), waves = blockDim.x / 64;
+    // (workgroups go round the eight dies in turn: with whole eights of products, those that share a product's lines share a die)
+    const uint32_t batch = blockIdx.x % p.batches, group = blockIdx.x / p.batches;
+    int64_t oa, ob, oc;
+    batch_offsets(p, batch, oa, ob, oc);
+    const uint32_t col = (group * LN + lane % LN) * 8, row = lane / LN;
+    const T* wp = w + ob + (col < p.N ? col : 0);   // (N is a multiple of 8; columns past it are never stored)
+    const T* xp[MR];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) xp[m] = x + oa + static_cast<int64_t>(static_cast<uint32_t>(m) < p.M ? m : 0) * p.a_rs;   // (rows past M are never stored)
+    float acc[MR * 8];
+#pragma unroll
+    for (int i = 0; i < MR * 8; ++i) acc[i] = 0.0f;
+    for (uint32_t first = 0; first < p.K; first += kRowsFewPass) {
+        const uint32_t here = p.K - first < kRowsFewPass ? p.K - first : kRowsFewPass;
+        const uint32_t k0 = wave * ROWS * UNROLL + row;
+        uint4r bits[UNROLL];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            const uint32_t k = k0 + u * ROWS;
+            bits[u] = uint4r{0, 0, 0, 0};
+            if (k < here) bits[u] = *reinterpret_cast<const uint4r*>(wp + static_cast<int64_t>(first + k) * p.b_rs);
+        }
+        if (first) __syncthreads();     // the pass before has been read
+        for (uint32_t k = threadIdx.x; k < here; k += blockDim.x)
+            values[k] = float4{static_cast<float>(widen(xp[0][first + k])), static_cast<float>(widen(xp[1][first + k])), static_cast<float>(widen(xp[2][first + k])),
+                               static_cast<float>(widen(xp[3][first + k]))};
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            const uint32_t k = k0 + u * ROWS;
+            const float4 v = k < here ? values[k] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+            const float f[MR] = {v.x, v.y, v.z, v.w};
+            T e[8];
+            __builtin_memcpy(e, &bits[u], 16);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float wide = static_cast<float>(widen(e[i]));
+#pragma unroll
+                for (int m = 0; m < MR; ++m) acc[m * 8 + i] += f[m] * wide;
+            }
+        }
+    }
+    scatter_sums<MR * 8, 32, LN>(acc, lane);
+    part[wave][lane] = acc[0];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        float sum = 0.0f;
+        for (uint32_t v = 0; v < waves; ++v) sum += part[v][lane];
+        uint32_t value = 0;
+#pragma unroll
+        for (int step = 32, half = MR * 4; step >= LN; step /= 2, half /= 2) value += lane & step ? half : 0;
+        const uint32_t m = value / 8, n = (group * LN + lane % LN) * 8 + value % 8;
+        if (m < p.M && n < p.N) y[oc + static_cast<int64_t>(m) * p.c_rs + n] = narrow_result<T>(sum);
+    }
+}
+
+// Few results of row-major matrices under a long K; above 8192 results the tiles and the kernel above have work enough.
+static bool rows_few_takes(const GemmProblem& p) {
+    if (p.M == 0 || p.M > 4 || p.N == 0 || p.N % 8 != 0 || p.K < 512 || p.K >= (1u << 31) || p.a_cs != 1 || p.b_cs != 1 || p.b_rs == 1 || p.row_bias || p.c_group || p.b_group_stride)
+        return false;
+    return static_cast<uint64_t>(p.N) * p.batches * p.M <= 8192;
+}
+
+template <class T>
+static int run_rows_few(const GemmProblem& p, const void* x, const void* w, void* y, hipStream_t stream) {
+    constexpr uint32_t per_wave = 32 * kRowsFewUnroll;
+    uint32_t waves = (p.K + per_wave - 1) / per_wave;
+    if (waves > kRowsBatchWaves) waves = kRowsBatchWaves;
+    const size_t lds = static_cast<size_t>(p.K < kRowsFewPass ? p.K : kRowsFewPass) * 16;
+    auto kernel = gemm_rows_few_kernel<T>;
+    static std::atomic<uint64_t> configured{0};
+    if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), kRowsFewPass * 16, configured)) return rc;
+    hipLaunchKernelGGL(kernel, dim3((p.N + 15) / 16 * p.batches), dim3(64 * waves), lds, stream, static_cast<const T*>(x), static_cast<const T*>(w), static_cast<T*>(y), p);
+    return launch_status("gemm_rows_few_kernel");
+}
+
+int gemm_rows_few(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream) {
+    if (!rows_few_takes(p)) return TANNIC_UNSUPPORTED_DTYPE;
+    if (dtype == TANNIC_FLOAT16) return run_rows_few<f16>(p, a, b, c, stream);
+    if (dtype == TANNIC_BFLOAT16) return run_rows_few<bf16>(p, a, b, c, stream);
+    return TANNIC_UNSUPPORTED_DTYPE;
+}
+
 // Which of the kernels takes a product: its lanes side by side along the columns, or 0 where none does.
 //
 // They are taken where the tiles would read an operand at any alignment (K, or a pitch or an address of x or W, that no 16 bytes divide)
