@@ -28,10 +28,16 @@ class DeviceLibrary:
         self.path = path
         self.cdll = C.CDLL(path)
         self.kernels = {}
+        # The same entry points for the operator interface, which keeps a tensor's descriptor as its bytes and a stream as its number: ctypes
+        # hands both on without building an object (one of 176 bytes each per call before; a descriptor is never written to).
+        self.calls = {}
         for name, (res, args) in abi.kernel_signatures(with_stream=True).items():
             fn = getattr(self.cdll, "tannic_hip_" + name)
             fn.restype, fn.argtypes = res, args
             self.kernels[name] = fn
+            call = self.cdll["tannic_hip_" + name]
+            call.restype, call.argtypes = res, [C.c_char_p if a is abi.TP else C.c_size_t if a is abi.stream_t else a for a in args]
+            self.calls[name] = call
         for name, (res, args) in abi.runtime_signatures().items():
             fn = getattr(self.cdll, "tannic_hip_" + name)
             fn.restype, fn.argtypes = res, args

@@ -35,10 +35,15 @@ class TannicError(RuntimeError):
 
 def _resolve(*tensors):
     """``resolve_two_environment`` / ``resolve_three_environment`` (``src/bindings.cpp:118-188``)."""
-    if len(tensors) == 2:
-        first, second = tensors[0].buffer, tensors[1].buffer
-        if first is not None and second is not None and first.environment is second.environment:
-            return first.environment
+    first = tensors[0].buffer
+    if first is not None:
+        # (the operands of a program share one Device object)
+        env = first.environment
+        for t in tensors:
+            if t.buffer is None or t.buffer.environment is not env:
+                break
+        else:
+            return env
     envs = [t.environment for t in tensors]
     devices = [e for e in envs if isinstance(e, Device)]
     if not devices:
@@ -50,19 +55,25 @@ def _resolve(*tensors):
 
 def _call(name, env, sources, dst, extra=(), scalar=None):
     """One backend call in the order the ABI expects: sources, [scalar], dst, [stream], extra."""
-    args = [s.reference() for s in sources]
-    if scalar is not None:
-        args.append(C.byref(scalar))
-    args.append(dst.reference())
     if env.kind == abi.DEVICE:
         lib = library()
-        status = lib.kernels[name](*args, env.stream(), *extra)
+        call = lib.calls[name]
+        if scalar is not None:
+            status = call(*[s.packed() for s in sources], C.byref(scalar), dst.packed(), env.stream_number(), *extra)
+        elif len(sources) == 2:
+            status = call(sources[0].packed(), sources[1].packed(), dst.packed(), env.stream_number(), *extra)
+        else:
+            status = call(*[s.packed() for s in sources], dst.packed(), env.stream_number(), *extra)
         if status == abi.SUCCESS:
             return dst
         detail = lib.error_message() if status == abi.ERROR else ""
     else:
         if _host_functions is None:
             raise BackendError(f"{name}: operands are on the host and tannic_amd holds device kernels only")
+        args = [s.reference() for s in sources]
+        if scalar is not None:
+            args.append(C.byref(scalar))
+        args.append(dst.reference())
         status = _host_functions[name](*args, *extra)
         detail = ""
     if status != abi.SUCCESS:
@@ -327,13 +338,26 @@ def _composition_dtype(a, b):
 
 def matmul(a, b):
     """``matmul(A, B)``: batch dims broadcast, transposed views reach the kernel as strides."""
+    key = (a.shape, b.shape, a.dtype, b.dtype)
+    rule = _PRODUCTS.get(key)
+    if rule is None:
+        rule = _product_rule(a, b)
+        if len(_PRODUCTS) > 4096:
+            _PRODUCTS.clear()
+        _PRODUCTS[key] = rule
+    env = _resolve(a, b)
+    return _call("gemm", env, (a, b), Tensor.fresh(rule[0], rule[1], env))
+
+
+_PRODUCTS = {}    # (shape, shape, dtype, dtype) -> dtype and shape of the product: the pairs of a program recur
+
+
+def _product_rule(a, b):
     if a.rank < 2 or b.rank < 2:
         raise TannicError("Inputs must have rank >= 2")
     if a.shape[-1] != b.shape[-2]:
         raise TannicError("Inner dimensions must match for matmul")
-    shape = broadcast(a.shape[:-2], b.shape[:-2]) + (a.shape[-2], b.shape[-1])
-    env = _resolve(a, b)
-    return _call("gemm", env, [a, b], _new(_composition_dtype(a.dtype, b.dtype), shape, env))
+    return _composition_dtype(a.dtype, b.dtype), broadcast(a.shape[:-2], b.shape[:-2]) + (a.shape[-2], b.shape[-1])
 
 
 # ---- convolution (include/tannic/convolutions.hpp:71-120) -----------------
@@ -341,8 +365,27 @@ def _pair(v):
     return (v, v) if isinstance(v, int) else tuple(v)
 
 
+_CONVOLUTIONS = {}    # (shapes, dtypes, stride, padding) -> shape of the result, padding and stride as the backend takes them
+
+
 def convolve2d(signal, kernel, bias=None, stride=1, padding=0):
     stride, padding = _pair(stride), _pair(padding)
+    key = (signal.shape, kernel.shape, None if bias is None else bias.shape, signal.dtype, kernel.dtype, None if bias is None else bias.dtype, stride, padding)
+    rule = _CONVOLUTIONS.get(key)
+    if rule is None:
+        rule = _convolution_rule(signal, kernel, bias, stride, padding)
+        if len(_CONVOLUTIONS) > 4096:
+            _CONVOLUTIONS.clear()
+        _CONVOLUTIONS[key] = rule
+    shape, extra = rule
+    if bias is None:
+        env = _resolve(signal, kernel)
+        return _call("conv2d", env, (signal, kernel), Tensor.fresh(signal.dtype, shape, env), extra)
+    env = _resolve(signal, kernel, bias)
+    return _call("conv2d_biased", env, (signal, kernel, bias), Tensor.fresh(signal.dtype, shape, env), extra)
+
+
+def _convolution_rule(signal, kernel, bias, stride, padding):
     if signal.dtype is not kernel.dtype or (bias is not None and bias.dtype is not signal.dtype):
         raise TannicError("Dtypes must match in convolutions.")
     if signal.rank != 4 or kernel.rank != 4:
@@ -354,10 +397,7 @@ def convolve2d(signal, kernel, bias=None, stride=1, padding=0):
     if bias is not None and (bias.rank != 1 or bias.shape[0] != c_out):
         raise TannicError("Bias shape must be [C_out].")
     shape = (n, c_out, (h + 2 * padding[0] - kh) // stride[0] + 1, (w + 2 * padding[1] - kw) // stride[1] + 1)
-    operands = [signal, kernel] + ([bias] if bias is not None else [])
-    env = _resolve(*operands)
-    extra = (abi.SIZE2(*padding), abi.SIZE2(*stride))
-    return _call("conv2d_biased" if bias is not None else "conv2d", env, operands, _new(signal.dtype, shape, env), extra=extra)
+    return shape, (abi.SIZE2(*padding), abi.SIZE2(*stride))
 
 
 def convolve1d(signal, kernel, stride=1, padding=0):

@@ -21,6 +21,7 @@ class Host:
     """Pageable host memory (``include/tannic/resources.hpp``, ``Host``)."""
 
     kind = abi.HOST
+    key = (abi.HOST, -1)
 
     def __eq__(self, other):
         return isinstance(other, Host)
@@ -33,6 +34,7 @@ class Host:
 
 
 _STREAMS = {}      # device id -> its stream (see Device.stream)
+_STREAM_NUMBERS = {}
 
 
 class Device:
@@ -46,6 +48,7 @@ class Device:
         if id < 0 or id >= count:
             raise IndexError("Invalid device ID")
         self.id = id
+        self.key = (abi.DEVICE, id)
         self._structure = abi.device_t(id)
         self.reference = C.byref(self._structure)    # what every backend call on this device passes
 
@@ -62,7 +65,13 @@ class Device:
             stream = lib.pop_stream(self.reference)
             lib.put_stream(self.reference, stream)
             _STREAMS[self.id] = stream
+            _STREAM_NUMBERS[self.id] = stream.address
         return stream
+
+    def stream_number(self):
+        """The same stream as the number a call of ``DeviceLibrary.calls`` takes."""
+        number = _STREAM_NUMBERS.get(self.id)
+        return self.stream().address if number is None else number
 
     def __eq__(self, other):
         return isinstance(other, Device) and other.id == self.id
@@ -78,15 +87,16 @@ class Buffer:
     """Owns one allocation; device memory goes back through ``deallocate``
     (``src/buffer.cpp:37-43`` -> ``Device::deallocate`` -> ``cuda::deallocate``)."""
 
+    __slots__ = ("nbytes", "environment", "array", "address", "__weakref__")
+
     def __init__(self, nbytes, environment):
         self.nbytes = nbytes
         self.environment = environment
         self.array, self.address = None, 0     # (what __del__ looks at, should the allocation raise)
         if environment.kind == abi.DEVICE:
-            self.address = library().allocate(environment.reference, max(nbytes, 1))
+            self.address = library().allocate(environment.reference, nbytes or 1)
             if not self.address:
                 raise BackendError("device allocation failed: " + library().error_message())
-            self.array = None
         else:
             self.array = np.zeros(max(nbytes, 1), dtype=np.uint8)
             self.address = self.array.ctypes.data
@@ -106,7 +116,9 @@ _PAD = [(0,) * (abi.DIMENSIONS - r) for r in range(abi.DIMENSIONS + 1)]
 assert _TENSOR_T.size == C.sizeof(abi.tensor_t)
 
 
+_ADDRESS = struct.Struct("<Q").pack
 _IMAGES = {}      # (shape, strides, dtype, environment) -> packed tensor_t without the address
+_FRESH = {}       # (shape, dtype, environment) -> what a new contiguous tensor is made of: strides, elements, bytes, packed tensor_t behind its address
 _STRIDES = {}     # shape -> (contiguous strides, number of elements); shapes recur, the table stays small
 
 
@@ -164,10 +176,21 @@ class Tensor:
         t = cls.__new__(cls)
         t.dtype = dtype
         t.shape = shape = tuple(shape)
-        t.strides, t.nelements = _shape_facts(shape)
         t.offset = 0
         t._contiguous = True
-        t.buffer = Buffer(types.nbytesof(dtype, t.nelements), environment)
+        key = (shape, dtype, environment.key)
+        facts = _FRESH.get(key)
+        if facts is None:
+            t.strides, t.nelements = _shape_facts(shape)
+            nbytes = types.nbytesof(dtype, t.nelements)
+            t.buffer = Buffer(nbytes, environment)
+            if len(_FRESH) > 4096:
+                _FRESH.clear()
+            _FRESH[key] = (t.strides, t.nelements, nbytes, t._image()[8:])
+            return t
+        t.strides, t.nelements, nbytes, tail = facts
+        t.buffer = buffer = Buffer(nbytes, environment)
+        t._packed = _ADDRESS(buffer.address) + tail
         return t
 
     def is_singleton(self):
@@ -193,6 +216,8 @@ class Tensor:
         if self.strides != contiguous_strides(self.shape) and data is not None:
             raise ValueError("initialize with data needs a contiguous tensor")
         self.buffer = Buffer(self.nbytes + self.offset, environment)
+        for cached in ("_descriptor", "_reference", "_packed"):    # (of a buffer before)
+            self.__dict__.pop(cached, None)
         if data is not None:
             self.write(data)
         return self
@@ -268,15 +293,11 @@ class Tensor:
         return out
 
     # ---- the descriptor handed to the backend ---------------------------
-    def descriptor(self):
-        """The ``tensor_t`` of this view; built once (a view's shape, strides, offset and buffer never change)."""
-        cached = self.__dict__.get("_descriptor")
-        if cached is not None:
-            return cached
-        # One packed image of ``tensor_t`` per (shape, strides, dtype, environment), kept; a tensor's own descriptor is a copy
-        # of it with the address filled in (offsets checked against the structure when ``abi`` is imported).
+    def _image(self):
+        """The packed ``tensor_t`` of this view without its address, one per (shape, strides, dtype, environment) (offsets checked against the
+        structure when ``abi`` is imported)."""
         env = self.buffer.environment
-        key = (self.shape, self.strides, self.dtype.code, env.kind, env.id if env.kind == abi.DEVICE else -1)
+        key = (self.shape, self.strides, self.dtype.code, env.key)
         image = _IMAGES.get(key)
         if image is None:
             rank = len(self.shape)
@@ -286,8 +307,23 @@ class Tensor:
             if len(_IMAGES) > 4096:
                 _IMAGES.clear()
             image = _IMAGES[key] = _TENSOR_T.pack(0, rank, *self.shape, *pad, *self.strides, *pad, self.dtype.code, env.kind, resource, self.nelements, layout)
-        t = abi.tensor_t.from_buffer_copy(image)
-        t.address = self.buffer.address + self.offset
+        return image
+
+    def packed(self):
+        """The ``tensor_t`` of this view as its bytes, what a call of ``DeviceLibrary.calls`` takes; built once (a view's shape, strides,
+        offset and buffer never change)."""
+        try:
+            return self._packed
+        except AttributeError:
+            self._packed = p = _ADDRESS(self.buffer.address + self.offset) + self._image()[8:]
+            return p
+
+    def descriptor(self):
+        """The ``tensor_t`` of this view as a structure; built once."""
+        cached = self.__dict__.get("_descriptor")
+        if cached is not None:
+            return cached
+        t = abi.tensor_t.from_buffer_copy(self.packed())
         self._descriptor = t
         self._reference = C.byref(t)
         return t
