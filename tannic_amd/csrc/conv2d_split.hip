@@ -655,8 +655,10 @@ int conv2d_split(const ConvProblem& p, int dtype, const void* x, const void* w, 
     // (a block's weights are loaded a tap ahead, the last ones behind the end)
     const size_t plane_bytes = (static_cast<size_t>(fragments) + 2) * 3 * 1024, largest_bytes = (static_cast<size_t>(fragments) * 4 + 255) / 256 * 256;
     char* scratch = nullptr;
-    if (scratch_acquire(reinterpret_cast<void**>(&scratch), plane_bytes + largest_bytes + (q.splits > 1 ? static_cast<size_t>(results) * q.splits * 4 : 0), stream) != TANNIC_SUCCESS)
-        return TANNIC_ERROR;
+    if (scratch_acquire(reinterpret_cast<void**>(&scratch), plane_bytes + largest_bytes + (q.splits > 1 ? static_cast<size_t>(results) * q.splits * 4 : 0), stream) != TANNIC_SUCCESS) {
+        (void)hipGetLastError();
+        return TANNIC_UNSUPPORTED_DTYPE;      // no memory for the split weights: conv2d_f32 needs none, or less
+    }
     q.weight_bytes = static_cast<uint32_t>(plane_bytes);
     uint4s* planes = reinterpret_cast<uint4s*>(scratch);
     uint32_t* largest = reinterpret_cast<uint32_t*>(scratch + plane_bytes);
