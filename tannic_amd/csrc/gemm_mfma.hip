@@ -612,15 +612,19 @@ int run16_split(const GemmProblem& p, bool ak, bool bk, uint32_t splits, const v
         }
         sk.partials = static_cast<float*>(workspace->base);
     } else if (scratch_acquire(reinterpret_cast<void**>(&sk.partials), bytes, stream) != TANNIC_SUCCESS) {
-        return TANNIC_ERROR;
+        if (BM != 256) return TANNIC_ERROR;
+        (void)hipGetLastError();
+        return TANNIC_UNSUPPORTED_DTYPE;
     }
     int status = TANNIC_UNSUPPORTED_DTYPE;
-    if constexpr (sizeof(T) == 2 && (BM == 128 || BM == 64)) status = gemm16_dtl_split<T>(p, BM, sk.splits, sk.k_chunk, sk.partials, a, b, stream);
-    if (status != TANNIC_UNSUPPORTED_DTYPE) {}
-    else if (ak && bk) status = launch16<T, BM, BN, 2, true, true, true>(p, a, b, c, stream, sk);
-    else if (ak) status = launch16<T, BM, BN, 2, true, false, true>(p, a, b, c, stream, sk);
-    else if (bk) status = launch16<T, BM, BN, 2, false, true, true>(p, a, b, c, stream, sk);
-    else status = launch16<T, BM, BN, 2, false, false, true>(p, a, b, c, stream, sk);
+    if constexpr (sizeof(T) == 2 && (BM == 128 || BM == 64 || BM == 256)) status = gemm16_dtl_split<T>(p, BM, sk.splits, sk.k_chunk, sk.partials, a, b, stream);
+    if constexpr (BM != 256) {                         // (256 rows: by direct loads only)
+        if (status != TANNIC_UNSUPPORTED_DTYPE) {}
+        else if (ak && bk) status = launch16<T, BM, BN, 2, true, true, true>(p, a, b, c, stream, sk);
+        else if (ak) status = launch16<T, BM, BN, 2, true, false, true>(p, a, b, c, stream, sk);
+        else if (bk) status = launch16<T, BM, BN, 2, false, true, true>(p, a, b, c, stream, sk);
+        else status = launch16<T, BM, BN, 2, false, false, true>(p, a, b, c, stream, sk);
+    }
     if (status == TANNIC_SUCCESS) {
         const uint32_t total = static_cast<uint32_t>(rows * quads_per_row);
         hipLaunchKernelGGL((gemm_split_reduce_kernel<T>), dim3((total + 255) / 256), dim3(256), 0, stream, sk.partials, static_cast<T*>(c), p, sk.splits,
@@ -634,6 +638,15 @@ int run16_split(const GemmProblem& p, bool ak, bool bk, uint32_t splits, const v
 // What a 256-row tile narrower than 256 columns loses per column it is narrower (operand bytes per multiply-add), as a
 // fraction of its time.
 constexpr double kNarrowTilePenalty = 0.001;
+// A step of a 128 x 96 tile, of one of 128 x 128: what it loses in operand bytes per multiply-add it more than gets back where tiles 128 wide
+// leave compute units idle (bf16, every W from memory, us on 128 wide / 96: 512 x 6144 x 4096 44 / 40, 512 x 5120 x 5120 54 / 48,
+// 768 x 3072 x 3072 34 / 31.4).  One round of them only, a long K, and more than 96 of them (the register-staged 64-row tiles are the better
+// ones under a short K or with few tiles: 256 x 7168 x 1536 19.2 / 20.1, 256 x 4096 x 2048 19.6 / 20.5; 512 x 4096 x 2048 21.9 / 20.9).
+constexpr double kNarrowStep = 0.85;
+// What of K a block with 256 rows gets at least where K is shared: half as many tiles, twice as many shares as with 128 rows, so the operands
+// cross the L2s less often and more partial sums are added (bf16, us with 128 rows / 256: 512 x 4096 x 14336 87 / 77, 768 x 7168 x 11008 183 / 147,
+// 1024 x 2048 x 16384 83 / 73; with shares of 2048 400 x 11008 x 8192 113 / 117, 400 x 4096 x 8192 44.1 / 44.5).
+constexpr uint32_t kTallShare = 2560;
 
 template <class T>
 int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream, const GemmWorkspace* workspace) {
@@ -717,8 +730,11 @@ int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream
     const bool tall = p.M > 64;
     const double steps_all = (p.K + 63) / 64;
     double best_cost = 1e30;
-    int best_bm = tall ? 128 : 64;
+    int best_bm = tall ? 128 : 64, best_bn = 128;
     uint32_t best_splits = 1;
+    // (what the direct-to-LDS tiles take, gemm16_dtl)
+    const bool direct = sizeof(T) == 2 && ak && bk && p.K % 64 == 0 && p.a_rs >= static_cast<int64_t>(p.K) && p.a_rs < (1 << 22) && p.b_cs >= static_cast<int64_t>(p.K) &&
+                        p.b_cs < (1 << 22);
     // (fp32: equal costs go to the 128-row tile, which is tried first)
     const int heights[3] = {sizeof(T) == 4 ? 128 : 256, sizeof(T) == 4 ? 256 : 128, 64};
     // Under a short K a block's start and end count: about 2 us for the 128- and 256-row tiles and 0.7 us for the 64-row
@@ -729,7 +745,9 @@ int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream
         const double block_fixed = short_k ? (bm == 64 ? 0.7 : 2.0) : 0.0;
         const uint64_t tiles = static_cast<uint64_t>((p.M + bm - 1) / bm) * ((p.N + 127) / 128) * p.batches;
         for (uint32_t splits : {1u, 2u, 4u, 8u, 16u}) {
-            if (splits > 1 && (bm == 256 || splits > p.K / (sizeof(T) == 4 ? 64 : 256))) break;
+            if (splits > 1 && splits > p.K / (sizeof(T) == 4 ? 64 : 256)) break;
+            // (a workspace too small for that many partial sums may hold those of the 128-row tiles)
+            if (splits > 1 && bm == 256 && (!direct || p.N % 4 != 0 || p.K / splits < kTallShare || (workspace && static_cast<uint64_t>(splits) * p.batches * p.M * p.N * sizeof(float) > workspace->bytes))) break;
             const double blocks = static_cast<double>(tiles) * splits;
             const double rounds = static_cast<double>((static_cast<uint64_t>(blocks) + 255) / 256);
             // a step costs more the more compute units pull operands through the L2s at the same time
@@ -746,13 +764,26 @@ int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream
             if (cost < best_cost) { best_cost = cost; best_bm = bm; best_splits = splits; }
         }
     }
+    if (direct && tall && p.K >= (best_bm == 64 ? 2048 : 1536)) {
+        const uint64_t tiles = static_cast<uint64_t>((p.M + 127) / 128) * ((p.N + 95) / 96) * p.batches;
+        const double cost = steps_all * kNarrowStep * (0.375 + 0.175 * (tiles / 256.0)) + 5.0;
+        if (tiles <= 256 && tiles > 96 && cost < best_cost) { best_cost = cost; best_bm = 128; best_bn = 96; best_splits = 1; }
+    }
     if (best_splits > 1) {
+        if constexpr (sizeof(T) == 2) {
+            if (best_bm == 256) {
+                const int rc = run16_split<T, 256>(p, ak, bk, best_splits, a, b, c, stream, workspace);
+                if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
+                best_bm = 128, best_splits /= 2;      // no memory for so many partial sums: as many blocks with half as many
+                if (best_splits == 1) return gemm16_dtl<T>(p, 128, 128, a, b, c, stream);
+            }
+        }
         if (best_bm == 128) return run16_split<T, 128>(p, ak, bk, best_splits, a, b, c, stream, workspace);
         return run16_split<T, 64>(p, ak, bk, best_splits, a, b, c, stream, workspace);
     }
     if constexpr (sizeof(T) == 2) {
         if (best_bm >= 128) {
-            const int rc = gemm16_dtl<T>(p, best_bm, 128, a, b, c, stream);
+            const int rc = gemm16_dtl<T>(p, best_bm, best_bn, a, b, c, stream);
             if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
         }
     }
