@@ -62,6 +62,7 @@ UNITS = [
     ("conv2d_pointwise.hip", "conv2d_pointwise.o", []),
     ("conv2d_stem.hip", "conv2d_stem.o", []),
     ("conv2d_split.hip", "conv2d_split.o", []),
+    ("conv2d_batch3.hip", "conv2d_batch3.o", []),
     ("conv2d_f32.hip", "conv2d_f32.o", []),
     ("conv2d_gather32.hip", "conv2d_gather32.o", []),
     ("conv2d_unfold.hip", "conv2d_unfold.o", []),

@@ -96,7 +96,8 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     p.bs = bias ? bias->strides.sizes[0] : 0;
     if (plan) {
         for (int i = 0; i < kConvPlanValues; ++i) plan[i] = 0;
-        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan)) conv2d_few_plan(p, x->dtype, plan);
+        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_few_plan(p, x->dtype, plan))
+            conv2d_batch3_plan(p, x->dtype, x->address, w->address, plan);
         return TANNIC_SUCCESS;
     }
     const void* pb = bias ? bias->address : nullptr;
@@ -111,6 +112,9 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     status = conv2d_f32(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     status = conv2d_few(p, x->dtype, x->address, w->address, pb, y->address, s);
+    if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
+    // a batch of small maps under many channels, 16-bit 3x3 (what it leaves to the kernels below: plan_batch3)
+    status = conv2d_batch3(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     if (pointwise) status = conv2d_k1(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (pointwise && status == TANNIC_UNSUPPORTED_DTYPE) status = conv2d_pointwise(p, x->dtype, x->address, w->address, pb, y->address, s);

@@ -20,8 +20,9 @@ struct ConvProblem {
 // The plan of the kernel that would take a problem, for tannic_hip_conv2d_plan: which of the kernels below, then its parameters and
 // the parts of its plan that say where a tile's windows lie (named in include/tannic_hip.h).
 constexpr int kConvPlanValues = 20;
-// true where the kernel takes the problem (conv2d_split, conv2d_f32 and conv2d_few launch what these report)
+// true where the kernel takes the problem (conv2d_split, conv2d_f32, conv2d_few and conv2d_batch3 launch what these report)
 bool conv2d_split_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
+bool conv2d_batch3_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_f32_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValues]);
 
@@ -37,6 +38,8 @@ int conv2d_resident(const ConvProblem& p, int dtype, const void* x, const void* 
 int conv2d_patch(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 // fp32 1x1 (from 140 channels on) and 3x3 on the 16-bit matrix pipe, every value as three bfloat16 values
 int conv2d_split(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
+// 16-bit 3x3, a batch of small maps under many channels, over the flattened batch
+int conv2d_batch3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 // the time (us) that conv2d_f32 is expected to take; negative where it does not take the problem
 double conv2d_f32_expected(const ConvProblem& p, int dtype, const void* x, const void* w);
 int conv2d_f32(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
