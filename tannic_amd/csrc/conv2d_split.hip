@@ -597,6 +597,9 @@ static int plan_split(const ConvProblem& p, int dtype, const void* x, const void
     if (p.xs[3] != 1 || p.xs[0] < 0 || p.xs[1] < 0 || p.xs[2] < 0 || p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO) || reinterpret_cast<uintptr_t>(x) % 4 != 0) return -1;
     if (p.KH == 1 && (p.pad_h || p.pad_w)) return -1;
     if (K * p.O * 4 >= (1ull << 31) || pixels >= (1ull << 28) || pixels * p.O >= (1ull << 31)) return -1;
+    // what is addressed is the weights as parts, six bytes a value with both kinds of channels rounded up: 32-bit byte offsets, two fragments ahead
+    const uint64_t fragments = (static_cast<uint64_t>(p.O) + 15) / 16 * ((static_cast<uint64_t>(p.C) + kSplitChannels - 1) / kSplitChannels) * (p.KH * p.KW);
+    if ((fragments + 2) * 3 * 1024 >= (1ull << 32)) return -1;
     // (few channels are a short K: what a tile starts and ends with counts, and 1x1 kernels are bound by their tensors; small problems by launches)
     if (p.KH == 1 ? p.C < (p.O >= 128 ? 100u : 140u) : p.C < 32) return -1;
     if (2.0 * K * p.O * pixels < 1.2e9) return -1;

@@ -93,6 +93,21 @@ def test_windows_lie_in_their_planes():
     assert taken >= 60, taken
 
 
+# channels in that are rounded up to whole chunks, and the output channels from which their three parts take more bytes than 32 bits count
+@pytest.mark.parametrize("x,beyond,neighbour", [((1, 68, 30, 30), 828497, True), ((1, 44, 18, 18), 1242753, True), ((22, 1774052, 7, 7), 33, False)], ids=["68", "44", "long"])
+def test_parts_of_the_weights_are_counted_in_32_bits(x, beyond, neighbour):
+    """(Below, the problem runs here; the longest K does not for another reason, and all go on to the kernel of the fp32 pipe.)"""
+    def parts(o):
+        return ((o + 15) // 16 * ((x[1] + 31) // 32) * 9 + 2) * 3 * 1024
+    assert parts(beyond - 1) < 2 ** 32 <= parts(beyond)
+    assert (split_plan(x, (beyond - 1, x[1], 3, 3), (1, 1), (1, 1)) is not None) == neighbour
+    w = (beyond, x[1], 3, 3)
+    assert split_plan(x, w, (1, 1), (1, 1)) is None
+    out = (C.c_uint32 * 20)()
+    args = [C.byref(descriptor("float32", s)) for s in (x, w, out_shape(x, w, (1, 1), (1, 1)))]
+    assert ta.library().conv2d_plan(*args, abi.SIZE2(1, 1), abi.SIZE2(1, 1), out) == abi.SUCCESS and out[0] == 1
+
+
 def run(xs, ws, stride, padding, device, change=lambda x, w: None):
     rng = np.random.default_rng(21)
     x, w, b = (rng.standard_normal(s, dtype=np.float32) for s in (xs, ws, ws[:1]))
