@@ -389,6 +389,9 @@ static int plan_batch3(const ConvProblem& p, int dtype, const void* x, const voi
     if (p.ws[3] != 1 || p.ws[2] != 3 || p.ws[1] != 9 || p.ws[0] != static_cast<int64_t>(K) || reinterpret_cast<uintptr_t>(w) % 2 != 0) return -1;
     if (p.xs[3] != 1 || p.xs[0] < 0 || p.xs[1] < 0 || p.xs[2] < 0 || p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO) || reinterpret_cast<uintptr_t>(x) % 2 != 0) return -1;
     if (K * p.O * 2 >= (1ull << 30) || pixels >= (1ull << 28) || pixels * p.O >= (1ull << 31)) return -1;
+    // (the ordered weights, both kinds of channels rounded up and a chunk ahead, are addressed by 32-bit byte offsets)
+    const uint64_t weight_blocks = (static_cast<uint64_t>(p.O) + 15) / 16 * ((static_cast<uint64_t>(p.C) + kBatch3Channels - 1) / kBatch3Channels);
+    if ((weight_blocks + 1) * kBatch3Taps * 1024 >= (1ull << 32)) return -1;
     // Where it is the faster one (fp16, us before / here, weights' kernel included; before: the patch kernel, or the unfolded batch as a product for
     // few pixels an image and for channels that are not whole chunks):
     //  * small problems are launches (256 -> 256, six images of 12 x 12 18.6 / 19.1, 128 -> 128, six of 24 x 24 16.2 / 13.4); 64 channels are two

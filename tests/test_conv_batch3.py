@@ -60,6 +60,19 @@ def test_variant_is_the_plan_of_its_shape(variant):
     assert q is not None and tuple(q[n] for n in NAMES[1:4]) == variant
 
 
+def test_ordered_weights_are_counted_in_32_bits():
+    """One output channel takes the room of sixteen: a signal of one value seen as any number of channels and images."""
+    def taken(channels):
+        x, w, y = (descriptor("float16", s) for s in ((200000, channels, 11, 11), (1, channels, 3, 3), (200000, 1, 11, 11)))
+        for d in range(3):
+            x.strides.sizes[d] = 0
+        out = (C.c_uint32 * 20)()
+        assert ta.library().conv2d_plan(*(C.byref(t) for t in (x, w, y)), abi.SIZE2(1, 1), abi.SIZE2(1, 1), out) == abi.SUCCESS
+        return out[0] == 4
+    fits = ((2 ** 32 - 1) // (9 * 1024) - 1) * 32
+    assert taken(fits) and not taken(fits + 1)
+
+
 def test_windows_lie_in_their_planes():
     """Every tap of every pixel of random problems: the place in the tile's plane holds the signal's value there, or a zero of the padding."""
     rng, taken = random.Random(5), 0
