@@ -15,9 +15,12 @@
 //    wavefront, and writes 16 bytes to each of three planes of 32 channels.  So nothing is asked of widths, alignments, strides or channels.
 //  * A wavefront's tile is 32 output channels by 16 PT pixels of the flattened batch; WO wavefronts of a block's four lie along the
 //    channels.  A tap of 32 channels is 12 PT MFMAs for six loads of weights and 3 PT reads of LDS.
-//  * Where a part cannot hold what it should (infinities and NaNs, values that round beyond the largest bfloat16, tiles whose largest value
-//    is below 2^-100 and whose low parts would be denormal), the block does its tile over again in fp32, straight from memory: every
-//    value's magnitude is looked at while it is split.
+//  * Both operands are split 2^24 times as large as they are, so that the last bit of the smallest fp32 value (2^-149) is a normal bfloat16: no
+//    part of any value is denormal, whatever lies beside it, and the sums are 2^48 times the results (powers of two change no rounding).
+//    What that puts out of range (values from 2^103 on, results from 2^79 on), infinities and NaNs leave a sum that is not finite: the wavefront
+//    does those sixteen pixels over again in fp32, straight from memory, thirty-six products at a time.  (Slow, and only there: 128 -> 256 3x3 over
+//    20 x 20, sixteen images, 35 us; one infinity 178, one in every ninth value of a channel 320; 52 on the fp32 pipe.  Weights or signals of 1e-37
+//    beside ordinary ones 1.1e-7 of their own results, 1.5e-7 on the fp32 pipe.)
 // With few tiles the channels are shared between `splits` blocks per tile, partial sums in fp32, added in split order by a second kernel.
 // Measured, 53 convolutions of a ResNet-50 and their additions, batch 32: 3351 -> 2777 us (the layers: plan_split).
 // What is left: the weights' kernel (3 - 5 us of a layer's 30 - 50), a block's start and end (some 9 us), the last round of tiles.
@@ -35,10 +38,8 @@ typedef unsigned short ushort2s __attribute__((ext_vector_type(2)));
 constexpr int kSplitThreads = 256;
 constexpr uint32_t kSplitOutside = 0x80000000u;   // byte offset no buffer reaches: loads zero
 constexpr uint32_t kSplitChannels = 32;           // per chunk: the K of one MFMA
-// High parts (bfloat16 magnitudes) from here on are infinities, NaNs, or values that round beyond the largest bfloat16 ...
-constexpr uint32_t kSplitLargest = 0x7F80;
-// ... and a tile whose largest value is below 2^-100 has low parts below the smallest bfloat16: both are done over in fp32
-constexpr uint32_t kSplitSmallest = (127 - 100) << 7;
+// the operands are split so many times as large as they are, and the sums brought back by the square of it
+constexpr float kSplitUp = 0x1p24f, kSplitSumUp = 0x1p48f, kSplitSumDown = 0x1p-48f;
 
 // The high products of so many chunks of a 1x1 kernel (the nine taps of one chunk of a 3x3 kernel) are one chain of additions, the chains'
 // sums added to a third set of accumulators.  The chain rounds as much as the square root of its length (K = 1024, 1024 -> 256 over 14 x 14:
@@ -76,30 +77,16 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t part[3]) {
     }
 }
 
-// the larger of two pairs of bfloat16 magnitudes, half by half
-__device__ __forceinline__ uint32_t split_larger(uint32_t largest, uint32_t high_part) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushort2s, largest), __builtin_bit_cast(ushort2s, high_part & 0x7FFF7FFFu)));
-}
-__device__ inline uint32_t split_largest_of_wave(uint32_t pair) {
-    uint32_t v = (pair & 0xFFFF) > (pair >> 16) ? pair & 0xFFFF : pair >> 16;
-#pragma unroll
-    for (int by = 32; by > 0; by /= 2) {
-        const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), by));
-        v = v > other ? v : other;
-    }
-    return v;
-}
-
 __device__ __forceinline__ float4s split_mfma(const uint4s& a, const uint4s& b, const float4s& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(split8, a), __builtin_bit_cast(split8, b), c, 0, 0, 0);
 }
 
-// The weights as MFMA operands: [16 channels out][32 channels in][tap][part][lane][8], and the largest magnitude of each such fragment.
+// The weights as MFMA operands: [16 channels out][32 channels in][tap][part][lane][8].
 // A block per 16 x 32 channels, whose weights are sixteen runs of 32 TAPS floats, through LDS; a wavefront per tap (1x1: four, of which
 // one goes on), as there is nothing here but the latency of one load, one pass through LDS and one store.
 template <int TAPS> constexpr int split_weight_threads = TAPS == 1 ? 256 : 64 * TAPS;
 template <int TAPS>
-__global__ __launch_bounds__(split_weight_threads<TAPS>) void conv2d_split_weights_kernel(const float* w, uint4s* planes, uint32_t* largest, uint32_t O, uint32_t C, FastDiv div_chunks) {
+__global__ __launch_bounds__(split_weight_threads<TAPS>) void conv2d_split_weights_kernel(const float* w, uint4s* planes, uint32_t O, uint32_t C, FastDiv div_chunks) {
     constexpr uint32_t RUN = kSplitChannels * TAPS, PITCH = RUN + 1, THREADS = split_weight_threads<TAPS>;
     __shared__ float held[16 * PITCH];
     const uint32_t tap = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -120,23 +107,18 @@ __global__ __launch_bounds__(split_weight_threads<TAPS>) void conv2d_split_weigh
     __syncthreads();
     if (tap >= TAPS) return;
     const float* mine = held + lane % 16 * PITCH + lane / 16 * (8 * TAPS) + tap;
-    uint32_t part[4][3], most = 0;
+    uint32_t part[4][3];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        split_pair(mine[2 * e * TAPS], mine[(2 * e + 1) * TAPS], part[e]);
-        most = split_larger(most, part[e][0]);
-    }
+    for (int e = 0; e < 4; ++e) split_pair(mine[2 * e * TAPS] * kSplitUp, mine[(2 * e + 1) * TAPS] * kSplitUp, part[e]);
     const uint32_t fragment = blockIdx.x * TAPS + tap;
 #pragma unroll
     for (int i = 0; i < 3; ++i) planes[(fragment * 3 + i) * 64 + lane] = uint4s{part[0][i], part[1][i], part[2][i], part[3][i]};
-    most = split_largest_of_wave(most);
-    if (lane == 0) largest[fragment] = most;
 }
 
 // KS: the kernel's side; PT: 16-pixel tiles per wavefront; WO: wavefronts along the output channels (32 each), the others along the
 // pixels; NL: places of a plane per lane.
 template <int KS, int PT, int WO, int NL>
-__global__ __launch_bounds__(kSplitThreads, NL <= 3 && (KS == 1 || PT <= 2) ? 2 : 1) void conv2d_split_kernel(const float* x, const float* w, const uint4s* planes, const uint32_t* largest, const float* bias, float* y,
+__global__ __launch_bounds__(kSplitThreads, NL <= 3 && (KS == 1 || PT <= 2) ? 2 : 1) void conv2d_split_kernel(const float* x, const float* w, const uint4s* planes, const float* bias, float* y,
                                                                                    float* partials, ConvProblem p, SplitPlan q) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass needs the launch stub only (and loses it over the body's device-only builtins)
     constexpr int TAPS = KS * KS;
@@ -206,11 +188,8 @@ __global__ __launch_bounds__(kSplitThreads, NL <= 3 && (KS == 1 || PT <= 2) ? 2 
         }
     };
     // two of a place's eight channels, split; all eight to LDS
-    uint32_t most = 0, part[4][3];
-    auto split_two = [&](int t, int e) __attribute__((always_inline)) {
-        split_pair(held[t][2 * e], held[t][2 * e + 1], part[e]);
-        most = split_larger(most, part[e][0]);
-    };
+    uint32_t part[4][3];
+    auto split_two = [&](int t, int e) __attribute__((always_inline)) { split_pair(held[t][2 * e] * kSplitUp, held[t][2 * e + 1] * kSplitUp, part[e]); };
     const uint32_t keep_at = lds_at + lane * PLACE + wave * 16;
     auto keep = [&](int t, uint32_t stage) __attribute__((always_inline)) {
 #pragma unroll
@@ -270,7 +249,7 @@ __global__ __launch_bounds__(kSplitThreads, NL <= 3 && (KS == 1 || PT <= 2) ? 2 
     float4s high[2][PT], low[2][PT], total[2][SETTLES ? PT : 1];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const float b = start_value(i);
+        const float b = start_value(i) * kSplitSumUp;
 #pragma unroll
         for (int j = 0; j < PT; ++j) {
             high[i][j] = SETTLES ? float4s{0.0f, 0.0f, 0.0f, 0.0f} : float4s{b, b, b, b};
@@ -384,80 +363,71 @@ __global__ __launch_bounds__(kSplitThreads, NL <= 3 && (KS == 1 || PT <= 2) ? 2 
 #pragma unroll
             for (int j = 0; j < PT; ++j) window[kh][j] += turn;
     }
+    uint32_t redo = 0;       // bit j: a sum of the pixels j is not finite
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < PT; ++j) {
+        bool finite = true;
 #pragma unroll
-        for (int j = 0; j < PT; ++j) {
+        for (int i = 0; i < 2; ++i) {
             high[i][j] += low[i][j];
             if constexpr (SETTLES) high[i][j] += total[i][j];
-        }
-
-    // ---- values that have no three parts: this tile over again, in fp32 --------------------------------------
-    uint32_t most_w = 0;
-    {
-        const uint32_t fragments = (chunk1 - chunk0) * TAPS, tiles = (p.O + 15) / 16;
-        for (uint32_t i = 0; i < 2 * WO && ct * WO * 2 + i < tiles; ++i)
-            for (uint32_t f = threadIdx.x; f < fragments; f += kSplitThreads) {
-                const uint32_t v = largest[(static_cast<size_t>(ct) * WO * 2 + i) * (q.chunks * TAPS) + chunk0 * TAPS + f];
-                most_w = most_w > v ? most_w : v;
-            }
-        uint32_t* told = reinterpret_cast<uint32_t*>(split_lds);
-        most = split_largest_of_wave(most);
-        most_w = split_largest_of_wave(most_w);
-        if (lane == 0) {
-            told[wave] = most;
-            told[4 + wave] = most_w;
-        }
-        meet();
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            most = most > told[i] ? most : told[i];
-            most_w = most_w > told[4 + i] ? most_w : told[4 + i];
+            for (int v = 0; v < 4; ++v) finite = finite && __builtin_isfinite(high[i][j][v]);
+            high[i][j] *= kSplitSumDown;
         }
+        if (__builtin_amdgcn_ballot_w64(!finite)) redo |= 1u << j;
     }
-    auto beyond = [](uint32_t v) { return v >= kSplitLargest || (v != 0 && v < kSplitSmallest); };
-    if (__builtin_amdgcn_readfirstlane(beyond(most) || beyond(most_w))) {
+
+    // ---- values and sums beyond the range: these pixels over again, in fp32 --------------------------------------
+    if (redo) {
+        constexpr int CHAIN = 9;        // MFMAs of four products, the loads of all on their way together
         const uint32_t k_first = chunk0 * kSplitChannels * TAPS, k_end = (chunk1 * kSplitChannels < p.C ? chunk1 * kSplitChannels : p.C) * TAPS;
 #pragma unroll 1
         for (int j = 0; j < PT; ++j) {
+            if (!(redo >> j & 1)) continue;
             const uint32_t pixel = p0 + wave_p * (16 * PT) + j * 16 + column;
             uint32_t n, r, oh, ow;
             q.div_hw.divmod(pixel < q.pixels ? pixel : q.pixels - 1, n, r);
             q.div_wo.divmod(r, oh, ow);
             const float* from_image = x + static_cast<int64_t>(n) * p.xs[0];
-            float4s sum[2], all[2];
+            float4s all[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const float b = start_value(i);
                 all[i] = float4s{b, b, b, b};
-                sum[i] = float4s{0.0f, 0.0f, 0.0f, 0.0f};
             }
-            uint32_t chained = 0;
-            for (uint32_t k0 = k_first; k0 < k_end; k0 += 4) {
-                const uint32_t k = k0 + quarter, c = k / TAPS, tap = k % TAPS;
-                const uint32_t ih = oh * p.stride_h + tap / KS - p.pad_h, iw = ow * p.stride_w + tap % KS - p.pad_w;
-                const bool there = k < k_end && pixel < q.pixels && ih < p.H && iw < p.W;
-                const float xv = there ? from_image[static_cast<int64_t>(c) * p.xs[1] + static_cast<int64_t>(ih) * p.xs[2] + iw] : 0.0f;
+#pragma unroll 1
+            for (uint32_t k0 = k_first; k0 < k_end; k0 += 4 * CHAIN) {
+                float xv[CHAIN], wk[CHAIN][2];
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const uint32_t co = co0 + i * 16 + column;
-                    const float wk = k < k_end && co < p.O ? w[static_cast<size_t>(co) * p.C * TAPS + k] : 0.0f;
-                    sum[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, wk, sum[i], 0, 0, 0);
-                }
-                if (++chained == 9) {
-                    chained = 0;
+                for (int u = 0; u < CHAIN; ++u) {
+                    const uint32_t k = k0 + 4 * u + quarter, c = k / TAPS, tap = k % TAPS;
+                    const uint32_t ih = oh * p.stride_h + tap / KS - p.pad_h, iw = ow * p.stride_w + tap % KS - p.pad_w;
+                    // (what is not there is the first element, and then zero)
+                    const bool there = k < k_end && pixel < q.pixels && ih < p.H && iw < p.W;
+                    const float value = from_image[there ? static_cast<int64_t>(c) * p.xs[1] + static_cast<int64_t>(ih) * p.xs[2] + iw : 0];
+                    xv[u] = there ? value : 0.0f;
 #pragma unroll
                     for (int i = 0; i < 2; ++i) {
-                        all[i] += sum[i];
-                        sum[i] = float4s{0.0f, 0.0f, 0.0f, 0.0f};
+                        const uint32_t co = co0 + i * 16 + column;
+                        const bool weighs = k < k_end && co < p.O;
+                        const float weight = w[weighs ? static_cast<size_t>(co) * p.C * TAPS + k : 0];
+                        wk[u][i] = weighs ? weight : 0.0f;
                     }
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    float4s sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int u = 0; u < CHAIN; ++u) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u], wk[u][i], sum, 0, 0, 0);
+                    all[i] += sum;
                 }
             }
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int to = 0; to < PT; ++to)
-                    if (to == j) high[i][to] = all[i] + sum[i];
+                    if (to == j) high[i][to] = all[i];
         }
     }
 
@@ -511,7 +481,6 @@ __global__ __launch_bounds__(256) void conv2d_split_sum_kernel(const float* part
 struct SplitOperands {
     const float *x, *w, *bias;
     const uint4s* planes;
-    const uint32_t* largest;
     float *y, *partials;
 };
 
@@ -522,7 +491,7 @@ static int launch_split(const ConvProblem& p, const SplitPlan& q, const SplitOpe
     constexpr size_t lds = 2 * 3 * NL * 64 * 80;
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds, configured)) return rc;
     const uint32_t blocks = (q.pixels + q.ptile - 1) / q.ptile * q.co_tiles * q.splits;
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSplitThreads), lds, stream, o.x, o.w, o.planes, o.largest, o.bias, o.y, o.partials, p, q);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSplitThreads), lds, stream, o.x, o.w, o.planes, o.bias, o.y, o.partials, p, q);
     return launch_status("conv2d_split_kernel");
 }
 
@@ -656,20 +625,19 @@ int conv2d_split(const ConvProblem& p, int dtype, const void* x, const void* w, 
     q.div_splits = FastDiv(q.splits);
     const uint32_t taps = p.KH * p.KW, fragments = (p.O + 15) / 16 * q.chunks * taps, results = q.pixels * p.O;
     // (a block's weights are loaded a tap ahead, the last ones behind the end)
-    const size_t plane_bytes = (static_cast<size_t>(fragments) + 2) * 3 * 1024, largest_bytes = (static_cast<size_t>(fragments) * 4 + 255) / 256 * 256;
+    const size_t plane_bytes = (static_cast<size_t>(fragments) + 2) * 3 * 1024;
     char* scratch = nullptr;
-    if (scratch_acquire(reinterpret_cast<void**>(&scratch), plane_bytes + largest_bytes + (q.splits > 1 ? static_cast<size_t>(results) * q.splits * 4 : 0), stream) != TANNIC_SUCCESS) {
+    if (scratch_acquire(reinterpret_cast<void**>(&scratch), plane_bytes + (q.splits > 1 ? static_cast<size_t>(results) * q.splits * 4 : 0), stream) != TANNIC_SUCCESS) {
         (void)hipGetLastError();
         return TANNIC_UNSUPPORTED_DTYPE;      // no memory for the split weights: conv2d_f32 needs none, or less
     }
     q.weight_bytes = static_cast<uint32_t>(plane_bytes);
     uint4s* planes = reinterpret_cast<uint4s*>(scratch);
-    uint32_t* largest = reinterpret_cast<uint32_t*>(scratch + plane_bytes);
-    const SplitOperands o{static_cast<const float*>(x), static_cast<const float*>(w), static_cast<const float*>(bias), planes, largest, static_cast<float*>(y),
-                          q.splits > 1 ? reinterpret_cast<float*>(scratch + plane_bytes + largest_bytes) : nullptr};
+    const SplitOperands o{static_cast<const float*>(x), static_cast<const float*>(w), static_cast<const float*>(bias), planes, static_cast<float*>(y),
+                          q.splits > 1 ? reinterpret_cast<float*>(scratch + plane_bytes) : nullptr};
     const uint32_t weight_blocks = (p.O + 15) / 16 * q.chunks;
-    if (taps == 1) hipLaunchKernelGGL((conv2d_split_weights_kernel<1>), dim3(weight_blocks), dim3(split_weight_threads<1>), 0, stream, o.w, planes, largest, p.O, p.C, FastDiv(q.chunks));
-    else hipLaunchKernelGGL((conv2d_split_weights_kernel<9>), dim3(weight_blocks), dim3(split_weight_threads<9>), 0, stream, o.w, planes, largest, p.O, p.C, FastDiv(q.chunks));
+    if (taps == 1) hipLaunchKernelGGL((conv2d_split_weights_kernel<1>), dim3(weight_blocks), dim3(split_weight_threads<1>), 0, stream, o.w, planes, p.O, p.C, FastDiv(q.chunks));
+    else hipLaunchKernelGGL((conv2d_split_weights_kernel<9>), dim3(weight_blocks), dim3(split_weight_threads<9>), 0, stream, o.w, planes, p.O, p.C, FastDiv(q.chunks));
     int status = launch_status("conv2d_split_weights_kernel");
     if (status == TANNIC_SUCCESS) {
         status = [&]() -> int {

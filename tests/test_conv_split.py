@@ -174,7 +174,16 @@ def beside_others(x, w):
     x[::2] *= 1e-34     # tiny images between others
 
 
-SPECIAL = [infinities_in_x, infinities_in_w, largest, smallest, smallest_weights, beside_others]
+def large_results(x, w):
+    x[1] *= 1e15
+    w *= 1e12
+
+
+def almost_infinite(x, w):
+    x[0, 0, 5, 5] = w[:, 0] = 1.999 * 2.0 ** 63     # (their product is finite, that of the nearest bfloat16 values is not)
+
+
+SPECIAL = [infinities_in_x, infinities_in_w, largest, smallest, smallest_weights, beside_others, large_results, almost_infinite]
 
 
 @pytest.mark.gpu
@@ -196,3 +205,32 @@ def test_values_without_three_parts(change, side, device):
         finite = np.isfinite(rounded[i])
         error = np.linalg.norm(got[i][finite] - want[i][finite]) / np.linalg.norm(want[i][finite])
         assert error < 5e-7, (i, error)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("side", [1, 3])
+@pytest.mark.parametrize("magnitude", [1e-33, 1e-36, 1e-38, 1e-40])
+def test_small_values_beside_ordinary_ones(magnitude, side, device):
+    """Output channels of small weights, and pixels of small values, in the same tiles as others: as exact as those, down to where fp32 ends
+    (a partial sum, the sum of all and the bias's are rounded to whole 2^-149 there)."""
+    xs, ws = ((16, 256, 24, 24), (512, 256, 1, 1)) if side == 1 else ((16, 128, 20, 20), (256, 128, 3, 3))
+    rng = np.random.default_rng(22)
+    q = split_plan(xs, ws, (1, 1), (0, 0))
+
+    def error(got, want):
+        return np.linalg.norm(got - want) - (q["splits"] + 2) * 2.0 ** -150 * want.size ** 0.5, np.linalg.norm(want)
+
+    def both(x, w):
+        return ops.convolve2d(ta.tensor(x, ta.float32, device), ta.tensor(w, ta.float32, device)).numpy(), reference(x, w, np.zeros(ws[0], np.float32), (1, 1), (0, 0))
+    x, w = (rng.standard_normal(s, dtype=np.float32) for s in (xs, ws))
+    small = w.copy()
+    small[::7] *= np.float32(magnitude)
+    got, want = both(x, small)
+    for channel in range(ws[0]):
+        off, norm = error(got[:, channel], want[:, channel])
+        assert off < 5e-7 * norm, ("channel", channel, off / norm)
+    x[:, :, 4:11, 4:11] *= np.float32(magnitude)
+    got, want = both(x, w)
+    for i in range(xs[0]):
+        off, norm = error(got[i, :, 4:12 - side, 4:12 - side], want[i, :, 4:12 - side, 4:12 - side])
+        assert off < 5e-7 * norm, ("pixels of image", i, off / norm)
