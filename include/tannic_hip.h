@@ -212,12 +212,14 @@ void tannic_hip_graph_destroy(void* recording);
 void tannic_hip_counters(uint64_t out[3]);
 /* Which kernel a convolution of these operands would run, without running it or reading what their addresses point at (for
  * tests, no reference twin).  out[0] is 1 for the fp32 kernel over the flattened batch, 2 for the 16-bit kernel over few
- * output pixels, 3 for the fp32 kernel on the 16-bit matrix pipe, 4 for the 16-bit 3x3 kernel over the flattened batch, 0 for any other.  After 1: the kernel's side, its template parameters U, PT, NL, RESIDENT, WO and WIDE, then
- * pixels per tile, tiles of channels, blocks sharing the channels, groups of kernel rows, groups per block, floats from plane to
- * plane, floats of a plane, rows per image and columns per row with the shared padding.  After 2: the kernel's side, tiles of
- * 16 channels and of 16 pixels per block, wavefronts, blocks.  After 3: the kernel's side, PT, WO and NL, pixels per tile, tiles
- * of channels, blocks sharing the channels, chunks of 32 channels, chunks per block, places of a plane, rows per image and columns
- * per row with the shared padding.  After 4: the same.  The status is the convolution's. */
+ * output pixels, 3 for the fp32 kernel on the 16-bit matrix pipe, 4 for the 16-bit 3x3 kernel over the flattened batch, 5 for the
+ * 16-bit 1x1 product whose tiles run over the images, 0 for any other.  After 1: the kernel's side, its template parameters U, PT, NL,
+ * RESIDENT, WO and WIDE, then pixels per tile, tiles of channels, blocks sharing the channels, groups of kernel rows, groups per block,
+ * floats from plane to plane, floats of a plane, rows per image and columns per row with the shared padding.  After 2: the kernel's
+ * side, tiles of 16 channels and of 16 pixels per block, wavefronts, blocks.  After 3: the kernel's side, PT, WO and NL, pixels per
+ * tile, tiles of channels, blocks sharing the channels, chunks of 32 channels, chunks per block, places of a plane, rows per image and
+ * columns per row with the shared padding.  After 4: the same.  After 5: the kernel's side, channels out of a tile, stages of its
+ * operands.  The status is the convolution's. */
 int tannic_hip_conv2d_plan(const tannic_tensor_t* x, const tannic_tensor_t* w, const tannic_tensor_t* y, const size_t pad[2],
                            const size_t stride[2], uint32_t out[20]);
 /* Whether the product of a few rows with narrow row-major matrices (16-bit, misaligned) takes these operands, asked the same way:

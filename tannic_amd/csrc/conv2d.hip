@@ -96,8 +96,9 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     p.bs = bias ? bias->strides.sizes[0] : 0;
     if (plan) {
         for (int i = 0; i < kConvPlanValues; ++i) plan[i] = 0;
-        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_few_plan(p, x->dtype, plan))
-            conv2d_batch3_plan(p, x->dtype, x->address, w->address, plan);
+        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_few_plan(p, x->dtype, plan) &&
+            !conv2d_batch3_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_k1_takes(p, x->dtype, x->address, w->address, y->address))
+            conv2d_pointwise_plan(p, x->dtype, x->address, w->address, plan);
         return TANNIC_SUCCESS;
     }
     const void* pb = bias ? bias->address : nullptr;

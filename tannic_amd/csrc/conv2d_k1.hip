@@ -328,34 +328,38 @@ int pick_k1(const ConvProblem& p, const K1Plan& q, uint32_t groups, const void* 
     }
 }
 
-template <class T>
-int run_k1(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
-    if (p.KH != 1 || p.KW != 1 || p.pad_h != 0 || p.pad_w != 0) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.stride_h != p.stride_w || (p.stride_w != 1 && p.stride_w != 2)) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.C == 0 || p.C % 64 != 0 || p.C > 256 || p.O == 0 || p.O % kK1CoBlock != 0) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.N == 0 || p.HO == 0 || p.WO == 0) return TANNIC_SUCCESS;
+static bool takes_k1(const ConvProblem& p, const void* x, const void* w, const void* y) {
+    if (p.KH != 1 || p.KW != 1 || p.pad_h != 0 || p.pad_w != 0) return false;
+    if (p.stride_h != p.stride_w || (p.stride_w != 1 && p.stride_w != 2)) return false;
+    if (p.C == 0 || p.C % 64 != 0 || p.C > 256 || p.O == 0 || p.O % kK1CoBlock != 0) return false;
+    if (p.N == 0 || p.HO == 0 || p.WO == 0) return true;
     const uint64_t pixels = static_cast<uint64_t>(p.HO) * p.WO;
-    if (pixels % 8 != 0 || pixels >= (1ull << 31)) return TANNIC_UNSUPPORTED_DTYPE;
+    if (pixels % 8 != 0 || pixels >= (1ull << 31)) return false;
     // weights: rows of C contiguous channels, 16-byte fragments
-    if (p.ws[1] != 1 || p.ws[0] % 8 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.ws[1] != 1 || p.ws[0] % 8 != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0) return false;
     // result: the pixels of a channel contiguous, rows written 16 bytes at a time
-    if (p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO) || p.ys[1] % 8 != 0 || p.ys[0] % 8 != 0 || reinterpret_cast<uintptr_t>(y) % 16 != 0)
-        return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO) || p.ys[1] % 8 != 0 || p.ys[0] % 8 != 0 || reinterpret_cast<uintptr_t>(y) % 16 != 0) return false;
     // signal: 16-byte loads along W
-    if (p.xs[3] != 1 || p.xs[2] % 8 != 0 || p.xs[1] % 8 != 0 || p.xs[0] % 8 != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.xs[3] != 1 || p.xs[2] % 8 != 0 || p.xs[1] % 8 != 0 || p.xs[0] % 8 != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0) return false;
     if (p.stride_w == 1) {
         // eight consecutive pixels are one load: a run must not cross a row
-        if (p.WO % 8 != 0) return TANNIC_UNSUPPORTED_DTYPE;
+        if (p.WO % 8 != 0) return false;
     } else {
         // four pixels are the even elements of one load of eight: the eighth must exist
-        if (p.WO % 4 != 0 || static_cast<uint64_t>(p.WO) * 2 > p.W) return TANNIC_UNSUPPORTED_DTYPE;
+        if (p.WO % 4 != 0 || static_cast<uint64_t>(p.WO) * 2 > p.W) return false;
     }
+    return p.N * ((pixels + kK1Pixels - 1) / kK1Pixels) < (1ull << 31);
+}
+
+template <class T>
+int run_k1(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
+    if (!takes_k1(p, x, w, y)) return TANNIC_UNSUPPORTED_DTYPE;
+    if (p.N == 0 || p.HO == 0 || p.WO == 0) return TANNIC_SUCCESS;
+    const uint64_t pixels = static_cast<uint64_t>(p.HO) * p.WO;
     K1Plan q{};
     q.pixels = static_cast<uint32_t>(pixels);
     const uint32_t tiles_per_image = (q.pixels + kK1Pixels - 1) / kK1Pixels;
-    const uint64_t tiles = static_cast<uint64_t>(p.N) * tiles_per_image;
-    if (tiles >= (1ull << 31)) return TANNIC_UNSUPPORTED_DTYPE;
-    q.tiles = static_cast<uint32_t>(tiles);
+    q.tiles = p.N * tiles_per_image;
     const uint32_t groups = p.O / kK1CoBlock;
     // one block per compute unit (up to 138 KB of LDS, every register): as many workers per group as that allows
     const uint32_t per_group = groups >= 256 ? 1 : 256 / groups;
@@ -364,6 +368,10 @@ int run_k1(const ConvProblem& p, const void* x, const void* w, const void* bias,
     q.div_tiles_per_image = FastDiv(tiles_per_image);
     if (p.stride_w == 1) return pick_k1<T, 1>(p, q, groups, x, w, bias, y, stream);
     return pick_k1<T, 2>(p, q, groups, x, w, bias, y, stream);
+}
+
+bool conv2d_k1_takes(const ConvProblem& p, int dtype, const void* x, const void* w, const void* y) {
+    return (dtype == TANNIC_FLOAT16 || dtype == TANNIC_BFLOAT16) && takes_k1(p, x, w, y);
 }
 
 int conv2d_k1(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {

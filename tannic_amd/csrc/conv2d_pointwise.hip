@@ -85,6 +85,29 @@ int product(const GemmProblem& g, int dtype, const void* a, const void* b, void*
     else return gemm_mfma_16bit(g, dtype, a, b, c, stream);
 }
 
+// The whole batch as one product O x C . C x (N * pitch), the columns of image n its pixels and what rounds them up to `pitch`: B the images where
+// they lie (a channel's pixels one run of memory), the result's columns to y[n].
+static GemmProblem batch_product(const ConvProblem& p, const void* bias, uint32_t pixels, uint32_t pitch) {
+    GemmProblem g{};
+    g.M = p.O;
+    g.N = p.N * pitch;
+    g.K = p.C;
+    g.a_rs = p.ws[0];
+    g.a_cs = 1;
+    g.b_rs = p.xs[1];
+    g.b_cs = 1;
+    g.c_rs = p.ys[1];
+    g.batches = 1;
+    for (int d = 0; d < 6; ++d) g.batch_extent[d] = 1;
+    g.row_bias = bias;
+    g.c_group = pitch;
+    g.c_group_live = pixels;
+    g.c_group_stride = p.ys[0];
+    g.c_group_div = FastDiv(pitch);
+    g.b_group_stride = p.xs[0];
+    return g;
+}
+
 template <class T>
 int run_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
     if (p.KH != 1 || p.KW != 1 || p.pad_h != 0 || p.pad_w != 0) return TANNIC_UNSUPPORTED_DTYPE;
@@ -122,30 +145,17 @@ int run_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w,
         const uint64_t in_rows = static_cast<uint64_t>(p.N) * p.C, out_rows = static_cast<uint64_t>(p.N) * p.O;
         if (in_rows * groups >= (1ull << 31) || out_rows * groups >= (1ull << 31) || static_cast<uint64_t>(p.N) * pitch >= (1ull << 31)) return TANNIC_UNSUPPORTED_DTYPE;
         const bool plane = dense && p.xs[3] == 1 && p.xs[2] == static_cast<int64_t>(p.W) && reinterpret_cast<uintptr_t>(x) % sizeof(T) == 0;
-        const uint64_t columns = static_cast<uint64_t>(p.N) * pitch;
-        // one product O x C . C x (N * pitch) for the whole batch; the columns of image n go to y[n], rows p.ys[1] apart
-        g.N = static_cast<uint32_t>(columns);
-        g.batch_rank = 0;
-        g.batches = 1;
-        g.batch_extent[0] = 1;
-        g.b_bs[0] = g.c_bs[0] = 0;
-        g.c_rs = p.ys[1];
-        g.c_group = pitch;
-        g.c_group_live = static_cast<uint32_t>(pixels);
-        g.c_group_stride = p.ys[0];
-        g.c_group_div = FastDiv(pitch);
+        g = batch_product(p, bias, static_cast<uint32_t>(pixels), pitch);
         if (plane) {
             // The pixels of a channel are one run of memory: the product reads the images where they lie, through the
             // direct-to-LDS tiles for columns in groups (whole steps of channels, an even number of pixels), or, with up to 256 channels,
             // its loaders take 16-byte pieces at whatever address they start.  (Those loads are slower than aligned ones and
             // the kernel that knows them walks all of K in one block; batch 32, fp16: 2048 -> 512 over 7 x 7 53 against 26 us through
             // re-pitched rows.)
-            g.b_rs = p.xs[1];
-            g.b_group_stride = p.xs[0];
             const int direct = product<T>(g, dtype, w, x, y, stream);
             if (direct != TANNIC_UNSUPPORTED_DTYPE) return direct;
-            g.b_group_stride = 0;
         }
+        g.b_group_stride = 0;
         T* dense_x = nullptr;
         if (scratch_acquire(reinterpret_cast<void**>(&dense_x), in_rows * pitch * sizeof(T), stream) != TANNIC_SUCCESS) return TANNIC_ERROR;
         const uint32_t total_in = static_cast<uint32_t>(in_rows * groups);
@@ -157,7 +167,7 @@ int run_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w,
                                static_cast<uint32_t>(pixels), pitch, FastDiv(groups), FastDiv(p.C), FastDiv(p.WO), total_in);
         int status = launch_status("conv_repitch_kernel");
         if (status == TANNIC_SUCCESS) {
-            g.b_rs = static_cast<int64_t>(columns);
+            g.b_rs = static_cast<int64_t>(g.N);
             status = product<T>(g, dtype, w, dense_x, y, stream);
             if (status == TANNIC_UNSUPPORTED_DTYPE) {
                 set_error_text("conv2d: internal: the 1x1 product refused a problem its caller had checked");
@@ -172,16 +182,7 @@ int run_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w,
         g.b_rs = p.xs[1];
         if (sizeof(T) == 2 && static_cast<uint64_t>(p.N) * pixels < (1ull << 31)) {
             // the whole batch as one product, tiles running over images (gemm16_dtl_grouped)
-            GemmProblem whole = g;
-            whole.N = static_cast<uint32_t>(p.N * pixels);
-            whole.batch_rank = 0;
-            whole.batches = 1;
-            whole.batch_extent[0] = 1;
-            whole.c_bs[0] = 0;
-            whole.c_group = whole.c_group_live = static_cast<uint32_t>(pixels);
-            whole.c_group_stride = p.ys[0];
-            whole.c_group_div = FastDiv(whole.c_group);
-            whole.b_group_stride = p.xs[0];
+            const GemmProblem whole = batch_product(p, bias, static_cast<uint32_t>(pixels), static_cast<uint32_t>(pixels));
             int status = TANNIC_UNSUPPORTED_DTYPE;
             if constexpr (sizeof(T) == 2) status = gemm16_dtl_grouped<T>(whole, w, x, y, stream);
             if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
@@ -218,6 +219,22 @@ int run_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w,
     }
     scratch_release(dense_x, stream);
     return status;
+}
+
+bool conv2d_pointwise_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]) {
+    if ((dtype != TANNIC_FLOAT16 && dtype != TANNIC_BFLOAT16) || p.KH != 1 || p.KW != 1 || p.pad_h || p.pad_w || p.stride_h != 1 || p.stride_w != 1) return false;
+    if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0 || p.C == 0 || p.N > 65535) return false;
+    if (p.ws[1] != 1 || p.ys[3] != 1 || p.ys[2] != static_cast<int64_t>(p.WO) || p.xs[3] != 1 || p.xs[2] != static_cast<int64_t>(p.W)) return false;
+    const uint64_t pixels = static_cast<uint64_t>(p.HO) * p.WO, pitch = (pixels + 7) / 8 * 8;
+    const uint64_t planes = static_cast<uint64_t>(p.N) * (p.C > p.O ? p.C : p.O);
+    if (p.N * pitch >= (1ull << 31) || (pixels != pitch && planes * (pitch / 8) >= (1ull << 31))) return false;
+    const GroupedTiles tiles = gemm16_dtl_grouped_tiles(batch_product(p, nullptr, static_cast<uint32_t>(pixels), static_cast<uint32_t>(pitch)), w, x);
+    if (tiles.rows == 0) return false;
+    out[0] = 5;
+    out[1] = 1;
+    out[2] = static_cast<uint32_t>(tiles.rows);
+    out[3] = static_cast<uint32_t>(tiles.stages);
+    return true;
 }
 
 int conv2d_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {

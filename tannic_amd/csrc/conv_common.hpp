@@ -20,8 +20,10 @@ struct ConvProblem {
 // The plan of the kernel that would take a problem, for tannic_hip_conv2d_plan: which of the kernels below, then its parameters and
 // the parts of its plan that say where a tile's windows lie (named in include/tannic_hip.h).
 constexpr int kConvPlanValues = 20;
-// true where the kernel takes the problem (conv2d_split, conv2d_f32, conv2d_few and conv2d_batch3 launch what these report)
+// true where the kernel takes the problem (conv2d_split, conv2d_f32, conv2d_few, conv2d_batch3 and, through the tiles over images,
+// conv2d_pointwise launch what these report)
 bool conv2d_split_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
+bool conv2d_pointwise_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_batch3_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_f32_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValues]);
@@ -30,6 +32,7 @@ bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValu
 // conditions, so that the caller can try the next, more general kernel.
 // 16-bit 1x1 and 3x3 over few output pixels
 int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
+bool conv2d_k1_takes(const ConvProblem& p, int dtype, const void* x, const void* w, const void* y);
 int conv2d_k1(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_stem(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);

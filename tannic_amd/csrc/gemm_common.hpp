@@ -112,7 +112,12 @@ template <class T> int gemm16_dtl(const GemmProblem& p, int bm, int bn, const vo
 // the 128 x 128 (bm = 128) or 64 x 128 (bm = 64) tiles with K shared between `splits` workgroups per tile (k_chunk elements each, a multiple of 64): fp32
 // partial sums go to partials[split][batch][M][N], which the caller adds up
 template <class T> int gemm16_dtl_split(const GemmProblem& p, int bm, uint32_t splits, uint32_t k_chunk, float* partials, const void* a, const void* b, hipStream_t stream);
-// the same kernel for B's columns in groups (b_group_stride), rows at any multiple of four bytes, C's columns in the same groups
+// the same kernel for B's columns in groups (b_group_stride), rows at any multiple of four bytes, C's columns in the same groups; its tiles
+// (rows, by 128 columns) and stages, no rows where it does not take the problem or leaves it to what there is beside it
+struct GroupedTiles {
+    int rows, stages;
+};
+GroupedTiles gemm16_dtl_grouped_tiles(const GemmProblem& p, const void* a, const void* b);
 template <class T> int gemm16_dtl_grouped(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream);
 // int8 x int8 -> int32 on the same tiles (v_mfma_i32_16x16x64_i8)
 int gemm_mfma_int8(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream);

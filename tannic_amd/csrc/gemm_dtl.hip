@@ -420,29 +420,14 @@ int gemm16_dtl_krows(const GemmProblem& p, int bm, int bn, bool a_t, bool b_t, S
     if (bm == 128 && bn == 128) return launch_dtl_krows<T, 128, 128, 4, false>(p, a_t, b_t, sk, a, b, c, stream);
     return TANNIC_UNSUPPORTED_DTYPE;
 }
-// B's columns in groups, at any multiple of four bytes (a buffer load of 16 bytes wants its address to be a multiple of four): a 1x1
-// convolution over a whole batch that reads the images where they lie.  Before, images of 14 x 14 were copied into aligned rows first or read
-// by the register-staged tiles for any alignment, and images of 28 x 28 were a product each, with a ragged last tile (fp16, batch 32, us before /
-// here: 1024 -> 256 over 14 x 14 28.2 / 13.8, 256 -> 1024 22.5 / 14.3, 1024 -> 512 29.2 / 17.5, 512 -> 256 over 28 x 28 22.4 / 17.2,
-// 128 -> 512 23.8 / 17.2).  Bound by a tile's start and end: K is 2 to 16 steps.
+// B's columns in groups (gemm16_dtl_grouped_tiles)
 template <class T>
 int gemm16_dtl_grouped(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream) {
-    if (p.K == 0 || p.K % 64 != 0 || p.batches != 1 || !p.c_group || p.c_group % 8 != 0 || p.c_group_live < 8 || p.N % p.c_group != 0) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.a_cs != 1 || p.a_rs < static_cast<int64_t>(p.K) || p.a_rs >= (1 << 22) || p.a_rs % 8 != 0 || reinterpret_cast<uintptr_t>(a) % 16 != 0) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.b_cs != 1 || p.b_rs % 2 != 0 || p.b_group_stride % 2 != 0 || p.c_group_live % 2 != 0 || p.b_rs <= 0 || p.b_group_stride <= 0 || reinterpret_cast<uintptr_t>(b) % 4 != 0)
-        return TANNIC_UNSUPPORTED_DTYPE;
-    // byte offsets stay below 2^31, so that a column past the last group is out of range
-    if ((static_cast<uint64_t>(p.N / p.c_group) * p.b_group_stride + static_cast<uint64_t>(p.K) * p.b_rs) * 2 >= (1ull << 31)) return TANNIC_UNSUPPORTED_DTYPE;
-    if (reinterpret_cast<uintptr_t>(c) % 2 != 0) return TANNIC_UNSUPPORTED_DTYPE;
-    // Tiles: 128 x 128 with two stages, two blocks on a compute unit, where there is more than one for each; else blocks enough come first,
-    // 64 x 128 unless the tiles of 128 rows are nearly enough and K is long (fp16, batch 32, us with 128 rows and two stages / 128 and
-    // four / 64 and three: 256 -> 1024 over 14 x 14 (400 tiles of 128 rows) 14.3 / 17.3 / 17.5, 512 -> 256 over 28 x 28 (392)
-    // 17.2 / 20.4 / 20.9, 1024 -> 512 over 14 x 14 (200) 18.2 / 17.5 / 20.8, 512 -> 128 over 28 x 28 (196) 16.9 / 14.8 / 14.2,
-    // 1024 -> 256 over 14 x 14 (100) 22.8 / 17.8 / 13.8; eight images of 256 -> 1024 10.3 / 10.6 / 9.7).
-    const uint64_t tiles = static_cast<uint64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
-    if (p.M > 64 && tiles > 256) return launch_dtl<T, 128, 128, 2, false, false, true, true>(p, a, b, c, stream);
-    if (p.M > 64 && tiles > 160 && p.K >= 768) return launch_dtl<T, 128, 128, 4, false, false, true, true>(p, a, b, c, stream);
-    return launch_dtl<T, 64, 128, 3, false, false, true, true>(p, a, b, c, stream);
+    const GroupedTiles tiles = gemm16_dtl_grouped_tiles(p, a, b);
+    if (tiles.rows == 0 || reinterpret_cast<uintptr_t>(c) % 2 != 0) return TANNIC_UNSUPPORTED_DTYPE;
+    if (tiles.rows == 64) return launch_dtl<T, 64, 128, 3, false, false, true, true>(p, a, b, c, stream);
+    if (tiles.stages == 2) return launch_dtl<T, 128, 128, 2, false, false, true, true>(p, a, b, c, stream);
+    return launch_dtl<T, 128, 128, 4, false, false, true, true>(p, a, b, c, stream);
 }
 
 #if TH_DTL_PART == 1
@@ -454,6 +439,50 @@ template int gemm16_dtl_krows<bf16>(const GemmProblem&, int, int, bool, bool, Sp
 #endif
 
 #else   // TH_DTL_PART == 0
+
+// B's columns in groups, at any multiple of four bytes (a buffer load of 16 bytes wants its address to be a multiple of four): a 1x1
+// convolution over a whole batch that reads the images where they lie.  Before, images of 14 x 14 were copied into aligned rows first or read
+// by the register-staged tiles for any alignment, and images of 28 x 28 were a product each, with a ragged last tile (fp16, batch 32, us before /
+// here: 1024 -> 256 over 14 x 14 28.2 / 13.8, 256 -> 1024 22.5 / 14.3, 1024 -> 512 29.2 / 17.5, 512 -> 256 over 28 x 28 22.4 / 17.2,
+// 128 -> 512 23.8 / 17.2).  Bound by a tile's start and end: K is 2 to 16 steps.
+GroupedTiles gemm16_dtl_grouped_tiles(const GemmProblem& p, const void* a, const void* b) {
+    const GroupedTiles none{0, 0};
+    if (p.M == 0 || p.N == 0 || p.K == 0 || p.K % 64 != 0 || p.batches != 1 || !p.c_group || p.c_group % 8 != 0 || p.c_group_live < 8 || p.N % p.c_group != 0) return none;
+    if (p.a_cs != 1 || p.a_rs < static_cast<int64_t>(p.K) || p.a_rs >= (1 << 22) || p.a_rs % 8 != 0 || reinterpret_cast<uintptr_t>(a) % 16 != 0) return none;
+    if (p.b_cs != 1 || p.b_rs % 2 != 0 || p.b_group_stride % 2 != 0 || p.c_group_live % 2 != 0 || p.b_rs <= 0 || p.b_group_stride <= 0 || reinterpret_cast<uintptr_t>(b) % 4 != 0)
+        return none;
+    // byte offsets stay below 2^31, so that a column past the last group is out of range
+    if ((static_cast<uint64_t>(p.N / p.c_group) * p.b_group_stride + static_cast<uint64_t>(p.K) * p.b_rs) * 2 >= (1ull << 31)) return none;
+    const uint64_t rows = p.M, columns = p.N, tiles = (rows + 127) / 128 * ((columns + 127) / 128), small_tiles = (rows + 63) / 64 * ((columns + 127) / 128);
+    // What else there is: with groups of whole pieces in aligned rows a product for each of them, without (and for any number of pixels)
+    // rows copied into aligned ones; both on the tiles of run16.
+    const bool whole = p.c_group_live == p.c_group, aligned = p.b_rs % 8 == 0 && p.b_group_stride % 8 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
+    //  * Few tiles under a long K: those share it between blocks (fp16, us there / here, 16 tiles of 64 x 128 under K = 2048 12.3 / 13.5, 3072
+    //    13.1 / 17.9, 8192 19.2 / 41; 50 tiles under 3072 16.6 / 23.5, 128 under 4096 23.7 / 25.0, 200 27.8 / 29.7; but 50 under 1536 1.05 of the time
+    //    here, 64 under 2048 1.05 .. 1.13, 128 under 3072 1.04, 256 under 8192 1.09; copied rows: 14 under 3072 17.7 / 22.9, 104 under 4096 27.4 / 29.3,
+    //    but 50 under 3072 and 88 under 4096 1.03).
+    if (whole ? aligned && small_tiles < 256 && p.K >= 1690 + 12 * small_tiles : small_tiles < 176 && p.K >= 2700 + 12 * small_tiles) return none;
+    //  * Tiles of 256 x 256 that (nearly) fill the chip read half as much for as many products.  They take whole rounds of 256, these pairs of 512
+    //    (fp16, us there / here: 8 images of 64 x 64 under 1024 -> 1024 65.1 / 73.2, 2048 -> 2048 230 / 313, 512 -> 2048 78.7 / 90.5, 2048 -> 320 57 / 70, 32 of
+    //    28 x 28 under 2048 -> 1024 121 / 149; but 16 of 48 x 48 under 512 -> 512, 288 tiles, 36.8 / 30.1, 1024 -> 320 53 / 34), and below K = 2048 images
+    //    that are no whole tiles leave them to the register-staged ones (32 of 28 x 28 under 1024 -> 1024 83 / 68, 512 -> 512 29.0 / 23.8).
+    if (whole && aligned && rows > 192 && p.K >= 512) {
+        const uint64_t images = columns / p.c_group, per_image = (p.c_group + 255) / 256, large = (rows + 255) / 256 * per_image * images;
+        const bool filled = p.c_group >= 0.75 * (per_image * 256.0) && large >= 200;      // (what run16 asks of them)
+        const uint64_t rounds = (large + 255) / 256, rounds_here = (tiles + 511) / 512;
+        // (under a short K what the last round here leaves idle is less: 8 of 64 x 64 under 512 -> 320 22.4 / 21.3, 16 of 48 x 48 under
+        // 512 -> 1024 57.7 / 49.7)
+        if (filled && (p.K >= 2048 || p.c_group % 256 == 0) && (p.K >= 1024 ? rounds_here * 10 >= rounds * 16 : tiles * 10 >= rounds * 8192)) return none;
+    }
+    // Tiles: 128 x 128 with two stages, two blocks on a compute unit, where there is more than one for each; else blocks enough come first,
+    // 64 x 128 unless the tiles of 128 rows are nearly enough and K is long (fp16, batch 32, us with 128 rows and two stages / 128 and
+    // four / 64 and three: 256 -> 1024 over 14 x 14 (400 tiles of 128 rows) 14.3 / 17.3 / 17.5, 512 -> 256 over 28 x 28 (392)
+    // 17.2 / 20.4 / 20.9, 1024 -> 512 over 14 x 14 (200) 18.2 / 17.5 / 20.8, 512 -> 128 over 28 x 28 (196) 16.9 / 14.8 / 14.2,
+    // 1024 -> 256 over 14 x 14 (100) 22.8 / 17.8 / 13.8; eight images of 256 -> 1024 10.3 / 10.6 / 9.7).
+    if (p.M > 64 && tiles > 256) return {128, 2};
+    if (p.M > 64 && tiles > 160 && p.K >= 768) return {128, 4};
+    return {64, 3};
+}
 
 // Whether the operands are this kernel's (tile bm x bn): each contiguous along K, or (16-bit types) along its other
 // index; whole K steps; rows that do not overlap; offsets that fit 32 bits.
