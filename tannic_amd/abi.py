@@ -153,6 +153,7 @@ def runtime_signatures():
         "counters": (None, [C.POINTER(C.c_uint64)]),
         "conv2d_plan": (C.c_int, [TP, TP, TP, SIZE2, SIZE2, C.POINTER(C.c_uint32)]),
         "gemm_rows_batch_lanes": (C.c_int, [TP, TP, TP]),
+        "gemm_plan": (C.c_int, [TP, TP, TP, C.POINTER(C.c_uint32)]),
         "event_create": (C.c_void_p, []),
         "event_destroy": (None, [C.c_void_p]),
         "event_record": (C.c_int, [C.c_void_p, stream_t]),

@@ -283,6 +283,17 @@ inline bool few_results_under_a_long_k(const GemmProblem& p, uint64_t most) {
     return p.M != 0 && p.N != 0 && p.batches != 0 && p.batches <= 65535 && p.K >= 256 && static_cast<uint64_t>(p.M) * p.N * p.batches <= most;
 }
 
+// Not where the tiles share K or W is streamed: aligned K-contiguous operands of the 16-bit types and fp32, of int8 up to 32 rows; nor the few
+// rows that the row-major kernel (gemm_rows_nn) streams
+template <class A>
+bool few_results_elsewhere(const GemmProblem& p, const void* a, const void* b) {
+    constexpr int64_t unit = 16 / sizeof(A);
+    const bool aligned_nt = p.a_cs == 1 && p.b_rs == 1 && p.K % (std::is_same_v<A, int8_t> ? 128 : unit) == 0 && p.a_rs % unit == 0 && p.b_cs % unit == 0 &&
+                            reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % 16 == 0;
+    if (aligned_nt && (!std::is_same_v<A, int8_t> || p.M <= 32)) return true;
+    return !std::is_same_v<A, int8_t> && p.M <= 8 && p.b_cs == 1 && p.b_rs != 1 && p.N >= 256 && p.N % 4 == 0;
+}
+
 template <class A, class B, class D>
 int run_few_results(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream) {
     const uint32_t tiles_m = (p.M + 3) / 4, tiles_n = (p.N + 3) / 4;
@@ -499,17 +510,8 @@ int gemm_entry(const tannic_tensor_t* a, const tannic_tensor_t* b, tannic_tensor
                 }
                 constexpr bool shares_k = std::is_same_v<A, B> && (is_16bit<A>::value || std::is_same_v<A, float> || std::is_same_v<A, int8_t>);
                 if (few_results_under_a_long_k(p, shares_k ? 8192 : 32768)) {
-                    // (not where the tiles share K or W is streamed: aligned K-contiguous operands of the 16-bit types and
-                    // fp32, of int8 up to 32 rows; nor the few rows that the row-major kernel below or the scalar kernel
-                    // for few rows streams)
-                    bool elsewhere = !shares_k && p.M <= 16 && p.a_cs == 1 && p.b_rs == 1;
-                    if constexpr (shares_k) {
-                        constexpr int64_t unit = 16 / sizeof(A);
-                        const bool aligned_nt = p.a_cs == 1 && p.b_rs == 1 && p.K % (std::is_same_v<A, int8_t> ? 128 : unit) == 0 && p.a_rs % unit == 0 && p.b_cs % unit == 0 &&
-                                                reinterpret_cast<uintptr_t>(first) % 16 == 0 && reinterpret_cast<uintptr_t>(second) % 16 == 0;
-                        if (aligned_nt && (!std::is_same_v<A, int8_t> || p.M <= 32)) elsewhere = true;
-                        if (!std::is_same_v<A, int8_t> && p.M <= 8 && p.b_cs == 1 && p.b_rs != 1 && p.N >= 256 && p.N % 4 == 0) elsewhere = true;   // gemm_rows_nn
-                    }
+                    bool elsewhere = !shares_k && p.M <= 16 && p.a_cs == 1 && p.b_rs == 1;     // (the scalar kernel for few rows streams them)
+                    if constexpr (shares_k) elsewhere = few_results_elsewhere<A>(p, first, second);
                     if (!elsewhere) {
                         if constexpr (std::is_same_v<A, B> && is_16bit<A>::value) {
                             status = gemm_rows_few(p, a->dtype, first, second, dst->address, s);
@@ -593,6 +595,22 @@ extern "C" int tannic_hip_gemm_noalloc(const tannic_tensor_t* a, const tannic_te
     if (int rc = scratch_address(&base)) return rc;
     const GemmWorkspace workspace{base, kNoAllocScratchBytes};
     return gemm_entry(a, b, dst, stream, &workspace);
+}
+
+extern "C" int tannic_hip_gemm_plan(const tannic_tensor_t* a, const tannic_tensor_t* b, const tannic_tensor_t* dst, uint32_t out[4]) {
+    for (int i = 0; i < 4; ++i) out[i] = 0;
+    if (!a || !b || !dst || a->dtype != b->dtype || !have_storage(a, b, dst)) return TANNIC_ERROR;
+    GemmProblem p;
+    tannic_tensor_t result = *dst;
+    if (const int status = describe_gemm(a, b, &result, p)) return status;
+    if ((a->dtype != TANNIC_FLOAT16 && a->dtype != TANNIC_BFLOAT16) || p.M == 0 || p.N == 0 || p.K == 0 || p.batches == 0 || (p.N == 1 && p.M > 1)) return TANNIC_SUCCESS;
+    if (const uint32_t lanes = gemm_rows_batch_lanes(p, a->dtype, a->address, b->address)) {
+        out[0] = 1;
+        out[1] = lanes;
+    } else if (few_results_under_a_long_k(p, 8192) && !few_results_elsewhere<f16>(p, a->address, b->address)) {
+        out[0] = gemm_rows_few_takes(p, a->dtype) ? 2 : 0;
+    }
+    return TANNIC_SUCCESS;
 }
 
 extern "C" int tannic_hip_gemm_rows_batch_lanes(const tannic_tensor_t* a, const tannic_tensor_t* b, const tannic_tensor_t* dst) {

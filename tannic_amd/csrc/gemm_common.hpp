@@ -91,6 +91,7 @@ int gemm_rows_nn(const GemmProblem& p, int dtype, const void* a, const void* b, 
 uint32_t gemm_rows_batch_lanes(const GemmProblem& p, int dtype, const void* a, const void* b);
 int gemm_rows_batch(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 // 16-bit, up to four rows and 8192 results, row-major matrices under a K of 512 or more (gemm_rows_batch.hip)
+bool gemm_rows_few_takes(const GemmProblem& p, int dtype);
 int gemm_rows_few(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 int gemm_few_results(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 int gemm_mfma_f64(const GemmProblem& p, const double* a, const double* b, double* c, hipStream_t stream);

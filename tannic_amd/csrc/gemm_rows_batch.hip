@@ -189,7 +189,18 @@ __global__ __launch_bounds__(64 * kRowsBatchWaves) void gemm_rows_few_kernel(con
 static bool rows_few_takes(const GemmProblem& p) {
     if (p.M == 0 || p.M > 4 || p.N == 0 || p.N % 8 != 0 || p.K < 512 || p.K >= (1u << 31) || p.a_cs != 1 || p.b_cs != 1 || p.b_rs == 1 || p.row_bias || p.c_group || p.b_group_stride)
         return false;
-    return static_cast<uint64_t>(p.N) * p.batches * p.M <= 8192;
+    if (static_cast<uint64_t>(p.N) * p.batches * p.M > 8192) return false;
+    // Rows of W that are an odd number of 16-byte pieces: a block's 32 bytes of one lie in two lines every other time, and fewer than 64 blocks
+    // under a long K are bound by the lines each has on its way (bf16, four rows, us on the kernel for few results / here, W in no cache: 104
+    // columns under 8192 22 / 27, 200 under 16384 39 / 50, two products 39 / 49, four 43 / 50; W in the caches 200 under 16384 33.4 / 35.6, 72 32 / 35, but
+    // 200 under 4096 14 / 12, 72 under 8192 15 / 13, two products 20 / 13; up to 64 columns from 32768 on, 40 under 65536 75 / 84, under 16384 23 / 19).  104 blocks of 200 columns under 16384 82 / 51, and
+    // 192 columns 45 / 46, two products of 128 46 / 44.
+    const uint64_t blocks = static_cast<uint64_t>((p.N + 15) / 16) * p.batches;
+    return p.N % 16 == 0 || p.N == 8 || blocks >= 64 || p.K < (p.N > 96 ? 6144u : p.N > 64 ? 12288u : 32768u);
+}
+
+bool gemm_rows_few_takes(const GemmProblem& p, int dtype) {
+    return (dtype == TANNIC_FLOAT16 || dtype == TANNIC_BFLOAT16) && rows_few_takes(p);
 }
 
 template <class T>

@@ -1,8 +1,11 @@
 """Which 16-bit products of a few rows with narrow row-major matrices run on the kernel for them, asked of the library without a GPU
 (``tannic_hip_gemm_rows_batch_lanes``)."""
+import ctypes as C
+
 import pytest
 
 import tannic_amd as ta
+from tannic_amd import abi
 from test_conv_plan import descriptor
 
 
@@ -48,3 +51,39 @@ def test_alignment_is_of_rows_and_addresses():
     assert lanes(64, 4, 128, 2048, x_start=1) == 4
     assert lanes(64, 4, 128, 2048, w_pitch=129) == 4
     assert lanes(128, 4, 128, 2048, w_pitch=129) == 0
+
+
+def product_plan(batches, m, n, k, dtype="bfloat16"):
+    out = (C.c_uint32 * 4)()
+    assert ta.library().gemm_plan(*(C.byref(descriptor(dtype, s)) for s in ((batches, m, k), (batches, k, n), (batches, m, n))), out) == abi.SUCCESS
+    return tuple(out)
+
+
+# batches, M, N, K of a few rows times row-major matrices with few results -> whether the kernel for them takes it
+FEW_RESULTS = {
+    "decoding": ((8, 4, 128, 2049), True),
+    "shortest": ((1, 1, 8, 512), True),
+    "shorter": ((1, 1, 8, 511), False),
+    "most_results": ((16, 4, 128, 4096), True),
+    "more_results": ((17, 4, 128, 4096), False),
+    "five_rows": ((8, 5, 128, 4096), False),
+    "columns_of_no_pieces": ((8, 4, 124, 4096), False),
+    # rows of an odd number of pieces under a long K
+    "odd_pieces": ((1, 4, 200, 6136), True),
+    "odd_pieces_long_k": ((1, 4, 200, 6144), False),
+    "odd_pieces_long_k_four_products": ((4, 4, 200, 16384), False),
+    "odd_pieces_long_k_more_blocks": ((8, 4, 200, 16384), True),
+    "fewer_odd_pieces": ((1, 4, 72, 12280), True),
+    "fewer_odd_pieces_long_k": ((1, 4, 72, 12288), False),
+    "even_pieces_long_k": ((1, 4, 192, 65536), True),
+    "few_odd_pieces": ((1, 4, 40, 32760), True),
+    "few_odd_pieces_long_k": ((1, 4, 40, 32768), False),
+    "one_piece": ((1, 4, 8, 200000), True),
+}
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("name", list(FEW_RESULTS))
+def test_few_results_of_row_major_matrices(name, dtype):
+    problem, taken = FEW_RESULTS[name]
+    assert (product_plan(*problem, dtype)[0] == 2) == taken
