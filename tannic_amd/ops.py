@@ -369,14 +369,18 @@ _CONVOLUTIONS = {}    # (shapes, dtypes, stride, padding) -> shape of the result
 
 
 def convolve2d(signal, kernel, bias=None, stride=1, padding=0):
+    whole = isinstance(stride, int) and isinstance(padding, int)
     stride, padding = _pair(stride), _pair(padding)
     key = (signal.shape, kernel.shape, None if bias is None else bias.shape, signal.dtype, kernel.dtype, None if bias is None else bias.dtype, stride, padding)
-    rule = _CONVOLUTIONS.get(key)
+    # (1.0 equals 1, and is refused: rules are kept for Python's whole numbers only)
+    kept = whole or all(isinstance(v, int) for v in stride + padding)
+    rule = _CONVOLUTIONS.get(key) if kept else None
     if rule is None:
         rule = _convolution_rule(signal, kernel, bias, stride, padding)
         if len(_CONVOLUTIONS) > 4096:
             _CONVOLUTIONS.clear()
-        _CONVOLUTIONS[key] = rule
+        if kept:
+            _CONVOLUTIONS[key] = rule
     shape, extra = rule
     if bias is None:
         env = _resolve(signal, kernel)
