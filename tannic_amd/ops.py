@@ -357,7 +357,9 @@ def _product_rule(a, b):
         raise TannicError("Inputs must have rank >= 2")
     if a.shape[-1] != b.shape[-2]:
         raise TannicError("Inner dimensions must match for matmul")
-    return _composition_dtype(a.dtype, b.dtype), broadcast(a.shape[:-2], b.shape[:-2]) + (a.shape[-2], b.shape[-1])
+    shape = broadcast(a.shape[:-2], b.shape[:-2]) + (a.shape[-2], b.shape[-1])
+    _resolve(a, b)      # (operands on different devices are reported before types that have no product)
+    return _composition_dtype(a.dtype, b.dtype), shape
 
 
 # ---- convolution (include/tannic/convolutions.hpp:71-120) -----------------
@@ -401,6 +403,7 @@ def _convolution_rule(signal, kernel, bias, stride, padding):
     if bias is not None and (bias.rank != 1 or bias.shape[0] != c_out):
         raise TannicError("Bias shape must be [C_out].")
     shape = (n, c_out, (h + 2 * padding[0] - kh) // stride[0] + 1, (w + 2 * padding[1] - kw) // stride[1] + 1)
+    _resolve(*((signal, kernel) if bias is None else (signal, kernel, bias)))      # (and here before strides that are no numbers of elements)
     return shape, (abi.SIZE2(*padding), abi.SIZE2(*stride))
 
 
