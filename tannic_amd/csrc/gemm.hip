@@ -609,6 +609,11 @@ extern "C" int tannic_hip_gemm_plan(const tannic_tensor_t* a, const tannic_tenso
         out[1] = lanes;
     } else if (few_results_under_a_long_k(p, 8192) && !few_results_elsewhere<f16>(p, a->address, b->address)) {
         out[0] = gemm_rows_few_takes(p, a->dtype) ? 2 : 0;
+    } else if (const Tiles16 tiles = gemm16_tiles(p, a->address, b->address); tiles.rows) {
+        out[0] = 3;
+        out[1] = static_cast<uint32_t>(tiles.rows);
+        out[2] = static_cast<uint32_t>(tiles.columns);
+        out[3] = tiles.splits;
     }
     return TANNIC_SUCCESS;
 }

@@ -95,6 +95,13 @@ bool gemm_rows_few_takes(const GemmProblem& p, int dtype);
 int gemm_rows_few(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 int gemm_few_results(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 int gemm_mfma_f64(const GemmProblem& p, const double* a, const double* b, double* c, hipStream_t stream);
+// 16-bit, more than 64 rows, both operands along K in 16-byte pieces: the tiles of a product that large ones do not fill the chip with and the
+// blocks that share K (no rows: another kernel's)
+struct Tiles16 {
+    int rows, columns;
+    uint32_t splits;
+};
+Tiles16 gemm16_tiles(const GemmProblem& p, const void* a, const void* b);
 int gemm_mfma_16bit(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream, const GemmWorkspace* workspace = nullptr);
 int gemm_mfma_f32(const GemmProblem& p, const float* a, const float* b, float* c, hipStream_t stream, const GemmWorkspace* workspace = nullptr);
 // Operands that do not lie as the tiled kernels want them, copied into dense K-contiguous rows (gemm_repack.hip).  SUCCESS:

@@ -648,6 +648,97 @@ constexpr double kNarrowStep = 0.85;
 // 1024 x 2048 x 16384 83 / 73; with shares of 2048 400 x 11008 x 8192 113 / 117, 400 x 4096 x 8192 44.1 / 44.5).
 constexpr uint32_t kTallShare = 2560;
 
+// Whether both operands are read in 16-byte pieces
+template <class T>
+static bool pieces16(const GemmProblem& p, bool ak, bool bk, const void* a, const void* b) {
+    // 16-byte accesses: addresses, leading dimensions, batch strides and the
+    // contiguous extent must be multiples of a chunk (8 elements of 16 bits, 4 of 32)
+    auto mult8 = [](int64_t v) { return v % kChunkOf<T> == 0; };
+    bool aligned = !(reinterpret_cast<uintptr_t>(a) % 16 || reinterpret_cast<uintptr_t>(b) % 16);
+    aligned = aligned && mult8(ak ? p.a_rs : p.a_cs) && mult8(bk ? p.b_cs : p.b_rs) && mult8(ak ? p.K : p.M) && mult8(bk ? p.K : p.N);
+    for (int d = 0; d < p.batch_rank; ++d) aligned = aligned && mult8(p.a_bs[d]) && mult8(p.b_bs[d]);
+    return aligned;
+}
+
+// How wide tiles of 256 rows are where they fill the chip, 0 where they do not.
+template <class T>
+static int large_width16(const GemmProblem& p, bool ak, bool bk) {
+    // (A tile taller than M multiplies padding.)  Large tiles when they give (nearly) every compute unit one.  Tile width: 256 unless a narrower one needs less time
+    // for its rounds over the 256 compute units (2048 x 14336: 448 tiles 256 wide are two rounds, the second three
+    // quarters full; 512 tiles 224 wide are two full rounds of tiles that take 7/8 of the time; 2048 x 6144 is 192 tiles
+    // 256 wide, and exactly 256 tiles 192 wide).  A narrower tile reads more operand bytes per multiply-add: it has to win
+    // by more than that.
+    const uint64_t tiles_m = (p.M + 255) / 256;
+    int width = 0;
+    double least = 1e30;
+    for (int w : {256, 224, 192}) {
+        if (w != 256 && (sizeof(T) != 2 || !(ak && bk))) continue;   // fp32 tiles and k-row tiles are powers of two wide
+        const uint64_t tiles = tiles_m * ((p.N + w - 1) / w) * p.batches;
+        if (tiles < 200) continue;
+        const double cost = static_cast<double>((tiles + 255) / 256) * w * (1.0 + (256 - w) * kNarrowTilePenalty);
+        if (cost < least) { least = cost; width = w; }
+    }
+    // Not when the last (or only) column of large tiles would be mostly empty (attention's P . V has 64 or 128 columns: fp16
+    // [200, 200] . [200, 64] x 384 takes 31 us on 256 x 256 tiles and 17-19 us on the smaller ones, fp32 140 against 60), and
+    // for fp32 only under a long K: its matrix pipe, not the operand traffic, sets the pace, so what counts is how little
+    // of a tile is padding and how many blocks overlap their starts and ends ([2048, 128] . [128, 2048] x 32: 437 us on
+    // 256 x 256 tiles, 383 on 128 x 128; 4096^3: 1094 against 1105).
+    const bool large_ok = static_cast<double>(p.N) >= 0.75 * (((p.N + 255) / 256) * 256.0) && (sizeof(T) == 2 || p.K >= 1024);
+    return large_ok && p.M > 192 ? width : 0;
+}
+
+// The tiles of a product that large ones do not fill the chip with, and the blocks that share K; `share_bytes`: what there is for partial
+// sums.
+template <class T>
+static Tiles16 small_tiles16(const GemmProblem& p, bool ak, bool bk, size_t share_bytes) {
+    // Fewer large tiles than compute units: choose between the smaller tiles (256 x 128, 128 x 128, 64 x 128) and between
+    // whole K per block and a share of it, by a model of the time (microseconds): blocks on the busiest compute unit x
+    // steps per block x the measured time of one 64-wide step of that tile, a fixed start-up and write-out, and for
+    // shared K the second pass over the fp32 partial sums.
+    const bool tall = p.M > 64;
+    const double steps_all = (p.K + 63) / 64;
+    double best_cost = 1e30;
+    Tiles16 best{tall ? 128 : 64, 128, 1};
+    // (what the direct-to-LDS tiles take, gemm16_dtl)
+    const bool direct = sizeof(T) == 2 && ak && bk && p.K % 64 == 0 && p.a_rs >= static_cast<int64_t>(p.K) && p.a_rs < (1 << 22) && p.b_cs >= static_cast<int64_t>(p.K) &&
+                        p.b_cs < (1 << 22);
+    // (fp32: equal costs go to the 128-row tile, which is tried first)
+    const int heights[3] = {sizeof(T) == 4 ? 128 : 256, sizeof(T) == 4 ? 256 : 128, 64};
+    // Under a short K a block's start and end count: about 2 us for the 128- and 256-row tiles and 0.7 us for the 64-row
+    // one, per round of blocks (fp16, K = 64, [192, 64] . [64, 192] x 384: 23 us on 128 x 128 tiles, 15 us on 64 x 128).
+    const bool short_k = steps_all <= 4 && sizeof(T) == 2;
+    for (int bm : heights) {
+        if ((bm == 128 && !tall) || (bm == 256 && p.M <= 192)) continue;
+        const double block_fixed = short_k ? (bm == 64 ? 0.7 : 2.0) : 0.0;
+        const uint64_t tiles = static_cast<uint64_t>((p.M + bm - 1) / bm) * ((p.N + 127) / 128) * p.batches;
+        for (uint32_t splits : {1u, 2u, 4u, 8u, 16u}) {
+            if (splits > 1 && splits > p.K / (sizeof(T) == 4 ? 64 : 256)) break;
+            // (a workspace too small for that many partial sums may hold those of the 128-row tiles)
+            if (splits > 1 && bm == 256 && (!direct || p.N % 4 != 0 || p.K / splits < kTallShare || static_cast<uint64_t>(splits) * p.batches * p.M * p.N * sizeof(float) > share_bytes)) break;
+            const double blocks = static_cast<double>(tiles) * splits;
+            const double rounds = static_cast<double>((static_cast<uint64_t>(blocks) + 255) / 256);
+            // a step costs more the more compute units pull operands through the L2s at the same time
+            const double busy = blocks < 256.0 ? blocks / 256.0 : 1.0;
+            // (A 64-row tile that walks all of K is register-staged with two stages: between other kernels, with its operands
+            // in no cache, its steps take a fifth longer than in a loop over the same product — 40 against 29 us for
+            // 512 x 4096 x 4096 inside a decoder layer — which those of the direct-to-LDS tiles do not: 33 us with K shared.)
+            double step_us = bm == 256 ? 1.0 : bm == 128 ? 0.375 + 0.175 * busy : splits == 1 ? 0.36 + 0.09 * busy : 0.30 + 0.075 * busy;
+            // fp32: the matrix pipe, sixteen times slower than for the 16-bit types, sets the pace of a step
+            // (2 * bm * 128 * 64 flops at 157.3 TFLOP/s over 256 compute units)
+            if constexpr (sizeof(T) == 4) step_us = std::max(step_us, 2.0 * bm * 128 * 64 / (157.3e6 / 256));
+            double cost = rounds * ((steps_all / splits) * step_us + block_fixed) + 5.0;
+            if (splits > 1) cost += 4.0 + (splits + 0.5) * static_cast<double>(p.M) * p.N * p.batches * 4.0 / 5.0e6;
+            if (cost < best_cost) { best_cost = cost; best.rows = bm; best.splits = splits; }
+        }
+    }
+    if (direct && tall && p.K >= (best.rows == 64 ? 2048 : 1536)) {
+        const uint64_t tiles = static_cast<uint64_t>((p.M + 127) / 128) * ((p.N + 95) / 96) * p.batches;
+        const double cost = steps_all * kNarrowStep * (0.375 + 0.175 * (tiles / 256.0)) + 5.0;
+        if (tiles <= 256 && tiles > 96 && cost < best_cost) best = Tiles16{128, 96, 1};
+    }
+    return best;
+}
+
 template <class T>
 int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream, const GemmWorkspace* workspace) {
     if (p.M == 0 || p.N == 0 || p.batches == 0) return TANNIC_SUCCESS;
@@ -658,12 +749,7 @@ int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream
     const bool ak = p.a_cs == 1, bk = p.b_rs == 1;
     if (!ak && p.a_rs != 1) return TANNIC_UNSUPPORTED_DTYPE;
     if (!bk && p.b_cs != 1) return TANNIC_UNSUPPORTED_DTYPE;
-    // 16-byte accesses: addresses, leading dimensions, batch strides and the
-    // contiguous extent must be multiples of a chunk (8 elements of 16 bits, 4 of 32)
-    auto mult8 = [](int64_t v) { return v % kChunkOf<T> == 0; };
-    bool aligned = !(reinterpret_cast<uintptr_t>(a) % 16 || reinterpret_cast<uintptr_t>(b) % 16);
-    aligned = aligned && mult8(ak ? p.a_rs : p.a_cs) && mult8(bk ? p.b_cs : p.b_rs) && mult8(ak ? p.K : p.M) && mult8(bk ? p.K : p.N);
-    for (int d = 0; d < p.batch_rank; ++d) aligned = aligned && mult8(p.a_bs[d]) && mult8(p.b_bs[d]);
+    const bool aligned = pieces16<T>(p, ak, bk, a, b);
     if (p.batches > 65535) return TANNIC_UNSUPPORTED_DTYPE;
     if (p.b_group_stride) {
         // B's columns in groups: the loaders for any alignment know about them; A is a parameter matrix, K-contiguous
@@ -689,107 +775,49 @@ int run16(const GemmProblem& p, const void* a, const void* b, void* c, hipStream
         if (bk) return launch16<T, 128, 128, 2, false, true, false, false>(p, a, b, c, stream);
         return launch16<T, 128, 128, 2, false, false, false, false>(p, a, b, c, stream);
     }
-    // Tile height by M (a tile taller than M multiplies padding).  Large tiles when they give (nearly) every compute unit one.  Tile width: 256 unless a narrower one needs less time
-    // for its rounds over the 256 compute units (2048 x 14336: 448 tiles 256 wide are two rounds, the second three
-    // quarters full; 512 tiles 224 wide are two full rounds of tiles that take 7/8 of the time; 2048 x 6144 is 192 tiles
-    // 256 wide, and exactly 256 tiles 192 wide).  A narrower tile reads more operand bytes per multiply-add: it has to win
-    // by more than that.
-    const uint64_t tiles_m = (p.M + 255) / 256;
-    int width = 0;
-    double least = 1e30;
-    for (int w : {256, 224, 192}) {
-        if (w != 256 && (sizeof(T) != 2 || !(ak && bk))) continue;   // fp32 tiles and k-row tiles are powers of two wide
-        const uint64_t tiles = tiles_m * ((p.N + w - 1) / w) * p.batches;
-        if (tiles < 200) continue;
-        const double cost = static_cast<double>((tiles + 255) / 256) * w * (1.0 + (256 - w) * kNarrowTilePenalty);
-        if (cost < least) { least = cost; width = w; }
-    }
-    // Not when the last (or only) column of large tiles would be mostly empty (attention's P . V has 64 or 128 columns: fp16
-    // [200, 200] . [200, 64] x 384 takes 31 us on 256 x 256 tiles and 17-19 us on the smaller ones, fp32 140 against 60), and
-    // for fp32 only under a long K: its matrix pipe, not the operand traffic, sets the pace, so what counts is how little
-    // of a tile is padding and how many blocks overlap their starts and ends ([2048, 128] . [128, 2048] x 32: 437 us on
-    // 256 x 256 tiles, 383 on 128 x 128; 4096^3: 1094 against 1105).
-    const bool large_ok = static_cast<double>(p.N) >= 0.75 * (((p.N + 255) / 256) * 256.0) && (sizeof(T) == 2 || p.K >= 1024);
+    const int width = large_width16<T>(p, ak, bk);
     if constexpr (sizeof(T) == 2) {
-        if (large_ok && p.M > 192 && width && width != 256) {
+        if (width && width != 256) {
             const int rc = gemm16_dtl<T>(p, 256, width, a, b, c, stream);
             if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
         }
     }
-    if (large_ok && p.M > 192 && tiles_m * ((p.N + 255) / 256) * p.batches >= 200) {
+    if (width && static_cast<uint64_t>((p.M + 255) / 256) * ((p.N + 255) / 256) * p.batches >= 200) {
         if constexpr (sizeof(T) == 2) {
             const int rc = gemm16_dtl<T>(p, 256, 256, a, b, c, stream);
             if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
         }
         return pick_layout16<T, 256, 256, 2>(p, ak, bk, a, b, c, stream);
     }
-    // Fewer large tiles than compute units: choose between the smaller tiles (256 x 128, 128 x 128, 64 x 128) and between
-    // whole K per block and a share of it, by a model of the time (microseconds): blocks on the busiest compute unit x
-    // steps per block x the measured time of one 64-wide step of that tile, a fixed start-up and write-out, and for
-    // shared K the second pass over the fp32 partial sums.
-    const bool tall = p.M > 64;
-    const double steps_all = (p.K + 63) / 64;
-    double best_cost = 1e30;
-    int best_bm = tall ? 128 : 64, best_bn = 128;
-    uint32_t best_splits = 1;
-    // (what the direct-to-LDS tiles take, gemm16_dtl)
-    const bool direct = sizeof(T) == 2 && ak && bk && p.K % 64 == 0 && p.a_rs >= static_cast<int64_t>(p.K) && p.a_rs < (1 << 22) && p.b_cs >= static_cast<int64_t>(p.K) &&
-                        p.b_cs < (1 << 22);
-    // (fp32: equal costs go to the 128-row tile, which is tried first)
-    const int heights[3] = {sizeof(T) == 4 ? 128 : 256, sizeof(T) == 4 ? 256 : 128, 64};
-    // Under a short K a block's start and end count: about 2 us for the 128- and 256-row tiles and 0.7 us for the 64-row
-    // one, per round of blocks (fp16, K = 64, [192, 64] . [64, 192] x 384: 23 us on 128 x 128 tiles, 15 us on 64 x 128).
-    const bool short_k = steps_all <= 4 && sizeof(T) == 2;
-    for (int bm : heights) {
-        if ((bm == 128 && !tall) || (bm == 256 && p.M <= 192)) continue;
-        const double block_fixed = short_k ? (bm == 64 ? 0.7 : 2.0) : 0.0;
-        const uint64_t tiles = static_cast<uint64_t>((p.M + bm - 1) / bm) * ((p.N + 127) / 128) * p.batches;
-        for (uint32_t splits : {1u, 2u, 4u, 8u, 16u}) {
-            if (splits > 1 && splits > p.K / (sizeof(T) == 4 ? 64 : 256)) break;
-            // (a workspace too small for that many partial sums may hold those of the 128-row tiles)
-            if (splits > 1 && bm == 256 && (!direct || p.N % 4 != 0 || p.K / splits < kTallShare || (workspace && static_cast<uint64_t>(splits) * p.batches * p.M * p.N * sizeof(float) > workspace->bytes))) break;
-            const double blocks = static_cast<double>(tiles) * splits;
-            const double rounds = static_cast<double>((static_cast<uint64_t>(blocks) + 255) / 256);
-            // a step costs more the more compute units pull operands through the L2s at the same time
-            const double busy = blocks < 256.0 ? blocks / 256.0 : 1.0;
-            // (A 64-row tile that walks all of K is register-staged with two stages: between other kernels, with its operands
-            // in no cache, its steps take a fifth longer than in a loop over the same product — 40 against 29 us for
-            // 512 x 4096 x 4096 inside a decoder layer — which those of the direct-to-LDS tiles do not: 33 us with K shared.)
-            double step_us = bm == 256 ? 1.0 : bm == 128 ? 0.375 + 0.175 * busy : splits == 1 ? 0.36 + 0.09 * busy : 0.30 + 0.075 * busy;
-            // fp32: the matrix pipe, sixteen times slower than for the 16-bit types, sets the pace of a step
-            // (2 * bm * 128 * 64 flops at 157.3 TFLOP/s over 256 compute units)
-            if constexpr (sizeof(T) == 4) step_us = std::max(step_us, 2.0 * bm * 128 * 64 / (157.3e6 / 256));
-            double cost = rounds * ((steps_all / splits) * step_us + block_fixed) + 5.0;
-            if (splits > 1) cost += 4.0 + (splits + 0.5) * static_cast<double>(p.M) * p.N * p.batches * 4.0 / 5.0e6;
-            if (cost < best_cost) { best_cost = cost; best_bm = bm; best_splits = splits; }
+    Tiles16 best = small_tiles16<T>(p, ak, bk, workspace ? workspace->bytes : SIZE_MAX);
+    if constexpr (sizeof(T) == 2) {
+        if (best.rows == 256 && best.splits > 1) {
+            const int rc = run16_split<T, 256>(p, ak, bk, best.splits, a, b, c, stream, workspace);
+            if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
+            best = Tiles16{128, 128, best.splits / 2};      // no memory for so many partial sums: as many blocks with half as many
+            if (best.splits == 1) return gemm16_dtl<T>(p, 128, 128, a, b, c, stream);
         }
     }
-    if (direct && tall && p.K >= (best_bm == 64 ? 2048 : 1536)) {
-        const uint64_t tiles = static_cast<uint64_t>((p.M + 127) / 128) * ((p.N + 95) / 96) * p.batches;
-        const double cost = steps_all * kNarrowStep * (0.375 + 0.175 * (tiles / 256.0)) + 5.0;
-        if (tiles <= 256 && tiles > 96 && cost < best_cost) { best_cost = cost; best_bm = 128; best_bn = 96; best_splits = 1; }
-    }
-    if (best_splits > 1) {
-        if constexpr (sizeof(T) == 2) {
-            if (best_bm == 256) {
-                const int rc = run16_split<T, 256>(p, ak, bk, best_splits, a, b, c, stream, workspace);
-                if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
-                best_bm = 128, best_splits /= 2;      // no memory for so many partial sums: as many blocks with half as many
-                if (best_splits == 1) return gemm16_dtl<T>(p, 128, 128, a, b, c, stream);
-            }
-        }
-        if (best_bm == 128) return run16_split<T, 128>(p, ak, bk, best_splits, a, b, c, stream, workspace);
-        return run16_split<T, 64>(p, ak, bk, best_splits, a, b, c, stream, workspace);
+    if (best.splits > 1) {
+        if (best.rows == 128) return run16_split<T, 128>(p, ak, bk, best.splits, a, b, c, stream, workspace);
+        return run16_split<T, 64>(p, ak, bk, best.splits, a, b, c, stream, workspace);
     }
     if constexpr (sizeof(T) == 2) {
-        if (best_bm >= 128) {
-            const int rc = gemm16_dtl<T>(p, best_bm, best_bn, a, b, c, stream);
+        if (best.rows >= 128) {
+            const int rc = gemm16_dtl<T>(p, best.rows, best.columns, a, b, c, stream);
             if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
         }
     }
-    if (best_bm == 256) return pick_layout16<T, 256, 128, 2>(p, ak, bk, a, b, c, stream);
-    if (best_bm == 128) return pick_layout16<T, 128, 128, 2>(p, ak, bk, a, b, c, stream);
+    if (best.rows == 256) return pick_layout16<T, 256, 128, 2>(p, ak, bk, a, b, c, stream);
+    if (best.rows == 128) return pick_layout16<T, 128, 128, 2>(p, ak, bk, a, b, c, stream);
     return pick_layout16<T, 64, 128, 2>(p, ak, bk, a, b, c, stream);
+}
+
+Tiles16 gemm16_tiles(const GemmProblem& p, const void* a, const void* b) {
+    // (the other kernels, of few rows or columns, for operands copied first or loaded at any alignment, come before or instead)
+    if (p.M <= 64 || p.N <= 32 || p.K == 0 || p.batches == 0 || p.batches > 65535 || p.a_cs != 1 || p.b_rs != 1 || p.c_group || p.b_group_stride) return Tiles16{0, 0, 0};
+    if (!pieces16<f16>(p, true, true, a, b) || large_width16<f16>(p, true, true)) return Tiles16{0, 0, 0};
+    return small_tiles16<f16>(p, true, true, SIZE_MAX);
 }
 
 int gemm_mfma_16bit(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream, const GemmWorkspace* workspace) {

@@ -6,6 +6,7 @@ import pytest
 
 import tannic_amd as ta
 from tannic_amd import abi
+import test_gpu_conv_columns
 from test_conv_plan import descriptor, out_shape
 
 
@@ -63,3 +64,23 @@ def test_signals_that_the_other_tiles_load_slowly_stay(x, w):
     assert columns_plan(x, w, start=2) is not None
     assert columns_plan(x, w, strides=(c * (plane + 2), plane + 2, wd, 1)) is not None
     assert columns_plan(x, w, strides=(c * plane + 2, plane, wd, 1)) is not None
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_the_shapes_on_the_gpu_are_these_tiles(dtype):
+    seen = set()
+    for name, (n, c, h, w, o) in test_gpu_conv_columns.SHAPES.items():
+        tiles = columns_plan((n, c, h, w), (o, c, 1, 1), dtype)
+        assert tiles, name
+        seen.add(tiles)
+    assert seen == {(64, 3), (128, 2), (128, 4)}
+    for name, (n, c, h, w, o) in test_gpu_conv_columns.FEW_PIXELS.items():
+        assert columns_plan((n, c, h, w), (o, c, 1, 1), dtype) is None, name
+
+
+@pytest.mark.parametrize("skip", [0, 1, 2, 3])
+def test_parts_of_a_tensor_on_the_gpu(skip):
+    """From an even element on a piece's address is a multiple of four bytes."""
+    c, h, w, o = test_gpu_conv_columns.PART
+    strides = ((c + 3) * h * w, h * w, w, 1)
+    assert bool(columns_plan((300, c, h, w), (o, c, 1, 1), strides=strides, start=skip + strides[0] + 2 * strides[1])) == (skip % 2 == 0)

@@ -1,10 +1,13 @@
 """Which 16-bit products of a few rows with narrow row-major matrices run on the kernel for them, asked of the library without a GPU
-(``tannic_hip_gemm_rows_batch_lanes``)."""
+(``tannic_hip_gemm_rows_batch_lanes``), and which tiles those of a few hundred rows (``tannic_hip_gemm_plan``): the products of the GPU
+tests are the kernels' that these name."""
 import ctypes as C
 
 import pytest
 
 import tannic_amd as ta
+import test_gpu_decode_ops
+import test_gpu_gemm_shares
 from tannic_amd import abi
 from test_conv_plan import descriptor
 
@@ -87,3 +90,34 @@ FEW_RESULTS = {
 def test_few_results_of_row_major_matrices(name, dtype):
     problem, taken = FEW_RESULTS[name]
     assert (product_plan(*problem, dtype)[0] == 2) == taken
+
+
+def plan_of(x, w, y):
+    out = (C.c_uint32 * 4)()
+    assert ta.library().gemm_plan(C.byref(x), C.byref(w), C.byref(y), out) == abi.SUCCESS
+    return tuple(out)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("batch,m,n,k", test_gpu_decode_ops.PRODUCTS)
+def test_few_results_on_the_gpu_are_that_kernel(batch, m, n, k, dtype):
+    x, w, y = (descriptor(dtype, s) for s in ((batch, m, k), (batch, k, n), (batch, m, n)))
+    x.address += 2
+    x.strides.sizes[:2] = m * (k + 3), k + 3
+    w.strides.sizes[0] = (k + 7) * n
+    assert plan_of(x, w, y)[0] == 2
+
+
+# rows and columns of a tile, and whether its K is shared
+TILES = {**{p: (128, 96, False) for p in test_gpu_gemm_shares.NARROW}, **{p: (256, 128, True) for p in test_gpu_gemm_shares.SHARED},
+         **{p: (64, 128, False) for p in test_gpu_gemm_shares.BESIDE}}
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("m,n,k", list(TILES))
+def test_tiles_of_long_products_on_the_gpu(m, n, k, dtype):
+    x, w, y = (descriptor(dtype, s) for s in ((m, k), (k, n), (m, n)))
+    x.strides.sizes[0] = k + 8
+    w.strides.sizes[:2] = 1, k + 16
+    kernel, rows, columns, shares = plan_of(x, w, y)
+    assert (kernel, rows, columns, shares > 1) == (3, *TILES[m, n, k])

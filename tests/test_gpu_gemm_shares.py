@@ -15,13 +15,15 @@ EPS = {ta.float16: 2.0 ** -11, ta.bfloat16: 2.0 ** -8}
 
 # M, N, K: rows that end in a tile's first half, its last row or with it, columns that end in a tile of 96 or in a piece of eight, K of whole
 # steps that the stages do not divide
-NARROW = [(129, 6144, 2112), (385, 5128, 1536), (300, 6150, 1600), (65, 22000, 2048), (768, 3000, 1536), (512, 6144, 2048)]
+NARROW = [(129, 6144, 2112), (385, 5128, 1536), (300, 6150, 2112), (65, 22000, 2048), (768, 3000, 1536), (512, 6144, 2048)]
 # and shares of K of different lengths
 SHARED = [(256, 4096, 20544), (250, 4092, 20544), (512, 4092, 10304), (511, 4084, 14400), (1020, 2044, 10368)]
+# and what goes to the 64-row tiles beside them
+BESIDE = [(300, 6150, 1600)]
 
 
 @pytest.mark.parametrize("dtype", [ta.float16, ta.bfloat16], ids=str)
-@pytest.mark.parametrize("m,n,k", NARROW + SHARED)
+@pytest.mark.parametrize("m,n,k", NARROW + SHARED + BESIDE)
 def test_tiles_of_long_products(m, n, k, dtype, device):
     """Both matrices are parts of larger ones; what lies beside them is infinite."""
     rng = np.random.default_rng(7)
