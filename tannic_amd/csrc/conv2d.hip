@@ -106,7 +106,8 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     // Kernels in order of preference.  A 1x1 kernel has no tap to amortise a staged patch over: its weights stay in
     // registers when they fit (conv2d_k1.hip), otherwise it is a matrix product per image (conv2d_pointwise.hip).
     const bool pointwise = p.KH == 1 && p.KW == 1;
-    // fp32 1x1, 3x3 and 7x7 (few channels) have a kernel of their own; what it refuses (weights that are not whole 16-byte pieces,
+    // fp32 1x1 and 3x3 run on the 16-bit matrix pipe where that takes less time than the kernel after it is expected to (plan_split).
+    // fp32 1x1, 3x3 and 7x7 (few channels) have a kernel of their own on the fp32 pipe; what it refuses (weights that are not whole 16-byte pieces,
     // planes wider than its LDS, few results, what others do in less time: plan_f32) goes on like the 16-bit types and the other kernel sizes.
     int status = conv2d_split(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;

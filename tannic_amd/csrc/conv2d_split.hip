@@ -1,10 +1,10 @@
 // conv2d in fp32 on the 16-bit matrix pipe: every value is the sum of three bfloat16 values, 1x1 and 3x3 kernels.
 //
-// The fp32 matrix pipe does 64 multiply-adds a clock and SIMD, the bfloat16 one 512.  A float is exactly the sum of three bfloat16 values
+// The fp32 matrix pipe does 32 multiply-adds a clock and SIMD, the bfloat16 one 512.  A float is exactly the sum of three bfloat16 values
 // (24 bits of mantissa, three times eight; each part the nearest to what the ones before left), and of the nine products of parts the
 // six largest carry everything above 2^-24 of the product: x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0, each exact, summed in fp32.  Six MFMAs of
-// 16 x 16 x 32 take the place of eight of 16 x 16 x 4 of twice the length: 2.7 times the rate of the fp32 pipe, 1.9 times after the clock that
-// this much work leaves (1.4 PFLOP/s of bfloat16 products, the rate of the large products; 233 TFLOP/s of fp32).
+// 16 x 16 x 32 take the place of eight of 16 x 16 x 4 of twice the length: 2.7 times the rate of the fp32 pipe, 1.5 times after the clock that
+// this much work leaves (1.4 PFLOP/s of bfloat16 products, the rate of the large products, are 233 TFLOP/s of fp32; the fp32 pipe does 157).
 // The error against 64 bits is below that of the fp32 pipe, which rounds after every product where this rounds after 32: the five small
 // products have accumulators of their own (a rounding there is 2^-8 of one beside the large ones), and the large ones' sums are
 // chains of nine taps (1x1: of 512 products).  256 -> 256 3x3 over 14 x 14: 1.07e-7 of the result's norm, 1.80e-7 on the fp32 pipe;
@@ -12,7 +12,9 @@
 //  * The weights are split by a kernel of their own, into the order in which the MFMAs want them; wavefronts load them straight into
 //    registers, 16 bytes a lane.  The signal is split on its way into LDS: a lane takes eight channels of a place of the tile's plane (the
 //    rows that the tile touches, padding made real, as in conv2d_f32.hip), eight loads of one float each, whole lines for the
-//    wavefront, and writes 16 bytes to each of three planes of 32 channels.  So nothing is asked of widths, alignments, strides or channels.
+//    wavefront, and writes 16 bytes to each of three planes of 32 channels.  So nothing is asked of the signal's widths, alignment or
+//    strides.  Of the weights plan_split asks what conv2d_f32.hip does (whole 16-byte pieces, a K that four divides): that kernel's
+//    expected time is what this one's is held against.
 //  * A wavefront's tile is 32 output channels by 16 PT pixels of the flattened batch; WO wavefronts of a block's four lie along the
 //    channels.  A tap of 32 channels is 12 PT MFMAs for six loads of weights and 3 PT reads of LDS.
 //  * Both operands are split 2^24 times as large as they are, so that the last bit of the smallest fp32 value (2^-149) is a normal bfloat16: no

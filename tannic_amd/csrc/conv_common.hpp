@@ -39,7 +39,7 @@ int conv2d_stem(const ConvProblem& p, int dtype, const void* x, const void* w, c
 int conv2d_k3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_resident(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_patch(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
-// fp32 1x1 (from 140 channels on) and 3x3 on the 16-bit matrix pipe, every value as three bfloat16 values
+// fp32 1x1 (from 100 channels on, 140 under fewer than 128 output channels) and 3x3 (from 32) on the 16-bit matrix pipe, every value as three bfloat16 values
 int conv2d_split(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 // 16-bit 3x3, a batch of small maps under many channels, over the flattened batch
 int conv2d_batch3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
