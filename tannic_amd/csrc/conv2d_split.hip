@@ -24,7 +24,7 @@
 //    20 x 20, sixteen images, 35 us; one infinity 178, one in every ninth value of a channel 320; 52 on the fp32 pipe.  Weights or signals of 1e-37
 //    beside ordinary ones 1.1e-7 of their own results, 1.5e-7 on the fp32 pipe.)
 // With few tiles the channels are shared between `splits` blocks per tile, partial sums in fp32, added in split order by a second kernel.
-// Measured, 53 convolutions of a ResNet-50 and their additions, batch 32: 3351 -> 2777 us (the layers: plan_split).
+// Measured, 53 convolutions of a ResNet-50 and their additions, batch 32: 3350 -> 2740 .. 2880 us by the card (the layers: plan_split).
 // What is left: the weights' kernel (3 - 5 us of a layer's 30 - 50), a block's start and end (some 9 us), the last round of tiles.
 #include "conv_common.hpp"
 
