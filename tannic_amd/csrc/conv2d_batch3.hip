@@ -323,10 +323,11 @@ static int launch_batch3(const ConvProblem& p, const Batch3Plan& q, const void* 
     return launch_status("conv2d_batch3_kernel");
 }
 
+constexpr uint32_t COMPUTE_UNITS = 256;
+
 // one of the kernels below as a candidate: its plan and the time it is expected to take
 template <int PT, int WO, int NL>
 static void consider_batch3(const ConvProblem& p, Batch3Plan& best, double& best_time, int& best_index, int index) {
-    constexpr uint32_t COMPUTE_UNITS = 256;
     Batch3Plan q{};
     q.pixels = p.N * p.HO * p.WO;
     q.ptile = 16 * PT * (4 / WO);
@@ -354,11 +355,18 @@ static void consider_batch3(const ConvProblem& p, Batch3Plan& best, double& best
         if (splits > 1 && (per_split * (splits - 1) >= q.chunks || tiles * (splits - 1) >= 2 * COMPUTE_UNITS)) continue;
         const uint64_t blocks = tiles * splits;
         if (blocks >= (1ull << 24)) continue;
-        // Microseconds: a chunk of a block, twice as long for both where two share a compute unit; a block's start and end; the weights' kernel;
-        // the pass over partial sums.
-        const double rounds = static_cast<double>((blocks + COMPUTE_UNITS - 1) / COMPUTE_UNITS);
-        const double chunk = (9.0 * 2 * PT * 16 + 600.0 + NL * 100.0) / 2100.0;
-        const double time = rounds * (per_split * chunk * (rounds > 1.0 && PT <= 4 ? 0.9 : 1.0) + 2.0) + 8.0 + (splits > 1 ? 4.0 + splits * static_cast<double>(q.pixels) * p.O * 8 / 4e6 : 0.0);
+        // Microseconds, within 4 % of 606 problems of one round and 8 % of 167 of more: a chunk of a block, alone on its compute unit with its loads'
+        // latency to wait for, or beside and behind others; launches, a block's start and end; the pass over partial sums.  (Before, a chunk alone was
+        // priced at two thirds of its time, and few blocks were left to walk all channels: 320 -> 512 over 20 x 24, one image, 64 blocks 23.5 us,
+        // with shares of K 20.9; 448 -> 624 over 13 x 16, three images, 100 blocks 31.7 / 24.6.)
+        const double rounds = static_cast<double>((blocks + COMPUTE_UNITS - 1) / COMPUTE_UNITS), results = static_cast<double>(q.pixels) * p.O;
+        double time;
+        if (rounds == 1.0) {
+            time = per_split * (0.113 * PT + 0.156 * NL + 0.4) + 8.4 + (splits > 1 ? 3.0 + 1.8e-6 * splits * results : 0.0);
+        } else {
+            const double chunk = (9.0 * 2 * PT * 16 + 600.0 + NL * 100.0) / 2100.0 * (PT <= 4 ? 0.9 : 1.0);
+            time = (PT <= 4 ? 1.35 : 1.35 + 0.05 * rounds) * (rounds * (per_split * chunk + 2.0) + 8.0 + (splits > 1 ? 4.0 + 2e-6 * splits * results : 0.0));
+        }
         if (time < best_time) {
             best_time = time;
             best = q;
@@ -402,7 +410,13 @@ static int plan_batch3(const ConvProblem& p, int dtype, const void* x, const voi
     //  * few pixels an image: the weights are brought into order for few pixels (512 -> 512 over 7 x 7: sixteen images 29 / 30, 32 images 32.5 / 31;
     //    with a stride, which leaves the unfolded operand small, from 14 x 14 32 / 37, 256 -> 256 from 28 x 28 32 images 37 / 29, eight 26.6 / 27.1)
     if (pixels < p.C || (image < 100 && pixels < 3ull * p.C)) return -1;
-    if ((p.stride_h > 1 || p.stride_w > 1) && (image < 100 || pixels < 3000)) return -1;
+    // (few pixels in all, where the unfolded batch is as small as the weights: 320 -> 512 over 20 x 24, one image, 18.6 / 20.9, 272 -> 592 over 19 x 18
+    // 16.8 / 18.7, 200 -> 560 over 12 x 9, four images, 16.2 / 17.2, 256 -> 736 over 25 x 22 19.7 / 21.5; but 136 -> 448 over 13 x 10, four images, 15.2 / 14.5,
+    // channels that eight does not divide, whose weights the product wants padded, 278 -> 512 over 22 x 24 25.2 / 21.7, and from 600 pixels on
+    // 448 -> 192 over 19 x 16, two images, 18.8 / 17.2)
+    const bool strided = p.stride_h > 1 || p.stride_w > 1;
+    if (!strided && pixels < 560 && p.C % 8 == 0 && p.C >= 150) return -1;
+    if (strided && (image < 100 || pixels < 3000)) return -1;
     //  * many pixels: the patch kernel fills the chip too.  While there is not a block here for every compute unit this one is ahead
     //    (256 -> 256, 32 images of 14 x 14 29.4 / 23.6, sixteen 30.9 / 20.4, sixteen of 20 x 20 35.9 / 22.3, 24 of 16 x 16 24.7 / 22.4; 128 -> 128, eight of
     //    28 x 28 19.4 / 15.3), beyond only where rows are no whole vectors (128 -> 128, 32 of 28 x 28 21.8 / 20.3, 512 -> 512, eight of 28 x 28
@@ -413,6 +427,19 @@ static int plan_batch3(const ConvProblem& p, int dtype, const void* x, const voi
     double time = 1e30;
     int index = -1, counter = 0;
     TH_BATCH3(TH_BATCH3_CONSIDER)
+    if (index < 0) return -1;
+    //  * the patch kernel in one round that is more than half full, where this one takes two or more (192 -> 512, nineteen images of 22 x 20
+    //    30.2 / 37.6, 128 -> 768, fifteen, 26.8 / 30.5, 576 -> 816, seven of 28 x 28 75 / 87, with a stride 480 -> 16, 42 images of 45 x 46 41.7 / 58;
+    //    less than half full 256 -> 278, 25 of 20 x 20 36.6 / 32.3, in two rounds 192 -> 691, twenty of 24 x 22 81 / 47); rows of an odd number of pixels
+    //    lie at odd addresses there (128 -> 816, twelve of 24 x 25 46 / 35, 160 -> 816, 53 of 16 x 19 83 / 71; but 576 -> 816, seven of 26 x 29, 78 / 87)
+    if (whole_chunks && p.W % 2 == 0) {
+        const K3Load there = conv2d_k3_load(p, x, w);
+        const uint64_t blocks = (pixels + q.ptile - 1) / q.ptile * q.co_tiles * q.splits;
+        if (blocks > COMPUTE_UNITS && there.blocks && there.blocks <= there.at_once && there.blocks * 100 >= there.at_once * 58ull) return -1;
+        //  * with a stride: rows in whole vectors of larger images there (160 -> 32, sixteen of 45 x 48 18.4 / 20, 224 -> 32 22.9 / 24.2; smaller ones
+        //    416 -> 128, thirty of 30 x 32, 0.90), and three chunks with two blocks on a compute unit (96 -> 28, 49 of 32 x 30 13.8 / 15.5)
+        if (strided && there.blocks && (there.flat ? p.C < 128 && there.at_once > 256 : image > 500)) return -1;
+    }
     return index;
 }
 

@@ -410,34 +410,43 @@ int launch_k3(bool flat, const ConvProblem& p, const K3Plan& q, size_t lds, uint
     return launch_k3_as<T, TN, ONE_STAGE, KH, KW, BPC, false>(p, q, lds, blocks, x, w, bias, y, stream);
 }
 
-template <class T, int KH, int KW>
-int run_k3(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
+// Rows of the result a block owns (none: the problem is not this kernel's), rows of its patch, 128 pixels a block `tn` times; mode 0: two
+// stages; 1: one stage, two blocks per compute unit; 2: one stage, one block.
+struct K3Tiles {
+    uint32_t R, IH;
+    int tn, mode;
+    bool flat, fits;      // `fits`: the operands lie as the kernel wants them
+};
+
+template <int KH, int KW>
+static K3Tiles choose_k3(const ConvProblem& p, const void* x, const void* w) {
     constexpr uint32_t TAPS = KH * KW, WEIGHT_ELEMS = TAPS * kK3BCO * kK3CH;
-    if (p.KH != KH || p.KW != KW) return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.C == 0 || p.C % kK3CH != 0 || p.xs[3] != 1) return TANNIC_UNSUPPORTED_DTYPE;
+    constexpr size_t ES = 2;
+    K3Tiles q{};
+    if (p.KH != KH || p.KW != KW) return q;
+    if (p.C == 0 || p.C % kK3CH != 0 || p.xs[3] != 1) return q;
     // 16-byte loads.  Aligned staging: rows a multiple of 8 wide, rows, channels and images starting at multiples of 8
     // elements.  Otherwise flat staging: rows that follow each other in memory (a channel plane is one run), at least four
     // columns, and at least eight elements of the image in every block's patch (its rows inside the image: KH - pad_h or more).
     const bool aligned = p.W % 8 == 0 && p.xs[2] % 8 == 0 && p.xs[1] % 8 == 0 && p.xs[0] % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
-    const bool flat = !aligned;
-    if (flat && (p.xs[2] != static_cast<int64_t>(p.W) || p.W < 4 || p.pad_h >= KH || p.H < KH - p.pad_h || static_cast<uint64_t>(KH - p.pad_h) * p.W < 8 ||
-                 reinterpret_cast<uintptr_t>(x) % sizeof(T) != 0))
-        return TANNIC_UNSUPPORTED_DTYPE;
+    q.flat = !aligned;
+    if (q.flat && (p.xs[2] != static_cast<int64_t>(p.W) || p.W < 4 || p.pad_h >= KH || p.H < KH - p.pad_h || static_cast<uint64_t>(KH - p.pad_h) * p.W < 8 ||
+                 reinterpret_cast<uintptr_t>(x) % ES != 0))
+        return q;
     if (p.ws[3] != 1 || p.ws[2] != KW || p.ws[1] != static_cast<int64_t>(TAPS) || p.ws[0] != static_cast<int64_t>(p.C) * TAPS || reinterpret_cast<uintptr_t>(w) % 16 != 0)
-        return TANNIC_UNSUPPORTED_DTYPE;
-    if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0) return TANNIC_SUCCESS;
-    K3Plan q{};
-    q.IWp = p.W + 2 * p.pad_w;
+        return q;
+    q.fits = true;
+    if (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0) return q;
+    const uint32_t IWp = p.W + 2 * p.pad_w;
     const size_t budget = 158 * 1024;
     // the largest number of output rows whose tile fits: pixels, LDS, staging registers
-    int tn = 0, mode = 0;   // mode 0: two stages; 1: one stage, two blocks per compute unit; 2: one stage, one block
     double best = 0.0;
     auto consider = [&](uint32_t R, int m, double weight) {
         const uint32_t IH = (R - 1) * p.stride_h + KH;
-        const size_t stage = (static_cast<size_t>(WEIGHT_ELEMS) + static_cast<size_t>(IH) * q.IWp * kK3CH) * sizeof(T);
-        const uint64_t microblocks = flat ? 4ull * ((static_cast<uint64_t>(p.W) * IH + 7) / 8) : 4ull * (p.W / 8) * IH;
+        const size_t stage = (static_cast<size_t>(WEIGHT_ELEMS) + static_cast<size_t>(IH) * IWp * kK3CH) * ES;
+        const uint64_t microblocks = q.flat ? 4ull * ((static_cast<uint64_t>(p.W) * IH + 7) / 8) : 4ull * (p.W / 8) * IH;
         const int t = R * p.WO > 256 ? 4 : 2;
-        const size_t out_bytes = static_cast<size_t>(kK3BCO) * (128 * t + 8) * sizeof(T);
+        const size_t out_bytes = static_cast<size_t>(kK3BCO) * (128 * t + 8) * ES;
         if (microblocks > (m == 1 ? 1 : kK3Passes) * kK3Threads) return;
         if (m == 0 && 2 * stage > budget) return;
         if (m == 1 && (stage > budget / 2 || out_bytes > budget / 2 || t != 2)) return;
@@ -446,7 +455,7 @@ int run_k3(const ConvProblem& p, const void* x, const void* w, const void* bias,
         const double rows = static_cast<double>(p.HO) / (((p.HO + R - 1) / R) * R);    // rows of the last block that exist
         const double halo = static_cast<double>(R * p.stride_h) / IH;                  // input rows read once
         const double score = weight * fill * rows * (0.5 + 0.5 * halo);
-        if (score >= best) { best = score; q.R = R; q.IH = IH; tn = t; mode = m; }
+        if (score >= best) { best = score; q.R = R; q.IH = IH; q.tn = t; q.mode = m; }
     };
     constexpr bool SMALL = TAPS <= 9;   // a larger kernel's chunk of weights leaves room for one stage of one block only
     if (SMALL)
@@ -459,7 +468,22 @@ int run_k3(const ConvProblem& p, const void* x, const void* w, const void* bias,
     // 5x5: one stage, the whole LDS, tiles of at most 256 pixels (what the registers hold next to 25 taps of weights).
     if (!SMALL)
         for (uint32_t R = 1; R <= p.HO && R * p.WO <= 256; ++R) consider(R, 2, 1.0);
-    if (best == 0.0) return TANNIC_UNSUPPORTED_DTYPE;
+    return q;
+}
+
+template <class T, int KH, int KW>
+int run_k3(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
+    constexpr uint32_t WEIGHT_ELEMS = KH * KW * kK3BCO * kK3CH;
+    constexpr bool SMALL = KH * KW <= 9;   // a larger kernel's chunk of weights leaves room for one stage of one block only
+    const K3Tiles tiles = choose_k3<KH, KW>(p, x, w);
+    if (tiles.fits && (p.N == 0 || p.O == 0 || p.HO == 0 || p.WO == 0)) return TANNIC_SUCCESS;
+    if (tiles.R == 0) return TANNIC_UNSUPPORTED_DTYPE;
+    const int tn = tiles.tn, mode = tiles.mode;
+    const bool flat = tiles.flat;
+    K3Plan q{};
+    q.IWp = p.W + 2 * p.pad_w;
+    q.R = tiles.R;
+    q.IH = tiles.IH;
     q.row_blocks = (p.HO + q.R - 1) / q.R;
     q.co_tiles = (p.O + kK3BCO - 1) / kK3BCO;
     q.patch_records = q.IH * q.IWp;
@@ -506,6 +530,12 @@ int conv2d_k5(const ConvProblem& p, int dtype, const void* x, const void* w, con
     return TANNIC_UNSUPPORTED_DTYPE;
 }
 #else
+K3Load conv2d_k3_load(const ConvProblem& p, const void* x, const void* w) {
+    const K3Tiles q = choose_k3<3, 3>(p, x, w);
+    if (q.R == 0) return K3Load{0, 0, false};
+    return K3Load{static_cast<uint64_t>(p.N) * ((p.HO + q.R - 1) / q.R) * ((p.O + kK3BCO - 1) / kK3BCO), q.mode == 1 ? 512u : 256u, q.flat};
+}
+
 int conv2d_k3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
     if (p.KH == 5 && p.KW == 5) return conv2d_k5(p, dtype, x, w, bias, y, stream);
     if (dtype == TANNIC_FLOAT16) return run_k3<f16, 3, 3>(p, x, w, bias, y, stream);

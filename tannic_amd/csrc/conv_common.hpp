@@ -41,6 +41,14 @@ int conv2d_resident(const ConvProblem& p, int dtype, const void* x, const void* 
 int conv2d_patch(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 // fp32 1x1 (from 100 channels on, 140 under fewer than 128 output channels) and 3x3 (from 32) on the 16-bit matrix pipe, every value as three bfloat16 values
 int conv2d_split(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
+// the blocks of conv2d_k3 for a 16-bit 3x3 problem (none where it does not take it), how many of them the chip runs at once, whether rows are no
+// whole aligned vectors
+struct K3Load {
+    uint64_t blocks;
+    uint32_t at_once;
+    bool flat;
+};
+K3Load conv2d_k3_load(const ConvProblem& p, const void* x, const void* w);
 // 16-bit 3x3, a batch of small maps under many channels, over the flattened batch
 int conv2d_batch3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 // the time (us) that conv2d_f32 is expected to take; negative where it does not take the problem
