@@ -358,7 +358,7 @@ static void consider_batch3(const ConvProblem& p, Batch3Plan& best, double& best
         // Microseconds, within 4 % of 606 problems of one round and 8 % of 167 of more: a chunk of a block, alone on its compute unit with its loads'
         // latency to wait for, or beside and behind others; launches, a block's start and end; the pass over partial sums.  (Before, a chunk alone was
         // priced at two thirds of its time, and few blocks were left to walk all channels: 320 -> 512 over 20 x 24, one image, 64 blocks 23.5 us,
-        // with shares of K 20.9; 448 -> 624 over 13 x 16, three images, 100 blocks 31.7 / 24.6.)
+        // with shares of K 20.9; 448 -> 624 over 13 x 16, three images, 100 blocks 31.7 / 25.2.)
         const double rounds = static_cast<double>((blocks + COMPUTE_UNITS - 1) / COMPUTE_UNITS), results = static_cast<double>(q.pixels) * p.O;
         double time;
         if (rounds == 1.0) {

@@ -642,7 +642,12 @@ constexpr double kNarrowTilePenalty = 0.001;
 // leave compute units idle (bf16, every W from memory, us on 128 wide / 96: 512 x 6144 x 4096 44 / 40, 512 x 5120 x 5120 54 / 48,
 // 768 x 3072 x 3072 34 / 31.4).  One round of them only, a long K, and more than 96 of them (the register-staged 64-row tiles are the better
 // ones under a short K or with few tiles: 256 x 7168 x 1536 19.2 / 20.1, 256 x 4096 x 2048 19.6 / 20.5; 512 x 4096 x 2048 21.9 / 20.9).
+// Below K = 4096, where the others share K, the estimate has to be a microsecond lower (77 x 12864 x 2560 23.5 / 24.8, 847 x 1504 x 3008 20.6 / 21.6), and two more where rows
+// of the result are no whole 16-byte pieces, which the pass over the partial sums and the 64-row tiles store faster (320 x 4084 x 2944 20.1 / 24.7,
+// 749 x 1708 x 2624 19.2 / 23.3, 451 x 2964 x 2048 16.2 / 18.8; but under a longer K 180 x 8436 x 7424 74 / 50, 533 x 3860 x 12160 0.76).  Beyond K = 14336 the times are uneven (733 x 3360 x 16320 124 / 149, 768 x 2764 x 14464
+// 107 / 121, 553 x 4416 x 14528 0.85).  Of 453 products that these tiles took 39 were slower for it, of those that they still take 5.
 constexpr double kNarrowStep = 0.85;
+constexpr uint32_t kNarrowLongest = 14336;
 // What of K a block with 256 rows gets at least where K is shared: half as many tiles, twice as many shares as with 128 rows, so the operands
 // cross the L2s less often and more partial sums are added (bf16, us with 128 rows / 256: 512 x 4096 x 14336 87 / 77, 768 x 7168 x 11008 183 / 147,
 // 1024 x 2048 x 16384 83 / 73; with shares of 2048 400 x 11008 x 8192 113 / 117, 400 x 4096 x 8192 44.1 / 44.5).
@@ -731,9 +736,11 @@ static Tiles16 small_tiles16(const GemmProblem& p, bool ak, bool bk, size_t shar
             if (cost < best_cost) { best_cost = cost; best.rows = bm; best.splits = splits; }
         }
     }
-    if (direct && tall && p.K >= (best.rows == 64 ? 2048 : 1536)) {
+    if (direct && tall && p.K >= (best.rows == 64 ? 2048 : 1536) && p.K <= kNarrowLongest) {
         const uint64_t tiles = static_cast<uint64_t>((p.M + 127) / 128) * ((p.N + 95) / 96) * p.batches;
-        const double cost = steps_all * kNarrowStep * (0.375 + 0.175 * (tiles / 256.0)) + 5.0;
+        const bool shares = best.splits > 1 && p.K < 4096, small = best.rows == 64 && best.splits == 1 && p.K <= 3072;
+        const double margin = (shares ? 1.0 : 0.0) + (p.N % 8 != 0 && (shares || small) ? 2.0 : 0.0);
+        const double cost = steps_all * kNarrowStep * (0.375 + 0.175 * (tiles / 256.0)) + 5.0 + margin;
         if (tiles <= 256 && tiles > 96 && cost < best_cost) best = Tiles16{128, 96, 1};
     }
     return best;

@@ -113,6 +113,18 @@ TILES = {**{p: (128, 96, False) for p in test_gpu_gemm_shares.NARROW}, **{p: (25
          **{p: (64, 128, False) for p in test_gpu_gemm_shares.BESIDE}}
 
 
+# rows of the result that are no whole pieces, and a K beyond the tiles' longest, go to other tiles
+NARROW_RULES = {(512, 3232, 2816): True, (437, 3944, 3200): False, (451, 2968, 2048): True, (451, 2964, 2048): False, (670, 3660, 2688): True,
+                (320, 4084, 2944): False, (180, 8436, 7424): True, (512, 4352, 14336): True, (512, 4352, 14400): False}
+
+
+@pytest.mark.parametrize("m,n,k", list(NARROW_RULES))
+def test_narrow_tiles(m, n, k):
+    x, w, y = (descriptor("bfloat16", s) for s in ((m, k), (k, n), (m, n)))
+    w.strides.sizes[:2] = 1, k
+    assert (plan_of(x, w, y)[2] == 96) == NARROW_RULES[m, n, k]
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("m,n,k", list(TILES))
 def test_tiles_of_long_products_on_the_gpu(m, n, k, dtype):

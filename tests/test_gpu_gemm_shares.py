@@ -15,11 +15,11 @@ EPS = {ta.float16: 2.0 ** -11, ta.bfloat16: 2.0 ** -8}
 
 # M, N, K: rows that end in a tile's first half, its last row or with it, columns that end in a tile of 96 or in a piece of eight, K of whole
 # steps that the stages do not divide
-NARROW = [(129, 6144, 2112), (385, 5128, 1536), (300, 6150, 2112), (65, 22000, 2048), (768, 3000, 1536), (512, 6144, 2048)]
+NARROW = [(129, 6144, 2112), (385, 5128, 1536), (201, 8789, 1536), (326, 5454, 1600), (65, 22000, 2048), (768, 3000, 1536), (512, 6144, 2048)]
 # and shares of K of different lengths
 SHARED = [(256, 4096, 20544), (250, 4092, 20544), (512, 4092, 10304), (511, 4084, 14400), (1020, 2044, 10368)]
 # and what goes to the 64-row tiles beside them
-BESIDE = [(300, 6150, 1600)]
+BESIDE = [(300, 6150, 1600), (300, 6150, 2112)]
 
 
 @pytest.mark.parametrize("dtype", [ta.float16, ta.bfloat16], ids=str)
