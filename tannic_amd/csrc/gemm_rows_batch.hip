@@ -193,10 +193,13 @@ static bool rows_few_takes(const GemmProblem& p) {
     // Rows of W that are an odd number of 16-byte pieces: a block's 32 bytes of one lie in two lines every other time, and fewer than 64 blocks
     // under a long K are bound by the lines each has on its way (bf16, four rows, us on the kernel for few results / here, W in no cache: 104
     // columns under 8192 22 / 27, 200 under 16384 39 / 50, two products 39 / 49, four 43 / 50; W in the caches 200 under 16384 33.4 / 35.6, 72 32 / 35, but
-    // 200 under 4096 14 / 12, 72 under 8192 15 / 13, two products 20 / 13; up to 64 columns from 32768 on, 40 under 65536 75 / 84, under 16384 23 / 19).  104 blocks of 200 columns under 16384 82 / 51, and
-    // 192 columns 45 / 46, two products of 128 46 / 44.
-    const uint64_t blocks = static_cast<uint64_t>((p.N + 15) / 16) * p.batches;
-    return p.N % 16 == 0 || p.N == 8 || blocks >= 64 || p.K < (p.N > 96 ? 6144u : p.N > 64 ? 12288u : 32768u);
+    // 200 under 4096 14 / 12, 72 under 8192 15 / 13, two products 20 / 13; up to 64 columns from 32768 on, 40 under 65536 75 / 84, under 16384 23 / 19;
+    // rows of an even number, under 16384: 192 columns 45 / 46, two products of 128 46 / 44).  And a last pass over less than 1024 rows costs nearly what a whole one does (two products of 72 columns under 4200 13.7 / 15.4, 6 of 40 12.0 / 13.2,
+    // two of 88 under 8250 20.2 / 22.2; under 5200 ten of 40 13.7 / 13.7, under 3000 72 12.8 / 11.4).  The kernel for few results does these in one round
+    // of workgroups; in two it takes twice as long (five products of 200 under 18417 53 / 57, six 94 / 58; twenty of 56 under 4200 22.2 / 14.6).
+    if (p.N % 16 == 0 || p.N == 8 || static_cast<uint64_t>((p.N + 3) / 4) * p.batches > 256) return true;
+    const uint32_t last = p.K % kRowsFewPass;
+    return p.K < (p.N > 96 ? 6144u : p.N > 64 ? 12288u : 32768u) && (p.K <= kRowsFewPass || last == 0 || last >= 1024);
 }
 
 bool gemm_rows_few_takes(const GemmProblem& p, int dtype) {

@@ -82,6 +82,15 @@ FEW_RESULTS = {
     "few_odd_pieces": ((1, 4, 40, 32760), True),
     "few_odd_pieces_long_k": ((1, 4, 40, 32768), False),
     "one_piece": ((1, 4, 8, 200000), True),
+    # and a short last pass of 4096 rows
+    "odd_pieces_one_pass": ((2, 2, 72, 4096), True),
+    "odd_pieces_short_pass": ((2, 2, 72, 4097), False),
+    "odd_pieces_shorter_pass": ((2, 2, 72, 5119), False),
+    "odd_pieces_longer_pass": ((2, 2, 72, 5120), True),
+    "odd_pieces_short_third_pass": ((2, 1, 88, 8250), False),
+    "odd_pieces_short_pass_more_blocks": ((15, 1, 72, 4200), True),
+    "odd_pieces_short_pass_fewer_blocks": ((14, 1, 72, 4200), False),
+    "even_pieces_short_pass": ((2, 2, 80, 4200), True),
 }
 
 
@@ -99,13 +108,13 @@ def plan_of(x, w, y):
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
-@pytest.mark.parametrize("batch,m,n,k", test_gpu_decode_ops.PRODUCTS)
+@pytest.mark.parametrize("batch,m,n,k", test_gpu_decode_ops.PRODUCTS + test_gpu_decode_ops.BESIDE)
 def test_few_results_on_the_gpu_are_that_kernel(batch, m, n, k, dtype):
     x, w, y = (descriptor(dtype, s) for s in ((batch, m, k), (batch, k, n), (batch, m, n)))
     x.address += 2
     x.strides.sizes[:2] = m * (k + 3), k + 3
     w.strides.sizes[0] = (k + 7) * n
-    assert plan_of(x, w, y)[0] == 2
+    assert (plan_of(x, w, y)[0] == 2) == ((batch, m, n, k) in test_gpu_decode_ops.PRODUCTS)
 
 
 # rows and columns of a tile, and whether its K is shared

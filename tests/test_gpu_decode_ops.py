@@ -14,11 +14,13 @@ pytestmark = pytest.mark.gpu
 EPS = {ta.float16: 2.0 ** -11, ta.bfloat16: 2.0 ** -8, ta.float32: 2.0 ** -24}
 
 # batches, M, N, K: one wavefront's rows and a row more, a pass of 4096 and a row more, columns that end in a block, aligned and odd
-PRODUCTS = [(8, 4, 128, 2049), (8, 4, 128, 2048), (3, 1, 8, 512), (2, 2, 24, 513), (5, 3, 40, 1000), (1, 4, 128, 4096), (1, 4, 16, 4097), (2, 4, 72, 9001), (16, 4, 128, 769)]
+PRODUCTS = [(8, 4, 128, 2049), (8, 4, 128, 2048), (3, 1, 8, 512), (2, 2, 24, 513), (5, 3, 40, 1000), (1, 4, 128, 4096), (1, 4, 16, 4097), (2, 4, 72, 9301), (16, 4, 128, 769)]
+# and one beside them: rows of an odd number of 16-byte pieces whose last pass would be short
+BESIDE = [(2, 4, 72, 9001)]
 
 
 @pytest.mark.parametrize("dtype", [ta.float16, ta.bfloat16], ids=str)
-@pytest.mark.parametrize("batch,m,n,k", PRODUCTS)
+@pytest.mark.parametrize("batch,m,n,k", PRODUCTS + BESIDE)
 def test_few_results_of_row_major_matrices(batch, m, n, k, dtype, device):
     """The matrices are the first rows of larger ones (a cache with room), x is a slice of rows of another length; what lies beside is infinite."""
     rng = np.random.default_rng(5)
