@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256, BLOCKS_PER_CU) void gemm16_dtl_kernel(const T*
 
     uint32_t tm, tn;
     const uint32_t split = SPLIT ? blockIdx.x % sk.splits : 0;
-    tile_of(SPLIT ? blockIdx.x / sk.splits : blockIdx.x, tiles_m, tiles_n, tm, tn);
+    tile_of<GROUPED>(SPLIT ? blockIdx.x / sk.splits : blockIdx.x, tiles_m, tiles_n, tm, tn);
     int64_t oa, ob, oc;
     batch_offsets(p, blockIdx.y, oa, ob, oc);
     const uint32_t m0 = tm * BM, n0 = tn * BN;
