@@ -474,6 +474,13 @@ GroupedTiles gemm16_dtl_grouped_tiles(const GemmProblem& p, const void* a, const
         // 512 -> 1024 57.7 / 49.7)
         if (filled && (p.K >= 2048 || p.c_group % 256 == 0) && (p.K >= 1024 ? rounds_here * 10 >= rounds * 16 : tiles * 10 >= rounds * 8192)) return none;
     }
+    //  * and where next to nothing of them is padding and there are two rounds of them, from K = 192 on (fp16 / bf16, us there / here: 33 images of 64 x 68
+    //    under 256 -> 1018 136 / 161, 60 of 76 x 72 under 320 -> 992 388 / 449, 31 of 74 x 72 under 256 -> 1954 354 / 389; with more padding 37 of 72 x 72
+    //    under 320 -> 1856 455 / 437, eight of 64 x 64 under 256 -> 1344 44 / 42, 55 of 43 x 40 under 256 -> 1952 227 / 228).
+    if (whole && aligned && rows > 192 && p.K >= 192) {
+        const uint64_t down = (rows + 255) / 256, per_image = (p.c_group + 255) / 256, large = down * per_image * (columns / p.c_group);
+        if (large >= 512 && static_cast<double>(rows) * p.c_group >= 0.925 * (65536.0 * down * per_image)) return none;
+    }
     // Tiles: 128 x 128 with two stages, two blocks on a compute unit, where there is more than one for each; else blocks enough come first,
     // 64 x 128 unless the tiles of 128 rows are nearly enough and K is long (fp16, batch 32, us with 128 rows and two stages / 128 and
     // four / 64 and three: 256 -> 1024 over 14 x 14 (400 tiles of 128 rows) 14.3 / 17.3 / 17.5, 512 -> 256 over 28 x 28 (392)

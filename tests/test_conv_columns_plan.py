@@ -33,6 +33,11 @@ PROBLEMS = {
     "large_ragged_images": ((32, 1024, 28, 28, 1024), (128, 2)),
     "large_few_channels_out": ((32, 1024, 32, 32, 192), (128, 2)),
     "large_odd_images": ((32, 2048, 14, 14, 2048), (128, 2)),
+    "large_hardly_padded": ((33, 256, 64, 68, 1018), None),
+    "large_hardly_padded_images": ((60, 320, 76, 72, 992), None),
+    "large_padded": ((37, 320, 72, 72, 1856), (128, 2)),
+    "large_hardly_padded_shortest_k": ((33, 128, 64, 68, 1018), (128, 2)),
+    "large_hardly_padded_one_round": ((7, 256, 64, 68, 1018), (128, 2)),
     # few tiles under a long K
     "long_k": ((1, 8192, 32, 32, 64), None),
     "long_k_sixteen_tiles": ((4, 2048, 16, 16, 128), None),
