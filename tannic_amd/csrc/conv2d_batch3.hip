@@ -432,14 +432,18 @@ static int plan_batch3(const ConvProblem& p, int dtype, const void* x, const voi
     //    30.2 / 37.6, 128 -> 768, fifteen, 26.8 / 30.5, 576 -> 816, seven of 28 x 28 75 / 87, with a stride 480 -> 16, 42 images of 45 x 46 41.7 / 58;
     //    less than half full 256 -> 278, 25 of 20 x 20 36.6 / 32.3, in two rounds 192 -> 691, twenty of 24 x 22 81 / 47); rows of an odd number of pixels
     //    lie at odd addresses there (128 -> 816, twelve of 24 x 25 46 / 35, 160 -> 816, 53 of 16 x 19 83 / 71; but 576 -> 816, seven of 26 x 29, 78 / 87)
+    const uint64_t blocks = (pixels + q.ptile - 1) / q.ptile * q.co_tiles * q.splits;
     if (whole_chunks && p.W % 2 == 0) {
         const K3Load there = conv2d_k3_load(p, x, w);
-        const uint64_t blocks = (pixels + q.ptile - 1) / q.ptile * q.co_tiles * q.splits;
         if (blocks > COMPUTE_UNITS && there.blocks && there.blocks <= there.at_once && there.blocks * 100 >= there.at_once * 58ull) return -1;
         //  * with a stride: rows in whole vectors of larger images there (160 -> 32, sixteen of 45 x 48 18.4 / 20, 224 -> 32 22.9 / 24.2; smaller ones
-        //    416 -> 128, thirty of 30 x 32, 0.90), and three chunks with two blocks on a compute unit (96 -> 28, 49 of 32 x 30 13.8 / 15.5)
-        if (strided && there.blocks && (there.flat ? p.C < 128 && there.at_once > 256 : image > 500)) return -1;
+        //    416 -> 128, thirty of 30 x 32, 0.90), and three or four chunks in one round, with whole vectors or two blocks on a compute unit (96 -> 28,
+        //    49 of 32 x 30 13.8 / 15.5, 128 -> 512, 27 of 23 x 20, 18.6 / 21.2, 128 -> 188, sixteen of 35 x 32, 17.1 / 18.1)
+        if (strided && there.blocks && ((!there.flat && image > 500) || (p.C <= 128 && blocks <= COMPUTE_UNITS && (!there.flat || there.at_once > COMPUTE_UNITS)))) return -1;
     }
+    //  * with a stride, more than one round where the unfolded batch has up to 4096 pixels (320 -> 693, nineteen of 24 x 27, 40 / 51, 408 -> 576 of
+    //    27 x 25 52 / 60, 615 -> 528, 29 of 20 x 23, 73 / 86; in one round 384 -> 560 of 26 x 26 49 / 37)
+    if (strided && blocks > COMPUTE_UNITS && pixels <= 4096 && K >= 2304) return -1;
     return index;
 }
 

@@ -71,6 +71,10 @@ RULES = {
     "stride": (((42, 480, 45, 46), (16, 480, 3, 3), 2), ((42, 480, 45, 47), (16, 480, 3, 3), 2)),
     "stride_whole_rows": (((16, 160, 45, 48), (32, 160, 3, 3), 2), ((30, 416, 30, 32), (128, 416, 3, 3), 2)),
     "stride_three_chunks": (((49, 96, 32, 30), (28, 96, 3, 3), 2), ((49, 96, 32, 31), (28, 96, 3, 3), 2)),
+    "stride_four_chunks": (((27, 128, 23, 20), (512, 128, 3, 3), 2), ((52, 128, 20, 22), (725, 128, 3, 3), 2)),
+    "stride_few_chunks_whole_rows": (((16, 128, 35, 32), (188, 128, 3, 3), 2), ((21, 192, 29, 32), (128, 192, 3, 3), 2)),
+    "stride_two_rounds": (((19, 320, 24, 27), (693, 320, 3, 3), 2), ((19, 384, 26, 26), (560, 384, 3, 3), 2)),
+    "stride_two_rounds_more_pixels": (((19, 408, 27, 25), (576, 408, 3, 3), 2), ((34, 352, 21, 22), (768, 352, 3, 3), 2)),
 }
 
 
