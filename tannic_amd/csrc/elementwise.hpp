@@ -32,6 +32,7 @@ struct Plan {
     uint32_t row_vectors;                  // vectors per row (set at launch)
     FastDiv row_div;                       // division by row_vectors
     uint32_t total_vectors;                // rows * row_vectors
+    uint32_t kept_from;                    // the block from which on results are stored through the caches
 };
 
 // Collapses `rank` dims.  strides[o][d] are element strides of operand o.
@@ -112,42 +113,57 @@ template <> struct RawBits<4> { using type = unsigned int; };
 template <> struct RawBits<2> { using type = unsigned short; };
 template <> struct RawBits<1> { using type = unsigned char; };
 
-#ifndef TH_NONTEMPORAL
-#define TH_NONTEMPORAL 1
-#endif
+// What is read or written past the caches (non-temporally): the BIG kernels.  A source of 96 MB or more could not stay in the memory-side
+// cache of 256 MB together with the result, and not putting it there leaves room for the result, which the next operator reads; of a
+// result, what comes before its last 208 MB cannot stay, and the rest is written back while the next operator runs.  Everything else
+// goes through the caches.  Before, everything went past them.  fp16, three operators in a row, us each, everything past the caches / by this
+// rule: one source 16 MB 7.0 / 6.6, 32 MB 12.3 / 11.1, 64 MB 22.8 / 20.3, 128 MB 43.5 / 40.5, 256 MB 84.7 / 78.0, 512 MB 167.3 / 165.5; two sources
+// 32 MB 17.2 / 15.6, 64 MB 32.2 / 29.2, 128 MB 62.5 / 61.2, 256 MB 124.6 / 118.4, 512 MB 248.7 / 246.6; eight operators over 512 MB 1508 / 1462 (the last
+// 128, 192, 224, 256 and 320 MB of a result kept 1495, 1480, 1478, 1496, 1541).  A decoder layer over a prompt of 512, whose results the next
+// product reads, 331 / 317, in the front end's own operators 571 / 551 (the loads alone through the caches 331 and 567, the stores alone 315 and 556);
+// one result of 8 MB that nothing reads afterwards 3.4 / 4.0.  Bound by HBM: 6.5 TB/s at 512 MB, 6.9 at 256.
+constexpr uint64_t kStreamedSource = 96ull << 20, kKeptResult = 208ull << 20;
 
-// Loads N consecutive elements with one access of sizeof(T)*N bytes.  Operand
-// streams are read once and results written once, so both bypass temporal
-// caching.
-template <class T, int N>
+// The first of `blocks` blocks of `bytes` bytes of results each whose results are kept
+inline uint32_t first_kept(uint32_t blocks, uint64_t bytes) { return blocks * bytes > kKeptResult ? static_cast<uint32_t>(blocks - kKeptResult / bytes) : 0; }
+
+// Loads N consecutive elements with one access of sizeof(T)*N bytes.
+template <class T, int N, bool STREAMED = false>
 __device__ inline Pack<T, N> load_pack(const T* p) {
     static_assert(sizeof(T) * N <= 16, "a pack is at most 16 bytes");
     using Raw = typename RawBits<sizeof(T) * N>::type;
-#if TH_NONTEMPORAL
-    const Raw raw = __builtin_nontemporal_load(reinterpret_cast<const Raw*>(p));
-#else
-    const Raw raw = *reinterpret_cast<const Raw*>(p);
-#endif
+    Raw raw;
+    if constexpr (STREAMED) raw = __builtin_nontemporal_load(reinterpret_cast<const Raw*>(p));
+    else raw = *reinterpret_cast<const Raw*>(p);
     Pack<T, N> r;
     __builtin_memcpy(&r, &raw, sizeof r);
     return r;
 }
 
-template <class T, int N>
+template <class T, int N, bool STREAMED = false>
 __device__ inline void store_pack(T* p, const Pack<T, N>& v) {
     using Raw = typename RawBits<sizeof(T) * N>::type;
     Raw raw;
     __builtin_memcpy(&raw, &v, sizeof raw);
-#if TH_NONTEMPORAL
-    __builtin_nontemporal_store(raw, reinterpret_cast<Raw*>(p));
-#else
-    *reinterpret_cast<Raw*>(p) = raw;
-#endif
+    if constexpr (STREAMED) __builtin_nontemporal_store(raw, reinterpret_cast<Raw*>(p));
+    else *reinterpret_cast<Raw*>(p) = raw;
 }
 
+// (the empty statements keep the two stores apart, which the compiler would merge into one that is not streamed)
 template <class T, int N>
+__device__ inline void store_kept(T* p, const Pack<T, N>& v, bool kept) {
+    if (kept) {
+        asm volatile("");
+        store_pack<T, N, false>(p, v);
+        asm volatile("");
+    } else {
+        store_pack<T, N, true>(p, v);
+    }
+}
+
+template <class T, int N, bool STREAMED>
 __device__ inline Pack<T, N> load_or_splat(const T* p, bool splat) {
-    if (!splat) return load_pack<T, N>(p);
+    if (!splat) return load_pack<T, N, STREAMED>(p);
     Pack<T, N> r;
     const T s = *p;
 #pragma unroll
@@ -185,55 +201,35 @@ __device__ inline Offsets decode(const Plan& p, uint32_t v) {
 
 // F: { using S0, S1, D; static constexpr int sources; const S0* a; const S1* b; D* out;
 //      __device__ D operator()(S0, S1) const; }   (S1/b unused when sources == 1)
-// UNROLL vectors per thread, kBlock apart.  One is best for plain contiguous operands; with a broadcast operand a
-// thread lives longer (row decoding, the dependent load of the repeated value) and two keep enough bytes in flight.
-template <class F, int VEC, int UNROLL>
+// One vector per thread.  (Two, kBlock apart, were 6 % faster for operands with a broadcast axis from 128 MB on while everything went
+// past the caches; with the rule at kStreamedSource one is as fast or faster at every size: fp16 with one repeated value, us with
+// two / one, 128 MB 41.5 / 40.0, 256 MB 85.9 / 77.9, 512 MB 170.4 / 169.5.)
+template <class F, int VEC, bool BIG>
 __global__ __launch_bounds__(kBlock) void elementwise_kernel(F f, Plan p) {
-    constexpr int kUnroll = UNROLL;
     using S0 = typename F::S0;
     using S1 = typename F::S1;
     using D = typename F::D;
     const int last = p.rank - 1;
-    const bool splat0 = p.stride[0][last] == 0;
-    const bool splat1 = p.stride[1][last] == 0;
-    const uint32_t base = blockIdx.x * (kBlock * kUnroll) + threadIdx.x;
+    const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
+    if (v >= p.total_vectors) return;
+    const Offsets o = decode<VEC>(p, v);
     if constexpr (VEC == 1) {
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const uint32_t v = base + u * kBlock;
-            if (v < p.total_vectors) {
-                const Offsets o = decode<1>(p, v);
-                if constexpr (F::sources == 2) f.out[o.od] = f(f.a[o.o0], f.b[o.o1]);
-                else f.out[o.od] = f(f.a[o.o0], S1{});
-            }
-        }
+        if constexpr (F::sources == 2) f.out[o.od] = f(f.a[o.o0], f.b[o.o1]);
+        else f.out[o.od] = f(f.a[o.o0], S1{});
     } else {
-        // all loads of the unrolled group are issued before any store
-        Pack<S0, VEC> a[kUnroll];
-        Pack<S1, VEC> b[kUnroll];
-        Offsets o[kUnroll];
-        bool live[kUnroll];
+        const Pack<S0, VEC> a = load_or_splat<S0, VEC, BIG>(f.a + o.o0, p.stride[0][last] == 0);
+        Pack<S1, VEC> b;
+        if constexpr (F::sources == 2) b = load_or_splat<S1, VEC, BIG>(f.b + o.o1, p.stride[1][last] == 0);
+        Pack<D, VEC> r;
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            const uint32_t v = base + u * kBlock;
-            live[u] = v < p.total_vectors;
-            if (live[u]) {
-                o[u] = decode<VEC>(p, v);
-                a[u] = load_or_splat<S0, VEC>(f.a + o[u].o0, splat0);
-                if constexpr (F::sources == 2) b[u] = load_or_splat<S1, VEC>(f.b + o[u].o1, splat1);
-            }
+        for (int i = 0; i < VEC; ++i) {
+            if constexpr (F::sources == 2) r.v[i] = f(a.v[i], b.v[i]);
+            else r.v[i] = f(a.v[i], S1{});
         }
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            if (live[u]) {
-                Pack<D, VEC> r;
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) {
-                    if constexpr (F::sources == 2) r.v[i] = f(a[u].v[i], b[u].v[i]);
-                    else r.v[i] = f(a[u].v[i], S1{});
-                }
-                store_pack<D, VEC>(f.out + o[u].od, r);
-            }
+        if constexpr (BIG) {
+            store_kept<D, VEC>(f.out + o.od, r, blockIdx.x >= p.kept_from);
+        } else {
+            store_pack<D, VEC>(f.out + o.od, r);
         }
     }
 }
@@ -262,11 +258,11 @@ __device__ inline int64_t outer_offset(const Plan& p, int o, uint32_t row) {
     return off;
 }
 
-template <class T, int VEC>
+template <class T, int VEC, bool BIG>
 __device__ inline Pack<T, VEC> flat_source(const FlatPlan& fp, int o, const T* base, uint64_t first, uint32_t row, uint32_t col, uint32_t live) {
     Pack<T, VEC> r;
     if (fp.full[o]) {
-        if (live == VEC) return load_pack<T, VEC>(base + first);
+        if (live == VEC) return load_pack<T, VEC, BIG>(base + first);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) r.v[i] = static_cast<uint32_t>(i) < live ? base[first + i] : T{};
         return r;
@@ -280,7 +276,7 @@ __device__ inline Pack<T, VEC> flat_source(const FlatPlan& fp, int o, const T* b
     return r;
 }
 
-template <class F, int VEC>
+template <class F, int VEC, bool BIG>
 __global__ __launch_bounds__(kBlock) void elementwise_flat_kernel(F f, FlatPlan fp, uint32_t vectors) {
     using S0 = typename F::S0;
     using S1 = typename F::S1;
@@ -291,9 +287,9 @@ __global__ __launch_bounds__(kBlock) void elementwise_flat_kernel(F f, FlatPlan 
     const uint32_t live = fp.elements - first < VEC ? static_cast<uint32_t>(fp.elements - first) : VEC;
     uint32_t row = 0, col = 0;
     if (fp.p.rank > 1) fp.p.row_div.divmod(static_cast<uint32_t>(first), row, col);   // fewer than 2^31 elements (the launch checks)
-    const Pack<S0, VEC> a = flat_source<S0, VEC>(fp, 0, f.a, first, row, col, live);
+    const Pack<S0, VEC> a = flat_source<S0, VEC, BIG>(fp, 0, f.a, first, row, col, live);
     Pack<S1, VEC> b;
-    if constexpr (F::sources == 2) b = flat_source<S1, VEC>(fp, 1, f.b, first, row, col, live);
+    if constexpr (F::sources == 2) b = flat_source<S1, VEC, BIG>(fp, 1, f.b, first, row, col, live);
     Pack<D, VEC> r;
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
@@ -301,7 +297,8 @@ __global__ __launch_bounds__(kBlock) void elementwise_flat_kernel(F f, FlatPlan 
         else r.v[i] = f(a.v[i], S1{});
     }
     if (live == VEC) {
-        store_pack<D, VEC>(f.out + first, r);
+        if constexpr (BIG) store_kept<D, VEC>(f.out + first, r, blockIdx.x >= fp.p.kept_from);
+        else store_pack<D, VEC>(f.out + first, r);
     } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i)
@@ -373,8 +370,13 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
                 fp.rows = static_cast<uint32_t>(rows);
                 p.row_div = FastDiv(p.extent[last]);
                 fp.p = p;
-                const uint32_t vectors = static_cast<uint32_t>((fp.elements + VEC - 1) / VEC);
-                hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC>), dim3((vectors + kBlock - 1) / kBlock), dim3(kBlock), 0, stream, f, fp, vectors);
+                const uint32_t vectors = static_cast<uint32_t>((fp.elements + VEC - 1) / VEC), grid = (vectors + kBlock - 1) / kBlock;
+                if (fp.elements * sizeof(S0) >= kStreamedSource) {
+                    fp.p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
+                    hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC, true>), dim3(grid), dim3(kBlock), 0, stream, f, fp, vectors);
+                } else {
+                    hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC, false>), dim3(grid), dim3(kBlock), 0, stream, f, fp, vectors);
+                }
                 return launch_status("elementwise_flat_kernel");
             }
         }
@@ -387,22 +389,19 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
     }
     p.total_vectors = static_cast<uint32_t>(rows * p.row_vectors);
     if (p.total_vectors == 0) return TANNIC_SUCCESS;
-    const bool repeats = p.rank > 1 || p.stride[0][last] == 0 || (F::sources == 2 && p.stride[1][last] == 0);
-    // Two vectors per thread pay only when the blocks are many generations deep (1 GiB with a broadcast operand: 6 %
-    // faster); at the sizes of a layer's activations (16 MB: one or two generations) one vector per thread and twice
-    // the blocks let stores of early blocks overlap loads of late ones (15 of a decoder layer's 600 us).
-    const bool two = repeats && p.total_vectors >= (1u << 23);
-    const uint32_t per_block = kBlock * (two ? 2 : 1);
-    const uint32_t grid = (p.total_vectors + per_block - 1) / per_block;
+    const uint32_t grid = (p.total_vectors + kBlock - 1) / kBlock;
     if constexpr (VEC > 1) {
         if (vec) {
-            if (two) hipLaunchKernelGGL((elementwise_kernel<F, VEC, 2>), dim3(grid), dim3(kBlock), 0, stream, f, p);
-            else hipLaunchKernelGGL((elementwise_kernel<F, VEC, 1>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+            if (static_cast<uint64_t>(p.total_vectors) * VEC * sizeof(S0) >= kStreamedSource) {
+                p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
+                hipLaunchKernelGGL((elementwise_kernel<F, VEC, true>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+            } else {
+                hipLaunchKernelGGL((elementwise_kernel<F, VEC, false>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+            }
             return launch_status("elementwise_kernel");
         }
     }
-    if (two) hipLaunchKernelGGL((elementwise_kernel<F, 1, 2>), dim3(grid), dim3(kBlock), 0, stream, f, p);
-    else hipLaunchKernelGGL((elementwise_kernel<F, 1, 1>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+    hipLaunchKernelGGL((elementwise_kernel<F, 1, false>), dim3(grid), dim3(kBlock), 0, stream, f, p);
     return launch_status("elementwise_kernel");
 }
 

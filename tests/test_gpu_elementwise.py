@@ -290,3 +290,17 @@ def test_int32_add_and_compare_reduced_size(device):
     # comparisons do not broadcast: the sum is compared with X itself
     n = want.nelements // 8
     support.assert_bit_exact(ops.gt(got, dx).raw()[:n], ops.gt(want, hx).raw()[:n], "int32 compare")
+
+
+@pytest.mark.parametrize("megabytes", [95, 96, 208, 209, 300], ids=lambda m: f"{m}MB")
+def test_operands_past_the_caches(device, megabytes):
+    """Sources from 96 MB on and what comes before the last 208 MB of a result go past the caches; a repeated operand does not.  Whole numbers: bit for bit."""
+    n = megabytes << 18
+    x = np.arange(n, dtype=np.int32)
+    dx = ta.tensor(x.reshape(-1, 64, 1024), ta.int32, device)
+    row = np.arange(1024, dtype=np.int32) * 7
+    dr = ta.tensor(row, ta.int32, device)
+    got = ops.sub(ops.add(dx, dx), dr)
+    want = (x + x).reshape(-1, 64, 1024) - row
+    np.testing.assert_array_equal(got.numpy(), want)
+    np.testing.assert_array_equal(ops.neg(got).numpy(), -want)
