@@ -213,10 +213,11 @@ void tannic_hip_counters(uint64_t out[3]);
 /* Which kernel a convolution of these operands would run, without running it or reading what their addresses point at (for
  * tests, no reference twin).  out[0] is 1 for the fp32 kernel over the flattened batch, 2 for the 16-bit kernel over few
  * output pixels, 3 for the fp32 kernel on the 16-bit matrix pipe, 4 for the 16-bit 3x3 kernel over the flattened batch, 5 for the
- * 16-bit 1x1 product whose tiles run over the images, 0 for any other.  After 1: the kernel's side, its template parameters U, PT, NL,
+ * 16-bit 1x1 product whose tiles run over the images, 6 for the one of 2 that stages its operands in LDS where it comes after 4, 0 for any other.  After 1: the kernel's side, its template parameters U, PT, NL,
  * RESIDENT, WO and WIDE, then pixels per tile, tiles of channels, blocks sharing the channels, groups of kernel rows, groups per block,
  * floats from plane to plane, floats of a plane, rows per image and columns per row with the shared padding.  After 2: the kernel's
- * side, tiles of 16 channels and of 16 pixels per block, wavefronts, blocks.  After 3: the kernel's side, PT, WO and NL, pixels per
+ * side, tiles of 16 channels and of 16 pixels per block, wavefronts, blocks, and where it stages its operands in LDS the channels per block
+ * and the pieces of the signal a lane has on their way; after 6 the same.  After 3: the kernel's side, PT, WO and NL, pixels per
  * tile, tiles of channels, blocks sharing the channels, chunks of 32 channels, chunks per block, places of a plane, rows per image and
  * columns per row with the shared padding.  After 4: the same.  After 5: the kernel's side, channels out of a tile, stages of its
  * operands.  The status is the convolution's. */

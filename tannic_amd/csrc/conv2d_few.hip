@@ -1,4 +1,5 @@
-// conv2d of 16-bit types over few output pixels (one image, or a handful): 1x1 and 3x3 kernels, C a multiple of 32.
+// conv2d of 16-bit types over few output pixels (one image, or a handful): 1x1 and 3x3 kernels, C a multiple of 32 (3x3 of more than a few
+// channels over plain rows goes to conv2d_few3.hip from here).
 //
 // With one image a layer's work is some 0.1 - 0.2 GFLOP and a megabyte of weights: a microsecond of the chip, if all of it
 // takes part.  The tiles of the other kernels (64 output channels x up to 512 pixels, or 64 x 128 of a product) leave four
@@ -16,38 +17,15 @@
 // tiles meet in LDS, in a fixed order.  The 53 convolutions and 16 additions of a ResNet-50 over one image, recorded: 867 -> 405 us
 // (512 -> 512 3x3 over 7 x 7 59 -> 13, 256 -> 256 over 14 x 14 26.7 -> 8.2, 256 -> 1024 1x1 10.7 -> 4.1).
 // (src/cpu/conv2d.cpp:17-64; sums in fp32, rounded once.)
-#include "conv_common.hpp"
-
-#include "gemm_tiles.hpp"
+#include "conv_few.hpp"
 
 namespace th {
-
-typedef _Float16 half8f __attribute__((ext_vector_type(8)));
-typedef __bf16 bfloat8f __attribute__((ext_vector_type(8)));
-typedef float float4f __attribute__((ext_vector_type(4)));
-typedef unsigned int uint4f __attribute__((ext_vector_type(4)));
-typedef unsigned int uint4f_any __attribute__((ext_vector_type(4), aligned(2)));
-
-template <class T> __device__ inline float4f few_mfma(uint4f a, uint4f b, float4f c) {
-    if constexpr (std::is_same_v<T, f16>) {
-        half8f x, y;
-        __builtin_memcpy(&x, &a, 16);
-        __builtin_memcpy(&y, &b, 16);
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, y, c, 0, 0, 0);
-    } else {
-        bfloat8f x, y;
-        __builtin_memcpy(&x, &a, 16);
-        __builtin_memcpy(&y, &b, 16);
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
-    }
-}
 
 struct FewPlan {
     uint32_t pixels, units, pixel_tiles, records;   // of the flattened batch; blocks of 32 channels; bytes of the signal
     FastDiv div_hw, div_wo, div_tiles;
 };
 
-constexpr uint32_t kFewPitch = 20;              // floats per row of a partial 16 x 16 tile: the four row groups of a write fall on different banks
 constexpr uint32_t kFewOutside = 0x80000000u;   // not below any signal's bytes that this kernel takes (records <= 2^31): the load gives zero
 
 template <class T, int KS, int MO, int NP, int WAVES>
@@ -169,7 +147,8 @@ static int launch_few(const ConvProblem& p, FewPlan q, const void* x, const void
 
 // Multiply-adds up to which this kernel is taken, its output channels counted in whole tiles of 16 (a tile costs its loads whatever it
 // holds): its loads grow with the work from the first pixel on, the other kernels' time hardly does while their blocks are few.
-// Where the lines lie (fp16, replayed calls on one box, us, this kernel / the others):
+// Where the lines lie (fp16, replayed calls on one box, us, this kernel / the others; 3x3 from before conv2d_few3.hip, which now has most of
+// what lies below them and is faster there):
 //   3x3, C = 64 or 128 with a stride   240 M   64 @56: batch 1 6.5 / 10.0, 2 8.7 / 10.1, 4 12.3 / 10.3; 128 @56 s2: 8.7 / 13.2, 11.3 / 16.6, 19.4 / 16.8
 //   other 3x3                          470 M   128 @28: batch 1 6.7 / 13.2, 4 12.7 / 19.3, 8 21.4 / 18.8; 256 @14: 8.2 / 26.7, 14.4 / 17.5, 26.8 / 24.8;
 //                                              512 @7: 13.0 / 58.9, 22.5 / 60.6, 37.5 / 20.0
@@ -233,7 +212,14 @@ static int run_few(const ConvProblem& p, const void* x, const void* w, const voi
         if (extent[d] > 1) last += (extent[d] - 1) * static_cast<uint64_t>(p.xs[d]);
         if (last >= (1ull << 30)) return TANNIC_UNSUPPORTED_DTYPE;
     }
-    if (pixels >= (1ull << 24) || !few_work(p, pixels)) return TANNIC_UNSUPPORTED_DTYPE;
+    if (pixels >= (1ull << 24)) return TANNIC_UNSUPPORTED_DTYPE;
+    const bool work = few_work(p, pixels);
+    if constexpr (KS == 3) {
+        // (from 256 output channels on also beyond the line: few3's own rule then says where it ends)
+        const int rc = work || p.O >= 256 ? conv2d_few3(p, dtype_code<T>(), x, w, bias, y, stream, plan) : TANNIC_UNSUPPORTED_DTYPE;
+        if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
+    }
+    if (!work) return TANNIC_UNSUPPORTED_DTYPE;
     FewPlan q{};
     q.pixels = static_cast<uint32_t>(pixels);
     q.units = p.C / 32;

@@ -32,6 +32,9 @@ bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValu
 // conditions, so that the caller can try the next, more general kernel.
 // 16-bit 1x1 and 3x3 over few output pixels
 int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
+// 16-bit 3x3 from 64 channels and 32 output channels on, few output pixels, the weights and the signal staged in LDS (what conv2d_few asks first, and
+// what conv2d_batch3 leaves); `plan`: only asked which tiles it would take
+int conv2d_few3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan = nullptr);
 bool conv2d_k1_takes(const ConvProblem& p, int dtype, const void* x, const void* w, const void* y);
 int conv2d_k1(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
