@@ -55,6 +55,7 @@ UNITS = [
     ("conv2d_mfma.hip", "conv2d_mfma.o", []),
     ("conv2d_few.hip", "conv2d_few.o", []),
     ("conv2d_few3.hip", "conv2d_few3.o", []),
+    ("conv2d_few1.hip", "conv2d_few1.o", []),
     ("conv2d_patch.hip", "conv2d_patch.o", []),
     ("conv2d_resident.hip", "conv2d_resident.o", []),
     ("conv2d_k3.hip", "conv2d_k3.o", ["-DTH_K3_PART=0"]),

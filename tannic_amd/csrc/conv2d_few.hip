@@ -219,6 +219,10 @@ static int run_few(const ConvProblem& p, const void* x, const void* w, const voi
         const int rc = work || p.O >= 256 ? conv2d_few3(p, dtype_code<T>(), x, w, bias, y, stream, plan) : TANNIC_UNSUPPORTED_DTYPE;
         if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
     }
+    if constexpr (KS == 1) {
+        const int rc = !work ? TANNIC_UNSUPPORTED_DTYPE : conv2d_few1(p, dtype_code<T>(), true, x, w, bias, y, stream, plan);
+        if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
+    }
     if (!work) return TANNIC_UNSUPPORTED_DTYPE;
     FewPlan q{};
     q.pixels = static_cast<uint32_t>(pixels);

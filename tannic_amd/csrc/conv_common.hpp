@@ -35,6 +35,8 @@ int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, co
 // 16-bit 3x3 from 64 channels and 32 output channels on, few output pixels, the weights and the signal staged in LDS (what conv2d_few asks first, and
 // what conv2d_batch3 leaves); `plan`: only asked which tiles it would take
 int conv2d_few3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan = nullptr);
+// 16-bit 1x1, stride 1, the same way; `few`: below conv2d_few's line
+int conv2d_few1(const ConvProblem& p, int dtype, bool few, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan = nullptr);
 bool conv2d_k1_takes(const ConvProblem& p, int dtype, const void* x, const void* w, const void* y);
 int conv2d_k1(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
 int conv2d_pointwise(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);

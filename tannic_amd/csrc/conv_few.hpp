@@ -29,6 +29,7 @@ template <class T> __device__ inline float4f few_mfma(uint4f a, uint4f b, float4
 
 constexpr uint32_t kFewPitch = 20;              // floats per row of a partial 16 x 16 tile: the four row groups of a write fall on different banks
 
+// what a block may have of LDS
 constexpr size_t kFew3Lds = 160 * 1024;
 
 }  // namespace th
