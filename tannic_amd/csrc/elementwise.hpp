@@ -25,14 +25,17 @@ namespace th {
 constexpr int kMaxOperands = 3;  // two sources + destination
 
 struct Plan {
+    // (what every thread needs comes first, so that it is one load of the arguments)
     int rank;                              // collapsed rank, >= 1
+    uint32_t total_vectors;                // rows * row_vectors
+    FastDiv row_div;                       // division by row_vectors
+    uint32_t row_vectors;                  // vectors per row (set at launch)
+    uint32_t kept_from;                    // the block from which on results are stored through the caches
+    uint32_t streamed;                     // whether the sources are loaded past them
+    int64_t row_stride[kMaxOperands];      // the last dim's element strides
     uint32_t extent[TANNIC_DIMENSIONS];    // collapsed extents
     FastDiv div[TANNIC_DIMENSIONS];        // division by extent[d]
     int64_t stride[kMaxOperands][TANNIC_DIMENSIONS];  // element strides per operand
-    uint32_t row_vectors;                  // vectors per row (set at launch)
-    FastDiv row_div;                       // division by row_vectors
-    uint32_t total_vectors;                // rows * row_vectors
-    uint32_t kept_from;                    // the block from which on results are stored through the caches
 };
 
 // Collapses `rank` dims.  strides[o][d] are element strides of operand o.
@@ -97,6 +100,7 @@ inline bool build_plan(Plan& p, int rank, const size_t* extent, const int64_t (*
         p.div[d] = FastDiv(p.extent[d]);
         for (int o = 0; o < kMaxOperands; ++o) p.stride[o][d] = (d < r && o < operands) ? st[o][d] : 0;
     }
+    for (int o = 0; o < kMaxOperands; ++o) p.row_stride[o] = p.stride[o][r - 1];
     return true;
 }
 
@@ -113,7 +117,7 @@ template <> struct RawBits<4> { using type = unsigned int; };
 template <> struct RawBits<2> { using type = unsigned short; };
 template <> struct RawBits<1> { using type = unsigned char; };
 
-// What is read or written past the caches (non-temporally): the BIG kernels.  A source of 96 MB or more could not stay in the memory-side
+// What is read or written past the caches (non-temporally).  A source of 96 MB or more could not stay in the memory-side
 // cache of 256 MB together with the result, and not putting it there leaves room for the result, which the next operator reads; of a
 // result, what comes before its last 208 MB cannot stay, and the rest is written back while the next operator runs.  Everything else
 // goes through the caches.  Before, everything went past them.  fp16, three operators in a row, us each, everything past the caches / by this
@@ -128,48 +132,70 @@ constexpr uint64_t kStreamedSource = 96ull << 20, kKeptResult = 208ull << 20;
 inline uint32_t first_kept(uint32_t blocks, uint64_t bytes) { return blocks * bytes > kKeptResult ? static_cast<uint32_t>(blocks - kKeptResult / bytes) : 0; }
 
 // Loads N consecutive elements with one access of sizeof(T)*N bytes.
-template <class T, int N, bool STREAMED = false>
+template <class T, int N>
 __device__ inline Pack<T, N> load_pack(const T* p) {
     static_assert(sizeof(T) * N <= 16, "a pack is at most 16 bytes");
     using Raw = typename RawBits<sizeof(T) * N>::type;
-    Raw raw;
-    if constexpr (STREAMED) raw = __builtin_nontemporal_load(reinterpret_cast<const Raw*>(p));
-    else raw = *reinterpret_cast<const Raw*>(p);
+    const Raw raw = *reinterpret_cast<const Raw*>(p);
     Pack<T, N> r;
     __builtin_memcpy(&r, &raw, sizeof r);
     return r;
 }
 
-template <class T, int N, bool STREAMED = false>
+template <class T, int N>
 __device__ inline void store_pack(T* p, const Pack<T, N>& v) {
     using Raw = typename RawBits<sizeof(T) * N>::type;
     Raw raw;
     __builtin_memcpy(&raw, &v, sizeof raw);
-    if constexpr (STREAMED) __builtin_nontemporal_store(raw, reinterpret_cast<Raw*>(p));
-    else *reinterpret_cast<Raw*>(p) = raw;
+    *reinterpret_cast<Raw*>(p) = raw;
 }
 
-// (the empty statements keep the two stores apart, which the compiler would merge into one that is not streamed)
+// The same, through the caches or past them.  (The empty statements keep the two accesses apart, which the compiler would merge into one
+// through the caches.)
 template <class T, int N>
 __device__ inline void store_kept(T* p, const Pack<T, N>& v, bool kept) {
+    using Raw = typename RawBits<sizeof(T) * N>::type;
+    Raw raw;
+    __builtin_memcpy(&raw, &v, sizeof raw);
     if (kept) {
         asm volatile("");
-        store_pack<T, N, false>(p, v);
+        *reinterpret_cast<Raw*>(p) = raw;
         asm volatile("");
     } else {
-        store_pack<T, N, true>(p, v);
+        __builtin_nontemporal_store(raw, reinterpret_cast<Raw*>(p));
     }
 }
 
-template <class T, int N, bool STREAMED>
-__device__ inline Pack<T, N> load_or_splat(const T* p, bool splat) {
-    if (!splat) return load_pack<T, N, STREAMED>(p);
-    Pack<T, N> r;
-    const T s = *p;
+// A source's vector as it is in its registers.  Nothing looks at them before both sources' loads are on their way: a value unpacked, or
+// repeated, right where it is loaded makes the second load wait for the first (an addition over 8 values 1.8 us, over 4096 2.0; a negation 1.65, 1.77).
+template <class T, int N>
+struct RawPack {
+    typename RawBits<sizeof(T) * N>::type bits;
+
+    // N elements, or, where the row repeats one, that one
+    __device__ inline void load(const T* p, bool splat, bool streamed) {
+        using Raw = typename RawBits<sizeof(T) * N>::type;
+        if (splat) {
+            typename RawBits<sizeof(T)>::type one = *reinterpret_cast<const typename RawBits<sizeof(T)>::type*>(p);
+            __builtin_memcpy(&bits, &one, sizeof one);
+        } else if (streamed) {
+            asm volatile("");
+            bits = __builtin_nontemporal_load(reinterpret_cast<const Raw*>(p));
+            asm volatile("");
+        } else {
+            bits = *reinterpret_cast<const Raw*>(p);
+        }
+    }
+    __device__ inline Pack<T, N> get(bool splat) const {
+        Pack<T, N> r;
+        __builtin_memcpy(&r, &bits, sizeof r);
+        if (splat) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) r.v[i] = s;
-    return r;
-}
+            for (int i = 1; i < N; ++i) r.v[i] = r.v[0];
+        }
+        return r;
+    }
+};
 
 constexpr int kBlock = 256;
 
@@ -180,15 +206,14 @@ struct Offsets {
 
 template <int VEC>
 __device__ inline Offsets decode(const Plan& p, uint32_t v) {
-    const int last = p.rank - 1;
     uint32_t row, col;
     p.row_div.divmod(v, row, col);
     col *= VEC;
     Offsets o;
-    o.o0 = static_cast<int64_t>(col) * p.stride[0][last];
-    o.o1 = static_cast<int64_t>(col) * p.stride[1][last];
-    o.od = static_cast<int64_t>(col) * p.stride[2][last];
-    for (int d = last - 1; d >= 0; --d) {
+    o.o0 = static_cast<int64_t>(col) * p.row_stride[0];
+    o.o1 = static_cast<int64_t>(col) * p.row_stride[1];
+    o.od = static_cast<int64_t>(col) * p.row_stride[2];
+    for (int d = p.rank - 2; d >= 0; --d) {
         uint32_t q, c;
         p.div[d].divmod(row, q, c);
         row = q;
@@ -204,12 +229,11 @@ __device__ inline Offsets decode(const Plan& p, uint32_t v) {
 // One vector per thread.  (Two, kBlock apart, were 6 % faster for operands with a broadcast axis from 128 MB on while everything went
 // past the caches; with the rule at kStreamedSource one is as fast or faster at every size: fp16 with one repeated value, us with
 // two / one, 128 MB 41.5 / 40.0, 256 MB 85.9 / 77.9, 512 MB 170.4 / 169.5.)
-template <class F, int VEC, bool BIG>
+template <class F, int VEC>
 __global__ __launch_bounds__(kBlock) void elementwise_kernel(F f, Plan p) {
     using S0 = typename F::S0;
     using S1 = typename F::S1;
     using D = typename F::D;
-    const int last = p.rank - 1;
     const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
     if (v >= p.total_vectors) return;
     const Offsets o = decode<VEC>(p, v);
@@ -217,21 +241,48 @@ __global__ __launch_bounds__(kBlock) void elementwise_kernel(F f, Plan p) {
         if constexpr (F::sources == 2) f.out[o.od] = f(f.a[o.o0], f.b[o.o1]);
         else f.out[o.od] = f(f.a[o.o0], S1{});
     } else {
-        const Pack<S0, VEC> a = load_or_splat<S0, VEC, BIG>(f.a + o.o0, p.stride[0][last] == 0);
+        const bool splat0 = p.row_stride[0] == 0, splat1 = p.row_stride[1] == 0;
+        RawPack<S0, VEC> ra;
+        RawPack<S1, VEC> rb;
+        ra.load(f.a + o.o0, splat0, p.streamed);
+        if constexpr (F::sources == 2) rb.load(f.b + o.o1, splat1, p.streamed);
+        const Pack<S0, VEC> a = ra.get(splat0);
         Pack<S1, VEC> b;
-        if constexpr (F::sources == 2) b = load_or_splat<S1, VEC, BIG>(f.b + o.o1, p.stride[1][last] == 0);
+        if constexpr (F::sources == 2) b = rb.get(splat1);
         Pack<D, VEC> r;
 #pragma unroll
         for (int i = 0; i < VEC; ++i) {
             if constexpr (F::sources == 2) r.v[i] = f(a.v[i], b.v[i]);
             else r.v[i] = f(a.v[i], S1{});
         }
-        if constexpr (BIG) {
-            store_kept<D, VEC>(f.out + o.od, r, blockIdx.x >= p.kept_from);
-        } else {
-            store_pack<D, VEC>(f.out + o.od, r);
-        }
+        store_kept<D, VEC>(f.out + o.od, r, blockIdx.x >= p.kept_from);
     }
+}
+
+// Every operand contiguous over everything, the most frequent call: no coordinates, and arguments of half a cache line that one load of them brings in
+// (of a whole plan several do, each after the one before).
+template <class F, int VEC>
+__global__ __launch_bounds__(kBlock) void elementwise_dense_kernel(F f, uint32_t total, uint32_t kept_from, uint32_t streamed) {
+    using S0 = typename F::S0;
+    using S1 = typename F::S1;
+    using D = typename F::D;
+    const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
+    if (v >= total) return;
+    const size_t at = static_cast<size_t>(v) * VEC;
+    RawPack<S0, VEC> ra;
+    RawPack<S1, VEC> rb;
+    ra.load(f.a + at, false, streamed);
+    if constexpr (F::sources == 2) rb.load(f.b + at, false, streamed);
+    const Pack<S0, VEC> a = ra.get(false);
+    Pack<S1, VEC> b;
+    if constexpr (F::sources == 2) b = rb.get(false);
+    Pack<D, VEC> r;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        if constexpr (F::sources == 2) r.v[i] = f(a.v[i], b.v[i]);
+        else r.v[i] = f(a.v[i], S1{});
+    }
+    store_kept<D, VEC>(f.out + at, r, blockIdx.x >= kept_from);
 }
 
 // Rows whose length is not a multiple of the vector (softmax over 197 columns: x - max, x / sum) when every operand is
@@ -258,11 +309,15 @@ __device__ inline int64_t outer_offset(const Plan& p, int o, uint32_t row) {
     return off;
 }
 
-template <class T, int VEC, bool BIG>
+template <class T, int VEC>
 __device__ inline Pack<T, VEC> flat_source(const FlatPlan& fp, int o, const T* base, uint64_t first, uint32_t row, uint32_t col, uint32_t live) {
     Pack<T, VEC> r;
     if (fp.full[o]) {
-        if (live == VEC) return load_pack<T, VEC, BIG>(base + first);
+        if (live == VEC) {
+            RawPack<T, VEC> raw;
+            raw.load(base + first, false, fp.p.streamed);
+            return raw.get(false);
+        }
 #pragma unroll
         for (int i = 0; i < VEC; ++i) r.v[i] = static_cast<uint32_t>(i) < live ? base[first + i] : T{};
         return r;
@@ -276,7 +331,7 @@ __device__ inline Pack<T, VEC> flat_source(const FlatPlan& fp, int o, const T* b
     return r;
 }
 
-template <class F, int VEC, bool BIG>
+template <class F, int VEC>
 __global__ __launch_bounds__(kBlock) void elementwise_flat_kernel(F f, FlatPlan fp, uint32_t vectors) {
     using S0 = typename F::S0;
     using S1 = typename F::S1;
@@ -287,9 +342,9 @@ __global__ __launch_bounds__(kBlock) void elementwise_flat_kernel(F f, FlatPlan 
     const uint32_t live = fp.elements - first < VEC ? static_cast<uint32_t>(fp.elements - first) : VEC;
     uint32_t row = 0, col = 0;
     if (fp.p.rank > 1) fp.p.row_div.divmod(static_cast<uint32_t>(first), row, col);   // fewer than 2^31 elements (the launch checks)
-    const Pack<S0, VEC> a = flat_source<S0, VEC, BIG>(fp, 0, f.a, first, row, col, live);
+    const Pack<S0, VEC> a = flat_source<S0, VEC>(fp, 0, f.a, first, row, col, live);
     Pack<S1, VEC> b;
-    if constexpr (F::sources == 2) b = flat_source<S1, VEC, BIG>(fp, 1, f.b, first, row, col, live);
+    if constexpr (F::sources == 2) b = flat_source<S1, VEC>(fp, 1, f.b, first, row, col, live);
     Pack<D, VEC> r;
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
@@ -297,8 +352,7 @@ __global__ __launch_bounds__(kBlock) void elementwise_flat_kernel(F f, FlatPlan 
         else r.v[i] = f(a.v[i], S1{});
     }
     if (live == VEC) {
-        if constexpr (BIG) store_kept<D, VEC>(f.out + first, r, blockIdx.x >= fp.p.kept_from);
-        else store_pack<D, VEC>(f.out + first, r);
+        store_kept<D, VEC>(f.out + first, r, blockIdx.x >= fp.p.kept_from);
     } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i)
@@ -371,12 +425,9 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
                 p.row_div = FastDiv(p.extent[last]);
                 fp.p = p;
                 const uint32_t vectors = static_cast<uint32_t>((fp.elements + VEC - 1) / VEC), grid = (vectors + kBlock - 1) / kBlock;
-                if (fp.elements * sizeof(S0) >= kStreamedSource) {
-                    fp.p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
-                    hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC, true>), dim3(grid), dim3(kBlock), 0, stream, f, fp, vectors);
-                } else {
-                    hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC, false>), dim3(grid), dim3(kBlock), 0, stream, f, fp, vectors);
-                }
+                fp.p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
+                fp.p.streamed = fp.elements * sizeof(S0) >= kStreamedSource;
+                hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, fp, vectors);
                 return launch_status("elementwise_flat_kernel");
             }
         }
@@ -392,16 +443,17 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
     const uint32_t grid = (p.total_vectors + kBlock - 1) / kBlock;
     if constexpr (VEC > 1) {
         if (vec) {
-            if (static_cast<uint64_t>(p.total_vectors) * VEC * sizeof(S0) >= kStreamedSource) {
-                p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
-                hipLaunchKernelGGL((elementwise_kernel<F, VEC, true>), dim3(grid), dim3(kBlock), 0, stream, f, p);
-            } else {
-                hipLaunchKernelGGL((elementwise_kernel<F, VEC, false>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+            p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
+            p.streamed = static_cast<uint64_t>(p.total_vectors) * VEC * sizeof(S0) >= kStreamedSource;
+            if (p.rank == 1 && p.stride[0][0] == 1 && (F::sources == 1 || p.stride[1][0] == 1)) {      // (vec: the result's is 1)
+                hipLaunchKernelGGL((elementwise_dense_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, p.total_vectors, p.kept_from, p.streamed);
+                return launch_status("elementwise_dense_kernel");
             }
+            hipLaunchKernelGGL((elementwise_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, p);
             return launch_status("elementwise_kernel");
         }
     }
-    hipLaunchKernelGGL((elementwise_kernel<F, 1, false>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+    hipLaunchKernelGGL((elementwise_kernel<F, 1>), dim3(grid), dim3(kBlock), 0, stream, f, p);
     return launch_status("elementwise_kernel");
 }
 
