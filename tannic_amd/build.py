@@ -45,6 +45,7 @@ UNITS = [
     ("gemm_small.hip", "gemm_small.o", []),
     ("gemm_f64.hip", "gemm_f64.o", []),
     ("gemm_rows_nn.hip", "gemm_rows_nn.o", []),
+    ("gemm_rows_dot.hip", "gemm_rows_dot.o", []),
     ("gemm_rows_batch.hip", "gemm_rows_batch.o", []),
     ("gemm_repack.hip", "gemm_repack.o", []),
     ("gemm_dtl.hip", "gemm_dtl.o", ["-DTH_DTL_PART=0"]),

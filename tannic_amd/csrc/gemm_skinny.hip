@@ -163,7 +163,7 @@ constexpr int kStreamBytesPerWave = 32 * 1024;
 
 template <class T, int MB, int NB>
 __global__ __launch_bounds__(64 * kStreamWaves) void gemm_skinny_stream_kernel(const T* x, const T* w, typename SkinnyTypes<T>::Out* c, GemmProblem p,
-                                                                               uint32_t windows_per_wave) {
+                                                                               uint32_t windows_per_wave, bool streamed) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using Acc = typename SkinnyTypes<T>::Acc;
     using Out = typename SkinnyTypes<T>::Out;
@@ -196,9 +196,19 @@ __global__ __launch_bounds__(64 * kStreamWaves) void gemm_skinny_stream_kernel(c
     }
     auto issue = [&](uint32_t window, uint32_t stage) {
         const uint32_t k_bytes = window * 128;
+        constexpr int PAST_CACHES = 2;      // (the non-temporal bit of a load)
+        if (streamed) {
 #pragma unroll
-        for (int j = 0; j < LOADS; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(j / 2 < NB ? rsrc_w : rsrc_x, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, 0);
+            for (int j = 0; j < 2 * NB; ++j)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, PAST_CACHES);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2 * NB; ++j)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, 0);
+        }
+#pragma unroll
+        for (int j = 2 * NB; j < LOADS; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_x, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, 0);
     };
     const uint32_t all = p.K / kBKof<T>;   // windows of 128 bytes per row: 64 elements of 16 bits, 32 of fp32
     const uint32_t first = wave * windows_per_wave;
@@ -287,7 +297,7 @@ static int launch_stream(const GemmProblem& p, const void* a, const void* b, voi
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds, configured)) return rc;
     const uint32_t windows = p.K / kBKof<T>, per_wave = (windows + kStreamWaves - 1) / kStreamWaves;
     hipLaunchKernelGGL(kernel, dim3((p.N + 16 * NB - 1) / (16 * NB), p.batches), dim3(64 * kStreamWaves), lds, stream, static_cast<const T*>(a), static_cast<const T*>(b),
-                       static_cast<typename SkinnyTypes<T>::Out*>(c), p, per_wave);
+                       static_cast<typename SkinnyTypes<T>::Out*>(c), p, per_wave, rows_past_caches(p, sizeof(T)));
     return launch_status("gemm_skinny_stream_kernel");
 }
 
@@ -301,6 +311,9 @@ int run_skinny(const GemmProblem& p, const void* a, const void* b, void* c, hipS
     if (reinterpret_cast<uintptr_t>(a) % 16 || reinterpret_cast<uintptr_t>(b) % 16) return TANNIC_UNSUPPORTED_DTYPE;
     for (int d = 0; d < p.batch_rank; ++d)
         if (!mult8(p.a_bs[d]) || !mult8(p.b_bs[d])) return TANNIC_UNSUPPORTED_DTYPE;
+    if constexpr (!std::is_same_v<T, int8_t>) {
+        if (gemm_rows_dot_takes(p, sizeof(T))) return gemm_rows_dot<T>(p, a, b, c, stream);
+    }
     // whole windows of 64 and rows that do not overlap: the streaming kernel (offsets inside a block are 32-bit byte counts)
     if (p.K % kBKof<T> == 0 && p.a_rs >= static_cast<int64_t>(p.K) && p.b_cs >= static_cast<int64_t>(p.K) && p.a_rs < (1 << 22) && p.b_cs < (1 << 22)) {
         // Many small products under a short K (the scores of attention while decoding: one row against [4096, 128] per head):
