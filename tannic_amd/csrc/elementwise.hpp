@@ -229,18 +229,25 @@ __device__ inline Offsets decode(const Plan& p, uint32_t v) {
 // One vector per thread.  (Two, kBlock apart, were 6 % faster for operands with a broadcast axis from 128 MB on while everything went
 // past the caches; with the rule at kStreamedSource one is as fast or faster at every size: fp16 with one repeated value, us with
 // two / one, 128 MB 41.5 / 40.0, 256 MB 85.9 / 77.9, 512 MB 170.4 / 169.5.)
-template <class F, int VEC>
+// Element by element a thread has UNROLL of them, two from 2^23 on (a slice at an odd place, fp16, us with one / two: 9 x 552 x 2802 27.1 / 23.1).
+template <class F, int VEC, int UNROLL = 1>
 __global__ __launch_bounds__(kBlock) void elementwise_kernel(F f, Plan p) {
+    static_assert(VEC == 1 || UNROLL == 1, "vectors: one per thread");
     using S0 = typename F::S0;
     using S1 = typename F::S1;
     using D = typename F::D;
-    const uint32_t v = blockIdx.x * kBlock + threadIdx.x;
-    if (v >= p.total_vectors) return;
-    const Offsets o = decode<VEC>(p, v);
+    const uint32_t v = blockIdx.x * (kBlock * UNROLL) + threadIdx.x;
     if constexpr (VEC == 1) {
-        if constexpr (F::sources == 2) f.out[o.od] = f(f.a[o.o0], f.b[o.o1]);
-        else f.out[o.od] = f(f.a[o.o0], S1{});
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            if (v + u * kBlock >= p.total_vectors) return;
+            const Offsets o = decode<1>(p, v + u * kBlock);
+            if constexpr (F::sources == 2) f.out[o.od] = f(f.a[o.o0], f.b[o.o1]);
+            else f.out[o.od] = f(f.a[o.o0], S1{});
+        }
     } else {
+        if (v >= p.total_vectors) return;
+        const Offsets o = decode<VEC>(p, v);
         const bool splat0 = p.row_stride[0] == 0, splat1 = p.row_stride[1] == 0;
         RawPack<S0, VEC> ra;
         RawPack<S1, VEC> rb;
@@ -453,7 +460,8 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
             return launch_status("elementwise_kernel");
         }
     }
-    hipLaunchKernelGGL((elementwise_kernel<F, 1>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+    if (p.total_vectors >= (1u << 23)) hipLaunchKernelGGL((elementwise_kernel<F, 1, 2>), dim3((p.total_vectors + 2 * kBlock - 1) / (2 * kBlock)), dim3(kBlock), 0, stream, f, p);
+    else hipLaunchKernelGGL((elementwise_kernel<F, 1>), dim3(grid), dim3(kBlock), 0, stream, f, p);
     return launch_status("elementwise_kernel");
 }
 
