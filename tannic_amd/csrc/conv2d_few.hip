@@ -1,5 +1,5 @@
-// conv2d of 16-bit types over few output pixels (one image, or a handful): 1x1 and 3x3 kernels, C a multiple of 32 (3x3 of more than a few
-// channels over plain rows goes to conv2d_few3.hip from here).
+// conv2d of 16-bit types over few output pixels (one image, or a handful): 1x1 and 3x3 kernels, C a multiple of 32 (3x3 from 64 channels
+// and 1x1 with stride 1, over plain rows and from 32 output channels on, mostly go on to conv2d_few3.hip and conv2d_few1.hip from here).
 //
 // With one image a layer's work is some 0.1 - 0.2 GFLOP and a megabyte of weights: a microsecond of the chip, if all of it
 // takes part.  The tiles of the other kernels (64 output channels x up to 512 pixels, or 64 x 128 of a product) leave four
@@ -147,8 +147,8 @@ static int launch_few(const ConvProblem& p, FewPlan q, const void* x, const void
 
 // Multiply-adds up to which this kernel is taken, its output channels counted in whole tiles of 16 (a tile costs its loads whatever it
 // holds): its loads grow with the work from the first pixel on, the other kernels' time hardly does while their blocks are few.
-// Where the lines lie (fp16, replayed calls on one box, us, this kernel / the others; 3x3 from before conv2d_few3.hip, which now has most of
-// what lies below them and is faster there):
+// Where the lines lie (fp16, replayed calls on one box, us, this kernel / the others; from before conv2d_few3.hip and conv2d_few1.hip, which now have
+// most of what lies below them and are faster there):
 //   3x3, C = 64 or 128 with a stride   240 M   64 @56: batch 1 6.5 / 10.0, 2 8.7 / 10.1, 4 12.3 / 10.3; 128 @56 s2: 8.7 / 13.2, 11.3 / 16.6, 19.4 / 16.8
 //   other 3x3                          470 M   128 @28: batch 1 6.7 / 13.2, 4 12.7 / 19.3, 8 21.4 / 18.8; 256 @14: 8.2 / 26.7, 14.4 / 17.5, 26.8 / 24.8;
 //                                              512 @7: 13.0 / 58.9, 22.5 / 60.6, 37.5 / 20.0
