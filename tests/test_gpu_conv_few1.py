@@ -25,6 +25,7 @@ VARIANTS = {
     (1, 2, 8, 1): ((7, 256, 12, 17), (33, 256, 1, 1)),
     (1, 2, 16, 1): ((18, 288, 3, 12), (73, 288, 1, 1)),
     (1, 2, 16, 2): ((19, 544, 6, 11), (33, 544, 1, 1)),
+    (2, 2, 2, 1): ((2, 32, 21, 22), (2842, 32, 1, 1)),
     (2, 2, 4, 1): ((14, 96, 36, 43), (33, 96, 1, 1)),
     (2, 2, 8, 1): ((10, 224, 4, 10), (620, 224, 1, 1)),
     (2, 2, 16, 1): ((19, 416, 12, 11), (37, 416, 1, 1)),
