@@ -226,10 +226,11 @@ int tannic_hip_conv2d_plan(const tannic_tensor_t* x, const tannic_tensor_t* w, c
 /* Whether the product of a few rows with narrow row-major matrices (16-bit, misaligned) takes these operands, asked the same way:
  * the lanes side by side along its columns, 0 if it does not. */
 int tannic_hip_gemm_rows_batch_lanes(const tannic_tensor_t* a, const tannic_tensor_t* b, const tannic_tensor_t* dst);
-/* Which of the kernels below a 16-bit product would run, asked the same way: out[0] is 1 for the one above (out[1] its lanes), 2 for
+/* Which of the kernels below a 16-bit or fp32 product would run, asked the same way: out[0] is 1 for the one above (out[1] its lanes), 2 for
  * the few rows times row-major matrices with few results, 3 for more than 64 rows, both operands along K in 16-byte pieces, on
- * tiles smaller than 256 x 192 (out[1], out[2] their rows and columns, out[3] the blocks that share K), 0 for any other.  The status is
- * the product's. */
+ * tiles smaller than 256 x 192 (out[1], out[2] their rows and columns, out[3] the blocks that share K), 4 for one row (two of fp32) times whole
+ * rows of the matrix, 5 for up to 64 rows by windows of K through LDS (out[2], out[3] rows and columns of a wavefront; for both out[1] is whether the matrix is loaded
+ * past the caches), 0 for any other; 1 to 3 of 16 bits only.  The status is the product's. */
 int tannic_hip_gemm_plan(const tannic_tensor_t* a, const tannic_tensor_t* b, const tannic_tensor_t* dst, uint32_t out[4]);
 /* The stream a recording captures: a caller that keeps a device's stream to itself checks that it is this one. */
 tannic_stream_t tannic_hip_graph_stream(void* recording);

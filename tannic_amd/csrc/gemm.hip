@@ -603,12 +603,16 @@ extern "C" int tannic_hip_gemm_plan(const tannic_tensor_t* a, const tannic_tenso
     GemmProblem p;
     tannic_tensor_t result = *dst;
     if (const int status = describe_gemm(a, b, &result, p)) return status;
-    if ((a->dtype != TANNIC_FLOAT16 && a->dtype != TANNIC_BFLOAT16) || p.M == 0 || p.N == 0 || p.K == 0 || p.batches == 0 || (p.N == 1 && p.M > 1)) return TANNIC_SUCCESS;
-    if (const uint32_t lanes = gemm_rows_batch_lanes(p, a->dtype, a->address, b->address)) {
+    if ((a->dtype != TANNIC_FLOAT16 && a->dtype != TANNIC_BFLOAT16 && a->dtype != TANNIC_FLOAT32) || p.M == 0 || p.N == 0 || p.K == 0 || p.batches == 0 || (p.N == 1 && p.M > 1))
+        return TANNIC_SUCCESS;
+    if (a->dtype == TANNIC_FLOAT32) {
+        if (!few_results_under_a_long_k(p, 8192) || few_results_elsewhere<float>(p, a->address, b->address)) gemm_skinny_plan(p, a->dtype, a->address, b->address, out);
+    } else if (const uint32_t lanes = gemm_rows_batch_lanes(p, a->dtype, a->address, b->address)) {
         out[0] = 1;
         out[1] = lanes;
     } else if (few_results_under_a_long_k(p, 8192) && !few_results_elsewhere<f16>(p, a->address, b->address)) {
         out[0] = gemm_rows_few_takes(p, a->dtype) ? 2 : 0;
+    } else if (gemm_skinny_plan(p, a->dtype, a->address, b->address, out); out[0]) {
     } else if (const Tiles16 tiles = gemm16_tiles(p, a->address, b->address); tiles.rows) {
         out[0] = 3;
         out[1] = static_cast<uint32_t>(tiles.rows);

@@ -88,12 +88,20 @@ int gemm_skinny_f32(const GemmProblem& p, const float* a, const float* b, float*
 int gemm_skinny_int8(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream);
 // One row (two of fp32) times a matrix whose rows are contiguous along K, by fused multiply-adds (gemm_rows_dot.hip)
 bool gemm_rows_dot_takes(const GemmProblem& p, size_t esize);
+bool rows_dot_past_caches(const GemmProblem& p, size_t esize);
 template <class T> int gemm_rows_dot(const GemmProblem& p, const void* x, const void* w, void* y, hipStream_t stream);
-// Whether a matrix that is read once for a few rows is loaded past the caches: from 40 MB on.  A layer's weights do not stay in a memory-side cache of 256 MB
-// anyway, and a load that does not put them there takes less time (bf16, one row, every W from memory, us through the caches / past them:
-// 6144 x 4096 14.3 / 13.1, 28672 x 4096 44.4 / 40.5, 4096 x 14336 23.3 / 20.2; four rows 28672 x 4096 45.5 / 41.2; a layer's step behind 2048 tokens 140.7 / 128.4).
-// Smaller ones may be a whole model's that does stay (16384 x 512, eight of them in turn, 12.8 / 14.6).
-inline bool rows_past_caches(const GemmProblem& p, size_t esize) { return static_cast<uint64_t>(p.N) * p.K * p.batches * esize >= (40ull << 20); }
+// Whether the matrix of a few rows is loaded past the caches: from `from` bytes on, a matrix that several products share counted once.  A load that
+// puts it into the memory-side cache (256 MB) takes more time and pushes out what is there; a matrix that is used again before anything else needs that room would
+// have stayed (the kernels say where their lines lie and why).
+inline bool rows_past_caches(const GemmProblem& p, size_t esize, uint64_t from) {
+    uint64_t bytes = static_cast<uint64_t>(p.N) * p.K * esize;
+    for (int d = 0; d < p.batch_rank; ++d)
+        if (p.b_bs[d] != 0) bytes *= p.batch_extent[d];
+    return bytes >= from;
+}
+// Which of these kernels a product of few rows would run: out[0] 4 for one row at a time (gemm_rows_dot.hip), 5 for windows of K through LDS (out[2] rows, out[3]
+// columns of a wavefront), out[1] whether W goes past the caches; else 0.
+void gemm_skinny_plan(const GemmProblem& p, int dtype, const void* a, const void* b, uint32_t out[4]);
 int gemm_rows_nn(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream);
 // 16-bit, two to four rows times narrow row-major matrices under a long K, misaligned (gemm_rows_batch.hip); the lanes it would take, 0 for none
 uint32_t gemm_rows_batch_lanes(const GemmProblem& p, int dtype, const void* a, const void* b);

@@ -85,13 +85,18 @@ __global__ __launch_bounds__(64 * kDotWaves) void gemm_rows_dot_kernel(const T* 
     }
 }
 
+// From 40 MB on.  us through the caches / past them, every W from memory, and the same W again and again: bf16 5248 x 4096 (42 MB) 11.0 / 9.9, 11.1 / 9.0;
+// 8576 x 4096 15.2 / 13.7, 14.4 / 12.5; 29440 x 4096 45.3 / 40.2, 37.2 / 36.6; fp32 3072 x 4096 12.9 / 11.8, 11.9 / 10.2; 14336 x 4096 45.7 / 42.5, 37.9 / 39.2.  Below, the same W
+// is as fast either way (bf16 2176 x 4096 6.3 / 6.4), and smaller ones may be a whole model's that does stay.
+bool rows_dot_past_caches(const GemmProblem& p, size_t esize) { return rows_past_caches(p, esize, 40ull << 20); }
+
 template <class T, int MR>
 static int launch_rows_dot(const GemmProblem& p, const void* x, const void* w, void* y, hipStream_t stream) {
     auto kernel = gemm_rows_dot_kernel<T, MR>;
     static std::atomic<uint64_t> configured{0};
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), kDotLds, configured)) return rc;
     hipLaunchKernelGGL(kernel, dim3((p.N + kDotWaves - 1) / kDotWaves, p.batches), dim3(64 * kDotWaves), MR * p.K * sizeof(T), stream, static_cast<const T*>(x),
-                       static_cast<const T*>(w), static_cast<T*>(y), p, rows_past_caches(p, sizeof(T)));
+                       static_cast<const T*>(w), static_cast<T*>(y), p, rows_dot_past_caches(p, sizeof(T)));
     return launch_status("gemm_rows_dot_kernel");
 }
 

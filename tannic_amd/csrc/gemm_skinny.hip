@@ -161,9 +161,10 @@ typedef __attribute__((address_space(3))) void* skinny_lds_void;
 constexpr int kStreamWaves = 4;
 constexpr int kStreamBytesPerWave = 32 * 1024;
 
-template <class T, int MB, int NB>
+// PAST: W is loaded past the caches (a parameter: tested in the loop it costs fp32 up to 5 %)
+template <class T, int MB, int NB, bool PAST>
 __global__ __launch_bounds__(64 * kStreamWaves) void gemm_skinny_stream_kernel(const T* x, const T* w, typename SkinnyTypes<T>::Out* c, GemmProblem p,
-                                                                               uint32_t windows_per_wave, bool streamed) {
+                                                                               uint32_t windows_per_wave) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using Acc = typename SkinnyTypes<T>::Acc;
     using Out = typename SkinnyTypes<T>::Out;
@@ -196,16 +197,10 @@ __global__ __launch_bounds__(64 * kStreamWaves) void gemm_skinny_stream_kernel(c
     }
     auto issue = [&](uint32_t window, uint32_t stage) {
         const uint32_t k_bytes = window * 128;
-        constexpr int PAST_CACHES = 2;      // (the non-temporal bit of a load)
-        if (streamed) {
+        constexpr int POLICY = PAST ? 2 : 0;      // (the non-temporal bit of a load)
 #pragma unroll
-            for (int j = 0; j < 2 * NB; ++j)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, PAST_CACHES);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 2 * NB; ++j)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, 0);
-        }
+        for (int j = 0; j < 2 * NB; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, POLICY);
 #pragma unroll
         for (int j = 2 * NB; j < LOADS; ++j)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_x, (skinny_lds_void)(ring + stage * STAGE_BYTES + j * 1024), 16, voff[j], k_bytes, 0, 0);
@@ -289,20 +284,44 @@ __global__ __launch_bounds__(64 * kStreamWaves) void gemm_skinny_stream_kernel(c
 #endif
 }
 
-template <class T, int MB, int NB>
-static int launch_stream(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream) {
-    auto kernel = gemm_skinny_stream_kernel<T, MB, NB>;
+// Which W goes past the caches.  us, through the caches / past them, every W from memory, and the same W again and again:
+//   up to four rows of 16 bits, from 56 MB on   14336 x 2048 (56 MB) 15.1 / 13.5, 13.8 / 12.8; 8192 x 4096 16.4 / 14.8, 15.7 / 14.4; 14336 x 4096 24.5 / 22.5,
+//                                               22.0 / 21.9; 20000 x 4096 35.1 / 32.3, 29.2 / 30.8; 28672 x 4096 46.5 / 43.3, 39.1 / 41.1; below: 6144 x 4096 14.7 / 13.2, 11.2 / 13.0
+//   more rows, int8: from 208 MB on             that much does not stay beside anything else.  16 rows of 14336 x 4096 (112 MB) 26.1 / 23.8, 22.0 / 23.4; of 12000 x 5120
+//                                               34.0 / 31.5, 24.7 / 30.0; of 28672 x 4096 (224 MB) 49.5 / 46.2, 39.9 / 44.3; a decoder layer's step of 16 sequences with
+//                                               matrices of 224, 112, 48 and 32 MB: all through the caches 173, the largest past them 158, from 56 MB on 156
+//   (8 products that share one of 4096 x 4096, 4 rows each, counted eight times and so past the caches: 27.1, through them 21.9)
+//   fp32: from 256 MB on, what cannot stay      16 rows of 4096 x 4096 18.3 / 17.2, 14.8 / 16.2; of 14336 x 4096 (224 MB) 56.5 / 55.4, 38.3 / 54.3; of 18304 x 4096
+//                                               83.7 / 79.1, 81.5 / 76.8
+template <class T>
+static bool stream_past_caches(const GemmProblem& p) {
+    return rows_past_caches(p, sizeof(T), sizeof(T) == 4 ? 256ull << 20 : sizeof(T) == 2 && p.M <= 4 ? 56ull << 20 : 208ull << 20);
+}
+
+template <class T, int MB, int NB, bool PAST>
+static int launch_stream(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream, uint32_t* plan) {
+    if (plan) {      // (only asked for)
+        const uint32_t values[4] = {5, PAST, 16 * MB, 16 * NB};
+        for (int i = 0; i < 4; ++i) plan[i] = values[i];
+        return TANNIC_SUCCESS;
+    }
+    auto kernel = gemm_skinny_stream_kernel<T, MB, NB, PAST>;
     constexpr size_t lds = kStreamWaves * kStreamBytesPerWave;
     static std::atomic<uint64_t> configured{0};
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds, configured)) return rc;
     const uint32_t windows = p.K / kBKof<T>, per_wave = (windows + kStreamWaves - 1) / kStreamWaves;
     hipLaunchKernelGGL(kernel, dim3((p.N + 16 * NB - 1) / (16 * NB), p.batches), dim3(64 * kStreamWaves), lds, stream, static_cast<const T*>(a), static_cast<const T*>(b),
-                       static_cast<typename SkinnyTypes<T>::Out*>(c), p, per_wave, rows_past_caches(p, sizeof(T)));
+                       static_cast<typename SkinnyTypes<T>::Out*>(c), p, per_wave);
     return launch_status("gemm_skinny_stream_kernel");
 }
 
+template <class T, int MB, int NB>
+static int launch_stream(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream, uint32_t* plan) {
+    return stream_past_caches<T>(p) ? launch_stream<T, MB, NB, true>(p, a, b, c, stream, plan) : launch_stream<T, MB, NB, false>(p, a, b, c, stream, plan);
+}
+
 template <class T>
-int run_skinny(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream) {
+int run_skinny(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream, uint32_t* plan = nullptr) {
     if (p.M == 0 || p.M > 64 || p.N == 0 || p.K == 0 || p.batches == 0 || p.batches > 65535 || p.row_bias || p.c_group) return TANNIC_UNSUPPORTED_DTYPE;
     // both operands K-contiguous; 16-byte chunks along K
     if (p.a_cs != 1 || p.b_rs != 1) return TANNIC_UNSUPPORTED_DTYPE;
@@ -312,7 +331,12 @@ int run_skinny(const GemmProblem& p, const void* a, const void* b, void* c, hipS
     for (int d = 0; d < p.batch_rank; ++d)
         if (!mult8(p.a_bs[d]) || !mult8(p.b_bs[d])) return TANNIC_UNSUPPORTED_DTYPE;
     if constexpr (!std::is_same_v<T, int8_t>) {
-        if (gemm_rows_dot_takes(p, sizeof(T))) return gemm_rows_dot<T>(p, a, b, c, stream);
+        if (gemm_rows_dot_takes(p, sizeof(T))) {
+            if (!plan) return gemm_rows_dot<T>(p, a, b, c, stream);
+            plan[0] = 4;
+            plan[1] = rows_dot_past_caches(p, sizeof(T));
+            return TANNIC_SUCCESS;
+        }
     }
     // whole windows of 64 and rows that do not overlap: the streaming kernel (offsets inside a block are 32-bit byte counts)
     if (p.K % kBKof<T> == 0 && p.a_rs >= static_cast<int64_t>(p.K) && p.b_cs >= static_cast<int64_t>(p.K) && p.a_rs < (1 << 22) && p.b_cs < (1 << 22)) {
@@ -323,8 +347,8 @@ int run_skinny(const GemmProblem& p, const void* a, const void* b, void* c, hipS
         if (sizeof(T) == 2 ? (p.batches >= 8 && p.K <= 512) : (p.batches >= 128 && p.K <= 128)) return TANNIC_UNSUPPORTED_DTYPE;
         // two column blocks per wavefront (half as many workgroups, x read half as often) while every compute unit still gets one
         const bool two = static_cast<uint64_t>((p.N + 31) / 32) * p.batches >= 400;
-        if (p.M <= 16) return two ? launch_stream<T, 1, 2>(p, a, b, c, stream) : launch_stream<T, 1, 1>(p, a, b, c, stream);
-        if (p.M <= 32) return two ? launch_stream<T, 2, 2>(p, a, b, c, stream) : launch_stream<T, 2, 1>(p, a, b, c, stream);
+        if (p.M <= 16) return two ? launch_stream<T, 1, 2>(p, a, b, c, stream, plan) : launch_stream<T, 1, 1>(p, a, b, c, stream, plan);
+        if (p.M <= 32) return two ? launch_stream<T, 2, 2>(p, a, b, c, stream, plan) : launch_stream<T, 2, 1>(p, a, b, c, stream, plan);
         // (fp32 stops here: with more row blocks its MFMAs, a sixteenth as fast, take longer than W takes to arrive; int8
         // beyond 32 rows has its tiles)
         if constexpr (sizeof(T) != 2) {
@@ -337,14 +361,14 @@ int run_skinny(const GemmProblem& p, const void* a, const void* b, void* c, hipS
             // (One product at a time: the many small products of an attention head - 64 x 64 x 64, a thousand of them - have one
             // window of K for four wavefronts and take 28 us here against 8 on tiles.)
             if (p.batches != 1 || p.K < 256 || static_cast<uint64_t>(p.N) * p.K > (20u << 20)) return TANNIC_UNSUPPORTED_DTYPE;
-            if (p.M <= 48) return launch_stream<T, 3, 1>(p, a, b, c, stream);
-            return launch_stream<T, 4, 1>(p, a, b, c, stream);
+            if (p.M <= 48) return launch_stream<T, 3, 1>(p, a, b, c, stream, plan);
+            return launch_stream<T, 4, 1>(p, a, b, c, stream, plan);
         }
     }
     if constexpr (sizeof(T) != 2) {
         return TANNIC_UNSUPPORTED_DTYPE;   // the kernel for other K is written for 16-bit fragments
     } else {
-        if (p.M > 32) return TANNIC_UNSUPPORTED_DTYPE;
+        if (p.M > 32 || plan) return TANNIC_UNSUPPORTED_DTYPE;
         // K is split evenly over the wavefronts, in whole steps of 32
         const uint32_t steps = (p.K + 31) / 32, per_wave = (steps + kSkinnyWaves - 1) / kSkinnyWaves;
         const uint32_t k_per_wave = per_wave * 32;
@@ -371,6 +395,12 @@ int gemm_skinny_f32(const GemmProblem& p, const float* a, const float* b, float*
 
 // int8 x int8 -> int32, at most 32 rows over whole windows of 128 k: W goes by once where the 128-row tiles walk it at their own pace
 int gemm_skinny_int8(const GemmProblem& p, const void* a, const void* b, void* c, hipStream_t stream) { return run_skinny<int8_t>(p, a, b, c, stream); }
+
+void gemm_skinny_plan(const GemmProblem& p, int dtype, const void* a, const void* b, uint32_t out[4]) {
+    if (dtype == TANNIC_FLOAT16) run_skinny<f16>(p, a, b, nullptr, nullptr, out);
+    else if (dtype == TANNIC_BFLOAT16) run_skinny<bf16>(p, a, b, nullptr, nullptr, out);
+    else if (dtype == TANNIC_FLOAT32) run_skinny<float>(p, a, b, nullptr, nullptr, out);
+}
 
 int gemm_skinny_16bit(const GemmProblem& p, int dtype, const void* a, const void* b, void* c, hipStream_t stream) {
     if (dtype == TANNIC_FLOAT16) return run_skinny<f16>(p, a, b, c, stream);

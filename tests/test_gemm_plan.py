@@ -142,3 +142,29 @@ def test_tiles_of_long_products_on_the_gpu(m, n, k, dtype):
     w.strides.sizes[:2] = 1, k + 16
     kernel, rows, columns, shares = plan_of(x, w, y)
     assert (kernel, rows, columns, shares > 1) == (3, *TILES[m, n, k])
+
+
+# rows, columns, K (and products that share one matrix) -> the matrix is loaded past the caches.  One row from 40 MB on; two to four rows of 16 bits from 56 MB, more
+# from 208 MB; fp32 from 256 MB: what stays in the memory-side cache from call to call is not kept out of it.
+PAST_CACHES = {
+    "bfloat16": [((1, 5120, 4096), 4, True), ((1, 5112, 4096), 4, False), ((2, 5120, 4096), 5, False), ((2, 14336, 2048), 5, True), ((4, 14336, 4096), 5, True),
+                 ((4, 7160, 4096), 5, False), ((5, 14336, 4096), 5, False), ((16, 14336, 4096), 5, False), ((16, 26624, 4096), 5, True), ((32, 26616, 4096), 5, False),
+                 ((2, 1, 4096, 4096), 5, False), ((8, 4, 6144, 4096), 5, False), ((8, 4, 7168, 4096), 5, True)],
+    "float32": [((1, 2560, 4096), 4, True), ((1, 2552, 4096), 4, False), ((2, 4096, 4096), 4, True), ((16, 4096, 4096), 5, False), ((4, 14336, 4096), 5, False),
+                ((4, 16384, 4096), 5, True), ((8, 4, 8192, 4096), 5, False)],
+}
+
+
+@pytest.mark.parametrize("dtype,problem,kernel,past", [(d, *c) for d in PAST_CACHES for c in PAST_CACHES[d]], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_matrices_of_few_rows_past_the_caches(dtype, problem, kernel, past):
+    *batch, m, n, k = problem
+    x, w, y = (descriptor(dtype, s) for s in ((*batch, m, k), (k, n), (*batch, m, n)))
+    w.strides.sizes[:2] = 1, k
+    assert plan_of(x, w, y)[:2] == (kernel, past)
+
+
+def test_matrices_of_many_products_count_together():
+    """Keys of 32 sequences, 8 heads each: 64 MB, every one its own product's."""
+    x, w, y = (descriptor("bfloat16", s) for s in ((32, 8, 4, 1024), (32, 8, 1024, 128), (32, 8, 4, 128)))
+    w.strides.sizes[:4] = 8 * 1024 * 128, 1024 * 128, 1, 1024
+    assert plan_of(x, w, y)[:2] == (5, 1)
