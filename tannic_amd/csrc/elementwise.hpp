@@ -226,13 +226,12 @@ __device__ inline Offsets decode(const Plan& p, uint32_t v) {
 
 // F: { using S0, S1, D; static constexpr int sources; const S0* a; const S1* b; D* out;
 //      __device__ D operator()(S0, S1) const; }   (S1/b unused when sources == 1)
-// One vector per thread.  (Two, kBlock apart, were 6 % faster for operands with a broadcast axis from 128 MB on while everything went
-// past the caches; with the rule at kStreamedSource one is as fast or faster at every size: fp16 with one repeated value, us with
-// two / one, 128 MB 41.5 / 40.0, 256 MB 85.9 / 77.9, 512 MB 170.4 / 169.5.)
-// Element by element a thread has UNROLL of them, two from 2^23 on (a slice at an odd place, fp16, us with one / two: 9 x 552 x 2802 27.1 / 23.1).
+// UNROLL vectors per thread, kBlock apart, two from 2^23 on: with rows to decode and a repeated value to wait for a thread lives longer, and two keep enough
+// bytes on their way.  fp16, X + a value per row (of [64, 4096, 1024]), us with one / two: 256 MB 91.0 / 88.1, 512 MB 177 / 169, 1 GB 347 / 336, into one buffer
+// again and again 512 MB 176 / 158; one value for all of it 512 MB 164 / 160 there; int32 128 MB 48.1 / 46.9.  Element by element: a slice at an odd place, fp16, 9 x 552 x
+// 2802 27.1 / 23.1.  Below 2^23 one is as fast (64 MB 22.5 / 22.4).
 template <class F, int VEC, int UNROLL = 1>
 __global__ __launch_bounds__(kBlock) void elementwise_kernel(F f, Plan p) {
-    static_assert(VEC == 1 || UNROLL == 1, "vectors: one per thread");
     using S0 = typename F::S0;
     using S1 = typename F::S1;
     using D = typename F::D;
@@ -246,23 +245,31 @@ __global__ __launch_bounds__(kBlock) void elementwise_kernel(F f, Plan p) {
             else f.out[o.od] = f(f.a[o.o0], S1{});
         }
     } else {
-        if (v >= p.total_vectors) return;
-        const Offsets o = decode<VEC>(p, v);
         const bool splat0 = p.row_stride[0] == 0, splat1 = p.row_stride[1] == 0;
-        RawPack<S0, VEC> ra;
-        RawPack<S1, VEC> rb;
-        ra.load(f.a + o.o0, splat0, p.streamed);
-        if constexpr (F::sources == 2) rb.load(f.b + o.o1, splat1, p.streamed);
-        const Pack<S0, VEC> a = ra.get(splat0);
-        Pack<S1, VEC> b;
-        if constexpr (F::sources == 2) b = rb.get(splat1);
-        Pack<D, VEC> r;
+        Offsets o[UNROLL];
+        RawPack<S0, VEC> ra[UNROLL];
+        RawPack<S1, VEC> rb[UNROLL];
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-            if constexpr (F::sources == 2) r.v[i] = f(a.v[i], b.v[i]);
-            else r.v[i] = f(a.v[i], S1{});
+        for (int u = 0; u < UNROLL; ++u) {
+            if (v + u * kBlock >= p.total_vectors) break;
+            o[u] = decode<VEC>(p, v + u * kBlock);
+            ra[u].load(f.a + o[u].o0, splat0, p.streamed);
+            if constexpr (F::sources == 2) rb[u].load(f.b + o[u].o1, splat1, p.streamed);
         }
-        store_kept<D, VEC>(f.out + o.od, r, blockIdx.x >= p.kept_from);
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u) {
+            if (v + u * kBlock >= p.total_vectors) break;
+            const Pack<S0, VEC> a = ra[u].get(splat0);
+            Pack<S1, VEC> b;
+            if constexpr (F::sources == 2) b = rb[u].get(splat1);
+            Pack<D, VEC> r;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                if constexpr (F::sources == 2) r.v[i] = f(a.v[i], b.v[i]);
+                else r.v[i] = f(a.v[i], S1{});
+            }
+            store_kept<D, VEC>(f.out + o[u].od, r, blockIdx.x >= p.kept_from);
+        }
     }
 }
 
@@ -447,7 +454,8 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
     }
     p.total_vectors = static_cast<uint32_t>(rows * p.row_vectors);
     if (p.total_vectors == 0) return TANNIC_SUCCESS;
-    const uint32_t grid = (p.total_vectors + kBlock - 1) / kBlock;
+    const bool two = p.total_vectors >= (1u << 23);
+    const uint32_t grid = (p.total_vectors + kBlock - 1) / kBlock, halves = (p.total_vectors + 2 * kBlock - 1) / (2 * kBlock);
     if constexpr (VEC > 1) {
         if (vec) {
             p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
@@ -456,11 +464,16 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
                 hipLaunchKernelGGL((elementwise_dense_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, p.total_vectors, p.kept_from, p.streamed);
                 return launch_status("elementwise_dense_kernel");
             }
-            hipLaunchKernelGGL((elementwise_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+            if (two) {
+                p.kept_from = first_kept(halves, 2 * sizeof(D) * VEC * kBlock);
+                hipLaunchKernelGGL((elementwise_kernel<F, VEC, 2>), dim3(halves), dim3(kBlock), 0, stream, f, p);
+            } else {
+                hipLaunchKernelGGL((elementwise_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, p);
+            }
             return launch_status("elementwise_kernel");
         }
     }
-    if (p.total_vectors >= (1u << 23)) hipLaunchKernelGGL((elementwise_kernel<F, 1, 2>), dim3((p.total_vectors + 2 * kBlock - 1) / (2 * kBlock)), dim3(kBlock), 0, stream, f, p);
+    if (two) hipLaunchKernelGGL((elementwise_kernel<F, 1, 2>), dim3(halves), dim3(kBlock), 0, stream, f, p);
     else hipLaunchKernelGGL((elementwise_kernel<F, 1>), dim3(grid), dim3(kBlock), 0, stream, f, p);
     return launch_status("elementwise_kernel");
 }

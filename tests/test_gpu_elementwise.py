@@ -304,3 +304,15 @@ def test_operands_past_the_caches(device, megabytes):
     want = (x + x).reshape(-1, 64, 1024) - row
     np.testing.assert_array_equal(got.numpy(), want)
     np.testing.assert_array_equal(ops.neg(got).numpy(), -want)
+
+
+@pytest.mark.parametrize("rows", [32896, 32897, 65800], ids=lambda r: f"{r}rows")
+def test_two_vectors_per_thread(device, rows):
+    """255 vectors a row next to a value per row and to one value: the last row count below 2^23 vectors, the first beyond it (a block of which only some threads have a
+    second vector), and one whose results go past the caches in part.  Whole numbers: bit for bit."""
+    x = np.arange(rows * 1020, dtype=np.int32).reshape(rows, 1020)
+    z = np.arange(rows, dtype=np.int32).reshape(rows, 1) * 5
+    dx = ta.tensor(x, ta.int32, device)
+    np.testing.assert_array_equal(ops.sub(dx, ta.tensor(z, ta.int32, device)).numpy(), x - z)
+    np.testing.assert_array_equal(ops.sub(ta.tensor(z, ta.int32, device), dx).numpy(), z - x)
+    np.testing.assert_array_equal(ops.add(dx, ta.tensor(np.array([7], np.int32), ta.int32, device)).numpy(), x + 7)
