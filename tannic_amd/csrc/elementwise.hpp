@@ -31,7 +31,7 @@ struct Plan {
     FastDiv row_div;                       // division by row_vectors
     uint32_t row_vectors;                  // vectors per row (set at launch)
     uint32_t kept_from;                    // the block from which on results are stored through the caches
-    uint32_t streamed;                     // whether the sources are loaded past them
+    uint32_t streamed;                     // the sources that are loaded past them: bit o for source o
     int64_t row_stride[kMaxOperands];      // the last dim's element strides
     uint32_t extent[TANNIC_DIMENSIONS];    // collapsed extents
     FastDiv div[TANNIC_DIMENSIONS];        // division by extent[d]
@@ -127,6 +127,17 @@ template <> struct RawBits<1> { using type = unsigned char; };
 // product reads, 331 / 317, in the front end's own operators 571 / 551 (the loads alone through the caches 331 and 567, the stores alone 315 and 556);
 // one result of 8 MB that nothing reads afterwards 3.4 / 4.0.  Bound by HBM: 6.5 TB/s at 512 MB, 6.9 at 256.
 constexpr uint64_t kStreamedSource = 96ull << 20, kKeptResult = 208ull << 20;
+
+// Source o as the plan walks it: its bit if it is loaded past the caches.  Counted is what the source itself has: a row or a plane that every outer index
+// reads again stays in the caches however large the tensor beside it is (fp16 [64, 4096, 1024] + [1024], us past the caches / through them 183 / 171, + [1, 4096, 1024] 217 / 178;
+// 1 GB of int32 + a plane 435 / 362).
+template <class S>
+inline uint32_t streamed_source(const Plan& p, int o) {
+    uint64_t bytes = sizeof(S);
+    for (int d = 0; d < p.rank; ++d)
+        if (p.stride[o][d] != 0) bytes *= p.extent[d];
+    return bytes >= kStreamedSource ? 1u << o : 0u;
+}
 
 // The first of `blocks` blocks of `bytes` bytes of results each whose results are kept
 inline uint32_t first_kept(uint32_t blocks, uint64_t bytes) { return blocks * bytes > kKeptResult ? static_cast<uint32_t>(blocks - kKeptResult / bytes) : 0; }
@@ -253,8 +264,8 @@ __global__ __launch_bounds__(kBlock) void elementwise_kernel(F f, Plan p) {
         for (int u = 0; u < UNROLL; ++u) {
             if (v + u * kBlock >= p.total_vectors) break;
             o[u] = decode<VEC>(p, v + u * kBlock);
-            ra[u].load(f.a + o[u].o0, splat0, p.streamed);
-            if constexpr (F::sources == 2) rb[u].load(f.b + o[u].o1, splat1, p.streamed);
+            ra[u].load(f.a + o[u].o0, splat0, p.streamed & 1);
+            if constexpr (F::sources == 2) rb[u].load(f.b + o[u].o1, splat1, p.streamed & 2);
         }
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) {
@@ -285,8 +296,8 @@ __global__ __launch_bounds__(kBlock) void elementwise_dense_kernel(F f, uint32_t
     const size_t at = static_cast<size_t>(v) * VEC;
     RawPack<S0, VEC> ra;
     RawPack<S1, VEC> rb;
-    ra.load(f.a + at, false, streamed);
-    if constexpr (F::sources == 2) rb.load(f.b + at, false, streamed);
+    ra.load(f.a + at, false, streamed & 1);
+    if constexpr (F::sources == 2) rb.load(f.b + at, false, streamed & 2);
     const Pack<S0, VEC> a = ra.get(false);
     Pack<S1, VEC> b;
     if constexpr (F::sources == 2) b = rb.get(false);
@@ -329,7 +340,7 @@ __device__ inline Pack<T, VEC> flat_source(const FlatPlan& fp, int o, const T* b
     if (fp.full[o]) {
         if (live == VEC) {
             RawPack<T, VEC> raw;
-            raw.load(base + first, false, fp.p.streamed);
+            raw.load(base + first, false, fp.p.streamed >> o & 1);
             return raw.get(false);
         }
 #pragma unroll
@@ -440,7 +451,7 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
                 fp.p = p;
                 const uint32_t vectors = static_cast<uint32_t>((fp.elements + VEC - 1) / VEC), grid = (vectors + kBlock - 1) / kBlock;
                 fp.p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
-                fp.p.streamed = fp.elements * sizeof(S0) >= kStreamedSource;
+                fp.p.streamed = streamed_source<S0>(p, 0) | (F::sources == 2 ? streamed_source<S1>(p, 1) : 0);
                 hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, fp, vectors);
                 return launch_status("elementwise_flat_kernel");
             }
@@ -459,7 +470,7 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
     if constexpr (VEC > 1) {
         if (vec) {
             p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
-            p.streamed = static_cast<uint64_t>(p.total_vectors) * VEC * sizeof(S0) >= kStreamedSource;
+            p.streamed = streamed_source<S0>(p, 0) | (F::sources == 2 ? streamed_source<S1>(p, 1) : 0);
             if (p.rank == 1 && p.stride[0][0] == 1 && (F::sources == 1 || p.stride[1][0] == 1)) {      // (vec: the result's is 1)
                 hipLaunchKernelGGL((elementwise_dense_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, p.total_vectors, p.kept_from, p.streamed);
                 return launch_status("elementwise_dense_kernel");

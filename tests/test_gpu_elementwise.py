@@ -316,3 +316,15 @@ def test_two_vectors_per_thread(device, rows):
     np.testing.assert_array_equal(ops.sub(dx, ta.tensor(z, ta.int32, device)).numpy(), x - z)
     np.testing.assert_array_equal(ops.sub(ta.tensor(z, ta.int32, device), dx).numpy(), z - x)
     np.testing.assert_array_equal(ops.add(dx, ta.tensor(np.array([7], np.int32), ta.int32, device)).numpy(), x + 7)
+
+
+@pytest.mark.parametrize("rows", [8192, 25600], ids=["32MB_plane", "100MB_plane"])
+def test_planes_and_rows_beside_large_tensors(device, rows):
+    """A plane and a row that every outer index reads again: the tensor beside them goes past the caches, they do by what they have themselves."""
+    x = np.arange(4 * rows * 1024, dtype=np.int32).reshape(4, rows, 1024)
+    plane, row = x[:1] * 3 + 1, np.arange(1024, dtype=np.int32) * 7
+    dx, dp, dr = (ta.tensor(v, ta.int32, device) for v in (x, plane, row))
+    np.testing.assert_array_equal(ops.sub(dx, dp).numpy(), x - plane)
+    np.testing.assert_array_equal(ops.sub(dp, dx).numpy(), plane - x)
+    np.testing.assert_array_equal(ops.sub(dr, dx).numpy(), row - x)
+    np.testing.assert_array_equal(ops.add(dp, dr).numpy(), plane + row)
