@@ -142,26 +142,29 @@ inline uint32_t streamed_source(const Plan& p, int o) {
 // The first of `blocks` blocks of `bytes` bytes of results each whose results are kept
 inline uint32_t first_kept(uint32_t blocks, uint64_t bytes) { return blocks * bytes > kKeptResult ? static_cast<uint32_t>(blocks - kKeptResult / bytes) : 0; }
 
-// Loads N consecutive elements with one access of sizeof(T)*N bytes.
-template <class T, int N>
+// Loads N consecutive elements with one access of sizeof(T)*N bytes, through the caches or past them.
+template <class T, int N, bool PAST>
 __device__ inline Pack<T, N> load_pack(const T* p) {
     static_assert(sizeof(T) * N <= 16, "a pack is at most 16 bytes");
     using Raw = typename RawBits<sizeof(T) * N>::type;
-    const Raw raw = *reinterpret_cast<const Raw*>(p);
+    Raw raw;
+    if constexpr (PAST) raw = __builtin_nontemporal_load(reinterpret_cast<const Raw*>(p));
+    else raw = *reinterpret_cast<const Raw*>(p);
     Pack<T, N> r;
     __builtin_memcpy(&r, &raw, sizeof r);
     return r;
 }
 
-template <class T, int N>
+template <class T, int N, bool PAST>
 __device__ inline void store_pack(T* p, const Pack<T, N>& v) {
     using Raw = typename RawBits<sizeof(T) * N>::type;
     Raw raw;
     __builtin_memcpy(&raw, &v, sizeof raw);
-    *reinterpret_cast<Raw*>(p) = raw;
+    if constexpr (PAST) __builtin_nontemporal_store(raw, reinterpret_cast<Raw*>(p));
+    else *reinterpret_cast<Raw*>(p) = raw;
 }
 
-// The same, through the caches or past them.  (The empty statements keep the two accesses apart, which the compiler would merge into one
+// The same with the choice made at run time.  (The empty statements keep the two accesses apart, which the compiler would merge into one
 // through the caches.)
 template <class T, int N>
 __device__ inline void store_kept(T* p, const Pack<T, N>& v, bool kept) {

@@ -215,7 +215,8 @@ __global__ __launch_bounds__(kBlock) void compare_kernel(const T* a, const T* b,
 
 // Contiguous operands: every lane reads ONE 16-byte vector per operand (fully coalesced) and turns it
 // into N = 16 / sizeof(T) result bits; lanes that hold less than a byte pass their bits down to the
-// first lane of their byte.
+// first lane of their byte.  The operands go past the caches: nothing but reads, which are as fast or faster so at every size (int32, two of 32 MB 12.2 us,
+// through the caches 13.7, of 256 MB 78 / 88, of 1 GB 344 / 356).
 template <class T, int K>
 __global__ __launch_bounds__(kBlock) void compare_flat_kernel(const T* a, const T* b, uint8_t* out, uint32_t ne) {
     constexpr int N = 16 / sizeof(T);
@@ -223,8 +224,8 @@ __global__ __launch_bounds__(kBlock) void compare_flat_kernel(const T* a, const 
     const uint32_t first = t * N;
     uint32_t bits = 0;
     if (first + N <= ne) {
-        const Pack<T, N> x = load_pack<T, N>(a + first);
-        const Pack<T, N> y = load_pack<T, N>(b + first);
+        const Pack<T, N> x = load_pack<T, N, true>(a + first);
+        const Pack<T, N> y = load_pack<T, N, true>(b + first);
 #pragma unroll
         for (int i = 0; i < N; ++i) bits |= static_cast<uint32_t>(compare<K>(x.v[i], y.v[i])) << i;
     } else if (first < ne) {

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kRowBlock) void rms_norm_kernel(const T* x, const T
     for (int i = 0; i < NCH; ++i) {
         const uint32_t c = t + i * G;
         if (live && c < chunks) {
-            v[i] = load_pack<T, VEC>(x + base + static_cast<size_t>(c) * VEC);
+            v[i] = load_pack<T, VEC, false>(x + base + static_cast<size_t>(c) * VEC);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const A a = static_cast<A>(widen(v[i].v[e]));
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kRowBlock) void rms_norm_kernel(const T* x, const T
             Pack<T, VEC> out;
 #pragma unroll
             for (int e = 0; e < VEC; ++e) out.v[e] = narrow<T>(static_cast<A>(widen(v[i].v[e])) * r * static_cast<A>(widen(g.v[e])));
-            store_pack<T, VEC>(y + base + static_cast<size_t>(c) * VEC, out);
+            store_pack<T, VEC, false>(y + base + static_cast<size_t>(c) * VEC, out);
         }
     }
 }
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kRowBlock) void softmax_kernel(const T* x, const T*
     for (int i = 0; i < NCH; ++i) {
         const uint32_t c = t + i * G;
         if (live && c < chunks) {
-            const Pack<T, VEC> v = load_pack<T, VEC>(x + base + static_cast<size_t>(c) * VEC);
+            const Pack<T, VEC> v = load_pack<T, VEC, false>(x + base + static_cast<size_t>(c) * VEC);
             Pack<T, VEC> m;
             if (MASK) m = *reinterpret_cast<const Pack<T, VEC>*>(mask + static_cast<size_t>(mrow) * L + static_cast<size_t>(c) * VEC);
 #pragma unroll
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(kRowBlock) void softmax_kernel(const T* x, const T*
             Pack<T, VEC> out;
 #pragma unroll
             for (int e = 0; e < VEC; ++e) out.v[e] = narrow<T>(s[i][e] * inv);
-            store_pack<T, VEC>(y + base + static_cast<size_t>(c) * VEC, out);
+            store_pack<T, VEC, false>(y + base + static_cast<size_t>(c) * VEC, out);
         }
     }
 }
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(kRowBlock) void rope_kernel(const T* x, const T* cs
     Pack<T, 2 * PAIRS> v;
     Pack<T, PAIRS> c, s;
     if constexpr (PAIRS > 1) {
-        v = load_pack<T, 2 * PAIRS>(x + off + col);
+        v = load_pack<T, 2 * PAIRS, false>(x + off + col);
         c = *reinterpret_cast<const Pack<T, PAIRS>*>(cs + table);
         s = *reinterpret_cast<const Pack<T, PAIRS>*>(sn + table);
     } else {
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(kRowBlock) void rope_kernel(const T* x, const T* cs
     }
     T* dst = y + static_cast<size_t>(row) * m.d + col;
     if constexpr (PAIRS > 1) {
-        store_pack<T, 2 * PAIRS>(dst, out);
+        store_pack<T, 2 * PAIRS, false>(dst, out);
     } else {
         dst[0] = out.v[0];
         dst[1] = out.v[1];
