@@ -49,7 +49,7 @@ template <class A> __device__ inline A fast_exp(A x, bool coarse) {
 }
 
 // ---- RMS normalisation ----------------------------------------------------------
-template <class T, int G, int NCH>
+template <class T, int G, int NCH, bool PAST>
 __global__ __launch_bounds__(kRowBlock) void rms_norm_kernel(const T* x, const T* gain, T* y, uint32_t rows, uint32_t L, double eps) {
     constexpr int VEC = 16 / sizeof(T);
     using A = RowAcc<T>;
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kRowBlock) void rms_norm_kernel(const T* x, const T
     for (int i = 0; i < NCH; ++i) {
         const uint32_t c = t + i * G;
         if (live && c < chunks) {
-            v[i] = load_pack<T, VEC, false>(x + base + static_cast<size_t>(c) * VEC);
+            v[i] = load_pack<T, VEC, PAST>(x + base + static_cast<size_t>(c) * VEC);
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const A a = static_cast<A>(widen(v[i].v[e]));
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kRowBlock) void rms_norm_kernel(const T* x, const T
             Pack<T, VEC> out;
 #pragma unroll
             for (int e = 0; e < VEC; ++e) out.v[e] = narrow<T>(static_cast<A>(widen(v[i].v[e])) * r * static_cast<A>(widen(g.v[e])));
-            store_pack<T, VEC, false>(y + base + static_cast<size_t>(c) * VEC, out);
+            store_pack<T, VEC, PAST>(y + base + static_cast<size_t>(c) * VEC, out);
         }
     }
 }
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kRowBlock) void rms_norm_any_kernel(const T* x, con
 }
 
 // ---- softmax ----------------------------------------------------------------------
-template <class T, int G, int NCH, bool MASK>
+template <class T, int G, int NCH, bool MASK, bool PAST>
 __global__ __launch_bounds__(kRowBlock) void softmax_kernel(const T* x, const T* mask, T* y, uint32_t rows, uint32_t L, FastDiv q, float scale) {
     constexpr int VEC = 16 / sizeof(T);
     using A = RowAcc<T>;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kRowBlock) void softmax_kernel(const T* x, const T*
     for (int i = 0; i < NCH; ++i) {
         const uint32_t c = t + i * G;
         if (live && c < chunks) {
-            const Pack<T, VEC> v = load_pack<T, VEC, false>(x + base + static_cast<size_t>(c) * VEC);
+            const Pack<T, VEC> v = load_pack<T, VEC, PAST>(x + base + static_cast<size_t>(c) * VEC);
             Pack<T, VEC> m;
             if (MASK) m = *reinterpret_cast<const Pack<T, VEC>*>(mask + static_cast<size_t>(mrow) * L + static_cast<size_t>(c) * VEC);
 #pragma unroll
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(kRowBlock) void softmax_kernel(const T* x, const T*
             Pack<T, VEC> out;
 #pragma unroll
             for (int e = 0; e < VEC; ++e) out.v[e] = narrow<T>(s[i][e] * inv);
-            store_pack<T, VEC, false>(y + base + static_cast<size_t>(c) * VEC, out);
+            store_pack<T, VEC, PAST>(y + base + static_cast<size_t>(c) * VEC, out);
         }
     }
 }
@@ -398,7 +398,7 @@ struct RopeMap {
 };
 
 // PAIRS rotations per thread: PAIRS * 2 consecutive elements of the last axis
-template <class T, int PAIRS>
+template <class T, int PAIRS, bool PAST>
 __global__ __launch_bounds__(kRowBlock) void rope_kernel(const T* x, const T* cs, const T* sn, T* y, RopeMap m) {
     using A = RowAcc<T>;
     const uint32_t idx = blockIdx.x * kRowBlock + threadIdx.x;
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(kRowBlock) void rope_kernel(const T* x, const T* cs
     Pack<T, 2 * PAIRS> v;
     Pack<T, PAIRS> c, s;
     if constexpr (PAIRS > 1) {
-        v = load_pack<T, 2 * PAIRS, false>(x + off + col);
+        v = load_pack<T, 2 * PAIRS, PAST>(x + off + col);
         c = *reinterpret_cast<const Pack<T, PAIRS>*>(cs + table);
         s = *reinterpret_cast<const Pack<T, PAIRS>*>(sn + table);
     } else {
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(kRowBlock) void rope_kernel(const T* x, const T* cs
     }
     T* dst = y + static_cast<size_t>(row) * m.d + col;
     if constexpr (PAIRS > 1) {
-        store_pack<T, 2 * PAIRS, false>(dst, out);
+        store_pack<T, 2 * PAIRS, PAST>(dst, out);
     } else {
         dst[0] = out.v[0];
         dst[1] = out.v[1];
@@ -473,10 +473,19 @@ inline bool row_shape(uint32_t chunks, uint32_t rows, int& group, int& nch) {
     return true;
 }
 
+// Operand and result go through the caches up to 128 MB each, which the memory-side cache of 256 MB holds together, and past them beyond.  us past / through
+// the caches, the operator again and again, and rms_norm with softmax behind it: bf16 rows of 4096, 64 MB 25.3 / 24.7, 53.4 / 49.5; 128 MB 45.2 / 43.5, 94.2 / 92.9; 160 MB 55.5 / 57.4,
+// 116 / 123; 256 MB 85.6 / 94.3, 176 / 190; 1 GB 337 / 357; fp32 rows of 512, 128 MB 43.3 / 42.4, 90.0 / 89.1; 256 MB 84.2 / 94.0, 170 / 188; 1 GB 339 / 364.  (16-bit rows of 512 are the
+// exception, 512 MB 177 / 173, and rope over 1 GB, 503 / 459.)
+template <class T>
+inline bool row_operands_past_caches(uint64_t elements) { return elements * sizeof(T) > (128ull << 20); }
+
 template <class T, int G, int NCH>
 int launch_rms(const T* x, const T* g, T* y, uint32_t rows, uint32_t L, double eps, hipStream_t stream) {
     const uint32_t per_block = kRowBlock / G;
-    hipLaunchKernelGGL((rms_norm_kernel<T, G, NCH>), dim3((rows + per_block - 1) / per_block), dim3(kRowBlock), 0, stream, x, g, y, rows, L, eps);
+    const dim3 grid((rows + per_block - 1) / per_block);
+    if (row_operands_past_caches<T>(static_cast<uint64_t>(rows) * L)) hipLaunchKernelGGL((rms_norm_kernel<T, G, NCH, true>), grid, dim3(kRowBlock), 0, stream, x, g, y, rows, L, eps);
+    else hipLaunchKernelGGL((rms_norm_kernel<T, G, NCH, false>), grid, dim3(kRowBlock), 0, stream, x, g, y, rows, L, eps);
     return launch_status("rms_norm_kernel");
 }
 
@@ -518,8 +527,12 @@ template <class T, int G, int NCH>
 int launch_softmax(const T* x, const T* mask, T* y, uint32_t rows, uint32_t L, uint32_t q, float scale, hipStream_t stream) {
     const uint32_t per_block = kRowBlock / G;
     const dim3 grid((rows + per_block - 1) / per_block);
-    if (mask) hipLaunchKernelGGL((softmax_kernel<T, G, NCH, true>), grid, dim3(kRowBlock), 0, stream, x, mask, y, rows, L, FastDiv(q), scale);
-    else hipLaunchKernelGGL((softmax_kernel<T, G, NCH, false>), grid, dim3(kRowBlock), 0, stream, x, mask, y, rows, L, FastDiv(1), scale);
+    auto launch = [&](auto with_mask, auto without) {
+        if (mask) hipLaunchKernelGGL(with_mask, grid, dim3(kRowBlock), 0, stream, x, mask, y, rows, L, FastDiv(q), scale);
+        else hipLaunchKernelGGL(without, grid, dim3(kRowBlock), 0, stream, x, mask, y, rows, L, FastDiv(1), scale);
+    };
+    if (row_operands_past_caches<T>(static_cast<uint64_t>(rows) * L)) launch(softmax_kernel<T, G, NCH, true, true>, softmax_kernel<T, G, NCH, false, true>);
+    else launch(softmax_kernel<T, G, NCH, true, false>, softmax_kernel<T, G, NCH, false, false>);
     return launch_status("softmax_kernel");
 }
 
@@ -638,14 +651,16 @@ int run_rope(const tannic_tensor_t* x, const tannic_tensor_t* cs, const tannic_t
             m.row_items = m.d / VEC;
             m.item_div = FastDiv(m.row_items);
             m.total = rows * m.row_items;
-            hipLaunchKernelGGL((rope_kernel<T, VEC / 2>), dim3((m.total + kRowBlock - 1) / kRowBlock), dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
+            const dim3 grid((m.total + kRowBlock - 1) / kRowBlock);
+            if (row_operands_past_caches<T>(count)) hipLaunchKernelGGL((rope_kernel<T, VEC / 2, true>), grid, dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
+            else hipLaunchKernelGGL((rope_kernel<T, VEC / 2, false>), grid, dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
             return launch_status("rope_kernel");
         }
     }
     m.row_items = m.d / 2;
     m.item_div = FastDiv(m.row_items);
     m.total = rows * m.row_items;
-    hipLaunchKernelGGL((rope_kernel<T, 1>), dim3((m.total + kRowBlock - 1) / kRowBlock), dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
+    hipLaunchKernelGGL((rope_kernel<T, 1, false>), dim3((m.total + kRowBlock - 1) / kRowBlock), dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
     return launch_status("rope_kernel");
 }
 

@@ -386,3 +386,23 @@ def test_rope_rejects_odd_width(device):
     t = ta.tensor(np.zeros((3, 2)), ta.float32, device)
     with pytest.raises(ops.TannicError):
         ops.rope(x, t, t)
+
+
+@pytest.mark.parametrize("name,length,repeats", [("bfloat16", 4096, 16), ("bfloat16", 4096, 17), ("float32", 512, 64), ("float32", 512, 65), ("float16", 2048, 33)],
+                         ids=lambda v: str(v))
+def test_large_row_operands(device, name, length, repeats):
+    """128 MB go through the caches, more past them: the same 1024 rows over and over give what the 1024 give, bit for bit."""
+    dtype = getattr(ta, name)
+    few = support.normal(51, 1, (1024, length)).astype(np.float32)
+    gain = support.uniform(51, 2, (length,), 0.5, 1.5).astype(np.float32)
+    angles = support.uniform(51, 3, (1024 * repeats, 64), -3, 3)
+    many = np.ascontiguousarray(np.broadcast_to(few, (repeats, 1024, length)))
+    df, dm, dg = (ta.tensor(v, dtype, device) for v in (few, many, gain))
+    for op in (lambda x: ops.rms_norm(x, dg, 1e-5), lambda x: ops.softmax(x, None, 0.5)):
+        want = op(df).raw()
+        np.testing.assert_array_equal(op(dm).raw().reshape(repeats, -1), np.broadcast_to(want, (repeats, want.size)))
+    heads = length // 128
+    cos, sin = (ta.tensor(f(angles[:1024]), dtype, device) for f in (np.cos, np.sin))
+    want = ops.rope(df.view(1024, heads, 128).transpose(0, 1), cos, sin).raw()
+    got = ops.rope(dm.view(repeats, 1024, heads, 128).transpose(1, 2), cos, sin).raw()
+    np.testing.assert_array_equal(got.reshape(repeats, -1), np.broadcast_to(want, (repeats, want.size)))
