@@ -104,7 +104,7 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
             plan[0] = 6;
             return true;
         };
-        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_few_plan(p, x->dtype, plan) &&
+        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_few_plan(p, x->dtype, x->address, w->address, plan) &&
             !conv2d_batch3_plan(p, x->dtype, x->address, w->address, plan) &&
             !staged_plan() && !conv2d_k1_takes(p, x->dtype, x->address, w->address, y->address))
             conv2d_pointwise_plan(p, x->dtype, x->address, w->address, plan);

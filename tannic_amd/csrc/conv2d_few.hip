@@ -250,8 +250,9 @@ int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, co
     return choose_few(p, dtype, x, w, bias, y, stream, nullptr);
 }
 
-bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValues]) {
-    return choose_few(p, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, out) == TANNIC_SUCCESS;
+// (the addresses are asked for their alignment: the staged kernels do not take every one)
+bool conv2d_few_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]) {
+    return choose_few(p, dtype, x, w, nullptr, nullptr, nullptr, out) == TANNIC_SUCCESS;
 }
 
 }  // namespace th

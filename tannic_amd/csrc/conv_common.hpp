@@ -26,7 +26,7 @@ bool conv2d_split_plan(const ConvProblem& p, int dtype, const void* x, const voi
 bool conv2d_pointwise_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_batch3_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_f32_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
-bool conv2d_few_plan(const ConvProblem& p, int dtype, uint32_t out[kConvPlanValues]);
+bool conv2d_few_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 
 // Each returns TANNIC_UNSUPPORTED_DTYPE when the problem does not meet its
 // conditions, so that the caller can try the next, more general kernel.

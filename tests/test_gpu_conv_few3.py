@@ -97,7 +97,7 @@ def test_edges(name, device):
 
 @pytest.mark.gpu
 def test_what_lies_beside_a_view(device):
-    """Images and channels that are slices of a tensor full of infinities, at an odd address; weights and results within larger tensors."""
+    """Images and channels that are slices of a tensor full of infinities, at an odd address; weights that are rows of a larger tensor."""
     x = np.full((3, 67, 7, 9), np.inf, np.float16)
     x[1, 1:65] = support.uniform(7, 1, (64, 7, 9), -1, 1)
     w = support.uniform(7, 2, (52, 64, 3, 3), -1, 1).astype(np.float16)
@@ -105,3 +105,54 @@ def test_what_lies_beside_a_view(device):
     want = ops.convolve2d(hx[1:2, 1:65], hw[3:50], None, 1, 1).numpy()
     got = ops.convolve2d(dx[1:2, 1:65], dw[3:50], None, 1, 1).numpy()
     support.assert_close(got, want, 2.0 ** -10, 64 * 9 * 2.0 ** -23, "view")
+
+
+def weights_at(start, pitch, rows=47, address=0x10000):
+    """Descriptors of a problem that is the kernel's (13 x 17 pixels under 64 channels), its weights ``start`` elements behind a multiple of 16 bytes, ``pitch`` from row to row."""
+    x, w, y = (descriptor("float16", s) for s in ((2, 64, 13, 17), (rows, 64, 3, 3), (2, rows, 13, 17)))
+    w.address = address + 2 * start
+    w.strides.sizes[0] = pitch
+    return x, w, y
+
+
+def runs_on_few3(x, w, y):
+    out = (C.c_uint32 * 20)()
+    assert ta.library().conv2d_plan(x, w, y, abi.SIZE2(1, 1), abi.SIZE2(1, 1), out) == abi.SUCCESS
+    return out[0] in (2, 6) and out[7] > 0
+
+
+# elements from a multiple of 16 bytes to the weights, from row to row -> loaded into LDS as they lie (at multiples of four bytes)
+STARTS = {(0, 576): True, (2, 612): True, (4, 578): True, (6, 584): True, (1, 612): False, (2, 613): False}
+
+
+@pytest.mark.parametrize("start,pitch", list(STARTS))
+def test_plan_of_weights_as_they_lie(start, pitch):
+    assert runs_on_few3(*map(C.byref, weights_at(start, pitch))) == STARTS[start, pitch]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("start,pitch", list(STARTS))
+def test_weights_as_they_lie(start, pitch, device):
+    """Rows of weights between infinities, and a result within a larger tensor whose other elements stay what they were."""
+    w = np.full(start + 47 * pitch + 8, np.inf, np.float16)
+    rows = np.lib.stride_tricks.as_strided(w[start:], (47, 576), (2 * pitch, 2))
+    rows[...] = support.uniform(8, 1, (47, 576), -1, 1)
+    x = support.uniform(8, 2, (2, 64, 13, 17), -1, 1).astype(np.float16)
+    dx, dw = ta.tensor(x, ta.float16, device), ta.tensor(w, ta.float16, device)._view((47, 64, 3, 3), (pitch, 9, 3, 1), 2 * start)
+    room = ta.tensor(np.full((3, 50, 14, 19), 7.0, np.float16), ta.float16, device)
+    y = room[1:, 2:49, 1:, 1:18]
+    assert runs_on_few3(dx.reference(), dw.reference(), y.reference()) == STARTS[start, pitch]
+    ops._call("conv2d", device, (dx, dw), y, (abi.SIZE2(1, 1), abi.SIZE2(1, 1)))
+    got = room.numpy()
+    padded = np.pad(x.astype(np.float32), ((0, 0), (0, 0), (1, 1), (1, 1)))
+    want = convolve64(padded, rows.reshape(47, 64, 3, 3).astype(np.float32), 1, 0)
+    support.assert_close(got[1:, 2:49, 1:, 1:18], want, 2.0 ** -10, 64 * 9 * 2.0 ** -23, f"{start} {pitch}")
+    beside = np.ones(got.shape, bool)
+    beside[1:, 2:49, 1:, 1:18] = False
+    assert (got[beside] == 7.0).all()
+
+
+@pytest.mark.gpu
+def test_the_view_above_is_the_kernels(device):
+    x, w = ta.tensor(np.zeros((3, 67, 7, 9)), ta.float16, device)[1:2, 1:65], ta.tensor(np.zeros((52, 64, 3, 3)), ta.float16, device)[3:50]
+    assert runs_on_few3(x.reference(), w.reference(), ta.Tensor(ta.float16, (1, 47, 7, 9)).initialize(device).reference())
