@@ -18,6 +18,8 @@
 // VEC = 1 and arbitrary row strides.
 #pragma once
 
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace th {
@@ -128,15 +130,36 @@ template <> struct RawBits<1> { using type = unsigned char; };
 // one result of 8 MB that nothing reads afterwards 3.4 / 4.0.  Bound by HBM: 6.5 TB/s at 512 MB, 6.9 at 256.
 constexpr uint64_t kStreamedSource = 96ull << 20, kKeptResult = 208ull << 20;
 
-// Source o as the plan walks it: its bit if it is loaded past the caches.  Counted is what the source itself has: a row or a plane that every outer index
+// What source o has, as the plan walks it.  That counts, not the index space: a row or a plane that every outer index
 // reads again stays in the caches however large the tensor beside it is (fp16 [64, 4096, 1024] + [1024], us past the caches / through them 183 / 171, + [1, 4096, 1024] 217 / 178;
 // 1 GB of int32 + a plane 435 / 362).
 template <class S>
-inline uint32_t streamed_source(const Plan& p, int o) {
+inline uint64_t source_bytes(const Plan& p, int o) {
     uint64_t bytes = sizeof(S);
     for (int d = 0; d < p.rank; ++d)
         if (p.stride[o][d] != 0) bytes *= p.extent[d];
-    return bytes >= kStreamedSource ? 1u << o : 0u;
+    return bytes;
+}
+
+// Two sources of which neither repeats anything go past the caches together also where both have 6 to 40 MB.  The shortcut additions of a network are of this
+// kind: what they read is hardly read again, and it pushed out what their convolutions left.  us through the caches / past them: 53 convolutions and 16 additions
+// recorded, fp16, 16 images (25 MB and less) 812 / 765, 24 images 1031 / 984, fp32, 6 images 1108 / 1090, 8 images 1240 / 1196, 12 images 1664 / 1629; an expression of eight
+// operators over fp16 tensors of 12 MB 49.2 / 49.1, 16 MB 60.0 / 58.7, 24 MB 82.1 / 82.6, 32 MB 102.4 / 103.0, but 48 MB 142.3 / 144.9 and 64 MB 184.2 / 186.6; smaller
+// ones are better off through the caches (one image, 1.6 MB and less, 306 / 312, four images 461 / 469).
+constexpr uint64_t kStreamedPair = 6ull << 20, kStreamedPairEnd = 40ull << 20;
+
+template <class F>
+inline uint32_t streamed_sources(const Plan& p) {
+    const uint64_t first = source_bytes<typename F::S0>(p, 0);
+    uint32_t streamed = first >= kStreamedSource ? 1 : 0;
+    if (F::sources == 2) {
+        const uint64_t second = source_bytes<typename F::S1>(p, 1);
+        if (second >= kStreamedSource) streamed |= 2;
+        bool repeats = false;
+        for (int d = 0; d < p.rank; ++d) repeats = repeats || p.stride[0][d] == 0 || p.stride[1][d] == 0;
+        if (!repeats && std::min(first, second) >= kStreamedPair && std::max(first, second) < kStreamedPairEnd) streamed = 3;
+    }
+    return streamed;
 }
 
 // The first of `blocks` blocks of `bytes` bytes of results each whose results are kept
@@ -454,7 +477,7 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
                 fp.p = p;
                 const uint32_t vectors = static_cast<uint32_t>((fp.elements + VEC - 1) / VEC), grid = (vectors + kBlock - 1) / kBlock;
                 fp.p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
-                fp.p.streamed = streamed_source<S0>(p, 0) | (F::sources == 2 ? streamed_source<S1>(p, 1) : 0);
+                fp.p.streamed = streamed_sources<F>(p);
                 hipLaunchKernelGGL((elementwise_flat_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, fp, vectors);
                 return launch_status("elementwise_flat_kernel");
             }
@@ -473,7 +496,7 @@ int launch_elementwise(F f, Plan p, hipStream_t stream) {
     if constexpr (VEC > 1) {
         if (vec) {
             p.kept_from = first_kept(grid, sizeof(D) * VEC * kBlock);
-            p.streamed = streamed_source<S0>(p, 0) | (F::sources == 2 ? streamed_source<S1>(p, 1) : 0);
+            p.streamed = streamed_sources<F>(p);
             if (p.rank == 1 && p.stride[0][0] == 1 && (F::sources == 1 || p.stride[1][0] == 1)) {      // (vec: the result's is 1)
                 hipLaunchKernelGGL((elementwise_dense_kernel<F, VEC>), dim3(grid), dim3(kBlock), 0, stream, f, p.total_vectors, p.kept_from, p.streamed);
                 return launch_status("elementwise_dense_kernel");

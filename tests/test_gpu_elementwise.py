@@ -328,3 +328,17 @@ def test_planes_and_rows_beside_large_tensors(device, rows):
     np.testing.assert_array_equal(ops.sub(dp, dx).numpy(), plane - x)
     np.testing.assert_array_equal(ops.sub(dr, dx).numpy(), row - x)
     np.testing.assert_array_equal(ops.add(dp, dr).numpy(), plane + row)
+
+
+@pytest.mark.parametrize("kilobytes", [6 * 1024 - 1, 6 * 1024, 40 * 1024 - 1, 40 * 1024], ids=lambda k: f"{k}KB")
+def test_pairs_past_the_caches(device, kilobytes):
+    """Two sources of 6 to 40 MB that repeat nothing go past the caches: contiguous ones, columns of larger tensors, rows that no vector divides.  Whole numbers: bit for bit."""
+    n = kilobytes << 8
+    x = np.arange(n, dtype=np.int32)
+    y = x[::-1] * 3
+    dx, dy = ta.tensor(x, ta.int32, device), ta.tensor(y, ta.int32, device)
+    np.testing.assert_array_equal(ops.sub(dx, dy).numpy(), x - y)
+    wide = ta.tensor(np.arange(2 * n, dtype=np.int32).reshape(-1, 512), ta.int32, device)
+    first, second = (np.arange(2 * n, dtype=np.int32).reshape(-1, 512)[:, part] for part in (slice(0, 256), slice(256, 512)))
+    np.testing.assert_array_equal(ops.mul(wide[:, 0:256], wide[:, 256:512]).numpy(), first * second)
+    np.testing.assert_array_equal(ops.add(dx[0:n - 1], dy[0:n - 1]).numpy(), x[:-1] + y[:-1])
