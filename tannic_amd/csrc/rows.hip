@@ -475,16 +475,27 @@ inline bool row_shape(uint32_t chunks, uint32_t rows, int& group, int& nch) {
 
 // Operand and result go through the caches up to 128 MB each, which the memory-side cache of 256 MB holds together, and past them beyond.  us past / through
 // the caches, the operator again and again, and rms_norm with softmax behind it: bf16 rows of 4096, 64 MB 25.3 / 24.7, 53.4 / 49.5; 128 MB 45.2 / 43.5, 94.2 / 92.9; 160 MB 55.5 / 57.4,
-// 116 / 123; 256 MB 85.6 / 94.3, 176 / 190; 1 GB 337 / 357; fp32 rows of 512, 128 MB 43.3 / 42.4, 90.0 / 89.1; 256 MB 84.2 / 94.0, 170 / 188; 1 GB 339 / 364.  (16-bit rows of 512 are the
-// exception, 512 MB 177 / 173, and rope over 1 GB, 503 / 459.)
+// 116 / 123; 256 MB 85.6 / 94.3, 176 / 190; 1 GB 337 / 357; fp32 rows of 512, 128 MB 43.3 / 42.4, 90.0 / 89.1; 256 MB 84.2 / 94.0, 170 / 188; 1 GB 339 / 364.
+// bf16 rows of one piece for each of 64 lanes are the exception (rms_norm 160 MB 61.1 / 60.3, 512 MB 188 / 180, 1 GB 374 / 351, softmax 57.8 / 55.8, 176 / 173, 350 / 339;
+// fp16 171 / 172 and 165 / 175 over 512 MB).  pieces: of 16 bytes, in a row.
 template <class T>
-inline bool row_operands_past_caches(uint64_t elements) { return elements * sizeof(T) > (128ull << 20); }
+inline bool row_operands_past_caches(uint64_t elements, uint32_t pieces) {
+    return elements * sizeof(T) > (128ull << 20) && !(std::is_same_v<T, bf16> && pieces == 64);
+}
+
+// rope likewise, while a die's share of the two tables, which every head reads again, stays in its L2 of 4 MB: us past / through the caches, bf16, heads of 128, 32 of them,
+// 512 MB (tables of 16 MB) 214 / 232, 768 MB (24 MB) 319 / 349, 1 GB (32 MB) 507 / 458, fp32 512 MB (16 MB) 179 / 228, 1 GB (32 MB) 478 / 452; where both tables are one, of
+// 16 MB, 1 GB 422 / 436, of 32 MB, 2 GB 942 / 864.
+template <class T>
+inline bool rope_past_caches(uint64_t elements, uint64_t table_elements) {
+    return elements * sizeof(T) > (128ull << 20) && table_elements * sizeof(T) < (32ull << 20);
+}
 
 template <class T, int G, int NCH>
 int launch_rms(const T* x, const T* g, T* y, uint32_t rows, uint32_t L, double eps, hipStream_t stream) {
     const uint32_t per_block = kRowBlock / G;
     const dim3 grid((rows + per_block - 1) / per_block);
-    if (row_operands_past_caches<T>(static_cast<uint64_t>(rows) * L)) hipLaunchKernelGGL((rms_norm_kernel<T, G, NCH, true>), grid, dim3(kRowBlock), 0, stream, x, g, y, rows, L, eps);
+    if (row_operands_past_caches<T>(static_cast<uint64_t>(rows) * L, L / (16 / sizeof(T)))) hipLaunchKernelGGL((rms_norm_kernel<T, G, NCH, true>), grid, dim3(kRowBlock), 0, stream, x, g, y, rows, L, eps);
     else hipLaunchKernelGGL((rms_norm_kernel<T, G, NCH, false>), grid, dim3(kRowBlock), 0, stream, x, g, y, rows, L, eps);
     return launch_status("rms_norm_kernel");
 }
@@ -531,7 +542,7 @@ int launch_softmax(const T* x, const T* mask, T* y, uint32_t rows, uint32_t L, u
         if (mask) hipLaunchKernelGGL(with_mask, grid, dim3(kRowBlock), 0, stream, x, mask, y, rows, L, FastDiv(q), scale);
         else hipLaunchKernelGGL(without, grid, dim3(kRowBlock), 0, stream, x, mask, y, rows, L, FastDiv(1), scale);
     };
-    if (row_operands_past_caches<T>(static_cast<uint64_t>(rows) * L)) launch(softmax_kernel<T, G, NCH, true, true>, softmax_kernel<T, G, NCH, false, true>);
+    if (row_operands_past_caches<T>(static_cast<uint64_t>(rows) * L, L / (16 / sizeof(T)))) launch(softmax_kernel<T, G, NCH, true, true>, softmax_kernel<T, G, NCH, false, true>);
     else launch(softmax_kernel<T, G, NCH, true, false>, softmax_kernel<T, G, NCH, false, false>);
     return launch_status("softmax_kernel");
 }
@@ -652,7 +663,7 @@ int run_rope(const tannic_tensor_t* x, const tannic_tensor_t* cs, const tannic_t
             m.item_div = FastDiv(m.row_items);
             m.total = rows * m.row_items;
             const dim3 grid((m.total + kRowBlock - 1) / kRowBlock);
-            if (row_operands_past_caches<T>(count)) hipLaunchKernelGGL((rope_kernel<T, VEC / 2, true>), grid, dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
+            if (rope_past_caches<T>(count, m.outer > 0 ? static_cast<uint64_t>(m.extent[m.outer - 1]) * m.d : m.d)) hipLaunchKernelGGL((rope_kernel<T, VEC / 2, true>), grid, dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
             else hipLaunchKernelGGL((rope_kernel<T, VEC / 2, false>), grid, dim3(kRowBlock), 0, stream, px, pc, ps, py, m);
             return launch_status("rope_kernel");
         }

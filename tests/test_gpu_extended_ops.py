@@ -406,3 +406,27 @@ def test_large_row_operands(device, name, length, repeats):
     want = ops.rope(df.view(1024, heads, 128).transpose(0, 1), cos, sin).raw()
     got = ops.rope(dm.view(repeats, 1024, heads, 128).transpose(1, 2), cos, sin).raw()
     np.testing.assert_array_equal(got.reshape(repeats, -1), np.broadcast_to(want, (repeats, want.size)))
+
+
+@pytest.mark.parametrize("positions", [65528, 65536], ids=lambda n: f"{n}positions")
+def test_rope_beside_large_tables(device, positions):
+    """Tables just below 32 MB and of 32 MB: the operand goes past the caches and through them; every head gives what it gives alone, bit for bit."""
+    x = support.normal(52, 1, (positions, 128)).astype(np.float32)
+    angles = support.uniform(52, 2, (positions, 64), -3, 3)
+    cos, sin = (ta.tensor(f(angles), ta.float32, device) for f in (np.cos, np.sin))
+    one = ta.tensor(x, ta.float32, device).view(1, positions, 128)
+    want = ops.rope(one, cos, sin).numpy()
+    got = ops.rope(ops.repeat(one, 5, 0), cos, sin).numpy()
+    for head in range(5):
+        np.testing.assert_array_equal(got[head], want[0])
+
+
+@pytest.mark.parametrize("rows", [131072, 131074, 140000], ids=lambda n: f"{n}rows")
+def test_large_rows_of_one_piece_a_lane(device, rows):
+    """bf16 rows of 512 at and beyond 128 MB: the same 2 rows over and over give what they give, bit for bit."""
+    few = support.normal(53, 1, (2, 512)).astype(np.float32)
+    dx = ta.tensor(np.broadcast_to(few, (rows // 2, 2, 512)), ta.bfloat16, device)
+    gain = ta.tensor(support.uniform(53, 2, (512,), 0.5, 1.5), ta.bfloat16, device)
+    for op in (lambda t: ops.rms_norm(t, gain, 1e-5), lambda t: ops.softmax(t, None, 0.5)):
+        want = op(ta.tensor(few, ta.bfloat16, device)).raw()
+        np.testing.assert_array_equal(op(dx).raw().reshape(rows // 2, -1), np.broadcast_to(want, (rows // 2, want.size)))
