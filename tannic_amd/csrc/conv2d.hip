@@ -96,16 +96,17 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     p.bs = bias ? bias->strides.sizes[0] : 0;
     if (plan) {
         for (int i = 0; i < kConvPlanValues; ++i) plan[i] = 0;
+        bool few3_asked = false;
         // (the staged kernels over few output pixels, where they come after the one over the flattened batch)
         auto staged_plan = [&] {
             if (conv2d_few1(p, x->dtype, false, x->address, w->address, nullptr, nullptr, nullptr, plan) != TANNIC_SUCCESS &&
-                conv2d_few3(p, x->dtype, x->address, w->address, nullptr, nullptr, nullptr, plan) != TANNIC_SUCCESS)
+                (few3_asked || conv2d_few3(p, x->dtype, x->address, w->address, nullptr, nullptr, nullptr, plan) != TANNIC_SUCCESS))
                 return false;
             plan[0] = 6;
             return true;
         };
-        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_few_plan(p, x->dtype, x->address, w->address, plan) &&
-            !conv2d_batch3_plan(p, x->dtype, x->address, w->address, plan) &&
+        if (!conv2d_split_plan(p, x->dtype, x->address, w->address, plan) && !conv2d_f32_plan(p, x->dtype, x->address, w->address, plan) &&
+            !conv2d_few_plan(p, x->dtype, x->address, w->address, plan, few3_asked) && !conv2d_batch3_plan(p, x->dtype, x->address, w->address, plan) &&
             !staged_plan() && !conv2d_k1_takes(p, x->dtype, x->address, w->address, y->address))
             conv2d_pointwise_plan(p, x->dtype, x->address, w->address, plan);
         return TANNIC_SUCCESS;
@@ -122,13 +123,15 @@ static int conv2d_entry(const tannic_tensor_t* x, const tannic_tensor_t* w, cons
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     status = conv2d_f32(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
-    status = conv2d_few(p, x->dtype, x->address, w->address, pb, y->address, s);
+    bool few3_asked = false;
+    status = conv2d_few(p, x->dtype, x->address, w->address, pb, y->address, s, few3_asked);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     // a batch of small maps under many channels, 16-bit 3x3 (what it leaves to the kernels below: plan_batch3)
     status = conv2d_batch3(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     // (what is left of the few output pixels beyond conv2d_few's line)
-    status = pointwise ? conv2d_few1(p, x->dtype, false, x->address, w->address, pb, y->address, s) : conv2d_few3(p, x->dtype, x->address, w->address, pb, y->address, s);
+    if (pointwise) status = conv2d_few1(p, x->dtype, false, x->address, w->address, pb, y->address, s);
+    else if (!few3_asked) status = conv2d_few3(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (status != TANNIC_UNSUPPORTED_DTYPE) return status;
     if (pointwise) status = conv2d_k1(p, x->dtype, x->address, w->address, pb, y->address, s);
     if (pointwise && status == TANNIC_UNSUPPORTED_DTYPE) status = conv2d_pointwise(p, x->dtype, x->address, w->address, pb, y->address, s);

@@ -195,7 +195,7 @@ static int few_shape(const ConvProblem& p, const FewPlan& q, uint64_t tiles, con
 }
 
 template <class T, int KS>
-static int run_few(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan) {
+static int run_few(const ConvProblem& p, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan, bool& few3_asked) {
     constexpr int64_t TAPS = KS * KS;
     const uint64_t pixels = static_cast<uint64_t>(p.N) * p.HO * p.WO;
     if (pixels == 0 || p.O == 0 || p.C == 0 || p.C % 32 != 0) return TANNIC_UNSUPPORTED_DTYPE;
@@ -216,7 +216,8 @@ static int run_few(const ConvProblem& p, const void* x, const void* w, const voi
     const bool work = few_work(p, pixels);
     if constexpr (KS == 3) {
         // (from 256 output channels on also beyond the line: few3's own rule then says where it ends)
-        const int rc = work || p.O >= 256 ? conv2d_few3(p, dtype_code<T>(), x, w, bias, y, stream, plan) : TANNIC_UNSUPPORTED_DTYPE;
+        few3_asked = work || p.O >= 256;
+        const int rc = few3_asked ? conv2d_few3(p, dtype_code<T>(), x, w, bias, y, stream, plan) : TANNIC_UNSUPPORTED_DTYPE;
         if (rc != TANNIC_UNSUPPORTED_DTYPE) return rc;
     }
     if constexpr (KS == 1) {
@@ -237,22 +238,23 @@ static int run_few(const ConvProblem& p, const void* x, const void* w, const voi
     return few_shape<T, KS, 2>(p, q, tiles, x, w, bias, y, stream, plan);
 }
 
-static int choose_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan) {
+static int choose_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan, bool& few3_asked) {
+    few3_asked = false;
     if (p.KH != p.KW) return TANNIC_UNSUPPORTED_DTYPE;
-    if (dtype == TANNIC_FLOAT16 && p.KH == 1) return run_few<f16, 1>(p, x, w, bias, y, stream, plan);
-    if (dtype == TANNIC_FLOAT16 && p.KH == 3) return run_few<f16, 3>(p, x, w, bias, y, stream, plan);
-    if (dtype == TANNIC_BFLOAT16 && p.KH == 1) return run_few<bf16, 1>(p, x, w, bias, y, stream, plan);
-    if (dtype == TANNIC_BFLOAT16 && p.KH == 3) return run_few<bf16, 3>(p, x, w, bias, y, stream, plan);
+    if (dtype == TANNIC_FLOAT16 && p.KH == 1) return run_few<f16, 1>(p, x, w, bias, y, stream, plan, few3_asked);
+    if (dtype == TANNIC_FLOAT16 && p.KH == 3) return run_few<f16, 3>(p, x, w, bias, y, stream, plan, few3_asked);
+    if (dtype == TANNIC_BFLOAT16 && p.KH == 1) return run_few<bf16, 1>(p, x, w, bias, y, stream, plan, few3_asked);
+    if (dtype == TANNIC_BFLOAT16 && p.KH == 3) return run_few<bf16, 3>(p, x, w, bias, y, stream, plan, few3_asked);
     return TANNIC_UNSUPPORTED_DTYPE;
 }
 
-int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream) {
-    return choose_few(p, dtype, x, w, bias, y, stream, nullptr);
+int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, bool& few3_asked) {
+    return choose_few(p, dtype, x, w, bias, y, stream, nullptr, few3_asked);
 }
 
 // (the addresses are asked for their alignment: the staged kernels do not take every one)
-bool conv2d_few_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]) {
-    return choose_few(p, dtype, x, w, nullptr, nullptr, nullptr, out) == TANNIC_SUCCESS;
+bool conv2d_few_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues], bool& few3_asked) {
+    return choose_few(p, dtype, x, w, nullptr, nullptr, nullptr, out, few3_asked) == TANNIC_SUCCESS;
 }
 
 }  // namespace th

@@ -26,12 +26,12 @@ bool conv2d_split_plan(const ConvProblem& p, int dtype, const void* x, const voi
 bool conv2d_pointwise_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_batch3_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
 bool conv2d_f32_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
-bool conv2d_few_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues]);
+bool conv2d_few_plan(const ConvProblem& p, int dtype, const void* x, const void* w, uint32_t out[kConvPlanValues], bool& few3_asked);
 
 // Each returns TANNIC_UNSUPPORTED_DTYPE when the problem does not meet its
 // conditions, so that the caller can try the next, more general kernel.
-// 16-bit 1x1 and 3x3 over few output pixels
-int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream);
+// 16-bit 1x1 and 3x3 over few output pixels; few3_asked: whether conv2d_few3 has been asked, and has refused if this returns UNSUPPORTED_DTYPE
+int conv2d_few(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, bool& few3_asked);
 // 16-bit 3x3 from 64 channels and 32 output channels on, few output pixels, the weights and the signal staged in LDS (what conv2d_few asks first, and
 // what conv2d_batch3 leaves); `plan`: only asked which tiles it would take
 int conv2d_few3(const ConvProblem& p, int dtype, const void* x, const void* w, const void* bias, void* y, hipStream_t stream, uint32_t* plan = nullptr);
