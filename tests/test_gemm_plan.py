@@ -7,6 +7,7 @@ import pytest
 
 import tannic_amd as ta
 import test_gpu_decode_ops
+import test_gpu_gemm_rows_dot
 import test_gpu_gemm_shares
 from tannic_amd import abi
 from test_conv_plan import descriptor
@@ -168,3 +169,35 @@ def test_matrices_of_many_products_count_together():
     x, w, y = (descriptor("bfloat16", s) for s in ((32, 8, 4, 1024), (32, 8, 1024, 128), (32, 8, 4, 128)))
     w.strides.sizes[:4] = 8 * 1024 * 128, 1024 * 128, 1, 1024
     assert plan_of(x, w, y)[:2] == (5, 1)
+
+
+@pytest.mark.parametrize("dtype", list(test_gpu_gemm_rows_dot.SHAPES))
+def test_whole_rows_on_the_gpu(dtype):
+    """The products of those tests, and the one of slices, are one row's (two of fp32) times whole rows."""
+    for m, n, k in test_gpu_gemm_rows_dot.SHAPES[dtype]:
+        x, w, y = (descriptor(dtype, s) for s in ((m, k), (k, n), (m, n)))
+        w.strides.sizes[:2] = 1, k
+        assert plan_of(x, w, y)[0] == 4, (m, n, k)
+    x, w, y = (descriptor("float16", s) for s in ((1, 2056), (2056, 34), (1, 34)))
+    x.address, w.address = x.address + 16, w.address + 16
+    x.strides.sizes[0] = 2072
+    w.strides.sizes[:2] = 1, 2072
+    assert plan_of(x, w, y)[0] == 4
+
+
+# one row (two of fp32): the shortest K, x as long as it may be for many and for few columns, and K whose last turn of eight loads would have one to three
+WHOLE_ROWS = {
+    "bfloat16": [((1, 64, 2048), True), ((1, 64, 2040), False), ((2, 64, 4096), False), ((1, 2056, 8192), True), ((1, 2056, 8200), False), ((1, 2048, 8200), True),
+                 ((1, 64, 32768), True), ((1, 64, 32776), False), ((1, 64, 4096), True), ((1, 64, 4160), False), ((1, 64, 5632), False), ((1, 64, 5696), True),
+                 ((1, 64, 4104), True), ((1, 64, 16448), True)],
+    "float32": [((1, 64, 1024), True), ((1, 64, 1016), False), ((2, 64, 1024), True), ((3, 64, 1024), False), ((2, 2056, 4096), True), ((2, 2056, 4104), False),
+                ((2, 64, 8192), True), ((2, 64, 8200), False), ((1, 64, 2080), False), ((1, 64, 2848), True)],
+}
+
+
+@pytest.mark.parametrize("dtype,problem,taken", [(d, *c) for d in WHOLE_ROWS for c in WHOLE_ROWS[d]], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_whole_rows(dtype, problem, taken):
+    m, n, k = problem
+    x, w, y = (descriptor(dtype, s) for s in ((m, k), (k, n), (m, n)))
+    w.strides.sizes[:2] = 1, k
+    assert (plan_of(x, w, y)[0] == 4) == taken

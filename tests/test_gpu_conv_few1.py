@@ -69,3 +69,12 @@ def test_what_lies_beside_a_view(device):
     w[:, 3:67] = support.uniform(7, 2, (52, 64, 1, 1), -1, 1)
     b = support.uniform(7, 3, (52,), -1, 1).astype(np.float16)
     check(x, w, b, ta.float16, device, lambda t, i: t[((slice(1, None), slice(1, 65)), (slice(2, 49), slice(3, 67)), (slice(2, 49),))[i]], "view")
+
+
+@pytest.mark.gpu
+def test_the_view_above_is_the_kernels(device):
+    x, w = ta.tensor(np.zeros((3, 67, 7, 9)), ta.float16, device)[1:, 1:65], ta.tensor(np.zeros((52, 71, 1, 1)), ta.float16, device)[2:49, 3:67]
+    out = (C.c_uint32 * 20)()
+    y = ta.Tensor(ta.float16, (2, 47, 7, 9)).initialize(device)
+    assert ta.library().conv2d_plan(x.reference(), w.reference(), y.reference(), abi.SIZE2(0, 0), abi.SIZE2(1, 1), out) == abi.SUCCESS
+    assert out[0] in (2, 6) and out[7]
