@@ -14,7 +14,8 @@
 // end, about 3.5 us.  fp16, recorded calls, weights from memory, us before / here: one image 64 -> 64 over 56 x 56 6.4 / 5.7, 128 -> 128 over 28 x 28
 // 7.5 / 5.0, 256 -> 256 over 14 x 14 9.0 / 5.1, 512 -> 512 over 7 x 7 14.7 / 7.1, with stride 2 128 at 56 9.3 / 6.6, 256 at 28 10.3 / 6.6, 512 at 14 16.9 / 6.4;
 // four images of 256 -> 256 15.2 / 7.4, of 512 -> 512 22.6 / 8.1, eight of them 19.0 / 12.8 and 21.1 / 10.0.
-// (src/cpu/conv2d.cpp:17-64; sums in fp32, in the order of conv2d_few.hip, rounded once.)
+// (src/cpu/conv2d.cpp:17-64; sums in fp32, the wavefronts' shares of the channels in a fixed order, rounded once; with another number of wavefronts than
+// conv2d_few.hip takes for the same problem the order is another.)
 #include "conv_few.hpp"
 
 namespace th {
@@ -197,7 +198,9 @@ struct Few3Shape {
 
 // The shape with `rows` and `pixel_tiles`, and the time (us) it is expected to take; negative where LDS does not hold it.  Fitted to
 // 370 timed calls (11 % off in the mean; the shape it picks 0.2 % slower than the best of them): start and end; every round of blocks waits
-// for its loads and its own products; and what a compute unit loads for 32 channels of a block, weights and pieces of the signal.
+// for its loads and its own products; and what a compute unit loads for 32 channels of a block, weights and pieces of the signal.  (The blocks at once
+// are counted by LDS and by eight wavefronts on a SIMD; registers hold two to four there, fewer blocks where a block is two wavefronts with little LDS.  The constants were fitted
+// with that count.)
 static double few3_expected(const ConvProblem& p, uint32_t rows, uint32_t pixel_tiles, Few3Shape& s) {
     const uint32_t pixels = p.HO * p.WO, units = p.C / 32, in_tile = 16 * pixel_tiles;
     s.rows = rows;

@@ -2,8 +2,8 @@
 //
 // The work is reading W once.  The kernel beside it (gemm_skinny_stream_kernel) reads 128 bytes of sixteen rows at a time, through LDS into
 // matrix fragments of which one row in sixteen is used, with one block of four wavefronts on a compute unit.  Here a wavefront owns a row of W: a load
-// instruction is a kilobyte of it, eight of them are on their way while the eight before are multiplied, eight blocks share a compute unit, and x
-// waits in LDS.  Bound by HBM, 6.5 TB/s of W where it is large (8 multiply-adds and their conversions for 16 bytes are a third of the
+// instruction is a kilobyte of it, eight of them are on their way while the eight before are multiplied, six blocks (five of two fp32 rows)
+// share a compute unit by their registers, and x waits in LDS.  Bound by HBM, 6.5 TB/s of W where it is large (8 multiply-adds and their conversions for 16 bytes are a third of the
 // time; two rows of 16-bit values are not worth it: 28672 x 4096 40.8 there, 44.0 here).  One row, W from memory, us there / here: bf16
 // 6144 x 4096 13.1 / 10.9, 28672 x 4096 40.5 / 36.0, 32000 x 2048 28.7 / 23.2, 12000 x 5000 30.6 / 22.5, 512 x 16384 12.8 / 8.8, fp32 4096 x 4096
 // 18.4 / 14.8, 14336 x 4096 51.0 / 38.3, 1024 x 1024 5.4 / 4.1, two rows 4096 x 4096 18.4 / 16.0.  (src/cpu/matmul.cpp:36-60)
