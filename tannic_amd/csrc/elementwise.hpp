@@ -141,12 +141,13 @@ inline uint64_t source_bytes(const Plan& p, int o) {
     return bytes;
 }
 
-// Two sources of which neither repeats anything go past the caches together also where both have 6 to 40 MB.  The shortcut additions of a network are of this
+// Two sources of which neither repeats anything go past the caches together also where both have 6 to 56 MB.  The shortcut additions of a network are of this
 // kind: what they read is hardly read again, and it pushed out what their convolutions left.  us through the caches / past them: 53 convolutions and 16 additions
-// recorded, fp16, 16 images (25 MB and less) 812 / 765, 24 images 1031 / 984, fp32, 6 images 1108 / 1090, 8 images 1240 / 1196, 12 images 1664 / 1629; an expression of eight
-// operators over fp16 tensors of 12 MB 49.2 / 49.1, 16 MB 60.0 / 58.7, 24 MB 82.1 / 82.6, 32 MB 102.4 / 103.0, but 48 MB 142.3 / 144.9 and 64 MB 184.2 / 186.6; smaller
-// ones are better off through the caches (one image, 1.6 MB and less, 306 / 312, four images 461 / 469).
-constexpr uint64_t kStreamedPair = 6ull << 20, kStreamedPairEnd = 40ull << 20;
+// recorded, fp16, 16 images (25 MB and less) 776 / 748, 20 images 895 / 832, 24 images 1003 / 975, 32 images (51 MB and less) 1114 / 1078 (with 25 MB and less past them 1114),
+// fp32, 6 images 1105 / 1094, 8 images 1262 / 1205, 12 images 1665 / 1642; an expression of eight operators over fp16 tensors of 12 MB 49.5 / 49.2, 16 MB 59.9 / 58.3, 24 MB
+// 81.3 / 81.4, 32 MB 104.1 / 102.9, 48 MB 142.6 / 144.4, 64 MB 184.2 / 186.6; smaller ones are better off through the caches (one image, 1.6 MB and less, 306 / 312, four
+// images 461 / 469).
+constexpr uint64_t kStreamedPair = 6ull << 20, kStreamedPairEnd = 56ull << 20;
 
 template <class F>
 inline uint32_t streamed_sources(const Plan& p) {

@@ -330,9 +330,9 @@ def test_planes_and_rows_beside_large_tensors(device, rows):
     np.testing.assert_array_equal(ops.add(dp, dr).numpy(), plane + row)
 
 
-@pytest.mark.parametrize("kilobytes", [6 * 1024 - 1, 6 * 1024, 40 * 1024 - 1, 40 * 1024], ids=lambda k: f"{k}KB")
+@pytest.mark.parametrize("kilobytes", [6 * 1024 - 1, 6 * 1024, 56 * 1024 - 1, 56 * 1024], ids=lambda k: f"{k}KB")
 def test_pairs_past_the_caches(device, kilobytes):
-    """Two sources of 6 to 40 MB that repeat nothing go past the caches: contiguous ones, columns of larger tensors, rows that no vector divides.  Whole numbers: bit for bit."""
+    """Two sources of 6 to 56 MB that repeat nothing go past the caches: contiguous ones, columns of larger tensors, rows that no vector divides.  Whole numbers: bit for bit."""
     n = kilobytes << 8
     x = np.arange(n, dtype=np.int32)
     y = x[::-1] * 3
