@@ -284,18 +284,17 @@ __global__ __launch_bounds__(64 * kStreamWaves) void gemm_skinny_stream_kernel(c
 #endif
 }
 
-// Which W goes past the caches.  us, through the caches / past them, every W from memory, and the same W again and again:
-//   up to four rows of 16 bits, from 56 MB on   14336 x 2048 (56 MB) 15.1 / 13.5, 13.8 / 12.8; 8192 x 4096 16.4 / 14.8, 15.7 / 14.4; 14336 x 4096 24.5 / 22.5,
-//                                               22.0 / 21.9; 20000 x 4096 35.1 / 32.3, 29.2 / 30.8; 28672 x 4096 46.5 / 43.3, 39.1 / 41.1; below: 6144 x 4096 14.7 / 13.2, 11.2 / 13.0
-//   more rows, int8: from 208 MB on             that much does not stay beside anything else.  16 rows of 14336 x 4096 (112 MB) 26.1 / 23.8, 22.0 / 23.4; of 12000 x 5120
-//                                               34.0 / 31.5, 24.7 / 30.0; of 28672 x 4096 (224 MB) 49.5 / 46.2, 39.9 / 44.3; a decoder layer's step of 16 sequences with
-//                                               matrices of 224, 112, 48 and 32 MB: all through the caches 173, the largest past them 158, from 56 MB on 156
+// Which W goes past the caches.  Weights of 16 bits and fewer are a model's, whose next layers push out what one of 40 MB and more leaves there: from 40 MB on.  us a step of three
+// decoder layers in turn (bf16, matrices of 224, 112, 48 and 32 MB), past the caches from 208 MB on / from 56 MB on / from 40 MB on: 4 sequences behind 2048 tokens - / 438 / 420, behind
+// 248 - / 393 / 393, 7 behind 832 464 / - / 431, 16 behind 248 450 / - / 425, behind 2048 555 / - / 549, 32 behind 248 515 / - / 485.  The price is a matrix that is used again at once with nothing in
+// between, through / past: 4 rows of 6144 x 4096 (48 MB) 11.2 / 13.0, from memory 14.7 / 13.2; 16 rows of 14336 x 4096 (112 MB) 22.0 / 23.4, from memory 26.1 / 23.8; of 12000 x 5120 24.7 / 30.0,
+// from memory 34.0 / 31.5; one such layer again and again 16 sequences behind 248 134 / 142, behind 2048 180 / 168.
 //   (8 products that share one of 4096 x 4096, 4 rows each, counted eight times and so past the caches: 27.1, through them 21.9)
-//   fp32: from 256 MB on, what cannot stay      16 rows of 4096 x 4096 18.3 / 17.2, 14.8 / 16.2; of 14336 x 4096 (224 MB) 56.5 / 55.4, 38.3 / 54.3; of 18304 x 4096
-//                                               83.7 / 79.1, 81.5 / 76.8
+//   fp32: from 256 MB on, what cannot stay, as little is gained from memory: 16 rows of 4096 x 4096 from memory 18.3 / 17.2, again and again 14.8 / 16.2; of 14336 x 4096 (224 MB)
+//   56.5 / 55.4, 38.3 / 54.3; of 18304 x 4096 83.7 / 79.1, 81.5 / 76.8
 template <class T>
 static bool stream_past_caches(const GemmProblem& p) {
-    return rows_past_caches(p, sizeof(T), sizeof(T) == 4 ? 256ull << 20 : sizeof(T) == 2 && p.M <= 4 ? 56ull << 20 : 208ull << 20);
+    return rows_past_caches(p, sizeof(T), sizeof(T) == 4 ? 256ull << 20 : 40ull << 20);
 }
 
 template <class T, int MB, int NB, bool PAST>

@@ -145,12 +145,12 @@ def test_tiles_of_long_products_on_the_gpu(m, n, k, dtype):
     assert (kernel, rows, columns, shares > 1) == (3, *TILES[m, n, k])
 
 
-# rows, columns, K (and products that share one matrix) -> the matrix is loaded past the caches.  One row from 40 MB on; two to four rows of 16 bits from 56 MB, more
-# from 208 MB; fp32 from 256 MB: what stays in the memory-side cache from call to call is not kept out of it.
+# rows, columns, K (and products that share one matrix) -> the matrix is loaded past the caches.  16 bits from 40 MB on, fp32 one row (two) from 40 MB, more from
+# 256 MB; a matrix that several products share counts once.
 PAST_CACHES = {
-    "bfloat16": [((1, 5120, 4096), 4, True), ((1, 5112, 4096), 4, False), ((2, 5120, 4096), 5, False), ((2, 14336, 2048), 5, True), ((4, 14336, 4096), 5, True),
-                 ((4, 7160, 4096), 5, False), ((5, 14336, 4096), 5, False), ((16, 14336, 4096), 5, False), ((16, 26624, 4096), 5, True), ((32, 26616, 4096), 5, False),
-                 ((2, 1, 4096, 4096), 5, False), ((8, 4, 6144, 4096), 5, False), ((8, 4, 7168, 4096), 5, True)],
+    "bfloat16": [((1, 5120, 4096), 4, True), ((1, 5112, 4096), 4, False), ((2, 5120, 4096), 5, True), ((2, 5112, 4096), 5, False), ((4, 14336, 4096), 5, True),
+                 ((5, 5120, 4096), 5, True), ((16, 14336, 4096), 5, True), ((32, 5112, 4096), 5, False), ((32, 26624, 4096), 5, True),
+                 ((2, 1, 4096, 4096), 5, False), ((8, 4, 5112, 4096), 5, False), ((8, 4, 5120, 4096), 5, True)],
     "float32": [((1, 2560, 4096), 4, True), ((1, 2552, 4096), 4, False), ((2, 4096, 4096), 4, True), ((16, 4096, 4096), 5, False), ((4, 14336, 4096), 5, False),
                 ((4, 16384, 4096), 5, True), ((8, 4, 8192, 4096), 5, False)],
 }
